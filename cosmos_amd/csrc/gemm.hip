@@ -4,7 +4,8 @@
 // to the fp32 accumulator in the epilogue).  A k-tile is 128 BYTES of K for both types, so the LDS
 // geometry, loads and swizzle are shared.
 //
-// Tiling: one workgroup computes a 256x256 tile with BK = 64.  Default: 8 waves (4x2), each owning a 64x128 sub-tile
+// Tiling: one workgroup computes a 256x256 tile with BK = 64 (launches with too few such tiles for the chip go to
+// gemm_tile.hip).  Default: 8 waves (4x2), each owning a 64x128 sub-tile
 // = 4x8 accumulators of 16x16 (128 fp32 registers per lane).  Cross-check: 4 waves (2x2) of 128x128 = 4x4
 // v_mfma_f32_32x32x16_bf16 accumulators (256 registers) on a plain two-stage pipeline.
 // Both operands are K-contiguous, so A and W fragments are plain 16-byte LDS reads.
@@ -17,7 +18,9 @@
 // on a compact block of tiles and its private L2 sees the reuse.
 #include <type_traits>
 
-#include "cdm_common.h"
+#include "gemm_common.h"
+
+using namespace cdm_gemm;
 
 namespace {
 
@@ -26,86 +29,6 @@ constexpr int kThreads = 256;
 constexpr int kTileBytes = BM * BK * 2;   // 32 KB per operand per stage
 
 typedef __attribute__((address_space(3))) void lds_void;
-
-typedef __attribute__((ext_vector_type(8))) int i32x8;
-
-constexpr int kMaxSeg = 8;
-
-// One launch covers up to kMaxSeg contiguous row segments of A / C / R, each with its own weights (the MoT
-// branches): the grid is the concatenation of the segments' tile lists, so the few tiles of a short segment (a
-// 256-token action run, a 512-token text run) fill the tail of the long segment's grid instead of paying for a
-// launch of their own that cannot fill the chip.
-struct GemmSeg {
-    int m_start, m_end;                  // token rows [m_start, m_end)
-    int tiles_m, tile_end;               // row tiles of the segment; tiles of segments 0..this one
-    const void* W; const void* W2;
-    const float* gate;
-    const float* sw; const float* sw2;   // fp8 only
-    const float* knw;                    // QKV_PACK only: the segment's K-norm weight row [head_dim] fp32, or null
-};
-
-struct GemmParams {
-    const void* A; int64_t lda;          // operand strides in BYTES
-    int64_t ldw;
-    const float* sa;                     // fp8 only: per-row scale of A, indexed by the global row
-    bf16_t* C; int64_t ldc;              // fp32 storage behind the same pointers for CDM_EPI_GATE_RESIDUAL_F32
-    int N, K;
-    const bf16_t* R; int64_t ldr;
-    const float* cos; const float* sin;
-    int rope_cols, head_dim;
-    // CDM_EPI_QKV_PACK: columns [0, d_q) are Q (written to C), [d_q, d_q + d_kv) K and the rest V; K and V leave as the
-    // attention kernel's tile images (64 keys x 128 channels per K / V head), with the largest key norm of every tile
-    char* kp; char* vp; float* kmax;
-    int d_q, d_kv, n_key_tiles;
-    float k_eps;                         // epsilon of the per-head RMSNorm of K (segments with a weight row)
-    // CDM_EPI_SWIGLU, optional: [M, amax_ld] fp32, entry (row, c) = largest |output| of the row within output columns
-    // 64 c .. 64 c + 63 (as stored): what a per-row quantiser of the output needs, without a pass of its own
-    float* row_amax; int64_t amax_ld;
-    int tiles_n, total_tiles, n_seg;
-    GemmSeg seg[kMaxSeg];
-};
-
-// what a workgroup works on
-struct Tile {
-    int m0, m_end, tn;
-    const void* W; const void* W2;
-    const float* gate; const float* sw; const float* sw2; const float* knw;
-};
-
-// XCD-aware tile assignment: workgroup ids are dealt round-robin over the 8 XCDs, so ids are remapped to give each
-// XCD a contiguous range of tiles; inside a segment, tiles are ordered in groups of 4 row tiles x all column tiles,
-// column-major inside the group, so that the 32 tiles an XCD runs at a time share 4 A slabs and 8 W slabs in its L2
-// (measured best among group heights 2, 3, 4, 6, 8, 16 once the output tiles are stored non-temporally).
-template <class T>
-__device__ __forceinline__ T* uniform_ptr(T* ptr) {      // wave-uniform value -> scalar registers
-    const uint64_t v = reinterpret_cast<uint64_t>(ptr);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return reinterpret_cast<T*>(((uint64_t)hi << 32) | lo);
-}
-
-__device__ __forceinline__ bool locate_tile(const GemmParams& p, Tile& t) {
-    const int per_xcd = (p.total_tiles + 7) >> 3;
-    int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (logical >= p.total_tiles) return false;
-    int si = 0;
-#pragma unroll
-    for (int i = 0; i < kMaxSeg - 1; ++i) si += (i < p.n_seg - 1 && logical >= p.seg[i].tile_end) ? 1 : 0;
-    const GemmSeg& sg = p.seg[si];
-    logical -= si ? p.seg[si - 1].tile_end : 0;
-    constexpr int GM = 4;
-    const int group = logical / (GM * p.tiles_n);
-    const int first_m = group * GM;
-    const int gsz = (sg.tiles_m - first_m) < GM ? (sg.tiles_m - first_m) : GM;
-    const int in_group = logical - group * GM * p.tiles_n;
-    // everything here is a function of blockIdx: pin it to scalar registers (the segment table is indexed
-    // dynamically, which the compiler would otherwise treat as a per-lane value)
-    t.m0 = __builtin_amdgcn_readfirstlane(sg.m_start + (first_m + in_group % gsz) * BM);
-    t.m_end = __builtin_amdgcn_readfirstlane(sg.m_end);
-    t.tn = __builtin_amdgcn_readfirstlane(in_group / gsz);
-    t.W = uniform_ptr(sg.W); t.W2 = uniform_ptr(sg.W2);
-    t.gate = uniform_ptr(sg.gate); t.sw = uniform_ptr(sg.sw); t.sw2 = uniform_ptr(sg.sw2); t.knw = uniform_ptr(sg.knw);
-    return true;
-}
 
 // chunk swizzle: 16-byte chunk c of tile row r lives at chunk position c ^ swz(r)
 __device__ __forceinline__ int swz(int row) { return (row ^ (row >> 3)) & 7; }
@@ -178,22 +101,12 @@ __device__ __forceinline__ void issue_loads(const char* abase, const char* wbase
 
 #endif
 
-// silu(g) = g / (1 + e^-g) with the hardware reciprocal (1 ulp) instead of an IEEE division: the result is rounded to
-// bf16 anyway, and a correctly rounded division is ten instructions per output value of a 128 x 64 result per wave
-__device__ __forceinline__ float silu_f(float g) {
-    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g));
-}
-
 // ---- epilogue shared by both pipelines.
 // The MFMAs are issued with the W fragment as the first operand, so an accumulator block holds C TRANSPOSED:
 // element v of block (mi, ni) is output row (token) lane % 32 and output column 8 (v / 4) + 4 (lane / 32) + v % 4 of
 // its 32x32 block.  A lane therefore owns ONE output row per mi and groups of FOUR consecutive columns, and every
 // global access of the epilogue (C, residual, gate, scales, rotary tables) is an 8- or 16-byte vector access.
 // N is a multiple of 8 (host-checked), so a group of four columns is either entirely inside or entirely outside.
-__device__ __forceinline__ uint2 pack4_bf16(float a, float b, float c, float d) {
-    return make_uint2(pack_bf16x2(a, b), pack_bf16x2(c, d));
-}
-
 constexpr int kStagePitch = 256 + 16;      // bytes per staged row (16-byte multiple; the pad spreads rows over banks)
 
 // wave-private staging area -> C: COLS (128 or 64) columns of ESIZE bytes (2 = bf16, 4 = fp32) of ROWS rows, whole rows
@@ -400,16 +313,18 @@ __device__ __forceinline__ void epilogue(const GemmParams& p, const Tile& t, ACC
                 if (hd128) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const float x1 = acc.get(rs, lo128, e), x2 = acc.get(rs, lo128 + HALF, e);
-                        acc.set(rs, lo128, e, x1 * cc[e] - x2 * sn[e]);
-                        acc.set(rs, lo128 + HALF, e, x2 * cc[e] + x1 * sn[e]);
+                        float x1 = acc.get(rs, lo128, e), x2 = acc.get(rs, lo128 + HALF, e);
+                        rotate_pair(x1, x2, cc[e], sn[e]);
+                        acc.set(rs, lo128, e, x1);
+                        acc.set(rs, lo128 + HALF, e, x2);
                     }
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const float x1 = acc.get(rs, lo64, e), x2 = acc.get(rs, lo64 + QUARTER, e);
-                        acc.set(rs, lo64, e, x1 * cc[e] - x2 * sn[e]);
-                        acc.set(rs, lo64 + QUARTER, e, x2 * cc[e] + x1 * sn[e]);
+                        float x1 = acc.get(rs, lo64, e), x2 = acc.get(rs, lo64 + QUARTER, e);
+                        rotate_pair(x1, x2, cc[e], sn[e]);
+                        acc.set(rs, lo64, e, x1);
+                        acc.set(rs, lo64 + QUARTER, e, x2);
                     }
                 }
             }
@@ -533,7 +448,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     __shared__ __attribute__((aligned(1024))) char sb1[kTileBytes];
 
     Tile tile;
-    if (!locate_tile(p, tile)) return;
+    if (!locate_tile<BM, 4>(p, tile)) return;
     const int tn = tile.tn;
 
     const int lane = threadIdx.x & 63;
@@ -632,14 +547,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
 // row block mi is the lane's address plus a constant.
 // ---------------------------------------------------------------------------------------------
 constexpr int kGranule = BM * 128;      // 32 KB
-__device__ __forceinline__ int swz16(int row) { return (row >> 1) & 7; }
 
 template <int EPI, bool FP8>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_ring_kernel(const GemmParams p) {
     __shared__ __attribute__((aligned(1024))) char s_ring[5 * kGranule];
 
     Tile tile;
-    if (!locate_tile(p, tile)) return;
+    if (!locate_tile<BM, 4>(p, tile)) return;
     const int tn = tile.tn;
 
     const int lane = threadIdx.x & 63;
@@ -853,27 +767,36 @@ struct HostSeg {
 // Launches the segments kMaxSeg at a time (one grid per batch).  p holds everything that is common to the segments.
 template <bool FP8>
 int32_t run(GemmParams p, const HostSeg* segs, int n_seg, int64_t N, int32_t epilogue, hipStream_t st, const char* who) {
-    const int tile_n = epilogue == CDM_EPI_SWIGLU ? BN / 2 : BN;
-    p.tiles_n = (int)((N + tile_n - 1) / tile_n);
-    // variant 0 = ring pipeline with eight waves and 16 x 16 MFMAs; 1 (cross-check build only) = two-stage pipeline, four
-    // waves, 32 x 32 MFMAs
+    // variant 0 = the rule of pick_tile; cross-check build only: 1 = two-stage pipeline, four waves, 32 x 32 MFMAs; 2 = the
+    // ring kernel for every size, 3 - 7 = one of the small tiles for every size
     const bool ring = cdm_get_variant(1) != 1;
-    (void)ring;
     int i = 0;
     while (i < n_seg) {
-        int ns = 0, total = 0;
+        int ns = 0;
         for (; i < n_seg && ns < kMaxSeg; ++i) {
             if (segs[i].len == 0) continue;
             GemmSeg& g = p.seg[ns++];
             g.m_start = (int)segs[i].start; g.m_end = (int)(segs[i].start + segs[i].len);
-            g.tiles_m = (int)((segs[i].len + BM - 1) / BM);
-            total += g.tiles_m * p.tiles_n;
-            g.tile_end = total;
             g.W = segs[i].W; g.W2 = segs[i].W2; g.gate = segs[i].gate; g.sw = segs[i].sw; g.sw2 = segs[i].sw2;
             g.knw = segs[i].knw;
         }
         if (ns == 0) break;
-        p.n_seg = ns; p.total_tiles = total;
+        p.n_seg = ns;
+        const TileShape shape = ring ? pick_tile(p, epilogue, FP8) : TileShape{BM, BN, 4, 2};
+        if (shape.tm != BM || shape.tn != BN) {
+            int32_t rc = launch_tile(p, epilogue, FP8, shape, st);
+            if (rc || (rc = cdm_check_launch(who))) return rc;
+            continue;
+        }
+        const int tile_n = epilogue == CDM_EPI_SWIGLU ? BN / 2 : BN;
+        p.tiles_n = (int)((N + tile_n - 1) / tile_n);
+        int total = 0;
+        for (int k = 0; k < ns; ++k) {
+            p.seg[k].tiles_m = (p.seg[k].m_end - p.seg[k].m_start + BM - 1) / BM;
+            total += p.seg[k].tiles_m * p.tiles_n;
+            p.seg[k].tile_end = total;
+        }
+        p.total_tiles = total;
         const int grid = ((total + 7) / 8) * 8;
 #ifdef CDM_CROSSCHECK
 #define CDM_LAUNCH(E)                                                         \

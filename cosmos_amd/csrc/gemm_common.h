@@ -1,0 +1,118 @@
+// What the GEMM kernels of this library share: the launch descriptor, the tile assignment and the small helpers of their
+// epilogues.
+#pragma once
+#include "cdm_common.h"
+
+namespace cdm_gemm {
+
+typedef __attribute__((ext_vector_type(8))) int i32x8;
+
+constexpr int kMaxSeg = 8;
+
+// One launch covers up to kMaxSeg contiguous row segments of A / C / R, each with its own weights (the MoT
+// branches): the grid is the concatenation of the segments' tile lists, so the few tiles of a short segment (a
+// 256-token action run, a 512-token text run) fill the tail of the long segment's grid instead of paying for a
+// launch of their own that cannot fill the chip.
+struct GemmSeg {
+    int m_start, m_end;                  // token rows [m_start, m_end)
+    int tiles_m, tile_end;               // row tiles of the segment; tiles of segments 0..this one
+    const void* W; const void* W2;
+    const float* gate;
+    const float* sw; const float* sw2;   // fp8 only
+    const float* knw;                    // QKV_PACK only: the segment's K-norm weight row [head_dim] fp32, or null
+};
+
+struct GemmParams {
+    const void* A; int64_t lda;          // operand strides in BYTES
+    int64_t ldw;
+    const float* sa;                     // fp8 only: per-row scale of A, indexed by the global row
+    bf16_t* C; int64_t ldc;              // fp32 storage behind the same pointers for CDM_EPI_GATE_RESIDUAL_F32
+    int N, K;
+    const bf16_t* R; int64_t ldr;
+    const float* cos; const float* sin;
+    int rope_cols, head_dim;
+    // CDM_EPI_QKV_PACK: columns [0, d_q) are Q (written to C), [d_q, d_q + d_kv) K and the rest V; K and V leave as the
+    // attention kernel's tile images (64 keys x 128 channels per K / V head), with the largest key norm of every tile
+    char* kp; char* vp; float* kmax;
+    int d_q, d_kv, n_key_tiles;
+    float k_eps;                         // epsilon of the per-head RMSNorm of K (segments with a weight row)
+    // CDM_EPI_SWIGLU, optional: [M, amax_ld] fp32, entry (row, c) = largest |output| of the row within output columns
+    // 64 c .. 64 c + 63 (as stored): what a per-row quantiser of the output needs, without a pass of its own
+    float* row_amax; int64_t amax_ld;
+    int tiles_n, total_tiles, n_seg;
+    GemmSeg seg[kMaxSeg];
+};
+
+// what a workgroup works on
+struct Tile {
+    int m0, m_end, tn;
+    const void* W; const void* W2;
+    const float* gate; const float* sw; const float* sw2; const float* knw;
+};
+
+template <class T>
+__device__ __forceinline__ T* uniform_ptr(T* ptr) {      // wave-uniform value -> scalar registers
+    const uint64_t v = reinterpret_cast<uint64_t>(ptr);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return reinterpret_cast<T*>(((uint64_t)hi << 32) | lo);
+}
+
+// XCD-aware tile assignment: workgroup ids are dealt round-robin over the 8 XCDs, so ids are remapped to give each
+// XCD a contiguous range of tiles; inside a segment, tiles of TM rows are ordered in groups of GM row tiles x all column
+// tiles, column-major inside the group, so that the 32 tiles an XCD runs at a time share GM A slabs and 32 / GM W slabs
+// in its L2 (256-row tiles: GM = 4 measured best among 2, 3, 4, 6, 8, 16 once the output tiles are stored
+// non-temporally).
+template <int TM, int GM>
+__device__ __forceinline__ bool locate_tile(const GemmParams& p, Tile& t) {
+    const int per_xcd = (p.total_tiles + 7) >> 3;
+    int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (logical >= p.total_tiles) return false;
+    int si = 0;
+#pragma unroll
+    for (int i = 0; i < kMaxSeg - 1; ++i) si += (i < p.n_seg - 1 && logical >= p.seg[i].tile_end) ? 1 : 0;
+    const GemmSeg& sg = p.seg[si];
+    logical -= si ? p.seg[si - 1].tile_end : 0;
+    const int group = logical / (GM * p.tiles_n);
+    const int first_m = group * GM;
+    const int gsz = (sg.tiles_m - first_m) < GM ? (sg.tiles_m - first_m) : GM;
+    const int in_group = logical - group * GM * p.tiles_n;
+    // everything here is a function of blockIdx: pin it to scalar registers (the segment table is indexed
+    // dynamically, which the compiler would otherwise treat as a per-lane value)
+    t.m0 = __builtin_amdgcn_readfirstlane(sg.m_start + (first_m + in_group % gsz) * TM);
+    t.m_end = __builtin_amdgcn_readfirstlane(sg.m_end);
+    t.tn = __builtin_amdgcn_readfirstlane(in_group / gsz);
+    t.W = uniform_ptr(sg.W); t.W2 = uniform_ptr(sg.W2);
+    t.gate = uniform_ptr(sg.gate); t.sw = uniform_ptr(sg.sw); t.sw2 = uniform_ptr(sg.sw2); t.knw = uniform_ptr(sg.knw);
+    return true;
+}
+
+// Chunk swizzle of a 128-byte tile row in LDS: 16-byte chunk c of row r lives at position c ^ swz16(r).  A fragment read
+// covers 16 rows x 4 chunks (lane = row % 16 + 16 x chunk), and the LDS serves 16 lanes of a 16-byte-per-lane read per
+// pass; (row / 2) % 8 puts the 16 rows of one chunk column on the 16 distinct 16-byte slots of the 256-byte bank window.
+__device__ __forceinline__ int swz16(int row) { return (row >> 1) & 7; }
+
+// silu(g) = g / (1 + e^-g) with the hardware reciprocal (1 ulp) instead of an IEEE division: the result is rounded to
+// bf16 anyway, and a correctly rounded division is ten instructions per output value of a 128 x 64 result per wave
+__device__ __forceinline__ float silu_f(float g) {
+    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g));
+}
+
+// rotate-half pair, (x1, x2) -> (x1 c - x2 s, x2 c + x1 s), with its roundings written out: kernels whose compiler-chosen
+// contractions differ would put K rows one bf16 rounding apart
+__device__ __forceinline__ void rotate_pair(float& x1, float& x2, float c, float s) {
+    const float a = x1, b = x2;
+    x1 = __builtin_fmaf(c, a, -(s * b));
+    x2 = __builtin_fmaf(s, a, c * b);
+}
+
+__device__ __forceinline__ uint2 pack4_bf16(float a, float b, float c, float d) {
+    return make_uint2(pack_bf16x2(a, b), pack_bf16x2(c, d));
+}
+
+// The kernels for launches too small for 256 x 256 tiles (gemm_tile.hip): shapes of their output tile, chosen by
+// pick_tile, and the launcher.  p holds everything but the tile counts.
+struct TileShape { int tm, tn, wm, wn; };
+TileShape pick_tile(const GemmParams& p, int epilogue, bool fp8);      // {256, 256} = the ring kernel
+int32_t launch_tile(GemmParams& p, int epilogue, bool fp8, TileShape shape, hipStream_t st);
+
+}  // namespace cdm_gemm

@@ -1,0 +1,535 @@
+// The "NT" GEMM C[M,N] = A[M,K] . W[N,K]^T for launches that 256 x 256 tiles (gemm.hip) leave the chip idle for: a text
+// run, an action run, one image, small models.  Same operands, same order of every sum (a row of C comes out bit for bit
+// the same whatever the tile), same epilogues; smaller output tiles.
+//
+// What bounds it: the feed of one CU.  With weights that no cache holds (every weight of a prompt is read exactly once) a CU
+// takes 57 - 72 bytes per ns into its LDS whatever the tile (0.40 us per k-tile at 64 x 128, 0.53 at 128 x 128), 78 with the
+// weights in the memory-side cache; a load-only loop over L2-resident rows reaches 110 - 137.  Removing the loads from the
+// 64 x 128 loop takes a third off, removing half of its LDS reads nothing.  So: all the LDS a CU has goes into ring stages
+// (over 100 KB in flight), loads go out one behind every few MFMAs, and the shape is chosen so that every CU has a tile.
+// At M = 512, K = 16384, N = 4096 (bf16, cold weights) the 64 x 128 tile takes 113 us where 32 tiles of 256 x 256 took 287;
+// M = 512, N = 12288, K = 4096 (QKV with images): 64 us against 85; M = 64, N = 4096, K = 4096: 14 us against 84.
+//
+// Layout: eight waves (four for the 32 x 32 tile) in a WM x WN grid, v_mfma_f32_16x16x32_bf16 / 16x16x128_f8f6f4, W
+// fragment first, so that a lane's accumulator quad is four consecutive columns of one output row.  The epilogue
+// first spreads the accumulators over the drained ring as fp32 rows; every thread then works on eight consecutive
+// columns of a row (16-byte accesses to C, residual, tables and images), whatever the wave grid was.
+#include <type_traits>
+
+#include "gemm_common.h"
+
+using namespace cdm_gemm;
+
+namespace {
+
+constexpr int kLds = 160 * 1024;
+
+template <int TM, int TN, int WM, int WN>
+struct Geo {
+    static constexpr int NT = 64 * WM * WN;                       // threads
+    static constexpr int MI = TM / WM / 16, NI = TN / WN / 16;    // accumulator blocks per wave
+    static constexpr int STAGE = (TM + TN) * 128;                 // bytes of one k-tile of both operands
+    static constexpr int LPW = (TM + TN) / 8 / (WM * WN);         // direct-to-LDS instructions (8 rows each) per wave and k-tile
+    static constexpr int PITCH = TN * 4 + 16;                     // bytes of a staged fp32 row (the pad spreads rows over banks)
+    static constexpr int KSQ = TM / 8 * 4;                        // QKV_PACK: one float per eight keys
+    static constexpr int MAXS = (TM + TN) >= 256 ? 5 : 8;
+    static constexpr int S = kLds / STAGE < MAXS ? kLds / STAGE : MAXS;      // ring stages
+    static constexpr int SMEM = S * STAGE > TM * PITCH + KSQ ? S * STAGE : TM * PITCH + KSQ;
+    static_assert((TM + TN) / 8 % (WM * WN) == 0 && S >= 3 && S <= 8 && SMEM <= kLds, "tile shape");
+};
+
+__device__ __forceinline__ void unpack4(const float4& v, float* f) { f[0] = v.x; f[1] = v.y; f[2] = v.z; f[3] = v.w; }
+
+// eight consecutive fp32 values from LDS or global memory
+__device__ __forceinline__ void load8(const void* src, float (&f)[8]) {
+    unpack4(reinterpret_cast<const float4*>(src)[0], f);
+    unpack4(reinterpret_cast<const float4*>(src)[1], f + 4);
+}
+__device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
+    return make_uint4(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7]));
+}
+__device__ __forceinline__ float amax8(const uint4& u) {      // largest magnitude among eight bf16
+    float m = 0.0f;
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) m = fmaxf(m, fmaxf(fabsf(bf16lo(w[i])), fabsf(bf16hi(w[i]))));
+    return m;
+}
+
+// rank-1 dequantisation: acc * (row scale * column scale), the order of the 256 x 256 kernel
+template <bool FP8>
+__device__ __forceinline__ void dequant8(float (&v)[8], const float* sw, int col, float sr) {
+    if constexpr (FP8) {
+        float w[8];
+        load8(sw + col, w);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] *= sr * w[e];
+    }
+}
+
+// K and V columns of the fused QKV projection: one 64-key x 128-column piece of the tile (its rows start at tile row r0, its
+// columns at tile column c0 = global column col0), as one image of a 128-channel head or two of 64-channel heads.
+template <bool FP8, int NT, int PITCH>
+__device__ __forceinline__ void pack_piece(const GemmParams& p, const Tile& t, const char* rows, float* ksq, int r0, int c0, int col0,
+                                           int tid) {
+    const bool is_k = col0 < p.d_q + p.d_kv;
+    const int hd = p.head_dim, half = hd >> 1, hshift = hd == 128 ? 7 : 6;
+    const int head0 = (col0 - (is_k ? p.d_q : p.d_q + p.d_kv)) >> hshift;
+    const int row0 = t.m0 + r0;                  // first key of the image (a multiple of 64)
+    const int key_tile = row0 >> 6;
+    const int64_t tile_bytes = (int64_t)hd * 128;
+    if (is_k) {
+        // eight threads per key; thread j holds both members of eight rotary pairs
+        const int j = tid & 7, hh = hd == 128 ? 0 : j >> 2, i0 = (hd == 128 ? j : (j & 3)) * 8;
+        char* img = p.kp + ((int64_t)(head0 + hh) * p.n_key_tiles + key_tile) * tile_bytes;
+        for (int key = tid >> 3; key < 64; key += NT / 8) {
+            const int row = row0 + key;
+            float a[8], b[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) a[e] = b[e] = 0.0f;      // padding keys of a ragged last tile are zero in the images
+            if (row < t.m_end) {
+                const char* src = rows + (r0 + key) * PITCH + (c0 + hh * hd + i0) * 4;
+                load8(src, a);
+                load8(src + half * 4, b);
+                if constexpr (FP8) {
+                    const float sr = p.sa[row];
+                    dequant8<true>(a, t.sw, col0 + hh * hd + i0, sr);
+                    dequant8<true>(b, t.sw, col0 + hh * hd + i0 + half, sr);
+                }
+                if (t.knw != nullptr) {
+                    float ss = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) ss += a[e] * a[e] + b[e] * b[e];
+                    ss += __shfl_xor(ss, 1, 64);
+                    ss += __shfl_xor(ss, 2, 64);
+                    if (hd == 128) ss += __shfl_xor(ss, 4, 64);
+                    const float rn = rsqrtf(ss * (hd == 128 ? 1.0f / 128.0f : 1.0f / 64.0f) + p.k_eps);
+                    float w1[8], w2[8];
+                    load8(t.knw + i0, w1);
+                    load8(t.knw + half + i0, w2);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) { a[e] *= rn * w1[e]; b[e] *= rn * w2[e]; }
+                }
+                if (p.cos != nullptr) {
+                    float c[8], s[8];
+                    load8(p.cos + (int64_t)row * half + i0, c);
+                    load8(p.sin + (int64_t)row * half + i0, s);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) rotate_pair(a[e], b[e], c[e], s[e]);
+                }
+            }
+            const uint4 ua = pack8(a), ub = pack8(b);
+            // K image, chunk-major [hd / 8 chunks][64 keys][16 bytes]
+            *reinterpret_cast<uint4*>(img + ((i0 >> 3) * 64 + key) * 16) = ua;
+            *reinterpret_cast<uint4*>(img + (((i0 + half) >> 3) * 64 + key) * 16) = ub;
+            const uint32_t w[8] = {ua.x, ua.y, ua.z, ua.w, ub.x, ub.y, ub.z, ub.w};
+            float sq = 0.0f;      // squared norm of the key as stored
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { const float lo = bf16lo(w[e]), hi = bf16hi(w[e]); sq += lo * lo + hi * hi; }
+            sq += __shfl_xor(sq, 1, 64);
+            sq += __shfl_xor(sq, 2, 64);
+            if (hd == 128) sq += __shfl_xor(sq, 4, 64);
+            // the largest among the eight keys of this wave instruction (hd 64: lanes 0-3 and 4-7 of every eight are two heads)
+            sq = fmaxf(sq, __shfl_xor(sq, 8, 64));
+            sq = fmaxf(sq, __shfl_xor(sq, 16, 64));
+            sq = fmaxf(sq, __shfl_xor(sq, 32, 64));
+            const int lane = tid & 63;
+            if (lane == 0 || (lane == 4 && hd == 64)) ksq[(key >> 3) * 2 + (lane >> 2)] = sq;
+        }
+    } else {
+        // V^T image [8 chunks][hd channel rows][8 keys]; chunk c = 4 s + g lists keys 32 s + 4 g + {0..3} and
+        // 32 s + 16 + 4 g + {0..3} (the order in which a lane of the attention kernel holds its probabilities)
+        const int h = tid & 127, hh = hd == 128 ? 0 : h >> 6;
+        char* img = p.vp + ((int64_t)(head0 + hh) * p.n_key_tiles + key_tile) * tile_bytes;
+        const float wsc = FP8 ? t.sw[col0 + h] : 1.0f;
+        for (int c = tid >> 7; c < 8; c += NT / 128) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int key = 32 * (c >> 2) + 4 * (c & 3) + 16 * (e >> 2) + (e & 3);
+                v[e] = 0.0f;
+                if (row0 + key < t.m_end) {
+                    v[e] = *reinterpret_cast<const float*>(rows + (r0 + key) * PITCH + (c0 + h) * 4);
+                    if constexpr (FP8) v[e] *= p.sa[row0 + key] * wsc;
+                }
+            }
+            *reinterpret_cast<uint4*>(img + (c * hd + (h & (hd - 1))) * 16) = pack8(v);
+        }
+    }
+}
+
+template <int EPI, bool FP8, int TM, int TN, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tile_kernel(const GemmParams p) {
+    using G = Geo<TM, TN, WM, WN>;
+    constexpr int NW = WM * WN, NT = G::NT, MI = G::MI, NI = G::NI, S = G::S, L = G::LPW;
+    static_assert(TM / 8 % NW == 0 || NW % (TM / 8) == 0, "a load instruction belongs to one operand");
+    __shared__ __attribute__((aligned(1024))) char smem[G::SMEM];
+
+    Tile tile;
+    if (!locate_tile<TM, 8>(p, tile)) return;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave % WN;
+    const int m0 = tile.m0;
+    const int n0 = tile.tn * (EPI == CDM_EPI_SWIGLU ? TN / 2 : TN);      // first output column
+
+    // ---- load instruction j of this wave covers tile rows 8 (NW j + wave) .. + 7 of [A rows | W rows]
+    uint32_t off[L];
+    const char* base[L];
+#pragma unroll
+    for (int j = 0; j < L; ++j) {
+        const int r8 = (NW * j + wave) * 8, row = r8 + (lane >> 3);
+        const int chunk = (lane & 7) ^ swz16(row);
+        if (r8 < TM) {
+            const int am = (m0 + row) < tile.m_end ? row : tile.m_end - 1 - m0;
+            off[j] = (uint32_t)(am * (int)p.lda + chunk * 16);
+            base[j] = uniform_ptr(reinterpret_cast<const char*>(p.A) + (int64_t)m0 * p.lda);
+        } else {
+            const int wr = row - TM;
+            // SWIGLU: 64-row groups of the tile alternate gate / up
+            const bool up = EPI == CDM_EPI_SWIGLU && (((r8 - TM) >> 6) & 1);
+            int bn = EPI == CDM_EPI_SWIGLU ? (wr >> 7) * 64 + (wr & 63) : wr;
+            bn = (n0 + bn) < p.N ? bn : p.N - 1 - n0;
+            off[j] = (uint32_t)(bn * (int)p.ldw + chunk * 16);
+            base[j] = uniform_ptr(reinterpret_cast<const char*>(up ? tile.W2 : tile.W) + (int64_t)n0 * p.ldw);
+        }
+    }
+    const uint32_t l0 = lds_addr_of(smem) + wave * 1024;
+    const int r16 = lane & 15, q = lane >> 4;
+    constexpr int KS = FP8 ? 1 : 2;
+    using T = typename std::conditional<FP8, i32x8, bf16x8>::type;
+    uint32_t fa[KS], fb[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        // bf16: 16-byte chunk 4 ks + q of the row; e4m3: chunks 2 q and 2 q + 1 (the second at the address ^ 16)
+        const int chunk = FP8 ? 2 * q : 4 * ks + q;
+        const uint32_t in_row = (uint32_t)(r16 * 128 + ((chunk ^ swz16(r16)) << 4));
+        fa[ks] = in_row + wm * (MI * 2048);
+        fb[ks] = in_row + TM * 128 + wn * (NI * 2048);
+    }
+    auto rd = [&](uint32_t o) {
+        if constexpr (FP8) {
+            const int4 lo = *reinterpret_cast<const int4*>(smem + o);
+            const int4 hi = *reinterpret_cast<const int4*>(smem + (o ^ 16));
+            return i32x8{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        } else {
+            return *reinterpret_cast<const bf16x8*>(smem + o);
+        }
+    };
+    f32x4 acc[MI][NI];
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+    T a[2][MI], b[2][NI];      // fragments of the k-step at hand and of the next one
+    auto read = [&](int slot, int ks, int set) {
+        const uint32_t s0 = slot * G::STAGE;
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) a[set][mi] = rd(fa[ks] + s0 + mi * 2048);
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni) b[set][ni] = rd(fb[ks] + s0 + ni * 2048);
+        __builtin_amdgcn_sched_barrier(0);      // the reads go out ahead of the MFMAs they run under
+    };
+    // the MFMAs of one k-step; LOADS: the refill of slot `slot` with tile t, one load behind every few MFMAs (a wave that
+    // issues its loads back to back sits in the vector-memory issue queue with the matrix pipe idle)
+    auto mma = [&](int set, auto loads_c, int t, int slot) {
+        constexpr bool LOADS = decltype(loads_c)::value;
+        constexpr int NM = MI * NI, GAP = NM / L > 0 ? NM / L : 1;
+        int nl = 0;
+#pragma unroll
+        for (int i = 0; i < NM; ++i) {
+            const int ni = i / MI, mi = i % MI;
+            if constexpr (FP8)
+                acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b[set][ni], a[set][mi], acc[mi][ni], 0 /*A: e4m3*/,
+                                                                               0 /*B: e4m3*/, 0, 0, 0, 0);
+            else
+                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[set][ni], a[set][mi], acc[mi][ni], 0, 0, 0);
+            if (LOADS && i % GAP == GAP - 1 && nl < L) {
+                lds_dma16(base[nl] + t * 128, off[nl], l0 + slot * G::STAGE + nl * (NW * 1024));
+                ++nl;
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (LOADS)
+            for (; nl < L; ++nl) lds_dma16(base[nl] + t * 128, off[nl], l0 + slot * G::STAGE + nl * (NW * 1024));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // ---- k-tiles.  Tile t lives in slot t % S.  A wave enters step t with the fragments of its first k-step in registers;
+    // the barrier sits ahead of the step's last k-step: every wave has then read all of tile t (whose slot is refilled with
+    // tile t + S) and tile t + 1 has landed, so the fragments the next step starts with are read under this step's last
+    // MFMAs.  Loads past the last tile are not issued: the last S steps count the loads still behind them instead.
+    const int KT = p.K / (FP8 ? 128 : 64);
+#pragma unroll
+    for (int t = 0; t < S; ++t)
+        if (t < KT) {
+#pragma unroll
+            for (int j = 0; j < L; ++j) lds_dma16(base[j] + t * 128, off[j], l0 + t * G::STAGE + j * (NW * 1024));
+        }
+    using std::false_type;
+    using std::true_type;
+    int slot = 0;
+    // SET: fragment set of the tile's first (e4m3: only) k-step - bf16 always 0, e4m3 alternating
+    auto step = [&](auto behind_c, auto refill_c, auto set_c, int t) {
+        constexpr int BEHIND = decltype(behind_c)::value;      // tiles that may still be in flight behind tile t + 1
+        constexpr int SET = decltype(set_c)::value;
+        const int next = slot == S - 1 ? 0 : slot + 1;
+        if constexpr (!FP8) {
+            read(slot, 1, 1);
+            mma(0, false_type{}, 0, 0);
+        }
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(BEHIND * L) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        read(next, 0, FP8 ? 1 - SET : 0);
+        mma(FP8 ? SET : 1, refill_c, t + S, slot);
+        slot = next;
+    };
+    using C0 = std::integral_constant<int, 0>;
+    using C1 = std::integral_constant<int, FP8 ? 1 : 0>;
+    using Deep = std::integral_constant<int, S - 2>;
+    // tile 0 has landed everywhere
+    if (KT >= S) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * L) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    read(0, 0, 0);
+    int t = 0;
+    if constexpr (FP8) {
+        for (; t + S < KT; t += 2) {
+            step(Deep{}, true_type{}, C0{}, t);
+            if (S % 2 == 0 || t + 1 + S < KT) step(Deep{}, true_type{}, C1{}, t + 1);      // KT is even
+        }
+    } else {
+        for (; t + S < KT; ++t) step(Deep{}, true_type{}, C0{}, t);
+    }
+    auto tail = [&](auto rem_c) {      // REM tiles behind this one; its index KT - 1 - REM has the parity of REM + 1
+        constexpr int REM = decltype(rem_c)::value;
+        if constexpr (REM > 0 && REM < S) {
+            if (KT > REM)
+                step(std::integral_constant<int, REM - 1>{}, false_type{}, std::integral_constant<int, FP8 ? (REM + 1) % 2 : 0>{}, 0);
+        }
+    };
+    tail(std::integral_constant<int, 7>{});
+    tail(std::integral_constant<int, 6>{});
+    tail(std::integral_constant<int, 5>{});
+    tail(std::integral_constant<int, 4>{});
+    tail(std::integral_constant<int, 3>{});
+    tail(std::integral_constant<int, 2>{});
+    tail(std::integral_constant<int, 1>{});
+    if constexpr (!FP8) {
+        read(slot, 1, 1);
+        mma(0, false_type{}, 0, 0);
+    }
+    mma(1, false_type{}, 0, 0);      // the last tile: an odd index
+
+    // ---- accumulators -> fp32 rows in LDS (every wave is done with the ring)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni)
+            *reinterpret_cast<f32x4*>(smem + ((wm * MI + mi) * 16 + r16) * G::PITCH + ((wn * NI + ni) * 16 + 4 * q) * 4) = acc[mi][ni];
+    __syncthreads();
+
+    constexpr int OC = EPI == CDM_EPI_SWIGLU ? TN / 2 : TN;      // output columns of the tile
+    constexpr int CPR = OC / 8;                                  // eight-column chunks per row
+    constexpr int ITERS = (TM * CPR + NT - 1) / NT;
+    if constexpr (EPI == CDM_EPI_QKV_PACK) {
+        float* ksq = reinterpret_cast<float*>(smem + TM * G::PITCH);
+#pragma unroll 1
+        for (int c0 = 0; c0 < TN; c0 += 128) {
+            const int col0 = n0 + c0;
+            if (col0 >= p.N) break;
+            if (col0 < p.d_q) {      // Q columns: plain rows
+                for (int idx = tid; idx < TM * 16; idx += NT) {
+                    const int rl = idx >> 4, row = m0 + rl, col = col0 + (idx & 15) * 8;
+                    if (row >= tile.m_end) continue;
+                    float v[8];
+                    load8(smem + rl * G::PITCH + (c0 + (idx & 15) * 8) * 4, v);
+                    dequant8<FP8>(v, tile.sw, col, FP8 ? p.sa[row] : 1.0f);
+                    *reinterpret_cast<uint4*>(p.C + (int64_t)row * p.ldc + col) = pack8(v);
+                }
+                continue;
+            }
+#pragma unroll 1
+            for (int r0 = 0; r0 < TM; r0 += 64) {
+                if (m0 + r0 >= tile.m_end) break;
+                pack_piece<FP8, NT, G::PITCH>(p, tile, smem, ksq, r0, c0, col0, tid);
+                if (col0 < p.d_q + p.d_kv) {      // largest key norm of the image(s)
+                    __syncthreads();
+                    const int heads = p.head_dim == 128 ? 1 : 2;
+                    if (tid < heads) {
+                        float m = 0.0f;
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) m = fmaxf(m, ksq[2 * i + tid]);
+                        const int head = (col0 - p.d_q) / p.head_dim + tid;
+                        p.kmax[(int64_t)head * p.n_key_tiles + ((m0 + r0) >> 6)] = sqrtf(m);
+                    }
+                    __syncthreads();
+                }
+            }
+        }
+        return;
+    }
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+        const int idx = it * NT + tid, rl = idx / CPR, cl = (idx % CPR) * 8;
+        const int row = m0 + rl, col = n0 + cl;
+        const bool in = (TM * CPR % NT == 0 || idx < TM * CPR) && row < tile.m_end && col < p.N;      // N is a multiple of 8: eight columns are in or out together
+        if (EPI != CDM_EPI_SWIGLU && !in) continue;
+        const float sr = FP8 && in ? p.sa[row] : 1.0f;
+        if constexpr (EPI == CDM_EPI_SWIGLU) {
+            uint4 o = make_uint4(0u, 0u, 0u, 0u);
+            if (in) {
+                const char* src = smem + rl * G::PITCH + ((cl >> 6) * 128 + (cl & 63)) * 4;
+                float g[8], u[8], h[8];
+                load8(src, g);
+                load8(src + 256, u);
+                dequant8<FP8>(g, tile.sw, col, sr);
+                dequant8<FP8>(u, tile.sw2, col, sr);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) h[e] = silu_f(g[e]) * u[e];
+                o = pack8(h);
+                *reinterpret_cast<uint4*>(p.C + (int64_t)row * p.ldc + col) = o;
+            }
+            if (p.row_amax != nullptr) {      // eight consecutive lanes hold a row's 64 columns
+                float m = amax8(o);
+                m = fmaxf(m, __shfl_xor(m, 1, 64));
+                m = fmaxf(m, __shfl_xor(m, 2, 64));
+                m = fmaxf(m, __shfl_xor(m, 4, 64));
+                if (in && (tid & 7) == 0) p.row_amax[(int64_t)row * p.amax_ld + (col >> 6)] = m;
+            }
+            continue;
+        }
+        float v[8];
+        load8(smem + rl * G::PITCH + cl * 4, v);
+        if constexpr (EPI == CDM_EPI_GATE_RESIDUAL_F32) {
+            const float* R = reinterpret_cast<const float*>(p.R) + (int64_t)row * p.ldr + col;
+            float* C = reinterpret_cast<float*>(p.C) + (int64_t)row * p.ldc + col;
+            float r[8], g[8];
+            load8(R, r);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) g[e] = 1.0f;
+            if (tile.gate) load8(tile.gate + col, g);
+            dequant8<FP8>(g, tile.sw, col, sr);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) r[e] = r[e] + g[e] * v[e];
+            *reinterpret_cast<float4*>(C) = make_float4(r[0], r[1], r[2], r[3]);
+            *reinterpret_cast<float4*>(C + 4) = make_float4(r[4], r[5], r[6], r[7]);
+            continue;
+        }
+        dequant8<FP8>(v, tile.sw, col, sr);
+        if constexpr (EPI == CDM_EPI_ROPE_QK) {
+            if (col < p.rope_cols) {      // whole heads: tile columns start on head boundaries
+                const int half = p.head_dim >> 1, in_head = col & (p.head_dim - 1), i = in_head & (half - 1);
+                const int pc = in_head < half ? cl + half : cl - half;
+                float w[8], c[8], s[8];
+                load8(smem + rl * G::PITCH + pc * 4, w);
+                dequant8<FP8>(w, tile.sw, n0 + pc, sr);
+                load8(p.cos + (int64_t)row * half + i, c);
+                load8(p.sin + (int64_t)row * half + i, s);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    float x1 = in_head < half ? v[e] : w[e], x2 = in_head < half ? w[e] : v[e];
+                    rotate_pair(x1, x2, c[e], s[e]);
+                    v[e] = in_head < half ? x1 : x2;
+                }
+            }
+        }
+        if constexpr (EPI == CDM_EPI_GATE_RESIDUAL) {
+            const uint4 r4 = *reinterpret_cast<const uint4*>(p.R + (int64_t)row * p.ldr + col);
+            const uint32_t rw[4] = {r4.x, r4.y, r4.z, r4.w};
+            float g[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) g[e] = 1.0f;
+            if (tile.gate) load8(tile.gate + col, g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[2 * e] = bf16lo(rw[e]) + g[2 * e] * v[2 * e];
+                v[2 * e + 1] = bf16hi(rw[e]) + g[2 * e + 1] * v[2 * e + 1];
+            }
+        }
+        *reinterpret_cast<uint4*>(p.C + (int64_t)row * p.ldc + col) = pack8(v);
+    }
+}
+
+template <int EPI, bool FP8>
+int32_t launch_epi(const GemmParams& p, TileShape s, int grid, hipStream_t st) {
+#define CDM_TILE(TM_, TN_, WM_, WN_) \
+    if (s.tm == TM_ && s.tn == TN_ && s.wm * 10 + s.wn == WM_ * 10 + WN_) { gemm_tile_kernel<EPI, FP8, TM_, TN_, WM_, WN_><<<grid, 64 * WM_ * WN_, 0, st>>>(p); return CDM_OK; }
+    CDM_TILE(128, 256, 2, 4)
+    CDM_TILE(128, 128, 4, 2)
+    CDM_TILE(64, 128, 2, 4)
+    if constexpr (EPI == CDM_EPI_NONE || EPI == CDM_EPI_GATE_RESIDUAL || EPI == CDM_EPI_GATE_RESIDUAL_F32) {
+        CDM_TILE(64, 64, 2, 4)
+        CDM_TILE(32, 32, 2, 2)
+    }
+#undef CDM_TILE
+    CDM_FAIL(CDM_ERR_LAUNCH, "gemm: no kernel for a %d x %d tile", s.tm, s.tn);
+}
+
+}  // namespace
+
+namespace cdm_gemm {
+
+// The shape with the least estimated time.  A round of 256 workgroups (one per CU; the 32 x 32 tile fits twice) takes a fixed
+// part - prologue latency, spreading the accumulators, epilogue - plus one slope per 128-byte k-tile, measured with weights
+// that no cache holds, in us:
+//     tile       fixed  per k-tile  example (M = 512, N = 4096, K = 16384, bf16: us, at the 256 x 256 tile 287)
+//     256 x 256   18    1.05 on up to half the CUs, 1.37 on all (power and L2)
+//     128 x 256   10    0.82        211
+//     128 x 128    7    0.53        142
+//      64 x 128    5    0.40        113
+//      64 x 64     4.5  0.25        138 (two rounds)
+//      32 x 32     4.5  0.14        220 (eight tiles per CU)
+// e4m3 k-tiles take the same time (twice the elements per 128 bytes at twice the matrix rate).
+TileShape pick_tile(const GemmParams& p, int epilogue, bool fp8) {
+    static const struct { TileShape s; double fixed, per_kt; } kShapes[] = {
+        {{128, 256, 2, 4}, 10.0, 0.82}, {{128, 128, 4, 2}, 7.0, 0.53}, {{64, 128, 2, 4}, 5.0, 0.40},
+        {{64, 64, 2, 4}, 4.5, 0.25},    {{32, 32, 2, 2}, 4.5, 0.14}};
+    const int v = cdm_get_variant(1);
+    if (v == 2) return TileShape{256, 256, 4, 2};      // cross-check build: one shape for everything
+    if (v > 2) return kShapes[(v - 3) % 5].s;
+    const bool narrow = epilogue == CDM_EPI_NONE || epilogue == CDM_EPI_GATE_RESIDUAL || epilogue == CDM_EPI_GATE_RESIDUAL_F32;
+    const double kt = p.K / (fp8 ? 128.0 : 64.0);
+    auto tiles = [&](int tm, int tn) {
+        const int64_t cols = epilogue == CDM_EPI_SWIGLU ? tn / 2 : tn;
+        int64_t rows = 0;
+        for (int i = 0; i < p.n_seg; ++i) rows += (p.seg[i].m_end - p.seg[i].m_start + tm - 1) / tm;
+        return rows * ((p.N + cols - 1) / cols);
+    };
+    const int64_t big = tiles(256, 256);
+    TileShape best{256, 256, 4, 2};
+    double best_us = (double)((big + 255) / 256) * (18.0 + kt * (big <= 128 ? 1.05 : 1.37));
+    for (const auto& k : kShapes) {
+        if (k.s.tn < 128 && !narrow) continue;
+        const int64_t n = tiles(k.s.tm, k.s.tn);
+        const double us = k.s.tm == 32 ? (n <= 256 ? k.fixed + kt * k.per_kt : (double)((n + 511) / 512) * (k.fixed + kt * 0.26))
+                                       : (double)((n + 255) / 256) * (k.fixed + kt * k.per_kt);
+        if (us < best_us) { best_us = us; best = k.s; }
+    }
+    return best;
+}
+
+int32_t launch_tile(GemmParams& p, int epilogue, bool fp8, TileShape s, hipStream_t st) {
+    const int cols = epilogue == CDM_EPI_SWIGLU ? s.tn / 2 : s.tn;
+    p.tiles_n = (p.N + cols - 1) / cols;
+    int total = 0;
+    for (int i = 0; i < p.n_seg; ++i) {
+        p.seg[i].tiles_m = (p.seg[i].m_end - p.seg[i].m_start + s.tm - 1) / s.tm;
+        total += p.seg[i].tiles_m * p.tiles_n;
+        p.seg[i].tile_end = total;
+    }
+    p.total_tiles = total;
+    const int grid = (total + 7) / 8 * 8;
+#define CDM_LAUNCH(E) return fp8 ? launch_epi<E, true>(p, s, grid, st) : launch_epi<E, false>(p, s, grid, st)
+    switch (epilogue) {
+        case CDM_EPI_NONE: CDM_LAUNCH(CDM_EPI_NONE);
+        case CDM_EPI_SWIGLU: CDM_LAUNCH(CDM_EPI_SWIGLU);
+        case CDM_EPI_GATE_RESIDUAL: CDM_LAUNCH(CDM_EPI_GATE_RESIDUAL);
+        case CDM_EPI_GATE_RESIDUAL_F32: CDM_LAUNCH(CDM_EPI_GATE_RESIDUAL_F32);
+        case CDM_EPI_QKV_PACK: CDM_LAUNCH(CDM_EPI_QKV_PACK);
+        default: CDM_LAUNCH(CDM_EPI_ROPE_QK);
+    }
+#undef CDM_LAUNCH
+}
+
+}  // namespace cdm_gemm

@@ -88,7 +88,8 @@ def time_ops(enable: bool):
 
 def set_variant(op: str, variant: int) -> int:
     """Cross-check aid (tests, measurements): run ``op`` ("attn" / "gemm") on a superseded kernel of the cross-check
-    build; 0 = back to the product library's kernel.  Returns the previous selection."""
+    build, or ("gemm", 2 - 7) on one tile shape whatever the size; 0 = back to the product library's kernel.  Returns the
+    previous selection."""
     return _lib.set_variant(op, variant)
 
 

@@ -102,6 +102,106 @@ def test_gemm_plain(M, N, K, variant):
     assert_close(c, ar @ wr.t(), 0.99999, 6e-3, f"gemm {M}x{N}x{K} variant={variant}")
 
 
+# tile shapes of the small launches: variant 2 = 256 x 256 for every size, 3 - 7 = 128 x 256, 128 x 128, 64 x 128, 64 x 64, 32 x 32
+# (the last two serve the epilogues without a column structure only)
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("M,N,K,epi", [(1, 8, 256, "none"), (65, 264, 512, "none"), (129, 1000, 2304, "gate_residual"),
+                                       (300, 136, 768, "gate_residual_f32"), (31, 72, 4096, "gate_residual_f32"),
+                                       (77, 200, 256, "swiglu"), (257, 1096, 1280, "swiglu"), (130, 768, 1024, "rope_qk")])
+def test_gemm_small_tiles_equal_the_large_one(M, N, K, epi, fp8, request):
+    """Every tile shape adds the products of an output element in the same order, so all of them give the bits of the
+    256 x 256 kernel: rows and columns off the tile edges, fewer k-tiles than ring stages, the partial row maxima."""
+    request.addfinalizer(lambda: ops.set_variant("gemm", 0))
+    g = gen(M + N + K)
+    a, ar = rand_bf16((M, K), g)
+    w, wr = rand_bf16((N, K), g, 0.05)
+    w2, w2r = rand_bf16((N, K), g, 0.05)
+    gate = torch.randn(N, generator=g)
+    r = torch.randn((M, N), generator=g).to(torch.float32 if epi.endswith("f32") else torch.bfloat16)
+    cos, sin = torch.rand((M, 64), generator=g), torch.rand((M, 64), generator=g)
+    kw = dict(epilogue="gate_residual" if epi.startswith("gate") else epi)
+    if epi.startswith("gate"):
+        kw.update(residual=r.to(dev()), gate=gate.to(dev()))
+    if epi == "rope_qk":
+        kw.update(cos=cos.to(dev()), sin=sin.to(dev()), rope_cols=512, head_dim=128)
+    if fp8:
+        (aq, sa), (wq, sw), (w2q, sw2) = ops.quant_rows(a), ops.quant_rows(w), ops.quant_rows(w2)
+        if epi == "swiglu":
+            kw.update(w2q=w2q, sw2=sw2)
+    elif epi == "swiglu":
+        kw.update(w2=w2)
+
+    def call():
+        out = torch.empty((M, N), dtype=r.dtype if epi.startswith("gate") else torch.bfloat16, device=dev())
+        amax = torch.zeros((M, (N + 63) // 64), device=dev()) if fp8 and epi == "swiglu" else None
+        if fp8:
+            ops.gemm_fp8(aq, sa, wq, sw, out=out, row_amax=amax, **kw)
+        else:
+            ops.gemm(a, w, out=out, **kw)
+        return out, amax
+
+    ops.set_variant("gemm", 2)
+    want, want_amax = call()
+    y = (aq.float().cpu() * sa.cpu()[:, None] @ (wq.float().cpu() * sw.cpu()[:, None]).t()) if fp8 else ar @ wr.t()
+    if epi == "swiglu":
+        u = (aq.float().cpu() * sa.cpu()[:, None] @ (w2q.float().cpu() * sw2.cpu()[:, None]).t()) if fp8 else ar @ w2r.t()
+        y = torch.nn.functional.silu(y) * u
+    elif epi.startswith("gate"):
+        y = r.float() + gate * y
+    if epi != "rope_qk":      # (the rotation is checked against the oracle by test_gemm_rope_qk)
+        assert_close(want, y, 0.9999, 1e-2, f"256x256 tile {M}x{N}x{K} {epi} fp8={fp8}")
+    for variant in range(3, 8 if epi.startswith(("none", "gate")) else 6):
+        ops.set_variant("gemm", variant)
+        got, amax = call()
+        assert torch.equal(got, want), f"tile variant {variant}: {M}x{N}x{K} {epi} fp8={fp8}"
+        assert amax is None or torch.equal(amax, want_amax), f"tile variant {variant}: row maxima"
+    ops.set_variant("gemm", 0)
+    assert torch.equal(call()[0], want)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("segs,H,Hkv,K,qkn,hd", [([(0, 64), (64, 77)], 2, 1, 512, False, 128), ([(0, 300)], 4, 2, 256, True, 64),
+                                                 ([(0, 128), (128, 1)], 3, 3, 768, True, 128)])
+def test_qkv_pack_small_tiles_equal_the_large_one(segs, H, Hkv, K, qkn, hd, fp8, request):
+    """The K / V tile images of the small tiles: bit-equal to those of the 256 x 256 kernel (with a K-norm the sum of squares
+    is added in another order: one bf16 rounding apart), key-norm bounds to fp32 accuracy."""
+    request.addfinalizer(lambda: ops.set_variant("gemm", 0))
+    n = sum(l for _, l in segs)
+    g = gen(n + K)
+    a, _ = rand_bf16((n, K), g)
+    rows = (H + 2 * Hkv) * hd
+    ws = [rand_bf16((rows, K), g, 0.05)[0] for _ in segs]
+    cos, sin = torch.rand((n, hd // 2), generator=g).to(dev()), torch.rand((n, hd // 2), generator=g).to(dev())
+    norm = None
+    if qkn:
+        kn = (1 + 0.2 * torch.randn((len(segs), hd), generator=g)).to(dev())
+        norm = (kn, kn, [s + l for s, l in segs], 1e-6)
+    sa = sws = None
+    if fp8:
+        (a, sa), quant = ops.quant_rows(a), [ops.quant_rows(w) for w in ws]
+        ws, sws = [q[0] for q in quant], [q[1] for q in quant]
+    one = (n + 63) // 64 * 64 * Hkv * hd * 2      # bytes of one image set
+    tiles = (n + 63) // 64 * Hkv
+
+    def call():
+        q = torch.zeros((n, H * hd), dtype=torch.bfloat16, device=dev())
+        img = torch.full((ops.attn_workspace_bytes(n, Hkv, hd),), 77, dtype=torch.uint8, device=dev())
+        ops.gemm_qkv_pack(a, sa, ws, sws, segs, H, Hkv, hd, q, img, cos, sin, norm)
+        return q, img[:one].view(torch.bfloat16), img[one:2 * one].view(torch.bfloat16), img[2 * one:2 * one + 4 * tiles].view(torch.float32)
+
+    ops.set_variant("gemm", 2)
+    q0, k0, v0, m0 = call()
+    for variant in (3, 4, 5):
+        ops.set_variant("gemm", variant)
+        q, k, v, m = call()
+        assert torch.equal(q, q0) and torch.equal(v, v0), f"tile variant {variant}"
+        if qkn:      # |difference| <= one unit in the last place of bf16 (2^-7 of the value at most)
+            assert bool(((k.float() - k0.float()).abs() <= k0.float().abs() * 2.0 ** -7).all()), f"tile variant {variant}: K image"
+        else:
+            assert torch.equal(k, k0), f"tile variant {variant}: K image"
+        assert bool(((m - m0).abs() <= m0 * (2.0 ** -7 if qkn else 1e-5)).all()), f"tile variant {variant}: key norms"
+
+
 def test_gemm_strided_views_and_determinism():
     g = gen(5)
     big, bigr = rand_bf16((200, 640), g)
