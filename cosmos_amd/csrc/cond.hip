@@ -1,0 +1,107 @@
+// Conditioning of a forward: the sinusoid of the timestep and the adaLN modulation vectors of every block.
+// The modulation streams one weight matrix per block once (12 d^2 bytes, 201 MB at d = 4096) and is bound by HBM there; at
+// small widths the launches are what counts.  One launch serves all blocks of a stack, where stock operators take ten
+// small ones per block (activation, GEMV, conversion, six copies); the sinusoid is one launch instead of eight.
+// A wave owns four output rows and reads 16 bytes per lane of each, four deep: 16 KB in flight per wave, 64 KB per CU.
+#include "cdm_common.h"
+
+namespace {
+
+constexpr int kRows = 4;             // output rows per wave
+constexpr int kWaves = 4;            // waves per workgroup
+constexpr int kMaxBlocks = 64;       // blocks per modulation launch
+
+__device__ __forceinline__ float silu_exact(float x) { return x / (1.0f + expf(-x)); }
+
+// [n, 2 half]: cos(t f_k) | sin(t f_k), f_k = 10000^(-k / half)
+__global__ __launch_bounds__(256) void timestep_sinusoid_kernel(const float* __restrict__ t, float* __restrict__ out, int half) {
+    const float tv = t[blockIdx.x];
+    for (int k = threadIdx.x; k < half; k += 256) {
+        const float a = tv * expf(-9.210340371976184f * (float)k / (float)half);      // ln(10000)
+        out[(int64_t)blockIdx.x * 2 * half + k] = cosf(a);
+        out[(int64_t)blockIdx.x * 2 * half + half + k] = sinf(a);
+    }
+}
+
+struct ModParams {
+    const float* c;                      // conditioning vector [d]
+    float* out;                          // [n_blocks, n_out]
+    int d, n_out, per_block;             // workgroups per block
+    const bf16_t* w[kMaxBlocks];         // [n_out, d]
+    const bf16_t* b[kMaxBlocks];         // [n_out]
+};
+
+// out[l] = W_l silu(c) + b_l for every block l.  The vector is rounded to bf16 ahead of the activation and behind it, and the
+// result to bf16, as the bf16 linear layer it stands for does; sums are fp32.
+__global__ __launch_bounds__(64 * kWaves) void modulation_kernel(const ModParams p) {
+    extern __shared__ float s[];         // silu(c), d values
+    for (int i = threadIdx.x; i < p.d; i += 64 * kWaves) {
+        const float c = bf16lo(pack_bf16x2(p.c[i], 0.0f));
+        s[i] = bf16lo(pack_bf16x2(silu_exact(c), 0.0f));
+    }
+    __syncthreads();
+    const int blk = blockIdx.x / p.per_block;
+    const int lane = threadIdx.x & 63;
+    const int row0 = ((blockIdx.x - blk * p.per_block) * kWaves + (threadIdx.x >> 6)) * kRows;
+    if (row0 >= p.n_out) return;
+    const bf16_t* w = p.w[blk];
+    const uint4* wr[kRows];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) wr[r] = reinterpret_cast<const uint4*>(w + (int64_t)(row0 + r < p.n_out ? row0 + r : p.n_out - 1) * p.d);
+    const int n8 = p.d >> 3;
+    float acc[kRows] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int i = lane; i < n8; i += 64) {
+        const float4 s0 = reinterpret_cast<const float4*>(s)[2 * i], s1 = reinterpret_cast<const float4*>(s)[2 * i + 1];
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+            const uint4 v = wr[r][i];
+            acc[r] += bf16lo(v.x) * s0.x + bf16hi(v.x) * s0.y + bf16lo(v.y) * s0.z + bf16hi(v.y) * s0.w + bf16lo(v.z) * s1.x +
+                      bf16hi(v.z) * s1.y + bf16lo(v.w) * s1.z + bf16hi(v.w) * s1.w;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+        acc[r] = wave_sum(acc[r]);
+        const int row = row0 + r;
+        if (lane == 0 && row < p.n_out)
+            p.out[(int64_t)blk * p.n_out + row] = bf16lo(pack_bf16x2(acc[r] + bf16lo(p.b[blk][row]), 0.0f));
+    }
+}
+
+}  // namespace
+
+extern "C" int32_t cdm_timestep_sinusoid_f32(const float* t, float* out, int64_t n, int64_t freq_dim, void* stream) {
+    CDM_REQUIRE(t && out, CDM_ERR_BAD_ARG, "timestep_sinusoid: null pointer");
+    CDM_REQUIRE(n >= 0 && n < (1ll << 31) && freq_dim >= 2 && freq_dim % 2 == 0 && freq_dim < (1ll << 24), CDM_ERR_BAD_SHAPE,
+                "timestep_sinusoid: n=%lld, freq_dim=%lld (even)", (long long)n, (long long)freq_dim);
+    if (n == 0) return CDM_OK;
+    int32_t rc = cdm_require_device();
+    if (rc) return rc;
+    timestep_sinusoid_kernel<<<(unsigned)n, 256, 0, (hipStream_t)stream>>>(t, out, (int)(freq_dim / 2));
+    return cdm_check_launch("timestep_sinusoid");
+}
+
+extern "C" int32_t cdm_adaln_modulation_bf16(const float* c, const void* const* w, const void* const* b, int32_t n_blocks, float* out,
+                                             int64_t d, int64_t n_out, void* stream) {
+    CDM_REQUIRE(c && w && b && out, CDM_ERR_BAD_ARG, "adaln_modulation: null pointer");
+    CDM_REQUIRE(n_blocks >= 0 && n_out > 0, CDM_ERR_BAD_ARG, "adaln_modulation: bad sizes");
+    CDM_REQUIRE(d > 0 && d % 8 == 0 && d <= 16384 && n_out < (1ll << 24), CDM_ERR_BAD_SHAPE,
+                "adaln_modulation: d=%lld must be a multiple of 8 up to 16384", (long long)d);
+    for (int i = 0; i < n_blocks; ++i)
+        CDM_REQUIRE(w[i] && b[i] && cdm_aligned16(w[i]), CDM_ERR_BAD_ARG, "adaln_modulation: weight or bias of block %d null or misaligned", i);
+    if (n_blocks == 0) return CDM_OK;
+    int32_t rc = cdm_require_device();
+    if (rc) return rc;
+    const int per = kWaves * kRows;
+    ModParams p;
+    p.c = c; p.d = (int)d; p.n_out = (int)n_out; p.per_block = (int)((n_out + per - 1) / per);
+    for (int at = 0; at < n_blocks; at += kMaxBlocks) {
+        const int nb = n_blocks - at < kMaxBlocks ? n_blocks - at : kMaxBlocks;
+        for (int i = 0; i < nb; ++i) { p.w[i] = (const bf16_t*)w[at + i]; p.b[i] = (const bf16_t*)b[at + i]; }
+        p.out = out + (int64_t)at * n_out;
+        modulation_kernel<<<(unsigned)(nb * p.per_block), 64 * kWaves, (size_t)d * 4, (hipStream_t)stream>>>(p);
+        if ((rc = cdm_check_launch("adaln_modulation"))) return rc;
+    }
+    return CDM_OK;
+}

@@ -39,12 +39,37 @@ __device__ __forceinline__ float block_reduce(float v, float (*slot)[4], int& pa
     return IS_MAX ? fmaxf(fmaxf(a, b), fmaxf(c, d)) : (a + b) + (c + d);
 }
 
+constexpr int kMaxSeg = 8;
+
+// Token runs with weights and modulation of their own (the branches of a joint sequence), one launch for all of them: a
+// workgroup belongs to one run and walks over its rows.
+struct NormSeg {
+    const uint4* w; const float* shift; const float* scale;
+    int64_t start, end;                  // token rows
+    int block_end;                       // workgroups of runs 0 .. this one
+};
+struct NormParams {
+    const void* x; void* y; float* s_tok;
+    int d, n_seg; float eps;
+    NormSeg seg[kMaxSeg];
+};
+
 // MAXC = chunks of 8 channels per thread (d <= 2048 * MAXC); XF32: the input rows are fp32 instead of bf16
 template <int MAXC, bool QUANT, bool XF32>
-__global__ __launch_bounds__(kThreads) void adaln_rmsnorm_kernel(
-    const void* __restrict__ x, const uint4* __restrict__ w, const float* __restrict__ shift,
-    const float* __restrict__ scale, void* __restrict__ y, float* __restrict__ s_tok, int64_t n_tokens,
-    int d, float eps) {
+__global__ __launch_bounds__(kThreads) void adaln_rmsnorm_kernel(const NormParams p) {
+    int si = 0;
+    while (si < p.n_seg - 1 && (int)blockIdx.x >= p.seg[si].block_end) ++si;
+    const int block0 = si ? p.seg[si - 1].block_end : 0;
+    const void* __restrict__ x = p.x;
+    const uint4* __restrict__ w = p.seg[si].w;
+    const float* __restrict__ shift = p.seg[si].shift;
+    const float* __restrict__ scale = p.seg[si].scale;
+    void* __restrict__ y = p.y;
+    float* __restrict__ s_tok = p.s_tok;
+    const int64_t n_tokens = p.seg[si].end, row0 = p.seg[si].start + ((int)blockIdx.x - block0);
+    const int row_step = p.seg[si].block_end - block0;
+    const int d = p.d;
+    const float eps = p.eps;
     __shared__ float slot_sum[2][4];
     __shared__ float slot_max[2][4];
     int par_sum = 0, par_max = 0;
@@ -89,8 +114,8 @@ __global__ __launch_bounds__(kThreads) void adaln_rmsnorm_kernel(
                 raw[c][h] = idx < nchunk ? xr[(XF32 ? 2 : 1) * idx + h] : make_uint4(0, 0, 0, 0);
         }
     };
-    if ((int64_t)blockIdx.x < n_tokens) fetch(blockIdx.x);
-    for (int64_t row = blockIdx.x; row < n_tokens; row += gridDim.x) {
+    if (row0 < n_tokens) fetch(row0);
+    for (int64_t row = row0; row < n_tokens; row += row_step) {
         float xv[MAXC][8];
         float ss = 0.0f;
 #pragma unroll
@@ -107,7 +132,7 @@ __global__ __launch_bounds__(kThreads) void adaln_rmsnorm_kernel(
 #pragma unroll
             for (int i = 0; i < 8; ++i) ss += xv[c][i] * xv[c][i];
         }
-        if (row + gridDim.x < n_tokens) fetch(row + gridDim.x);
+        if (row + row_step < n_tokens) fetch(row + row_step);
         ss = block_reduce<false>(ss, slot_sum, par_sum);
         const float r = rsqrtf(ss * inv_d + eps);
         float amax = 0.0f;
@@ -242,17 +267,21 @@ __global__ __launch_bounds__(kThreads) void quant_rows_parts_kernel(const bf16_t
 }
 
 template <bool QUANT, bool XF32>
-int32_t launch_norm(const void* x, const void* w, const float* shift, const float* scale, void* y, float* s_tok,
-                    int64_t n_tokens, int64_t d, float eps, hipStream_t st) {
+int32_t launch_norm(NormParams& p, hipStream_t st) {
     // 64 workgroups per CU's worth of rows in flight: at 56 k rows a workgroup walks over three or four rows.  Measured in
     // the 56,832 x 4096 stack (fp32 rows in, bf16 out): 2048 workgroups 5.37 TB/s, 4096 5.53, 8192 5.63, 16384 5.75, 32768
-    // 5.52, one row each 5.04 (the per-channel vectors are then loaded as often as the rows)
+    // 5.52, one row each 5.04 (the per-channel vectors are then loaded as often as the rows).  Several runs share them out
+    // by their rows.
     const int64_t max_blocks = 256 * 64;
-    const int grid = (int)(n_tokens < max_blocks ? n_tokens : max_blocks);
-    const int chunks = (int)((d / 8 + kThreads - 1) / kThreads);
-#define CDM_NORM_LAUNCH(C)                                                                                  \
-    adaln_rmsnorm_kernel<C, QUANT, XF32><<<grid, kThreads, 0, st>>>(x, (const uint4*)w, shift, scale, y, s_tok, \
-                                                                    n_tokens, (int)d, eps)
+    int64_t total = 0, grid = 0;
+    for (int i = 0; i < p.n_seg; ++i) total += p.seg[i].end - p.seg[i].start;
+    for (int i = 0; i < p.n_seg; ++i) {
+        const int64_t rows = p.seg[i].end - p.seg[i].start;
+        grid += total <= max_blocks ? rows : (rows * max_blocks + total - 1) / total;
+        p.seg[i].block_end = (int)grid;
+    }
+    const int chunks = (p.d / 8 + kThreads - 1) / kThreads;
+#define CDM_NORM_LAUNCH(C) adaln_rmsnorm_kernel<C, QUANT, XF32><<<(unsigned)grid, kThreads, 0, st>>>(p)
     if (chunks <= 1) CDM_NORM_LAUNCH(1);
     else if (chunks == 2) CDM_NORM_LAUNCH(2);
     else CDM_NORM_LAUNCH(4);
@@ -271,46 +300,69 @@ int32_t check_norm_args(const void* x, const void* w, const void* y, int64_t n_t
     return CDM_OK;
 }
 
+// runs [start, start + len) of x / y, kMaxSeg per launch; s_tok != null: e4m3 rows and their scales
+int32_t norm_runs(const void* x, bool x_f32, const void* const* w, const float* const* shift, const float* const* scale,
+                  const int64_t* start, const int64_t* len, int32_t n_seg, void* y, float* s_tok, int64_t d, float eps,
+                  void* stream) {
+    for (int i = 0; i < n_seg; ++i) {
+        int32_t rc = check_norm_args(x, w[i], y, len[i], d, shift ? shift[i] : nullptr, scale ? scale[i] : nullptr);
+        if (rc) return rc;
+        CDM_REQUIRE(start[i] >= 0 && start[i] + len[i] < (1ll << 31), CDM_ERR_BAD_ARG, "adaln_rmsnorm: bad token run %d", i);
+    }
+    int32_t rc = cdm_require_device();
+    if (rc) return rc;
+    NormParams p;
+    p.x = x; p.y = y; p.s_tok = s_tok; p.d = (int)d; p.eps = eps;
+    for (int i = 0; i < n_seg;) {
+        p.n_seg = 0;
+        for (; i < n_seg && p.n_seg < kMaxSeg; ++i)
+            if (len[i] > 0)
+                p.seg[p.n_seg++] = NormSeg{(const uint4*)w[i], shift ? shift[i] : nullptr, scale ? scale[i] : nullptr, start[i],
+                                           start[i] + len[i], 0};
+        if (p.n_seg == 0) continue;
+        hipStream_t st = (hipStream_t)stream;
+        rc = s_tok == nullptr ? (x_f32 ? launch_norm<false, true>(p, st) : launch_norm<false, false>(p, st))
+                              : (x_f32 ? launch_norm<true, true>(p, st) : launch_norm<true, false>(p, st));
+        if (rc) return rc;
+    }
+    return CDM_OK;
+}
+
 }  // namespace
 
 extern "C" int32_t cdm_adaln_rmsnorm_bf16(const void* x, const void* w, const float* shift, const float* scale,
                                           void* y, int64_t n_tokens, int64_t d, float eps, void* stream) {
-    int32_t rc = check_norm_args(x, w, y, n_tokens, d, shift, scale);
-    if (rc) return rc;
-    if ((rc = cdm_require_device())) return rc;
-    if (n_tokens == 0) return CDM_OK;
-    return launch_norm<false, false>(x, w, shift, scale, y, nullptr, n_tokens, d, eps, (hipStream_t)stream);
+    const int64_t start = 0;
+    return norm_runs(x, false, &w, &shift, &scale, &start, &n_tokens, 1, y, nullptr, d, eps, stream);
 }
 
 extern "C" int32_t cdm_adaln_rmsnorm_f32(const float* x, const void* w, const float* shift, const float* scale,
                                          void* y, int64_t n_tokens, int64_t d, float eps, void* stream) {
-    int32_t rc = check_norm_args(x, w, y, n_tokens, d, shift, scale);
-    if (rc) return rc;
-    if ((rc = cdm_require_device())) return rc;
-    if (n_tokens == 0) return CDM_OK;
-    return launch_norm<false, true>(x, w, shift, scale, y, nullptr, n_tokens, d, eps, (hipStream_t)stream);
+    const int64_t start = 0;
+    return norm_runs(x, true, &w, &shift, &scale, &start, &n_tokens, 1, y, nullptr, d, eps, stream);
 }
 
 extern "C" int32_t cdm_adaln_rmsnorm_quant_e4m3(const void* x, const void* w, const float* shift,
                                                 const float* scale, void* yq, float* s_tok, int64_t n_tokens,
                                                 int64_t d, float eps, void* stream) {
-    int32_t rc = check_norm_args(x, w, yq, n_tokens, d, shift, scale);
-    if (rc) return rc;
+    const int64_t start = 0;
     CDM_REQUIRE(s_tok, CDM_ERR_BAD_ARG, "adaln_rmsnorm_quant: null s_tok");
-    if ((rc = cdm_require_device())) return rc;
-    if (n_tokens == 0) return CDM_OK;
-    return launch_norm<true, false>(x, w, shift, scale, yq, s_tok, n_tokens, d, eps, (hipStream_t)stream);
+    return norm_runs(x, false, &w, &shift, &scale, &start, &n_tokens, 1, yq, s_tok, d, eps, stream);
 }
 
 extern "C" int32_t cdm_adaln_rmsnorm_f32_quant_e4m3(const float* x, const void* w, const float* shift,
                                                     const float* scale, void* yq, float* s_tok, int64_t n_tokens,
                                                     int64_t d, float eps, void* stream) {
-    int32_t rc = check_norm_args(x, w, yq, n_tokens, d, shift, scale);
-    if (rc) return rc;
+    const int64_t start = 0;
     CDM_REQUIRE(s_tok, CDM_ERR_BAD_ARG, "adaln_rmsnorm_quant: null s_tok");
-    if ((rc = cdm_require_device())) return rc;
-    if (n_tokens == 0) return CDM_OK;
-    return launch_norm<true, true>(x, w, shift, scale, yq, s_tok, n_tokens, d, eps, (hipStream_t)stream);
+    return norm_runs(x, true, &w, &shift, &scale, &start, &n_tokens, 1, yq, s_tok, d, eps, stream);
+}
+
+extern "C" int32_t cdm_adaln_rmsnorm_grouped(const void* x, int32_t x_is_f32, const void* const* w, const float* const* shift,
+                                             const float* const* scale, const int64_t* seg_start, const int64_t* seg_len,
+                                             int32_t n_seg, void* y, float* s_tok, int64_t d, float eps, void* stream) {
+    CDM_REQUIRE(w && seg_start && seg_len && n_seg >= 0 && n_seg <= 64, CDM_ERR_BAD_ARG, "adaln_rmsnorm_grouped: bad token runs");
+    return norm_runs(x, x_is_f32 != 0, w, shift, scale, seg_start, seg_len, n_seg, y, s_tok, d, eps, stream);
 }
 
 extern "C" int32_t cdm_quant_rows_e4m3(const void* a, int64_t lda, void* q, float* s, int64_t rows, int64_t cols,

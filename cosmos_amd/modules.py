@@ -10,7 +10,6 @@ Per-branch ("Mixture-of-Transformers") weights: branch b of a layer owns
     attn.out_weight[b]  = to_add_out (DM) / to_out (AR)
     norm1_weight[b], norm2_weight[b], gate_weight[b], up_weight[b], down_weight[b] = the branch's norms and MLP
 (parameter names as in transformers models/cosmos3_omni/modeling_cosmos3_omni.py:39-60).
-Only timestep conditioning (a one-row MLP) is left to torch ops.
 """
 from __future__ import annotations
 
@@ -401,6 +400,21 @@ def _routed_linear(a, sa, weights, qweights, weights2, segments, *, out, epilogu
                          head_dim=head_dim, out=out, row_amax=row_amax)
 
 
+def _modulations(blocks: Sequence["DMBlock"], temb: torch.Tensor) -> List[Tuple[torch.Tensor, ...]]:
+    """(shift1, scale1, gate1, shift2, scale2, gate2), each [d] fp32, of every block: one launch over all of them."""
+    lins = [b.adaLN_modulation for b in blocks]
+    if not lins:
+        return []
+    w = lins[0].weight
+    if w.is_cuda and all(l.weight.dtype == torch.bfloat16 and l.weight.is_contiguous() and l.bias is not None and
+                         l.weight.shape == w.shape for l in lins):
+        m = ops.adaln_modulation(temb.reshape(-1).to(torch.float32), [l.weight for l in lins], [l.bias for l in lins])
+    else:      # other parameter types: the layer itself
+        m = torch.stack([l(torch.nn.functional.silu(temb.reshape(1, -1).to(l.weight.dtype))).float().reshape(-1) for l in lins])
+    rows = m.view(6 * len(lins), -1).unbind(0)
+    return [rows[6 * i:6 * i + 6] for i in range(len(lins))]
+
+
 class DMBlock(nn.Module):
     """One Mixture-of-Transformers layer (generator side)."""
 
@@ -441,24 +455,16 @@ class DMBlock(nn.Module):
 
     def modulation(self, temb: torch.Tensor) -> Tuple[torch.Tensor, ...]:
         """(shift1, scale1, gate1, shift2, scale2, gate2), each [d] fp32, from the conditioning vector."""
-        c = temb.reshape(1, -1).to(self.adaLN_modulation.weight.dtype)
-        m = self.adaLN_modulation(torch.nn.functional.silu(c)).float().reshape(-1)
-        return tuple(t.contiguous() for t in m.chunk(6))
+        return _modulations([self], temb)[0]
 
     def _norm(self, x, weights, shift, scale, segments, ws):
         """Per-branch adaLN-RMSNorm of x (bf16 or fp32) into the workspace: y (bf16), or (e4m3, per-token scale) for
         the fp8 variant."""
-        if not self.fp8:
-            y = ws.y
-            for (s0, ln, b, modulated) in segments:
-                ops.adaln_rmsnorm(x[s0:s0 + ln], weights[b], shift if modulated else None, scale if modulated else None,
-                                  self.eps, out=y[s0:s0 + ln])
-            return y, None
-        yq, st = ws.yq, ws.ys
-        for (s0, ln, b, modulated) in segments:
-            ops.adaln_rmsnorm_quant(x[s0:s0 + ln], weights[b], shift if modulated else None,
-                                    scale if modulated else None, self.eps, out_q=yq[s0:s0 + ln], out_s=st[s0:s0 + ln])
-        return yq, st
+        y, st = (ws.yq, ws.ys) if self.fp8 else (ws.y, None)
+        ops.adaln_rmsnorm_grouped(x, [weights[b] for (_, _, b, _) in segments], [shift if m else None for (_, _, _, m) in segments],
+                                  [scale if m else None for (_, _, _, m) in segments], [(s0, ln) for (s0, ln, _, _) in segments],
+                                  self.eps, y, st)
+        return y, st
 
     def forward(self, hidden_states: torch.Tensor, temb: torch.Tensor,
                 image_rotary_emb: Tuple[torch.Tensor, torch.Tensor],
@@ -499,7 +505,7 @@ class DMBlock(nn.Module):
 
 
 class TimestepEmbedder(nn.Module):
-    """256-d sinusoidal embedding of t -> Linear -> SiLU -> Linear (stays in torch: a one-row MLP)."""
+    """256-d sinusoidal embedding of t -> Linear -> SiLU -> Linear (the one-row MLP stays in torch)."""
 
     def __init__(self, d_model: int, freq_dim: int = 256, device=None, dtype=torch.float32):
         super().__init__()
@@ -509,6 +515,8 @@ class TimestepEmbedder(nn.Module):
 
     def sinusoid(self, t: torch.Tensor) -> torch.Tensor:
         half = self.freq_dim // 2
+        if t.is_cuda and self.freq_dim % 2 == 0:
+            return ops.timestep_sinusoid(t.reshape(-1).to(torch.float32).contiguous(), self.freq_dim)
         k = torch.arange(half, dtype=torch.float32, device=t.device)
         f = torch.exp(-math.log(10000.0) * k / half)
         a = t.to(torch.float32).reshape(-1, 1) * f.reshape(1, -1)
@@ -588,9 +596,7 @@ class DMStack(nn.Module):
             raise RuntimeError("context reuse needs the hybrid mask (DMConfig.hybrid_mask)")
         if c.n_text == 0:
             raise ValueError("context reuse needs a text run")
-        x = self._stream(_as2d(encoder_hidden_states))
-        if x.shape != (c.n_text, c.d_model):
-            raise ValueError(f"context has shape {tuple(x.shape)}, expected {(c.n_text, c.d_model)}")
+        x = self._stream([_as2d(encoder_hidden_states)], c.n_text, "context")
         cos, sin = self.rotary(x.device)
         rot = (cos[:c.n_text].contiguous(), sin[:c.n_text].contiguous())
         segs = [(0, c.n_text, 0, False)]
@@ -627,16 +633,15 @@ class DMStack(nn.Module):
             parts.append(_as2d(encoder_hidden_states))
         parts.append(_as2d(hidden_states))
         parts += self._generator_extras(audio_states, action_states)
-        x = self._stream(torch.cat(parts, dim=0) if len(parts) > 1 else parts[0])
-        if x.shape != (c.n_tokens, c.d_model):
-            raise ValueError(f"joint sequence has shape {tuple(x.shape)}, expected {(c.n_tokens, c.d_model)}")
+        x = self._stream(parts, c.n_tokens, "joint")
         rot = self.rotary(x.device)
         segs = self.segments()
         temb = self.time_embedder(timestep.reshape(-1)[:1])
         if self._ws is None or not self._ws.fits(c.n_tokens, c.d_model, c.hidden, c.fp8) or self._ws.y.device != x.device:
             self._ws = Workspace(c.n_tokens, c.d_model, c.hidden, c.n_heads, c.head_dim, x.device, c.kv_heads, c.fp8)
-        for blk in self.blocks:
-            blk(x, temb, rot, segs, inplace=True, workspace=self._ws, causal_prefix=c.n_text if c.hybrid_mask else 0)
+        for blk, mod in zip(self.blocks, _modulations(self.blocks, temb)):
+            blk(x, temb, rot, segs, inplace=True, modulation=mod, workspace=self._ws,
+                causal_prefix=c.n_text if c.hybrid_mask else 0)
         return self._result(x, c.n_text, hidden_states.dim() == 3, return_dict)
 
     def capture(self, hidden_states: torch.Tensor, timestep: torch.Tensor,
@@ -650,10 +655,19 @@ class DMStack(nn.Module):
                                        encoder_hidden_states=encoder_hidden_states, action_states=action_states,
                                        audio_states=audio_states), context_cache)
 
-    def _stream(self, x: torch.Tensor) -> torch.Tensor:
-        """A private, contiguous copy of the joint sequence in the dtype the residual stream is kept in."""
-        dt = torch.float32 if self.cfg.residual_fp32 else torch.bfloat16
-        return x.to(dt).contiguous() if x.dtype != dt else x.contiguous().clone()
+    def _stream(self, parts: Sequence[torch.Tensor], n: int, what: str) -> torch.Tensor:
+        """A private, contiguous copy of the sequence (its runs joined) in the dtype the residual stream is kept in: one
+        converting copy per run."""
+        d = self.cfg.d_model
+        rows = sum(p.shape[0] for p in parts)
+        if rows != n or any(p.dim() != 2 or p.shape[1] != d for p in parts):
+            raise ValueError(f"{what} sequence has shape {(rows, *parts[0].shape[1:])}, expected {(n, d)}")
+        x = torch.empty((n, d), dtype=torch.float32 if self.cfg.residual_fp32 else torch.bfloat16, device=parts[0].device)
+        at = 0
+        for p in parts:
+            x[at:at + p.shape[0]].copy_(p)
+            at += p.shape[0]
+        return x
 
     def _result(self, x: torch.Tensor, first_video: int, batched: bool, return_dict: bool):
         """The video rows of the final stream as bf16 (the transformer's output dtype); "joint" is the stream itself."""
@@ -681,10 +695,8 @@ class DMStack(nn.Module):
         if cache.n_tokens != P or len(cache.images) != len(self.blocks):
             raise ValueError("context cache does not belong to this stack")
         parts = [_as2d(hidden_states)] + self._generator_extras(audio_states, action_states)
-        x = self._stream(torch.cat(parts, dim=0) if len(parts) > 1 else parts[0])
         n = c.n_tokens - P
-        if x.shape != (n, c.d_model):
-            raise ValueError(f"generator sequence has shape {tuple(x.shape)}, expected {(n, c.d_model)}")
+        x = self._stream(parts, n, "generator")
         if self._rot_gen is None or self._rot_gen[0].device != x.device:
             cos, sin = self.rotary(x.device)
             self._rot_gen = (cos[P:].contiguous(), sin[P:].contiguous())
@@ -692,8 +704,8 @@ class DMStack(nn.Module):
         temb = self.time_embedder(timestep.reshape(-1)[:1])
         if self._ws_gen is None or not self._ws_gen.fits(n, c.d_model, c.hidden, c.fp8) or self._ws_gen.y.device != x.device:
             self._ws_gen = Workspace(n, c.d_model, c.hidden, c.n_heads, c.head_dim, x.device, c.kv_heads, c.fp8)
-        for blk, img in zip(self.blocks, cache.images):
-            blk(x, temb, self._rot_gen, segs, inplace=True, workspace=self._ws_gen, prefix=(img, P))
+        for blk, img, mod in zip(self.blocks, cache.images, _modulations(self.blocks, temb)):
+            blk(x, temb, self._rot_gen, segs, inplace=True, modulation=mod, workspace=self._ws_gen, prefix=(img, P))
         return self._result(x, 0, hidden_states.dim() == 3, return_dict)
 
 

@@ -135,6 +135,31 @@ def adaln_rmsnorm_quant(x, w, shift=None, scale=None, eps: float = 1e-6, out_q: 
     return yq, s
 
 
+@_timed("norm")
+def adaln_rmsnorm_grouped(x: torch.Tensor, ws: Sequence[torch.Tensor], shifts: Sequence[Optional[torch.Tensor]],
+                          scales: Sequence[Optional[torch.Tensor]], segments: Sequence[Tuple[int, int]], eps: float,
+                          out: torch.Tensor, out_s: Optional[torch.Tensor] = None) -> None:
+    """``adaln_rmsnorm`` (or, with ``out_s``, ``adaln_rmsnorm_quant``) of the token runs [start, start + len) of x, each with
+    its own weights and modulation, in one launch; ``out`` [n, d] bf16 (e4m3 with ``out_s`` [n] fp32)."""
+    lib = _lib.load()
+    n, d = x.shape
+    f32 = x.dtype == torch.float32
+    if not x.is_contiguous() or not out.is_contiguous() or out.shape != x.shape or (out_s is not None and out_s.shape != (n,)):
+        raise ValueError("x and out must be contiguous [n, d], out_s [n]")
+    if any(s < 0 or l < 0 or s + l > n for s, l in segments):
+        raise ValueError("token run outside x")
+    k = len(segments)
+    PP, I64 = C.c_void_p * k, C.c_int64 * k
+    rc = lib.cdm_adaln_rmsnorm_grouped(_chk(x, "x", x.dtype if f32 else torch.bfloat16, 2), int(f32),
+                                       PP(*[_chk(w, "w", torch.bfloat16, 1) for w in ws]),
+                                       PP(*[_f32vec(t, "shift", d) or None for t in shifts]),
+                                       PP(*[_f32vec(t, "scale", d) or None for t in scales]),
+                                       I64(*[s for s, _ in segments]), I64(*[l for _, l in segments]), k,
+                                       _chk(out, "out", torch.bfloat16 if out_s is None else FP8_DTYPE, 2),
+                                       _chk(out_s, "out_s", torch.float32, 1) or None, d, float(eps), _stream())
+    _lib.check(rc, "cdm_adaln_rmsnorm_grouped")
+
+
 @_timed("quant")
 def quant_rows(a: torch.Tensor, out_q: Optional[torch.Tensor] = None,
                out_s: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -547,6 +572,35 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, n_heads: int, h
     # two-stage form: prefix images, or HIP events around the attention kernel alone while timing is on
     attention_pack_kv(k, v, n_kv_heads, head_dim, workspace, cos, sin, qk_norm)
     return attention_packed(q, workspace, n_heads, head_dim, out, cos, sin, qk_norm, prefix, causal_prefix, n_kv_heads)
+
+
+# ----------------------------------------------------------------------------- conditioning
+@_timed("cond")
+def timestep_sinusoid(t: torch.Tensor, freq_dim: int) -> torch.Tensor:
+    """[n, freq_dim] fp32: [cos | sin](t f_k) of n timesteps, f_k = 10000^(-k / (freq_dim / 2))."""
+    lib = _lib.load()
+    n = t.numel()
+    out = torch.empty((n, freq_dim), dtype=torch.float32, device=t.device)
+    rc = lib.cdm_timestep_sinusoid_f32(_f32vec(t, "t", n), out.data_ptr(), n, freq_dim, _stream())
+    _lib.check(rc, "cdm_timestep_sinusoid_f32")
+    return out
+
+
+@_timed("cond")
+def adaln_modulation(c: torch.Tensor, ws: Sequence[torch.Tensor], bs: Sequence[torch.Tensor]) -> torch.Tensor:
+    """[n_blocks, n_out] fp32: the modulation vectors w silu(c) + b of every block in one launch; ``c`` [d] fp32 (any
+    shape of d elements), ``ws[l]`` [n_out, d] bf16, ``bs[l]`` [n_out] bf16."""
+    lib = _lib.load()
+    n_out, d = ws[0].shape
+    if any(w.shape != ws[0].shape or not w.is_contiguous() for w in ws) or any(b.shape != (n_out,) for b in bs) or len(bs) != len(ws):
+        raise ValueError("modulation weights must be contiguous and share one shape [n_out, d], biases [n_out]")
+    PP = C.c_void_p * len(ws)
+    out = torch.empty((len(ws), n_out), dtype=torch.float32, device=c.device)
+    rc = lib.cdm_adaln_modulation_bf16(_f32vec(c, "c", d), PP(*[_chk(w, "w", torch.bfloat16, 2) for w in ws]),
+                                       PP(*[_chk(b, "b", torch.bfloat16, 1) for b in bs]), len(ws), out.data_ptr(), d, n_out,
+                                       _stream())
+    _lib.check(rc, "cdm_adaln_modulation_bf16")
+    return out
 
 
 @_timed("step")

@@ -92,6 +92,15 @@ int32_t cdm_adaln_rmsnorm_f32_quant_e4m3(const float* x, const void* w, const fl
                                          void* stream);      /* x fp32 */
 
 /*
+ * The norms above over the token runs of a joint sequence in one launch: rows [seg_start[g], seg_start[g] + seg_len[g]) of x
+ * use w[g], shift[g], scale[g] (shift / scale: null arrays or null entries = un-modulated).  x_is_f32: x holds fp32 rows;
+ * s_tok null: y is bf16, else y is e4m3 and s_tok[row] receives the row's scale.
+ */
+int32_t cdm_adaln_rmsnorm_grouped(const void* x, int32_t x_is_f32, const void* const* w, const float* const* shift,
+                                  const float* const* scale, const int64_t* seg_start, const int64_t* seg_len, int32_t n_seg,
+                                  void* y, float* s_tok, int64_t d, float eps, void* stream);
+
+/*
  * Per-row dynamic e4m3 quantisation of a bf16 matrix (activations before a quantised linear):
  *   s[i] = max_j |a[i,j]| / 448 (0 -> 1);  q[i,j] = e4m3(a[i,j] / s[i]).  cols % 8 == 0, cols <= 32768.
  * Also used offline for weights W[out, in] (per-output-channel scales).
@@ -275,6 +284,21 @@ int32_t cdm_attn_fwd_static_bf16(const void* q, int64_t ldq, const void* k, int6
  */
 int32_t cdm_linear_bias_bf16(const void* A, int64_t lda, const void* W, int64_t ldw, const void* bias, void* C,
                              int64_t ldc, int64_t M, int64_t N, int64_t K, void* stream);
+
+/*
+ * Sinusoidal embedding ahead of the time_embedder's MLP (parameter names: transformers
+ * models/cosmos3_omni/modeling_cosmos3_omni.py:50): out[i] = [cos | sin](t[i] f_k), f_k = 10000^(-k / (freq_dim / 2)).
+ * t: [n] fp32; out: [n, freq_dim] fp32.
+ */
+int32_t cdm_timestep_sinusoid_f32(const float* t, float* out, int64_t n, int64_t freq_dim, void* stream);
+
+/*
+ * adaLN modulation vectors of n_blocks blocks at once - replaces SiLU + nn.Linear(d, 6 d) of each block's modulation:
+ *   out[l] = W_l silu(c) + b_l, rounded to bf16 where the bf16 linear layer rounds (c, silu(c), the result), fp32 sums.
+ *   c: [d] fp32; w[l]: [n_out, d] bf16 row-major, b[l]: [n_out] bf16; out: [n_blocks, n_out] fp32.
+ */
+int32_t cdm_adaln_modulation_bf16(const float* c, const void* const* w, const void* const* b, int32_t n_blocks, float* out,
+                                  int64_t d, int64_t n_out, void* stream);
 
 /*
  * Mixture-of-Transformers routed linear: contiguous token segments, one weight set each

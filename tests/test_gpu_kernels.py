@@ -53,6 +53,54 @@ def test_adaln_rmsnorm_fp32_stream(n, d):
     assert torch.equal(q1.view(torch.uint8), q2.view(torch.uint8)) and torch.equal(s1, s2)
 
 
+@pytest.mark.parametrize("xdt,quant", [(torch.float32, False), (torch.bfloat16, False), (torch.float32, True), (torch.bfloat16, True)])
+def test_adaln_rmsnorm_grouped_equals_the_single_runs(xdt, quant):
+    """Ten token runs (more than one launch holds), empty ones and gaps among them: the bits of one call per run."""
+    g = gen(77)
+    d, lens = 1168, [3, 0, 64, 1, 130, 7, 2, 5, 1, 40]
+    segs, at = [], 2
+    for n in lens:
+        segs.append((at, n)); at += n + (1 if n == 64 else 0)
+    x = torch.randn((at, d), generator=g).to(dev(), xdt)
+    vec = lambda: torch.randn(d, generator=g).to(dev())
+    ws = [torch.randn(d, generator=g).to(dev(), torch.bfloat16) for _ in segs]
+    sh, sc = [vec() if i % 3 else None for i in range(10)], [vec() if i % 3 else None for i in range(10)]
+    out = torch.zeros((at, d), dtype=ops.FP8_DTYPE if quant else torch.bfloat16, device=dev())
+    ref, s, s_ref = torch.zeros_like(out), torch.zeros(at, device=dev()), torch.zeros(at, device=dev())
+    ops.adaln_rmsnorm_grouped(x, ws, sh, sc, segs, 1e-6, out, s if quant else None)
+    for (s0, n), w, a, b in zip(segs, ws, sh, sc):
+        if n and quant:
+            ops.adaln_rmsnorm_quant(x[s0:s0 + n], w, a, b, 1e-6, out_q=ref[s0:s0 + n], out_s=s_ref[s0:s0 + n])
+        elif n:
+            ops.adaln_rmsnorm(x[s0:s0 + n], w, a, b, 1e-6, out=ref[s0:s0 + n])
+    assert torch.equal(out.view(torch.uint8), ref.view(torch.uint8)) and torch.equal(s, s_ref)
+
+
+@pytest.mark.parametrize("d,n_out,L", [(64, 384, 1), (1024, 6144, 3), (520, 13, 70)])
+def test_adaln_modulation(d, n_out, L):
+    """All blocks' modulation vectors in one call (70 blocks: two launches) against the fp64 product of the rounded
+    activation.  The result is rounded once to bf16: at most half a unit in the last place, 2^-8 of it, plus fp32 sums."""
+    g = gen(d)
+    c = torch.randn(d, generator=g)
+    ws = [(torch.randn((n_out, d), generator=g) * 0.05).to(torch.bfloat16) for _ in range(L)]
+    bs = [torch.randn(n_out, generator=g).to(torch.bfloat16) for _ in range(L)]
+    got = ops.adaln_modulation(c.to(dev()), [w.to(dev()) for w in ws], [b.to(dev()) for b in bs]).cpu()
+    s = torch.nn.functional.silu(c.to(torch.bfloat16)).double()
+    for l in range(L):
+        want = ws[l].double() @ s + bs[l].double()
+        assert bool(((got[l].double() - want).abs() <= want.abs() * 2.0 ** -8 + 1e-5).all())
+
+
+@pytest.mark.parametrize("freq", [2, 256, 600])
+def test_timestep_sinusoid(freq):
+    t = torch.tensor([0.0, 1.5, 999.9])
+    got = ops.timestep_sinusoid(t.to(dev()), freq).cpu()
+    k = torch.arange(freq // 2, dtype=torch.float64)
+    a = t.double()[:, None] * torch.exp(-math.log(10000.0) * k / (freq // 2))
+    # the fp32 angle (up to 1000) carries a relative error of a few 2^-24
+    assert bool(((got.double() - torch.cat([a.cos(), a.sin()], -1)).abs() <= a.abs().amax() * 2.0 ** -22 + 1e-6).all())
+
+
 def test_adaln_rmsnorm_closed_form():
     d = 512
     x = torch.full((3, d), 2.5, dtype=torch.bfloat16, device=dev())
