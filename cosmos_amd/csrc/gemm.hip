@@ -764,12 +764,46 @@ struct HostSeg {
     const float* gate; const float* sw; const float* sw2; const float* knw;
 };
 
-// Launches the segments kMaxSeg at a time (one grid per batch).  p holds everything that is common to the segments.
+// One launch over the segments in p.
 template <bool FP8>
-int32_t run(GemmParams p, const HostSeg* segs, int n_seg, int64_t N, int32_t epilogue, hipStream_t st, const char* who) {
-    // variant 0 = the rule of pick_tile; cross-check build only: 1 = two-stage pipeline, four waves, 32 x 32 MFMAs; 2 = the
-    // ring kernel for every size, 3 - 7 = one of the small tiles for every size
-    const bool ring = cdm_get_variant(1) != 1;
+int32_t launch(GemmParams& p, TileShape shape, int32_t epilogue, hipStream_t st, const char* who) {
+    if (shape.tm != BM || shape.tn != BN) {
+        int32_t rc = launch_tile(p, epilogue, FP8, shape, st);
+        return rc ? rc : cdm_check_launch(who);
+    }
+    const int tile_n = epilogue == CDM_EPI_SWIGLU ? BN / 2 : BN;
+    p.tiles_n = (p.N + tile_n - 1) / tile_n;
+    p.total_tiles = 0;
+    for (int k = 0; k < p.n_seg; ++k) {
+        p.seg[k].tiles_m = (p.seg[k].m_end - p.seg[k].m_start + BM - 1) / BM;
+        p.total_tiles += p.seg[k].tiles_m * p.tiles_n;
+        p.seg[k].tile_end = p.total_tiles;
+    }
+    const int grid = ((p.total_tiles + 7) / 8) * 8;
+#ifdef CDM_CROSSCHECK
+#define CDM_LAUNCH(E)                                                                          \
+    if (cdm_get_variant(1) != 1) gemm_ring_kernel<E, FP8><<<grid, 512, 0, st>>>(p);            \
+    else gemm_kernel<E, FP8><<<grid, kThreads, 0, st>>>(p)
+#else
+#define CDM_LAUNCH(E) gemm_ring_kernel<E, FP8><<<grid, 512, 0, st>>>(p)
+#endif
+    switch (epilogue) {
+        case CDM_EPI_NONE: CDM_LAUNCH(CDM_EPI_NONE); break;
+        case CDM_EPI_SWIGLU: CDM_LAUNCH(CDM_EPI_SWIGLU); break;
+        case CDM_EPI_GATE_RESIDUAL: CDM_LAUNCH(CDM_EPI_GATE_RESIDUAL); break;
+        case CDM_EPI_GATE_RESIDUAL_F32: CDM_LAUNCH(CDM_EPI_GATE_RESIDUAL_F32); break;
+        case CDM_EPI_QKV_PACK: gemm_ring_kernel<CDM_EPI_QKV_PACK, FP8><<<grid, 512, 0, st>>>(p); break;   // ring only
+        default: CDM_LAUNCH(CDM_EPI_ROPE_QK); break;
+    }
+#undef CDM_LAUNCH
+    return cdm_check_launch(who);
+}
+
+// Launches the segments kMaxSeg at a time.  p holds everything that is common to the segments.
+// variant 0 = the rule of plan_gemm; cross-check build only: 1 = two-stage pipeline, four waves, 32 x 32 MFMAs; 2 = the ring
+// kernel for every size, 3 - 7 = one of the small tiles for every size
+template <bool FP8>
+int32_t run(GemmParams p, const HostSeg* segs, int n_seg, int32_t epilogue, hipStream_t st, const char* who) {
     int i = 0;
     while (i < n_seg) {
         int ns = 0;
@@ -782,40 +816,25 @@ int32_t run(GemmParams p, const HostSeg* segs, int n_seg, int64_t N, int32_t epi
         }
         if (ns == 0) break;
         p.n_seg = ns;
-        const TileShape shape = ring ? pick_tile(p, epilogue, FP8) : TileShape{BM, BN, 4, 2};
-        if (shape.tm != BM || shape.tn != BN) {
-            int32_t rc = launch_tile(p, epilogue, FP8, shape, st);
-            if (rc || (rc = cdm_check_launch(who))) return rc;
+        const GemmPlan plan = cdm_get_variant(1) == 1 ? GemmPlan{1, -1, {{BM, BN, 4, 2}, {}}} : plan_gemm(p, epilogue, FP8);
+        int32_t rc;
+        if (plan.parts == 1) {
+            if ((rc = launch<FP8>(p, plan.shape[0], epilogue, st, who))) return rc;
             continue;
         }
-        const int tile_n = epilogue == CDM_EPI_SWIGLU ? BN / 2 : BN;
-        p.tiles_n = (int)((N + tile_n - 1) / tile_n);
-        int total = 0;
+        GemmParams head = p, tail = p;
+        head.n_seg = tail.n_seg = 0;
+        int left = plan.row_tiles;
         for (int k = 0; k < ns; ++k) {
-            p.seg[k].tiles_m = (p.seg[k].m_end - p.seg[k].m_start + BM - 1) / BM;
-            total += p.seg[k].tiles_m * p.tiles_n;
-            p.seg[k].tile_end = total;
+            const GemmSeg& g = p.seg[k];
+            const int t = (g.m_end - g.m_start + BM - 1) / BM, take = t < left ? t : left;
+            const int cut = take == t ? g.m_end : g.m_start + take * BM;
+            left -= take;
+            if (cut > g.m_start) { head.seg[head.n_seg] = g; head.seg[head.n_seg++].m_end = cut; }
+            if (cut < g.m_end) { tail.seg[tail.n_seg] = g; tail.seg[tail.n_seg++].m_start = cut; }
         }
-        p.total_tiles = total;
-        const int grid = ((total + 7) / 8) * 8;
-#ifdef CDM_CROSSCHECK
-#define CDM_LAUNCH(E)                                                         \
-    if (ring) gemm_ring_kernel<E, FP8><<<grid, 512, 0, st>>>(p);            \
-    else gemm_kernel<E, FP8><<<grid, kThreads, 0, st>>>(p)
-#else
-#define CDM_LAUNCH(E) gemm_ring_kernel<E, FP8><<<grid, 512, 0, st>>>(p)
-#endif
-        switch (epilogue) {
-            case CDM_EPI_NONE: CDM_LAUNCH(CDM_EPI_NONE); break;
-            case CDM_EPI_SWIGLU: CDM_LAUNCH(CDM_EPI_SWIGLU); break;
-            case CDM_EPI_GATE_RESIDUAL: CDM_LAUNCH(CDM_EPI_GATE_RESIDUAL); break;
-            case CDM_EPI_GATE_RESIDUAL_F32: CDM_LAUNCH(CDM_EPI_GATE_RESIDUAL_F32); break;
-            case CDM_EPI_QKV_PACK: gemm_ring_kernel<CDM_EPI_QKV_PACK, FP8><<<grid, 512, 0, st>>>(p); break;   // ring only
-            default: CDM_LAUNCH(CDM_EPI_ROPE_QK); break;
-        }
-#undef CDM_LAUNCH
-        int32_t rc = cdm_check_launch(who);
-        if (rc) return rc;
+        if ((rc = launch<FP8>(head, plan.shape[0], epilogue, st, who))) return rc;
+        if ((rc = launch<FP8>(tail, plan.shape[1], epilogue, st, who))) return rc;
     }
     return CDM_OK;
 }
@@ -879,7 +898,7 @@ int32_t grouped(const char* who, const void* A, int64_t lda, const float* sa, co
         p.kp = pack->kp; p.vp = pack->vp; p.kmax = pack->kmax;
         p.d_q = pack->d_q; p.d_kv = pack->d_kv; p.n_key_tiles = pack->n_key_tiles; p.k_eps = pack->k_eps;
     }
-    return run<FP8>(p, segs, n_seg, N, epilogue, (hipStream_t)stream, who);
+    return run<FP8>(p, segs, n_seg, epilogue, (hipStream_t)stream, who);
 }
 
 // QKV projection whose K and V columns leave as the attention kernel's tile images (see the header for the contract)

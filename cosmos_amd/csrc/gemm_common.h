@@ -109,10 +109,15 @@ __device__ __forceinline__ uint2 pack4_bf16(float a, float b, float c, float d) 
     return make_uint2(pack_bf16x2(a, b), pack_bf16x2(c, d));
 }
 
-// The kernels for launches too small for 256 x 256 tiles (gemm_tile.hip): shapes of their output tile, chosen by
-// pick_tile, and the launcher.  p holds everything but the tile counts.
-struct TileShape { int tm, tn, wm, wn; };
-TileShape pick_tile(const GemmParams& p, int epilogue, bool fp8);      // {256, 256} = the ring kernel
+// The kernels for launches too small for 256 x 256 tiles (gemm_tile.hip), the rule that chooses between the shapes, and the
+// launcher.  p holds everything but the tile counts.
+struct TileShape { int tm, tn, wm, wn; };      // {256, 256}: the ring kernel
+struct GemmPlan {
+    int parts;             // launches: 1, or 2 = the first `row_tiles` 256-row tiles of the segments in shape[0], the rest in shape[1]
+    int row_tiles;
+    TileShape shape[2];
+};
+GemmPlan plan_gemm(const GemmParams& p, int epilogue, bool fp8);
 int32_t launch_tile(GemmParams& p, int epilogue, bool fp8, TileShape shape, hipStream_t st);
 
 }  // namespace cdm_gemm

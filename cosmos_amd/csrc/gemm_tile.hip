@@ -468,45 +468,85 @@ int32_t launch_epi(const GemmParams& p, TileShape s, int grid, hipStream_t st) {
 
 }  // namespace
 
-namespace cdm_gemm {
+namespace {
 
-// The shape with the least estimated time.  A round of 256 workgroups (one per CU; the 32 x 32 tile fits twice) takes a fixed
-// part - prologue latency, spreading the accumulators, epilogue - plus one slope per 128-byte k-tile, measured with weights
-// that no cache holds, in us:
-//     tile       fixed  per k-tile  example (M = 512, N = 4096, K = 16384, bf16: us, at the 256 x 256 tile 287)
-//     256 x 256   18    1.05 on up to half the CUs, 1.37 on all (power and L2)
-//     128 x 256   10    0.82        211
-//     128 x 128    7    0.53        142
-//      64 x 128    5    0.40        113
-//      64 x 64     4.5  0.25        138 (two rounds)
-//      32 x 32     4.5  0.14        220 (eight tiles per CU)
+// Estimated time of a launch of n tiles, in us.  A round of 256 workgroups (one per CU; the 32 x 32 tile fits twice) takes a
+// fixed part - prologue latency, spreading the accumulators, epilogue - plus one slope per 128-byte k-tile; a last round on
+// up to half the CUs runs at the slope on the left (power, L2), and its fixed part half overlaps the round before it.
+// Measured with weights that no cache holds:
+//     tile       fixed  per k-tile   example (M = 512, N = 4096, K = 16384, bf16: us, at the 256 x 256 tile 287)
+//     256 x 256   18    1.08 / 1.37
+//     128 x 256   10    0.64 / 0.84  211
+//     128 x 128    7    0.50 / 0.53  142
+//      64 x 128    5    0.40         113
+//      64 x 64     4.5  0.25         138 (two rounds)
+//      32 x 32     4.5  0.14         220 (eight tiles per CU)
 // e4m3 k-tiles take the same time (twice the elements per 128 bytes at twice the matrix rate).
-TileShape pick_tile(const GemmParams& p, int epilogue, bool fp8) {
-    static const struct { TileShape s; double fixed, per_kt; } kShapes[] = {
-        {{128, 256, 2, 4}, 10.0, 0.82}, {{128, 128, 4, 2}, 7.0, 0.53}, {{64, 128, 2, 4}, 5.0, 0.40},
-        {{64, 64, 2, 4}, 4.5, 0.25},    {{32, 32, 2, 2}, 4.5, 0.14}};
-    const int v = cdm_get_variant(1);
-    if (v == 2) return TileShape{256, 256, 4, 2};      // cross-check build: one shape for everything
-    if (v > 2) return kShapes[(v - 3) % 5].s;
+struct ShapeCost { TileShape s; double fixed, half, full; };
+const ShapeCost kShapes[] = {{{256, 256, 4, 2}, 18.0, 1.08, 1.37}, {{128, 256, 2, 4}, 10.0, 0.64, 0.84},
+                             {{128, 128, 4, 2}, 7.0, 0.50, 0.53},  {{64, 128, 2, 4}, 5.0, 0.40, 0.40},
+                             {{64, 64, 2, 4}, 4.5, 0.25, 0.25},    {{32, 32, 2, 2}, 4.5, 0.14, 0.26}};
+
+double estimate(const ShapeCost& c, int64_t n, double kt) {
+    const int64_t cap = c.s.tm == 32 ? 512 : 256, full = n / cap, rest = n % cap;
+    double us = (double)full * (c.fixed + kt * c.full);
+    if (rest > 0) {
+        const double f = rest <= cap / 2 ? 0.0 : rest >= 3 * cap / 4 ? 1.0 : (double)(rest - cap / 2) / (cap / 4);
+        us += (full > 0 ? 0.5 : 1.0) * c.fixed + kt * (c.half + f * (c.full - c.half));
+    }
+    return us;
+}
+
+struct Best { TileShape s; double us; };
+Best best_shape(const int64_t* rows, int n_seg, int64_t N, double kt, int epilogue) {
     const bool narrow = epilogue == CDM_EPI_NONE || epilogue == CDM_EPI_GATE_RESIDUAL || epilogue == CDM_EPI_GATE_RESIDUAL_F32;
-    const double kt = p.K / (fp8 ? 128.0 : 64.0);
-    auto tiles = [&](int tm, int tn) {
-        const int64_t cols = epilogue == CDM_EPI_SWIGLU ? tn / 2 : tn;
-        int64_t rows = 0;
-        for (int i = 0; i < p.n_seg; ++i) rows += (p.seg[i].m_end - p.seg[i].m_start + tm - 1) / tm;
-        return rows * ((p.N + cols - 1) / cols);
-    };
-    const int64_t big = tiles(256, 256);
-    TileShape best{256, 256, 4, 2};
-    double best_us = (double)((big + 255) / 256) * (18.0 + kt * (big <= 128 ? 1.05 : 1.37));
-    for (const auto& k : kShapes) {
-        if (k.s.tn < 128 && !narrow) continue;
-        const int64_t n = tiles(k.s.tm, k.s.tn);
-        const double us = k.s.tm == 32 ? (n <= 256 ? k.fixed + kt * k.per_kt : (double)((n + 511) / 512) * (k.fixed + kt * 0.26))
-                                       : (double)((n + 255) / 256) * (k.fixed + kt * k.per_kt);
-        if (us < best_us) { best_us = us; best = k.s; }
+    Best best{kShapes[0].s, 1e30};
+    for (const ShapeCost& c : kShapes) {
+        if (c.s.tn < 128 && !narrow) continue;
+        const int64_t cols = epilogue == CDM_EPI_SWIGLU ? c.s.tn / 2 : c.s.tn;
+        int64_t n = 0;
+        for (int i = 0; i < n_seg; ++i) n += (rows[i] + c.s.tm - 1) / c.s.tm;
+        const double us = estimate(c, n * ((N + cols - 1) / cols), kt);
+        if (us < best.us) best = Best{c.s, us};
     }
     return best;
+}
+
+}  // namespace
+
+namespace cdm_gemm {
+
+// How a launch is cut: one shape for all of it, or - where 256 x 256 tiles end in a poorly filled round - whole rounds of
+// those tiles and a second launch for the rows behind them in the shape that suits it.  N = 4096, one launch of 256 x 256
+// tiles against the cut: M = 4352 (1.06 rounds) 184 -> 141 us at K = 4096, 667 -> 459 at K = 16384; M = 9000 (2.25) 295 ->
+// 264 and 1043 -> 907; M = 14080 (3.44) 427 -> 414 and 1453 -> 1381; M = 11000 (2.69) keeps one launch.
+// The second launch costs about 5 us of its own (it starts when the first has drained).
+GemmPlan plan_gemm(const GemmParams& p, int epilogue, bool fp8) {
+    const int v = cdm_get_variant(1);
+    if (v >= 2) return GemmPlan{1, -1, {kShapes[(v - 2) % 6].s, {}}};      // cross-check build: one shape for everything
+    const double kt = p.K / (fp8 ? 128.0 : 64.0);
+    int64_t rows[kMaxSeg];
+    int64_t tm = 0;                                                         // row tiles of 256
+    for (int i = 0; i < p.n_seg; ++i) {
+        rows[i] = p.seg[i].m_end - p.seg[i].m_start;
+        tm += (rows[i] + 255) / 256;
+    }
+    const Best one = best_shape(rows, p.n_seg, p.N, kt, epilogue);
+    GemmPlan plan{1, -1, {one.s, {}}};
+    const int64_t cols = epilogue == CDM_EPI_SWIGLU ? 128 : 256, tn = (p.N + cols - 1) / cols;
+    const int64_t first = tm * tn / 256 * 256 / tn;                         // row tiles of the whole rounds
+    if (first == 0 || first == tm) return plan;
+    int64_t head[kMaxSeg], tail[kMaxSeg], left = first;
+    for (int i = 0; i < p.n_seg; ++i) {
+        const int64_t t = (rows[i] + 255) / 256, take = t < left ? t : left;
+        head[i] = take == t ? rows[i] : take * 256;
+        tail[i] = rows[i] - head[i];
+        left -= take;
+    }
+    const double us = estimate(kShapes[0], first * tn, kt) + best_shape(tail, p.n_seg, p.N, kt, epilogue).us + 5.0;
+    if (us < 0.98 * one.us)
+        plan = GemmPlan{2, (int)first, {kShapes[0].s, best_shape(tail, p.n_seg, p.N, kt, epilogue).s}};
+    return plan;
 }
 
 int32_t launch_tile(GemmParams& p, int epilogue, bool fp8, TileShape s, hipStream_t st) {

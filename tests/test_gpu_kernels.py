@@ -155,7 +155,8 @@ def test_gemm_plain(M, N, K, variant):
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("M,N,K,epi", [(1, 8, 256, "none"), (65, 264, 512, "none"), (129, 1000, 2304, "gate_residual"),
                                        (300, 136, 768, "gate_residual_f32"), (31, 72, 4096, "gate_residual_f32"),
-                                       (77, 200, 256, "swiglu"), (257, 1096, 1280, "swiglu"), (130, 768, 1024, "rope_qk")])
+                                       (77, 200, 256, "swiglu"), (257, 1096, 1280, "swiglu"), (130, 768, 1024, "rope_qk"),
+                                       (2100, 8192, 1024, "none")])      # the last: 288 large tiles, cut behind a whole round
 def test_gemm_small_tiles_equal_the_large_one(M, N, K, epi, fp8, request):
     """Every tile shape adds the products of an output element in the same order, so all of them give the bits of the
     256 x 256 kernel: rows and columns off the tile edges, fewer k-tiles than ring stages, the partial row maxima."""
@@ -205,6 +206,22 @@ def test_gemm_small_tiles_equal_the_large_one(M, N, K, epi, fp8, request):
         assert amax is None or torch.equal(amax, want_amax), f"tile variant {variant}: row maxima"
     ops.set_variant("gemm", 0)
     assert torch.equal(call()[0], want)
+
+
+def test_grouped_gemm_cut_behind_a_whole_round():
+    """Two segments and 9 row tiles x 32 column tiles: the launch is cut behind 8 row tiles, inside the second segment."""
+    g = gen(99)
+    M, N, K, segs = 2150, 8192, 512, [(0, 1000), (1020, 1130)]
+    a, _ = rand_bf16((M, K), g)
+    ws = [rand_bf16((N, K), g, 0.05)[0] for _ in segs]
+    r = torch.randn((M, N), generator=g).to(dev())
+    gates = [None, torch.randn(N, generator=g).to(dev())]
+    out, ref = r.clone(), r.clone()
+    ops.grouped_gemm(a, ws, segs, epilogue="gate_residual", residual=out, gates=gates, out=out)
+    for (s0, ln), w, gt in zip(segs, ws, gates):
+        ops.gemm(a[s0:s0 + ln], w, epilogue="gate_residual", residual=ref[s0:s0 + ln], gate=gt, out=ref[s0:s0 + ln])
+    assert torch.equal(out, ref)
+    assert torch.equal(out[1000:1020], r[1000:1020])
 
 
 @pytest.mark.parametrize("fp8", [False, True])
