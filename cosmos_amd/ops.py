@@ -28,7 +28,9 @@ def _epilogue(name: str, out: torch.Tensor, residual: Optional[torch.Tensor]):
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current HIP stream of the current device (the raw handle: building a ``torch.cuda.Stream`` for it costs more
+    than the rest of a launch)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _chk(t: Optional[torch.Tensor], name: str, dtype=None, ndim: Optional[int] = None) -> int:
@@ -603,6 +605,17 @@ def adaln_modulation(c: torch.Tensor, ws: Sequence[torch.Tensor], bs: Sequence[t
     return out
 
 
+def _flat(t: torch.Tensor, name: str, dtype, n: int) -> int:
+    """Pointer of a contiguous tensor of n elements, whatever its shape."""
+    if t.numel() != n or not t.is_contiguous():
+        raise ValueError(f"{name} must be contiguous with {n} elements")
+    if not t.is_cuda:
+        raise RuntimeError(f"{name} must live on the GPU (the HIP path has no CPU fallback)")
+    if t.dtype != dtype:
+        raise TypeError(f"{name} must be {dtype}, got {t.dtype}")
+    return t.data_ptr()
+
+
 @_timed("step")
 def cfg_multistep(x: torch.Tensor, v_cond: torch.Tensor, v_uncond: Optional[torch.Tensor], guidance: float,
                   coef: Sequence[Sequence[float]], hist: Sequence[torch.Tensor], outs: Sequence[torch.Tensor]) -> None:
@@ -613,18 +626,13 @@ def cfg_multistep(x: torch.Tensor, v_cond: torch.Tensor, v_uncond: Optional[torc
     n = x.numel()
     if not 1 <= len(outs) <= 3 or len(coef) != len(outs) or any(len(r) != 2 + len(hist) for r in coef):
         raise ValueError("coef must have one row of 2 + len(hist) values per output (1..3 outputs)")
-    for t, name, dt in [(x, "x", torch.float32), (v_cond, "v_cond", torch.bfloat16)] + \
-                       ([(v_uncond, "v_uncond", torch.bfloat16)] if v_uncond is not None else []) + \
-                       [(h, "hist", torch.float32) for h in hist] + [(o, "out", torch.float32) for o in outs]:
-        if t.numel() != n or not t.is_contiguous():
-            raise ValueError(f"{name} must be contiguous with {n} elements")
-        _chk(t.reshape(-1), name, dt)
-    hp = (C.c_void_p * max(len(hist), 1))(*[h.data_ptr() for h in hist])
-    op = (C.c_void_p * len(outs))(*[o.data_ptr() for o in outs])
-    flat = [float(c) for row in coef for c in row]
-    cf = (C.c_float * len(flat))(*flat)
-    rc = lib.cdm_cfg_step_f32(x.data_ptr(), v_cond.data_ptr(), v_uncond.data_ptr() if v_uncond is not None else None,
-                              float(guidance), hp, len(hist), cf, op, len(outs), n, _stream())
+    f32, bf16 = torch.float32, torch.bfloat16
+    ptr = lambda t, name, dt: _flat(t, name, dt, n)
+    px, pc, pu = ptr(x, "x", f32), ptr(v_cond, "v_cond", bf16), None if v_uncond is None else ptr(v_uncond, "v_uncond", bf16)
+    hp = (C.c_void_p * max(len(hist), 1))(*[ptr(h, "hist", f32) for h in hist])
+    op = (C.c_void_p * len(outs))(*[ptr(o, "out", f32) for o in outs])
+    cf = (C.c_float * (len(coef) * (2 + len(hist))))(*[float(c) for row in coef for c in row])
+    rc = lib.cdm_cfg_step_f32(px, pc, pu, float(guidance), hp, len(hist), cf, op, len(outs), n, _stream())
     _lib.check(rc, "cdm_cfg_step_f32")
 
 

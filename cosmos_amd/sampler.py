@@ -95,6 +95,9 @@ class _Update:
         if corrector:
             if order == 1:
                 rhos = [0.5]
+            elif order == 2:           # [[1, 1], [rk, 1]] rhos = b (an abscissa at -inf gives rho 0)
+                r = (b[1] - b[0]) / (rks[0] - 1.0)
+                rhos = [r, b[0] - r]
             else:
                 R = np.array([[rk ** (i - 1) for rk in rks] for i in range(1, order + 1)], dtype=np.float64)
                 rhos = list(np.linalg.solve(R, np.array(b, dtype=np.float64)))
@@ -103,9 +106,9 @@ class _Update:
                 rhos = []
             elif order == 2:
                 rhos = [0.5]
-            else:
-                R = np.array([[rk ** (i - 1) for rk in rks[:-1]] for i in range(1, order)], dtype=np.float64)
-                rhos = list(np.linalg.solve(R, np.array(b[:-1], dtype=np.float64)))
+            else:                      # order 3: [[1, 1], [rk0, rk1]] rhos = b
+                r = (b[1] - rks[0] * b[0]) / (rks[1] - rks[0])
+                rhos = [b[0] - r, r]
             rhos = rhos + [0.0]            # no term for a prediction at st
         self.c_x = st / s0
         self.c_old = [-alpha_t * B_h * r * ir for r, ir in zip(rhos[:-1], inv_rk)]
@@ -158,19 +161,15 @@ class UniPCStepper:
         olds = list(reversed(self.m_hist))                     # m_{i-1}, m_{i-2}, ...
         old_sig = list(reversed(self.sig_hist))
         n_old = len(olds)
-        width = 3 + n_old                                       # basis: x, v, last_sample, m_{i-1}, m_{i-2}, ...
-        e = lambda k, c=1.0: [c if j == k else 0.0 for j in range(width)]
-        add = lambda a, b, cb=1.0: [p + cb * q for p, q in zip(a, b)]
-        m_row = add(e(0), e(1), -sigma)                         # m_i = x - sigma v
-        corrected = self.use_corrector and i > 0 and self.last_sample is not None
-        if corrected:
+        # rows over the basis x, v, last_sample, m_{i-1}, m_{i-2}, ...
+        pad = [0.0] * n_old
+        m_row = [1.0, -sigma, 0.0] + pad                        # m_i = x - sigma v
+        if self.use_corrector and i > 0 and self.last_sample is not None:
             u = _Update(sigma, old_sig[0], old_sig[1:self.this_order], True, self.solver_type)
-            xc_row = add(e(2, u.c_x), e(3, u.c_m0))
-            for k, c in enumerate(u.c_old):
-                xc_row = add(xc_row, e(4 + k, c))
-            xc_row = add(xc_row, m_row, u.c_new)
+            xc_row = [u.c_new, -u.c_new * sigma, u.c_x, u.c_m0] + u.c_old
+            xc_row += [0.0] * (3 + n_old - len(xc_row))
         else:
-            xc_row = e(0)
+            xc_row = [1.0, 0.0, 0.0] + pad
         order = min(self.solver_order, n_steps - i) if self.lower_order_final else self.solver_order
         order = min(order, self.lower_order_nums + 1)
         # a kept level at sigma = 1 (lambda = -inf) cannot enter the solved coefficients of order 3
@@ -180,17 +179,18 @@ class UniPCStepper:
             order = 1                                           # the step to sigma = 0 returns the data prediction
         self.this_order = order
         u = _Update(sigma_next, sigma, old_sig[:order - 1], False, self.solver_type)
-        nx_row = add([u.c_x * c for c in xc_row], m_row, u.c_m0)
+        nx_row = [u.c_x * c for c in xc_row]
+        nx_row[0] += u.c_m0
+        nx_row[1] -= u.c_m0 * sigma
         for k, c in enumerate(u.c_old):
-            nx_row = add(nx_row, e(3 + k, c))
+            nx_row[3 + k] += c
         # tensors: inputs (a dummy for the slots that do not exist yet - their coefficients are zero)
         fill = sample
         hist = [self.last_sample if self.last_sample is not None else fill] + olds
         m_new = self._spare.pop() if self._spare else torch.empty_like(sample)
         if self.last_sample is None:
             self.last_sample = torch.empty_like(sample)
-        rows = [[r[0], r[1]] + r[2:] for r in (nx_row, m_row, xc_row)]
-        ops.cfg_multistep(sample, v_cond, v_uncond, self.guidance_scale, rows, hist, [sample, m_new, self.last_sample])
+        ops.cfg_multistep(sample, v_cond, v_uncond, self.guidance_scale, (nx_row, m_row, xc_row), hist, [sample, m_new, self.last_sample])
         self.m_hist.append(m_new)
         self.sig_hist.append(sigma)
         if len(self.m_hist) > self.solver_order:
