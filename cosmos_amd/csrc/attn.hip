@@ -20,7 +20,7 @@
 namespace {
 
 constexpr int BN = 64;       // keys per tile
-constexpr int BMQ = 256;     // query rows per workgroup
+constexpr int BMQ = 256;     // query rows per workgroup (the smaller form for small grids: 128)
 constexpr int KB = BN / 16;  // 16-key blocks per tile
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
@@ -311,10 +311,12 @@ constexpr float kSafeLog2 = 60.0f;      // largest excess over the reference tha
 constexpr int kMaxKm = 2048;            // key tiles that get a decision of their own (131,072 keys); longer sequences: one per head
 constexpr int kMaxSplit = 8;            // most key ranges a query block of the last round is split into
 
-template <int HD, int QS, bool LATE>
+// NW = waves per workgroup.  (The bound is given for eight waves also where four are launched: for a 256-thread workgroup
+// the compiler splits the register file and copies accumulators between its halves.)
+template <int HD, int QS, int NW, bool LATE>
 __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS, 2 / QS))) void attn_fwd_pipe_kernel(
     const PackedParams p) {
-    constexpr int NW = 8 / QS;
+    constexpr int ROWS = NW * 32 * QS;                 // query rows per workgroup
     constexpr int QB = 2 * QS;                         // 16-row query blocks per wave
     constexpr int KS = HD / 32, HB = HD / 16;
     constexpr int TILE_BYTES = BN * HD * 2;            // same for K and V tiles
@@ -357,7 +359,7 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
         if (hi >= hpx || head >= nh) return;
     }
     const int kv_head = head / p.kv_group;
-    const int q0 = qblk * BMQ + wave * (32 * QS);
+    const int q0 = qblk * ROWS + wave * (32 * QS);
 
     // ---- Q fragments: rotate-half mRoPE (if tables are given) and the factor log2(e)/sqrt(HD), both in fp32 and
     // with ONE rounding to bf16.  The lane holds channels 32ks + 8g .. +7 (g = lane / 16) of its query row for every
@@ -382,7 +384,7 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
         const float* km = p.kmax + (int64_t)kv_head * NM - p.n_prefix_tiles + t0;      // indexed by the frame's tile number
         const float* kmp = p.kmax_prefix + (int64_t)kv_head * p.n_prefix_tiles + t0;
         if (per_tile) {
-            for (int i = threadIdx.x; i < kMaxKm; i += 512 / QS) s_km[i] = i >= NT ? 0.0f : (i < NP ? kmp[i] : km[i]);
+            for (int i = threadIdx.x; i < kMaxKm; i += 64 * NW) s_km[i] = i >= NT ? 0.0f : (i < NP ? kmp[i] : km[i]);
         } else {
             for (int i = lane; i < NT; i += 64) kmax_all = fmaxf(kmax_all, i < NP ? kmp[i] : km[i]);
             kmax_all = wave_max(kmax_all);
@@ -485,7 +487,7 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
     const int last_valid = n_keys - (NT - 1) * BN;
     // per-row key limit and the tiles this workgroup needs: a query block inside the causal prefix stops at its
     // own last row, and every tile it visits is masked per row
-    const int b0 = qblk * BMQ;
+    const int b0 = qblk * ROWS;
     const bool causal_wg = b0 < p.causal_prefix;
     int klim[QB];
 #pragma unroll
@@ -493,7 +495,7 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
         const int qrow = q0 + qb * 16 + r16;
         klim[qb] = qrow < p.causal_prefix ? qrow + 1 : n_keys;
     }
-    const int kmax = (causal_wg && b0 + BMQ <= p.causal_prefix) ? (b0 + BMQ < n_keys ? b0 + BMQ : n_keys) : n_keys;
+    const int kmax = (causal_wg && b0 + ROWS <= p.causal_prefix) ? (b0 + ROWS < n_keys ? b0 + ROWS : n_keys) : n_keys;
     const int NTW = (kmax + BN - 1) / BN;
     const uint32_t lane_off = (uint32_t)(wave * 1024 + lane * 16);
     // tile t of the key sequence [prefix tiles | main tiles] lives at pre + t * TILE_BYTES (t < NP) or at
@@ -587,7 +589,7 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
     // VALU-heavy block the other is in its MFMA block.  Such a wave reads K(j+1) and the first fragments of V(j)
     // before barrier j: both tiles are complete at barrier j - 1 (neither is the most recently issued group there),
     // and their slots are not refilled before barrier j + 1.
-    const bool late_sync = QS == 1 && wave >= 4;
+    const bool late_sync = NW == 8 && wave >= 4;
 #define CDM_ATTN_STEP(SCUR, SNEXT)                                                                              \
     {                                                                                                           \
         const int k_fill = ks_cur;                              /* slot of K(j)   == j % 3     */               \
@@ -993,16 +995,25 @@ extern "C" int32_t cdm_attn_fwd_packed_bf16(const void* q, int64_t ldq, const fl
     const float mant = frexpf(full, &ex);                 // full = mant * 2^ex, mant in [0.5, 1)
     p.scale_log2e = late ? ldexpf(1.0f, ex - 1) : full;
     p.late_r = late ? 2.0f * mant : 1.0f;
-    p.n_qblocks = (int)((n_tokens + BMQ - 1) / BMQ);
     // 1-D grid of 8 x ceil(heads / 8) x query blocks ids: id % 8 = XCD, see the kernel's placement rule
     // variant 0 = 32 query rows per wave (8 waves, two per SIMD), row maxima dropped where the norm bound allows;
-    // cross-check build only: 1 = 64 query rows per wave (4 waves), 2 = variant 0 with the row maxima always taken
+    // cross-check build only: 1 = 64 query rows per wave (4 waves), 2 = variant 0 with the row maxima always taken, 3 =
+    // 128-row workgroups and 4 = 256-row workgroups whatever the grid
     const int variant = cdm_get_variant(0);
+    // Small grids: 128-row workgroups of four waves (same arithmetic per row, bit-equal).  A wave then has its SIMD to
+    // itself and nothing runs under its exponentials, so such a workgroup takes 0.7 of the time of one with twice the
+    // rows; it pays where the larger ones would leave half of an XCD's 32 CUs idle, i.e. up to 16 per XCD.  Measured,
+    // 256-row against 128-row workgroups: 32 heads x 128, 512 keys 23.2 -> 17.4 us, 1024 keys (16 per XCD) 34.6 -> 27.2, 2048
+    // keys (32 per XCD) 64.6 against 84.8; 16 heads x 64, 1024 keys 21.8 -> 17.3, 4096 keys (32 per XCD) equal.
+    const int64_t per_xcd = (n_heads + 7) / 8 * ((n_tokens + BMQ - 1) / BMQ);
+    const bool half_blocks = variant == 3 || ((variant == 0 || variant == 2) && per_xcd <= 16);
+    const int rows_wg = half_blocks ? BMQ / 2 : BMQ;
+    p.n_qblocks = (int)((n_tokens + rows_wg - 1) / rows_wg);
     p.always_max = variant == 2;
     // the last round's query blocks by key range, if the caller brought the scratch memory for it
     p.split = 1; p.split_tail = 0; p.part_o = nullptr; p.part_lse = nullptr;
     const SplitPlan plan = split_plan(n_tokens, n_heads, head_dim, causal_prefix);
-    if (split_scratch != nullptr && plan.split > 1 && split_scratch_bytes >= plan.bytes && variant != 1) {
+    if (split_scratch != nullptr && plan.split > 1 && split_scratch_bytes >= plan.bytes && variant != 1 && !half_blocks) {
         p.split = plan.split; p.split_tail = plan.tail;
         p.part_o = (bf16_t*)split_scratch;
         p.part_lse = (float*)((char*)split_scratch + 8ll * plan.tail * plan.split * BMQ * head_dim * 2);
@@ -1011,16 +1022,17 @@ extern "C" int32_t cdm_attn_fwd_packed_bf16(const void* q, int64_t ldq, const fl
     CDM_REQUIRE(nwg < (1ll << 31), CDM_ERR_BAD_SHAPE, "attn_fwd_packed: grid too large");
     dim3 grid((unsigned)nwg);
     hipStream_t st = (hipStream_t)stream;
-#define CDM_ATTN_LAUNCH(QS_, THREADS)                                                                      \
-    if (head_dim == 128 && late) attn_fwd_pipe_kernel<128, QS_, true><<<grid, THREADS, 0, st>>>(p);       \
-    else if (head_dim == 128) attn_fwd_pipe_kernel<128, QS_, false><<<grid, THREADS, 0, st>>>(p);         \
-    else if (late) attn_fwd_pipe_kernel<64, QS_, true><<<grid, THREADS, 0, st>>>(p);                      \
-    else attn_fwd_pipe_kernel<64, QS_, false><<<grid, THREADS, 0, st>>>(p)
+#define CDM_ATTN_LAUNCH(QS_, NW_)                                                                                     \
+    if (head_dim == 128 && late) attn_fwd_pipe_kernel<128, QS_, NW_, true><<<grid, 64 * NW_, 0, st>>>(p);            \
+    else if (head_dim == 128) attn_fwd_pipe_kernel<128, QS_, NW_, false><<<grid, 64 * NW_, 0, st>>>(p);              \
+    else if (late) attn_fwd_pipe_kernel<64, QS_, NW_, true><<<grid, 64 * NW_, 0, st>>>(p);                           \
+    else attn_fwd_pipe_kernel<64, QS_, NW_, false><<<grid, 64 * NW_, 0, st>>>(p)
 #ifdef CDM_CROSSCHECK
-    if (variant == 1) { CDM_ATTN_LAUNCH(2, 256); }
+    if (variant == 1) { CDM_ATTN_LAUNCH(2, 4); }
     else
 #endif
-    { CDM_ATTN_LAUNCH(1, 512); }
+    if (half_blocks) { CDM_ATTN_LAUNCH(1, 4); }
+    else { CDM_ATTN_LAUNCH(1, 8); }
 #undef CDM_ATTN_LAUNCH
     if (p.split > 1) {
         if ((rc = cdm_check_launch("attn_fwd_packed"))) return rc;

@@ -533,6 +533,31 @@ def test_attention_vs_oracle(n, H, hd, variant):
     assert_close(o, want.reshape(n, d), 0.9999, 1e-2, f"attention n={n} H={H} hd={hd} variant={variant}")
 
 
+@pytest.mark.parametrize("n,H,Hkv,hd,P,causal,qkn", [(1, 1, 1, 128, 0, 0, False), (129, 2, 1, 128, 70, 0, True), (500, 3, 3, 64, 0, 190, False),
+                                                     (1000, 8, 2, 128, 0, 0, True), (385, 16, 16, 64, 64, 0, False),
+                                                     (4096, 8, 8, 128, 0, 0, False), (4097, 8, 8, 128, 0, 0, False)])
+def test_attention_128_row_workgroups_equal_the_256_row_ones(n, H, Hkv, hd, P, causal, qkn, request):
+    """Small grids run on workgroups of 128 query rows (the last two sizes lie on either side of the rule): a row's
+    arithmetic does not depend on the workgroup's size, so the bits do not either."""
+    request.addfinalizer(lambda: ops.set_variant("attn", 0))
+    g = gen(n + H)
+    q, _ = rand_bf16((n, H * hd), g)
+    k, _ = rand_bf16((n, Hkv * hd), g, 0.2)
+    v, _ = rand_bf16((n, Hkv * hd), g)
+    cos, sin = torch.rand((n, hd // 2), generator=g).to(dev()), torch.rand((n, hd // 2), generator=g).to(dev())
+    w = torch.randn((1, hd), generator=g).to(dev())
+    norm = (w, w, (n,), 1e-6) if qkn else None
+    img = ops.attention_pack_kv(k, v, Hkv, hd, None, cos, sin, norm)
+    prefix = (ops.attention_pack_kv(k[:P].contiguous(), v[:P].contiguous(), Hkv, hd), P) if P else None
+    res = {}
+    for variant in (4, 3, 0):
+        ops.set_variant("attn", variant)
+        amax = torch.zeros((n, H), device=dev())
+        res[variant] = (ops.attention_packed(q, img, H, hd, None, cos, sin, norm, prefix, causal, Hkv, row_amax=amax), amax)
+    for variant in (3, 0):
+        assert torch.equal(res[variant][0], res[4][0]) and torch.equal(res[variant][1], res[4][1]), f"variant {variant}"
+
+
 @pytest.mark.parametrize("variant", [0, 1])
 @pytest.mark.parametrize("n,H,hd,sections", [(300, 2, 128, (32, 48, 48)), (130, 3, 64, (16, 24, 24))])
 def test_attention_with_rope_in_registers(n, H, hd, sections, variant):
