@@ -62,6 +62,7 @@ SIGNATURES = {
                                         _I64, _P]),
     "cdm_attn_split_scratch_bytes": (_I64, [_I64, _I32, _I32]),
     "cdm_timestep_sinusoid_f32": (_I32, [_P, _P, _I64, _I64, _P]),
+    "cdm_timestep_mlp_f32": (_I32, [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _P]),
     "cdm_adaln_modulation_bf16": (_I32, [_P, C.POINTER(_P), C.POINTER(_P), _I32, _P, _I64, _I64, _P]),
     "cdm_linear_bias_bf16": (_I32, [_P, _I64, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _P]),
     "cdm_grouped_gemm_fp8": (_I32, [_P, _I64, _P, C.POINTER(_P), C.POINTER(_P), _I64, C.POINTER(_P), C.POINTER(_P), _P, _I64,

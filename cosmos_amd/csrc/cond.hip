@@ -1,7 +1,8 @@
 // Conditioning of a forward: the sinusoid of the timestep and the adaLN modulation vectors of every block.
 // The modulation streams one weight matrix per block once (12 d^2 bytes, 201 MB at d = 4096) and is bound by HBM there; at
 // small widths the launches are what counts.  One launch serves all blocks of a stack, where stock operators take ten
-// small ones per block (activation, GEMV, conversion, six copies); the sinusoid is one launch instead of eight.
+// small ones per block (activation, GEMV, conversion, six copies); the timestep's MLP - sinusoid, linear, silu, linear - is
+// two launches instead of fourteen.
 // A wave owns four output rows and reads 16 bytes per lane of each, four deep: 16 KB in flight per wave, 64 KB per CU.
 #include "cdm_common.h"
 
@@ -20,6 +21,41 @@ __global__ __launch_bounds__(256) void timestep_sinusoid_kernel(const float* __r
         const float a = tv * expf(-9.210340371976184f * (float)k / (float)half);      // ln(10000)
         out[(int64_t)blockIdx.x * 2 * half + k] = cosf(a);
         out[(int64_t)blockIdx.x * 2 * half + half + k] = sinf(a);
+    }
+}
+
+// One row through a linear layer in fp32, y = [silu](W x + b) with W [n_out, K]: the two halves of the timestep's MLP.  With
+// FREQ x is not read but built: the sinusoid of t, every workgroup for itself (K cosines and sines cost less than the
+// launch that would share them), and the activation follows.  A wave owns one output row, 16 bytes per lane four deep.
+// Bound by the weights' read (W2: 4 d^2 bytes, 67 MB at d = 4096) or, at small widths, by the launch alone.
+template <bool FREQ>
+__global__ __launch_bounds__(64 * kWaves) void linear_row_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                 const float* __restrict__ b, float* __restrict__ y, int K, int n_out) {
+    extern __shared__ float s[];         // K values
+    if (FREQ) {
+        const float tv = x[0];
+        const int half = K >> 1;
+        for (int k = threadIdx.x; k < half; k += 64 * kWaves) {
+            const float a = tv * expf(-9.210340371976184f * (float)k / (float)half);      // ln(10000)
+            s[k] = cosf(a);
+            s[half + k] = sinf(a);
+        }
+    } else {
+        for (int i = threadIdx.x; i < K >> 2; i += 64 * kWaves) reinterpret_cast<float4*>(s)[i] = reinterpret_cast<const float4*>(x)[i];
+    }
+    const int lane = threadIdx.x & 63, row = blockIdx.x * kWaves + (threadIdx.x >> 6);
+    const float4* wr = reinterpret_cast<const float4*>(w + (int64_t)(row < n_out ? row : n_out - 1) * K);
+    float acc = 0.0f;
+    __syncthreads();
+#pragma unroll 4
+    for (int i = lane; i < K >> 2; i += 64) {
+        const float4 v = wr[i], u = reinterpret_cast<const float4*>(s)[i];
+        acc += v.x * u.x + v.y * u.y + v.z * u.z + v.w * u.w;
+    }
+    acc = wave_sum(acc);
+    if (lane == 0 && row < n_out) {
+        const float v = acc + b[row];
+        y[row] = FREQ ? silu_exact(v) : v;
     }
 }
 
@@ -80,6 +116,22 @@ extern "C" int32_t cdm_timestep_sinusoid_f32(const float* t, float* out, int64_t
     if (rc) return rc;
     timestep_sinusoid_kernel<<<(unsigned)n, 256, 0, (hipStream_t)stream>>>(t, out, (int)(freq_dim / 2));
     return cdm_check_launch("timestep_sinusoid");
+}
+
+extern "C" int32_t cdm_timestep_mlp_f32(const float* t, const float* w1, const float* b1, const float* w2, const float* b2,
+                                        float* hidden, float* out, int64_t freq_dim, int64_t d, void* stream) {
+    CDM_REQUIRE(t && w1 && b1 && w2 && b2 && hidden && out, CDM_ERR_BAD_ARG, "timestep_mlp: null pointer");
+    CDM_REQUIRE(freq_dim > 0 && freq_dim % 4 == 0 && freq_dim <= 16384 && d > 0 && d % 4 == 0 && d <= 16384, CDM_ERR_BAD_SHAPE,
+                "timestep_mlp: freq_dim=%lld and d=%lld must be multiples of 4 up to 16384", (long long)freq_dim, (long long)d);
+    CDM_REQUIRE(cdm_aligned16(w1) && cdm_aligned16(w2) && cdm_aligned16(hidden), CDM_ERR_BAD_ALIGN,
+                "timestep_mlp: weights and hidden must be 16-byte aligned");
+    int32_t rc = cdm_require_device();
+    if (rc) return rc;
+    const unsigned grid = (unsigned)((d + kWaves - 1) / kWaves);
+    linear_row_kernel<true><<<grid, 64 * kWaves, (size_t)freq_dim * 4, (hipStream_t)stream>>>(t, w1, b1, hidden, (int)freq_dim, (int)d);
+    if ((rc = cdm_check_launch("timestep_mlp"))) return rc;
+    linear_row_kernel<false><<<grid, 64 * kWaves, (size_t)d * 4, (hipStream_t)stream>>>(hidden, w2, b2, out, (int)d, (int)d);
+    return cdm_check_launch("timestep_mlp");
 }
 
 extern "C" int32_t cdm_adaln_modulation_bf16(const float* c, const void* const* w, const void* const* b, int32_t n_blocks, float* out,

@@ -400,16 +400,23 @@ def _routed_linear(a, sa, weights, qweights, weights2, segments, *, out, epilogu
                          head_dim=head_dim, out=out, row_amax=row_amax)
 
 
+def _plain(lin: nn.Module, device: torch.device, dtype: torch.dtype) -> bool:
+    """An ``nn.Linear`` with bias as it stands - no subclass, wrapper or hook whose forward a kernel on its parameters would
+    pass by - whose parameters such a kernel can read."""
+    return (type(lin) is nn.Linear and lin.bias is not None and not lin._forward_hooks and not lin._forward_pre_hooks
+            and all(p.device == device and p.dtype == dtype and p.is_contiguous() for p in (lin.weight, lin.bias))
+            and lin.weight.data_ptr() % 16 == 0 and lin.in_features % 8 == 0 and lin.in_features <= 16384)
+
+
 def _modulations(blocks: Sequence["DMBlock"], temb: torch.Tensor) -> List[Tuple[torch.Tensor, ...]]:
     """(shift1, scale1, gate1, shift2, scale2, gate2), each [d] fp32, of every block: one launch over all of them."""
     lins = [b.adaLN_modulation for b in blocks]
     if not lins:
         return []
     w = lins[0].weight
-    if w.is_cuda and all(l.weight.dtype == torch.bfloat16 and l.weight.is_contiguous() and l.bias is not None and
-                         l.weight.shape == w.shape for l in lins):
+    if temb.is_cuda and all(_plain(l, temb.device, torch.bfloat16) and l.weight.shape == w.shape for l in lins):
         m = ops.adaln_modulation(temb.reshape(-1).to(torch.float32), [l.weight for l in lins], [l.bias for l in lins])
-    else:      # other parameter types: the layer itself
+    else:      # other parameter types, wrapped layers: the layer itself
         m = torch.stack([l(torch.nn.functional.silu(temb.reshape(1, -1).to(l.weight.dtype))).float().reshape(-1) for l in lins])
     rows = m.view(6 * len(lins), -1).unbind(0)
     return [rows[6 * i:6 * i + 6] for i in range(len(lins))]
@@ -505,7 +512,8 @@ class DMBlock(nn.Module):
 
 
 class TimestepEmbedder(nn.Module):
-    """256-d sinusoidal embedding of t -> Linear -> SiLU -> Linear (the one-row MLP stays in torch)."""
+    """256-d sinusoidal embedding of t -> Linear -> SiLU -> Linear (one timestep, fp32 parameters: two launches of the HIP
+    kernels; anything else through torch)."""
 
     def __init__(self, d_model: int, freq_dim: int = 256, device=None, dtype=torch.float32):
         super().__init__()
@@ -523,6 +531,11 @@ class TimestepEmbedder(nn.Module):
         return torch.cat([a.cos(), a.sin()], dim=-1)
 
     def forward(self, t: torch.Tensor) -> torch.Tensor:
+        l1, l2 = self.linear_1, self.linear_2
+        if (t.is_cuda and t.numel() == 1 and not torch.is_grad_enabled() and _plain(l1, t.device, torch.float32)
+                and _plain(l2, t.device, torch.float32) and l1.in_features == self.freq_dim
+                and l2.weight.shape == (l1.out_features, l1.out_features)):
+            return ops.timestep_mlp(t.reshape(-1).to(torch.float32), l1.weight, l1.bias, l2.weight, l2.bias)
         e = self.sinusoid(t).to(self.linear_1.weight.dtype)
         return self.linear_2(torch.nn.functional.silu(self.linear_1(e)))
 

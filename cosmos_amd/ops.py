@@ -589,6 +589,21 @@ def timestep_sinusoid(t: torch.Tensor, freq_dim: int) -> torch.Tensor:
 
 
 @_timed("cond")
+def timestep_mlp(t: torch.Tensor, w1: torch.Tensor, b1: torch.Tensor, w2: torch.Tensor, b2: torch.Tensor) -> torch.Tensor:
+    """[1, d] fp32: w2 silu(w1 e + b1) + b2 of one timestep's sinusoid e (``w1`` [d, freq_dim], ``w2`` [d, d], fp32)."""
+    lib = _lib.load()
+    d, freq_dim = w1.shape
+    if w2.shape != (d, d) or not w1.is_contiguous() or not w2.is_contiguous():
+        raise ValueError("timestep MLP weights must be contiguous [d, freq_dim] and [d, d]")
+    f32 = torch.float32
+    both = torch.empty((2, d), dtype=f32, device=w1.device)      # hidden | out
+    rc = lib.cdm_timestep_mlp_f32(_f32vec(t, "t", 1), _chk(w1, "w1", f32, 2), _f32vec(b1, "b1", d), _chk(w2, "w2", f32, 2),
+                                  _f32vec(b2, "b2", d), both.data_ptr(), both.data_ptr() + 4 * d, freq_dim, d, _stream())
+    _lib.check(rc, "cdm_timestep_mlp_f32")
+    return both[1:]
+
+
+@_timed("cond")
 def adaln_modulation(c: torch.Tensor, ws: Sequence[torch.Tensor], bs: Sequence[torch.Tensor]) -> torch.Tensor:
     """[n_blocks, n_out] fp32: the modulation vectors w silu(c) + b of every block in one launch; ``c`` [d] fp32 (any
     shape of d elements), ``ws[l]`` [n_out, d] bf16, ``bs[l]`` [n_out] bf16."""

@@ -293,6 +293,14 @@ int32_t cdm_linear_bias_bf16(const void* A, int64_t lda, const void* W, int64_t 
 int32_t cdm_timestep_sinusoid_f32(const float* t, float* out, int64_t n, int64_t freq_dim, void* stream);
 
 /*
+ * The time_embedder of one timestep, all in fp32: out = W2 silu(W1 e + b1) + b2 with e = the sinusoid above.
+ *   t: [1]; w1: [d, freq_dim], w2: [d, d] row-major, 16-byte aligned; b1, b2, out: [d]; hidden: [d] scratch, 16-byte aligned.
+ *   freq_dim and d are multiples of 4 up to 16384.
+ */
+int32_t cdm_timestep_mlp_f32(const float* t, const float* w1, const float* b1, const float* w2, const float* b2, float* hidden,
+                             float* out, int64_t freq_dim, int64_t d, void* stream);
+
+/*
  * adaLN modulation vectors of n_blocks blocks at once - replaces SiLU + nn.Linear(d, 6 d) of each block's modulation:
  *   out[l] = W_l silu(c) + b_l, rounded to bf16 where the bf16 linear layer rounds (c, silu(c), the result), fp32 sums.
  *   c: [d] fp32; w[l]: [n_out, d] bf16 row-major, b[l]: [n_out] bf16; out: [n_blocks, n_out] fp32.

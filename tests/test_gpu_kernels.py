@@ -112,6 +112,32 @@ def test_adaln_rmsnorm_closed_form():
 
 
 # ------------------------------------------------------------------ mRoPE
+@pytest.mark.parametrize("freq,d", [(256, 1024), (4, 4), (260, 68), (256, 4096)])
+def test_timestep_mlp(freq, d):
+    """Against the same MLP in 64 bits behind the same sinusoid; fp32 sums of up to 4096 terms: 1e-5."""
+    g = torch.Generator().manual_seed(freq + d)
+    w1, b1 = torch.randn(d, freq, generator=g) * 0.05, torch.randn(d, generator=g) * 0.1
+    w2, b2 = torch.randn(d, d, generator=g) * 0.05, torch.randn(d, generator=g) * 0.1
+    t = torch.tensor([731.25])
+    got = ops.timestep_mlp(t.to(dev()), w1.to(dev()), b1.to(dev()), w2.to(dev()), b2.to(dev())).cpu().double()
+    e = ops.timestep_sinusoid(t.to(dev()), freq).cpu().double()
+    want = torch.nn.functional.linear(torch.nn.functional.silu(torch.nn.functional.linear(e, w1.double(), b1.double())), w2.double(), b2.double())
+    assert got.shape == (1, d)
+    assert ((got - want).norm() / want.norm()).item() < 1e-5
+
+
+def test_conditioning_honours_wrapped_layers():
+    """A hook on a conditioning layer takes the layer's own forward: the kernels on its parameters would pass it by."""
+    from cosmos_amd import TimestepEmbedder
+    te = TimestepEmbedder(64, device=dev())
+    t = torch.tensor([3.0], device=dev())
+    with torch.no_grad():
+        plain = te(t)
+        te.linear_2.register_forward_hook(lambda m, i, o: o + 1.0)
+        hooked = te(t)
+    assert torch.allclose(hooked, plain + 1.0, rtol=1e-5, atol=1e-5)      # fp32 sums in two orders
+
+
 @pytest.mark.parametrize("hd,H,sections", [(64, 16, (16, 24, 24)), (128, 4, (32, 48, 48))])
 def test_mrope_standalone(hd, H, sections):
     g = gen(hd)
