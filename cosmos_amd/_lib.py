@@ -45,6 +45,8 @@ SIGNATURES = {
     "cdm_adaln_rmsnorm_f32_quant_e4m3": (_I32, [_P, _P, _P, _P, _P, _P, _I64, _I64, _F32, _P]),
     "cdm_adaln_rmsnorm_grouped": (_I32, [_P, _I32, C.POINTER(_P), C.POINTER(_P), C.POINTER(_P), C.POINTER(_I64), C.POINTER(_I64),
                                          _I32, _P, _P, _I64, _F32, _P]),
+    "cdm_adaln_rmsnorm_join": (_I32, [C.POINTER(_P), _P, C.POINTER(_P), C.POINTER(_P), C.POINTER(_P), C.POINTER(_I64), C.POINTER(_I64),
+                                      _I32, _P, _P, _I64, _F32, _P]),
     "cdm_quant_rows_e4m3": (_I32, [_P, _I64, _P, _P, _I64, _I64, _P]),
     "cdm_quant_rows_from_parts_e4m3": (_I32, [_P, _I64, _P, _I64, _I64, _P, _P, _I64, _I64, _P]),
     "cdm_gemm_bf16": (_I32, [_P, _I64, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I32, _P, _I64, _P, _P, _P, _I64,

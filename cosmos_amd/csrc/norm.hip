@@ -47,20 +47,27 @@ struct NormSeg {
     const uint4* w; const float* shift; const float* scale;
     int64_t start, end;                  // token rows
     int block_end;                       // workgroups of runs 0 .. this one
+    const void* src;                     // Join: the run's own rows (bf16, row 0 = token row `start`)
 };
+enum NormInput { kBf16 = 0, kF32 = 1, kJoin = 2 };
 struct NormParams {
     const void* x; void* y; float* s_tok;
+    float* stream;                       // Join: the fp32 stream the rows are written to
     int d, n_seg; float eps;
     NormSeg seg[kMaxSeg];
 };
 
-// MAXC = chunks of 8 channels per thread (d <= 2048 * MAXC); XF32: the input rows are fp32 instead of bf16
-template <int MAXC, bool QUANT, bool XF32>
+// MAXC = chunks of 8 channels per thread (d <= 2048 * MAXC); IN: bf16 rows, fp32 rows, or bf16 rows of separate runs that are
+// also left behind as the joined fp32 stream.  The last form stands at the head of a stack: it writes 6 and reads 2 bytes per
+// value where a converting copy (2 + 4) and the norm behind it (4 + 2) moved 12.
+template <int MAXC, bool QUANT, int IN>
 __global__ __launch_bounds__(kThreads) void adaln_rmsnorm_kernel(const NormParams p) {
     int si = 0;
     while (si < p.n_seg - 1 && (int)blockIdx.x >= p.seg[si].block_end) ++si;
     const int block0 = si ? p.seg[si - 1].block_end : 0;
-    const void* __restrict__ x = p.x;
+    constexpr bool XF32 = IN == kF32;
+    const void* __restrict__ x = IN == kJoin ? p.seg[si].src : p.x;
+    const int64_t x_row0 = IN == kJoin ? p.seg[si].start : 0;      // token row of x's first row
     const uint4* __restrict__ w = p.seg[si].w;
     const float* __restrict__ shift = p.seg[si].shift;
     const float* __restrict__ scale = p.seg[si].scale;
@@ -105,7 +112,7 @@ __global__ __launch_bounds__(kThreads) void adaln_rmsnorm_kernel(const NormParam
     // XF32 (residual stream kept in fp32): a chunk of 8 channels is 32 bytes of the row instead of 16
     uint4 raw[MAXC][XF32 ? 2 : 1];
     auto fetch = [&](int64_t row) {
-        const uint4* xr = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(x) + row * (int64_t)d * (XF32 ? 4 : 2));
+        const uint4* xr = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(x) + (row - x_row0) * (int64_t)d * (XF32 ? 4 : 2));
 #pragma unroll
         for (int c = 0; c < MAXC; ++c) {
             const int idx = c * kThreads + tid;
@@ -133,6 +140,17 @@ __global__ __launch_bounds__(kThreads) void adaln_rmsnorm_kernel(const NormParam
             for (int i = 0; i < 8; ++i) ss += xv[c][i] * xv[c][i];
         }
         if (row + row_step < n_tokens) fetch(row + row_step);
+        if constexpr (IN == kJoin) {
+            float4* so = reinterpret_cast<float4*>(p.stream + row * d);
+#pragma unroll
+            for (int c = 0; c < MAXC; ++c) {
+                const int idx = c * kThreads + tid;
+                if (idx < nchunk) {
+                    so[2 * idx] = make_float4(xv[c][0], xv[c][1], xv[c][2], xv[c][3]);
+                    so[2 * idx + 1] = make_float4(xv[c][4], xv[c][5], xv[c][6], xv[c][7]);
+                }
+            }
+        }
         ss = block_reduce<false>(ss, slot_sum, par_sum);
         const float r = rsqrtf(ss * inv_d + eps);
         float amax = 0.0f;
@@ -266,7 +284,7 @@ __global__ __launch_bounds__(kThreads) void quant_rows_parts_kernel(const bf16_t
     }
 }
 
-template <bool QUANT, bool XF32>
+template <bool QUANT, int IN>
 int32_t launch_norm(NormParams& p, hipStream_t st) {
     // 64 workgroups per CU's worth of rows in flight: at 56 k rows a workgroup walks over three or four rows.  Measured in
     // the 56,832 x 4096 stack (fp32 rows in, bf16 out): 2048 workgroups 5.37 TB/s, 4096 5.53, 8192 5.63, 16384 5.75, 32768
@@ -281,7 +299,7 @@ int32_t launch_norm(NormParams& p, hipStream_t st) {
         p.seg[i].block_end = (int)grid;
     }
     const int chunks = (p.d / 8 + kThreads - 1) / kThreads;
-#define CDM_NORM_LAUNCH(C) adaln_rmsnorm_kernel<C, QUANT, XF32><<<(unsigned)grid, kThreads, 0, st>>>(p)
+#define CDM_NORM_LAUNCH(C) adaln_rmsnorm_kernel<C, QUANT, IN><<<(unsigned)grid, kThreads, 0, st>>>(p)
     if (chunks <= 1) CDM_NORM_LAUNCH(1);
     else if (chunks == 2) CDM_NORM_LAUNCH(2);
     else CDM_NORM_LAUNCH(4);
@@ -300,29 +318,33 @@ int32_t check_norm_args(const void* x, const void* w, const void* y, int64_t n_t
     return CDM_OK;
 }
 
-// runs [start, start + len) of x / y, kMaxSeg per launch; s_tok != null: e4m3 rows and their scales
-int32_t norm_runs(const void* x, bool x_f32, const void* const* w, const float* const* shift, const float* const* scale,
+// runs [start, start + len) of x / y, kMaxSeg per launch; s_tok != null: e4m3 rows and their scales; kJoin: run i's rows are
+// src[i], x is the stream they are written to
+int32_t norm_runs(const void* const* src, const void* x, NormInput in, const void* const* w, const float* const* shift, const float* const* scale,
                   const int64_t* start, const int64_t* len, int32_t n_seg, void* y, float* s_tok, int64_t d, float eps,
                   void* stream) {
     for (int i = 0; i < n_seg; ++i) {
         int32_t rc = check_norm_args(x, w[i], y, len[i], d, shift ? shift[i] : nullptr, scale ? scale[i] : nullptr);
         if (rc) return rc;
+        CDM_REQUIRE(in != kJoin || len[i] == 0 || (src[i] && cdm_aligned16(src[i])), CDM_ERR_BAD_ALIGN,
+                    "adaln_rmsnorm_join: rows of run %d null or misaligned", i);
         CDM_REQUIRE(start[i] >= 0 && start[i] + len[i] < (1ll << 31), CDM_ERR_BAD_ARG, "adaln_rmsnorm: bad token run %d", i);
     }
     int32_t rc = cdm_require_device();
     if (rc) return rc;
     NormParams p;
-    p.x = x; p.y = y; p.s_tok = s_tok; p.d = (int)d; p.eps = eps;
+    p.x = x; p.stream = in == kJoin ? (float*)x : nullptr; p.y = y; p.s_tok = s_tok; p.d = (int)d; p.eps = eps;
     for (int i = 0; i < n_seg;) {
         p.n_seg = 0;
         for (; i < n_seg && p.n_seg < kMaxSeg; ++i)
             if (len[i] > 0)
                 p.seg[p.n_seg++] = NormSeg{(const uint4*)w[i], shift ? shift[i] : nullptr, scale ? scale[i] : nullptr, start[i],
-                                           start[i] + len[i], 0};
+                                           start[i] + len[i], 0, in == kJoin ? src[i] : nullptr};
         if (p.n_seg == 0) continue;
         hipStream_t st = (hipStream_t)stream;
-        rc = s_tok == nullptr ? (x_f32 ? launch_norm<false, true>(p, st) : launch_norm<false, false>(p, st))
-                              : (x_f32 ? launch_norm<true, true>(p, st) : launch_norm<true, false>(p, st));
+        if (in == kJoin) rc = s_tok == nullptr ? launch_norm<false, kJoin>(p, st) : launch_norm<true, kJoin>(p, st);
+        else if (in == kF32) rc = s_tok == nullptr ? launch_norm<false, kF32>(p, st) : launch_norm<true, kF32>(p, st);
+        else rc = s_tok == nullptr ? launch_norm<false, kBf16>(p, st) : launch_norm<true, kBf16>(p, st);
         if (rc) return rc;
     }
     return CDM_OK;
@@ -333,13 +355,13 @@ int32_t norm_runs(const void* x, bool x_f32, const void* const* w, const float* 
 extern "C" int32_t cdm_adaln_rmsnorm_bf16(const void* x, const void* w, const float* shift, const float* scale,
                                           void* y, int64_t n_tokens, int64_t d, float eps, void* stream) {
     const int64_t start = 0;
-    return norm_runs(x, false, &w, &shift, &scale, &start, &n_tokens, 1, y, nullptr, d, eps, stream);
+    return norm_runs(nullptr, x, kBf16, &w, &shift, &scale, &start, &n_tokens, 1, y, nullptr, d, eps, stream);
 }
 
 extern "C" int32_t cdm_adaln_rmsnorm_f32(const float* x, const void* w, const float* shift, const float* scale,
                                          void* y, int64_t n_tokens, int64_t d, float eps, void* stream) {
     const int64_t start = 0;
-    return norm_runs(x, true, &w, &shift, &scale, &start, &n_tokens, 1, y, nullptr, d, eps, stream);
+    return norm_runs(nullptr, x, kF32, &w, &shift, &scale, &start, &n_tokens, 1, y, nullptr, d, eps, stream);
 }
 
 extern "C" int32_t cdm_adaln_rmsnorm_quant_e4m3(const void* x, const void* w, const float* shift,
@@ -347,7 +369,7 @@ extern "C" int32_t cdm_adaln_rmsnorm_quant_e4m3(const void* x, const void* w, co
                                                 int64_t d, float eps, void* stream) {
     const int64_t start = 0;
     CDM_REQUIRE(s_tok, CDM_ERR_BAD_ARG, "adaln_rmsnorm_quant: null s_tok");
-    return norm_runs(x, false, &w, &shift, &scale, &start, &n_tokens, 1, yq, s_tok, d, eps, stream);
+    return norm_runs(nullptr, x, kBf16, &w, &shift, &scale, &start, &n_tokens, 1, yq, s_tok, d, eps, stream);
 }
 
 extern "C" int32_t cdm_adaln_rmsnorm_f32_quant_e4m3(const float* x, const void* w, const float* shift,
@@ -355,14 +377,21 @@ extern "C" int32_t cdm_adaln_rmsnorm_f32_quant_e4m3(const float* x, const void* 
                                                     int64_t d, float eps, void* stream) {
     const int64_t start = 0;
     CDM_REQUIRE(s_tok, CDM_ERR_BAD_ARG, "adaln_rmsnorm_quant: null s_tok");
-    return norm_runs(x, true, &w, &shift, &scale, &start, &n_tokens, 1, yq, s_tok, d, eps, stream);
+    return norm_runs(nullptr, x, kF32, &w, &shift, &scale, &start, &n_tokens, 1, yq, s_tok, d, eps, stream);
 }
 
 extern "C" int32_t cdm_adaln_rmsnorm_grouped(const void* x, int32_t x_is_f32, const void* const* w, const float* const* shift,
                                              const float* const* scale, const int64_t* seg_start, const int64_t* seg_len,
                                              int32_t n_seg, void* y, float* s_tok, int64_t d, float eps, void* stream) {
     CDM_REQUIRE(w && seg_start && seg_len && n_seg >= 0 && n_seg <= 64, CDM_ERR_BAD_ARG, "adaln_rmsnorm_grouped: bad token runs");
-    return norm_runs(x, x_is_f32 != 0, w, shift, scale, seg_start, seg_len, n_seg, y, s_tok, d, eps, stream);
+    return norm_runs(nullptr, x, x_is_f32 != 0 ? kF32 : kBf16, w, shift, scale, seg_start, seg_len, n_seg, y, s_tok, d, eps, stream);
+}
+
+extern "C" int32_t cdm_adaln_rmsnorm_join(const void* const* src, float* x, const void* const* w, const float* const* shift,
+                                          const float* const* scale, const int64_t* seg_start, const int64_t* seg_len,
+                                          int32_t n_seg, void* y, float* s_tok, int64_t d, float eps, void* stream) {
+    CDM_REQUIRE(src && w && seg_start && seg_len && n_seg >= 0 && n_seg <= 64, CDM_ERR_BAD_ARG, "adaln_rmsnorm_join: bad token runs");
+    return norm_runs(src, x, kJoin, w, shift, scale, seg_start, seg_len, n_seg, y, s_tok, d, eps, stream);
 }
 
 extern "C" int32_t cdm_quant_rows_e4m3(const void* a, int64_t lda, void* q, float* s, int64_t rows, int64_t cols,

@@ -464,22 +464,24 @@ class DMBlock(nn.Module):
         """(shift1, scale1, gate1, shift2, scale2, gate2), each [d] fp32, from the conditioning vector."""
         return _modulations([self], temb)[0]
 
-    def _norm(self, x, weights, shift, scale, segments, ws):
+    def _norm(self, x, weights, shift, scale, segments, ws, sources=None):
         """Per-branch adaLN-RMSNorm of x (bf16 or fp32) into the workspace: y (bf16), or (e4m3, per-token scale) for
-        the fp8 variant."""
+        the fp8 variant.  ``sources``: x is still to be joined from these runs, in the same pass."""
         y, st = (ws.yq, ws.ys) if self.fp8 else (ws.y, None)
         ops.adaln_rmsnorm_grouped(x, [weights[b] for (_, _, b, _) in segments], [shift if m else None for (_, _, _, m) in segments],
                                   [scale if m else None for (_, _, _, m) in segments], [(s0, ln) for (s0, ln, _, _) in segments],
-                                  self.eps, y, st)
+                                  self.eps, y, st, sources)
         return y, st
 
     def forward(self, hidden_states: torch.Tensor, temb: torch.Tensor,
                 image_rotary_emb: Tuple[torch.Tensor, torch.Tensor],
                 modality_segments: Optional[Sequence[Segment]] = None, *, inplace: bool = False,
                 modulation: Optional[Sequence[torch.Tensor]] = None, workspace: Optional[Workspace] = None,
-                causal_prefix: int = 0, prefix=None, kv_images: Optional[torch.Tensor] = None):
+                causal_prefix: int = 0, prefix=None, kv_images: Optional[torch.Tensor] = None,
+                sources: Optional[Sequence[torch.Tensor]] = None):
         """``hidden_states`` [N, d] (or [1, N, d]) is the residual stream, bf16 or fp32; the result has its dtype (a
-        stack keeps the stream in fp32 between blocks: only the operands of the matrix products are bf16)."""
+        stack keeps the stream in fp32 between blocks: only the operands of the matrix products are bf16).  ``sources``
+        (with ``inplace``): the bf16 rows of every segment; the first norm joins them into ``hidden_states``."""
         batched = hidden_states.dim() == 3
         x = _as2d(hidden_states)
         if not inplace:
@@ -494,7 +496,7 @@ class DMBlock(nn.Module):
                 self._ws = ws
         sh1, sc1, g1, sh2, sc2, g2 = modulation if modulation is not None else self.modulation(temb)
 
-        y, sy = self._norm(x, self.norm1_weight, sh1, sc1, segs, ws)
+        y, sy = self._norm(x, self.norm1_weight, sh1, sc1, segs, ws, sources)
         self.attn(y, image_rotary_emb=image_rotary_emb, modality_segments=segs, residual=x, gate=g1, quant_scale=sy,
                   workspace=ws, causal_prefix=causal_prefix, prefix=prefix, kv_images=kv_images)
         y, sy = self._norm(x, self.norm2_weight, sh2, sc2, segs, ws)
@@ -609,7 +611,7 @@ class DMStack(nn.Module):
             raise RuntimeError("context reuse needs the hybrid mask (DMConfig.hybrid_mask)")
         if c.n_text == 0:
             raise ValueError("context reuse needs a text run")
-        x = self._stream([_as2d(encoder_hidden_states)], c.n_text, "context")
+        x, sources = self._stream([_as2d(encoder_hidden_states)], c.n_text, "context")
         cos, sin = self.rotary(x.device)
         rot = (cos[:c.n_text].contiguous(), sin[:c.n_text].contiguous())
         segs = [(0, c.n_text, 0, False)]
@@ -619,7 +621,8 @@ class DMStack(nn.Module):
         for blk in self.blocks:
             img = torch.empty((nbytes,), dtype=torch.uint8, device=x.device)
             blk(x, None, rot, segs, inplace=True, workspace=ws, modulation=(None,) * 6, causal_prefix=c.n_text,
-                kv_images=img)
+                kv_images=img, sources=sources)
+            sources = None
             images.append(img)
         return ContextCache(images, c.n_text)
 
@@ -627,7 +630,8 @@ class DMStack(nn.Module):
     def forward(self, hidden_states: torch.Tensor, timestep: torch.Tensor,
                 encoder_hidden_states: Optional[torch.Tensor] = None, action_states: Optional[torch.Tensor] = None,
                 return_dict: bool = False, context_cache: Optional["ContextCache"] = None,
-                audio_states: Optional[torch.Tensor] = None):
+                audio_states: Optional[torch.Tensor] = None, *, joint_only: bool = False):
+        """``joint_only`` (one sample): {"joint": the final stream} without the bf16 copy of its video rows."""
         c = self.cfg
         batch = _batch_size(hidden_states, 3)
         if batch > 1:
@@ -638,7 +642,7 @@ class DMStack(nn.Module):
                                                       _sample(audio_states, b, 3, batch)),
                                batch, return_dict)
         if context_cache is not None:
-            return self._forward_cached(hidden_states, timestep, action_states, return_dict, context_cache, audio_states)
+            return self._forward_cached(hidden_states, timestep, action_states, return_dict, context_cache, audio_states, joint_only)
         parts = []
         if c.n_text:
             if encoder_hidden_states is None:
@@ -646,7 +650,7 @@ class DMStack(nn.Module):
             parts.append(_as2d(encoder_hidden_states))
         parts.append(_as2d(hidden_states))
         parts += self._generator_extras(audio_states, action_states)
-        x = self._stream(parts, c.n_tokens, "joint")
+        x, sources = self._stream(parts, c.n_tokens, "joint")
         rot = self.rotary(x.device)
         segs = self.segments()
         temb = self.time_embedder(timestep.reshape(-1)[:1])
@@ -654,8 +658,9 @@ class DMStack(nn.Module):
             self._ws = Workspace(c.n_tokens, c.d_model, c.hidden, c.n_heads, c.head_dim, x.device, c.kv_heads, c.fp8)
         for blk, mod in zip(self.blocks, _modulations(self.blocks, temb)):
             blk(x, temb, rot, segs, inplace=True, modulation=mod, workspace=self._ws,
-                causal_prefix=c.n_text if c.hybrid_mask else 0)
-        return self._result(x, c.n_text, hidden_states.dim() == 3, return_dict)
+                causal_prefix=c.n_text if c.hybrid_mask else 0, sources=sources)
+            sources = None
+        return self._result(x, c.n_text, hidden_states.dim() == 3, return_dict, joint_only)
 
     def capture(self, hidden_states: torch.Tensor, timestep: torch.Tensor,
                 encoder_hidden_states: Optional[torch.Tensor] = None, action_states: Optional[torch.Tensor] = None,
@@ -668,22 +673,30 @@ class DMStack(nn.Module):
                                        encoder_hidden_states=encoder_hidden_states, action_states=action_states,
                                        audio_states=audio_states), context_cache)
 
-    def _stream(self, parts: Sequence[torch.Tensor], n: int, what: str) -> torch.Tensor:
-        """A private, contiguous copy of the sequence (its runs joined) in the dtype the residual stream is kept in: one
-        converting copy per run."""
+    def _stream(self, parts: Sequence[torch.Tensor], n: int, what: str):
+        """(stream, sources): a private, contiguous tensor for the sequence (its runs joined) in the dtype the residual stream
+        is kept in.  Where the first block's norm can join the runs as it reads them, it is not filled yet and ``sources``
+        are the runs; otherwise it is filled - one converting copy per run - and ``sources`` is None."""
         d = self.cfg.d_model
         rows = sum(p.shape[0] for p in parts)
         if rows != n or any(p.dim() != 2 or p.shape[1] != d for p in parts):
             raise ValueError(f"{what} sequence has shape {(rows, *parts[0].shape[1:])}, expected {(n, d)}")
         x = torch.empty((n, d), dtype=torch.float32 if self.cfg.residual_fp32 else torch.bfloat16, device=parts[0].device)
+        first = self.blocks[0] if len(self.blocks) else None      # a subclass or a hook may read its input: it gets it filled
+        if (type(first) is DMBlock and not first._forward_pre_hooks and self.cfg.residual_fp32 and x.is_cuda and d % 8 == 0
+                and all(p.dtype == torch.bfloat16 and p.device == x.device and p.is_contiguous() and p.data_ptr() % 16 == 0
+                        for p in parts)):
+            return x, list(parts)
         at = 0
         for p in parts:
             x[at:at + p.shape[0]].copy_(p)
             at += p.shape[0]
-        return x
+        return x, None
 
-    def _result(self, x: torch.Tensor, first_video: int, batched: bool, return_dict: bool):
+    def _result(self, x: torch.Tensor, first_video: int, batched: bool, return_dict: bool, joint_only: bool):
         """The video rows of the final stream as bf16 (the transformer's output dtype); "joint" is the stream itself."""
+        if joint_only:
+            return {"joint": x}
         video = x[first_video:first_video + self.cfg.n_video].to(torch.bfloat16)
         out = video.unsqueeze(0) if batched else video
         if return_dict:
@@ -702,14 +715,14 @@ class DMStack(nn.Module):
         return parts
 
     def _forward_cached(self, hidden_states, timestep, action_states, return_dict, cache: "ContextCache",
-                        audio_states=None):
+                        audio_states=None, joint_only=False):
         c = self.cfg
         P = c.n_text
         if cache.n_tokens != P or len(cache.images) != len(self.blocks):
             raise ValueError("context cache does not belong to this stack")
         parts = [_as2d(hidden_states)] + self._generator_extras(audio_states, action_states)
         n = c.n_tokens - P
-        x = self._stream(parts, n, "generator")
+        x, sources = self._stream(parts, n, "generator")
         if self._rot_gen is None or self._rot_gen[0].device != x.device:
             cos, sin = self.rotary(x.device)
             self._rot_gen = (cos[P:].contiguous(), sin[P:].contiguous())
@@ -718,8 +731,9 @@ class DMStack(nn.Module):
         if self._ws_gen is None or not self._ws_gen.fits(n, c.d_model, c.hidden, c.fp8) or self._ws_gen.y.device != x.device:
             self._ws_gen = Workspace(n, c.d_model, c.hidden, c.n_heads, c.head_dim, x.device, c.kv_heads, c.fp8)
         for blk, img, mod in zip(self.blocks, cache.images, _modulations(self.blocks, temb)):
-            blk(x, temb, self._rot_gen, segs, inplace=True, modulation=mod, workspace=self._ws_gen, prefix=(img, P))
-        return self._result(x, 0, hidden_states.dim() == 3, return_dict)
+            blk(x, temb, self._rot_gen, segs, inplace=True, modulation=mod, workspace=self._ws_gen, prefix=(img, P), sources=sources)
+            sources = None
+        return self._result(x, 0, hidden_states.dim() == 3, return_dict, joint_only)
 
 
 class GraphedStack:
@@ -878,9 +892,11 @@ class DMTransformer(nn.Module):
             if given[name] is None:
                 raise ValueError(f"this configuration expects {name}_states")
             emb[name] = _edge_linear(p_in, _as2d(given[name]).to(dt)) + embed
+        # only the stream is read here (a subclass or a hook sees the whole result)
+        kw = {"joint_only": True} if type(self.stack) is DMStack and not self.stack._forward_hooks else {}
         res = self.stack(tok, timestep, encoder_hidden_states=None if context_cache is not None else encoder_hidden_states,
                          action_states=emb.get("action"), return_dict=True, context_cache=context_cache,
-                         audio_states=emb.get("audio"))
+                         audio_states=emb.get("audio"), **kw)
         joint = res["joint"]            # with a context cache: the generator tokens only
         first = 0 if context_cache is not None else c.n_text
         y = ops.adaln_rmsnorm(joint, self.norm_out.data, None, None, c.eps)

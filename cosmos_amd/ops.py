@@ -140,9 +140,11 @@ def adaln_rmsnorm_quant(x, w, shift=None, scale=None, eps: float = 1e-6, out_q: 
 @_timed("norm")
 def adaln_rmsnorm_grouped(x: torch.Tensor, ws: Sequence[torch.Tensor], shifts: Sequence[Optional[torch.Tensor]],
                           scales: Sequence[Optional[torch.Tensor]], segments: Sequence[Tuple[int, int]], eps: float,
-                          out: torch.Tensor, out_s: Optional[torch.Tensor] = None) -> None:
+                          out: torch.Tensor, out_s: Optional[torch.Tensor] = None,
+                          sources: Optional[Sequence[torch.Tensor]] = None) -> None:
     """``adaln_rmsnorm`` (or, with ``out_s``, ``adaln_rmsnorm_quant``) of the token runs [start, start + len) of x, each with
-    its own weights and modulation, in one launch; ``out`` [n, d] bf16 (e4m3 with ``out_s`` [n] fp32)."""
+    its own weights and modulation, in one launch; ``out`` [n, d] bf16 (e4m3 with ``out_s`` [n] fp32).  With ``sources`` (run
+    g's rows, contiguous [len, d] bf16) x is an fp32 output as well: the runs joined."""
     lib = _lib.load()
     n, d = x.shape
     f32 = x.dtype == torch.float32
@@ -152,13 +154,16 @@ def adaln_rmsnorm_grouped(x: torch.Tensor, ws: Sequence[torch.Tensor], shifts: S
         raise ValueError("token run outside x")
     k = len(segments)
     PP, I64 = C.c_void_p * k, C.c_int64 * k
-    rc = lib.cdm_adaln_rmsnorm_grouped(_chk(x, "x", x.dtype if f32 else torch.bfloat16, 2), int(f32),
-                                       PP(*[_chk(w, "w", torch.bfloat16, 1) for w in ws]),
-                                       PP(*[_f32vec(t, "shift", d) or None for t in shifts]),
-                                       PP(*[_f32vec(t, "scale", d) or None for t in scales]),
-                                       I64(*[s for s, _ in segments]), I64(*[l for _, l in segments]), k,
-                                       _chk(out, "out", torch.bfloat16 if out_s is None else FP8_DTYPE, 2),
-                                       _chk(out_s, "out_s", torch.float32, 1) or None, d, float(eps), _stream())
+    if sources is None:
+        fn, given = lib.cdm_adaln_rmsnorm_grouped, (_chk(x, "x", x.dtype if f32 else torch.bfloat16, 2), int(f32))
+    else:
+        if not f32 or len(sources) != k or any(t.shape != (l, d) or not t.is_contiguous() for t, (_, l) in zip(sources, segments)):
+            raise ValueError("sources must be contiguous [len, d] rows of every run, x fp32")
+        fn, given = lib.cdm_adaln_rmsnorm_join, (PP(*[_chk(t, "source", torch.bfloat16, 2) for t in sources]), _chk(x, "x"))
+    rc = fn(*given, PP(*[_chk(w, "w", torch.bfloat16, 1) for w in ws]), PP(*[_f32vec(t, "shift", d) or None for t in shifts]),
+            PP(*[_f32vec(t, "scale", d) or None for t in scales]), I64(*[s for s, _ in segments]), I64(*[l for _, l in segments]), k,
+            _chk(out, "out", torch.bfloat16 if out_s is None else FP8_DTYPE, 2), _chk(out_s, "out_s", torch.float32, 1) or None, d,
+            float(eps), _stream())
     _lib.check(rc, "cdm_adaln_rmsnorm_grouped")
 
 

@@ -101,6 +101,14 @@ int32_t cdm_adaln_rmsnorm_grouped(const void* x, int32_t x_is_f32, const void* c
                                   void* y, float* s_tok, int64_t d, float eps, void* stream);
 
 /*
+ * The head of a stack: the runs of a joint sequence, run g's rows in src[g] ([seg_len[g], d] bf16, 16-byte aligned), are joined
+ * into the fp32 stream x (rows seg_start[g] ..) and normalised into y / s_tok as above, in one pass.
+ */
+int32_t cdm_adaln_rmsnorm_join(const void* const* src, float* x, const void* const* w, const float* const* shift,
+                               const float* const* scale, const int64_t* seg_start, const int64_t* seg_len, int32_t n_seg,
+                               void* y, float* s_tok, int64_t d, float eps, void* stream);
+
+/*
  * Per-row dynamic e4m3 quantisation of a bf16 matrix (activations before a quantised linear):
  *   s[i] = max_j |a[i,j]| / 448 (0 -> 1);  q[i,j] = e4m3(a[i,j] / s[i]).  cols % 8 == 0, cols <= 32768.
  * Also used offline for weights W[out, in] (per-output-channel scales).

@@ -76,6 +76,45 @@ def test_adaln_rmsnorm_grouped_equals_the_single_runs(xdt, quant):
     assert torch.equal(out.view(torch.uint8), ref.view(torch.uint8)) and torch.equal(s, s_ref)
 
 
+@pytest.mark.parametrize("quant", [False, True])
+@pytest.mark.parametrize("d", [8, 1168, 4096, 8192])
+def test_adaln_rmsnorm_join_equals_copy_and_norm(d, quant):
+    """Runs joined and normalised in one pass: the bits of a converting copy per run and the norm of the joined stream; more
+    runs than one launch holds, an empty one, and enough rows that a workgroup walks over several."""
+    g = gen(d)
+    lens = [3, 0, 64, 1, 130, 7, 2, 5, 1, 20000 if d == 1168 else 40]
+    src = [torch.randn((n, d), generator=g).to(dev(), torch.bfloat16) for n in lens]
+    at = [sum(lens[:i]) for i in range(len(lens))]
+    segs, n = list(zip(at, lens)), sum(lens)
+    vec = lambda: torch.randn(d, generator=g).to(dev())
+    ws = [torch.randn(d, generator=g).to(dev(), torch.bfloat16) for _ in segs]
+    sh, sc = [vec() if i % 3 else None for i in range(10)], [vec() if i % 3 else None for i in range(10)]
+    out = torch.zeros((n, d), dtype=ops.FP8_DTYPE if quant else torch.bfloat16, device=dev())
+    ref, s, s_ref = torch.zeros_like(out), torch.zeros(n, device=dev()), torch.zeros(n, device=dev())
+    x = torch.full((n, d), float("nan"), device=dev())
+    ops.adaln_rmsnorm_grouped(x, ws, sh, sc, segs, 1e-6, out, s if quant else None, src)
+    joined = torch.cat(src).float()
+    ops.adaln_rmsnorm_grouped(joined, ws, sh, sc, segs, 1e-6, ref, s_ref if quant else None)
+    assert torch.equal(x, joined) and torch.equal(out.view(torch.uint8), ref.view(torch.uint8)) and torch.equal(s, s_ref)
+
+
+def test_stack_fills_the_stream_for_hooked_blocks():
+    """A hook ahead of the first block sees the joined runs; results are the same bits either way, as with fp32 inputs."""
+    from cosmos_amd import DMConfig, DMStack
+    cfg = DMConfig("t", 256, 2, 128, 512, 2, (2, 4, 9), n_text=37)
+    st = DMStack(cfg, device=dev())
+    st.reset_parameters(3)
+    g = gen(4)
+    ctx, x = (torch.randn((1, n, 256), generator=g).to(dev(), torch.bfloat16) for n in (37, 72))
+    t = torch.tensor([500.0], device=dev())
+    want = st(x, t, encoder_hidden_states=ctx)[0]
+    assert torch.equal(st(x.float(), t, encoder_hidden_states=ctx)[0], want)
+    seen = []
+    st.blocks[0].register_forward_pre_hook(lambda m, a: seen.append(a[0].clone()))
+    assert torch.equal(st(x, t, encoder_hidden_states=ctx)[0], want)
+    assert torch.equal(seen[0], torch.cat([ctx[0], x[0]]).float())
+
+
 @pytest.mark.parametrize("d,n_out,L", [(64, 384, 1), (1024, 6144, 3), (520, 13, 70)])
 def test_adaln_modulation(d, n_out, L):
     """All blocks' modulation vectors in one call (70 blocks: two launches) against the fp64 product of the rounded
