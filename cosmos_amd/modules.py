@@ -611,7 +611,7 @@ class DMStack(nn.Module):
             raise RuntimeError("context reuse needs the hybrid mask (DMConfig.hybrid_mask)")
         if c.n_text == 0:
             raise ValueError("context reuse needs a text run")
-        x, sources = self._stream([_as2d(encoder_hidden_states)], c.n_text, "context")
+        x, sources = self._joined([_as2d(encoder_hidden_states)], c.n_text, "context")
         cos, sin = self.rotary(x.device)
         rot = (cos[:c.n_text].contiguous(), sin[:c.n_text].contiguous())
         segs = [(0, c.n_text, 0, False)]
@@ -650,7 +650,7 @@ class DMStack(nn.Module):
             parts.append(_as2d(encoder_hidden_states))
         parts.append(_as2d(hidden_states))
         parts += self._generator_extras(audio_states, action_states)
-        x, sources = self._stream(parts, c.n_tokens, "joint")
+        x, sources = self._joined(parts, c.n_tokens, "joint")
         rot = self.rotary(x.device)
         segs = self.segments()
         temb = self.time_embedder(timestep.reshape(-1)[:1])
@@ -673,25 +673,30 @@ class DMStack(nn.Module):
                                        encoder_hidden_states=encoder_hidden_states, action_states=action_states,
                                        audio_states=audio_states), context_cache)
 
-    def _stream(self, parts: Sequence[torch.Tensor], n: int, what: str):
-        """(stream, sources): a private, contiguous tensor for the sequence (its runs joined) in the dtype the residual stream
-        is kept in.  Where the first block's norm can join the runs as it reads them, it is not filled yet and ``sources``
-        are the runs; otherwise it is filled - one converting copy per run - and ``sources`` is None."""
-        d = self.cfg.d_model
-        rows = sum(p.shape[0] for p in parts)
-        if rows != n or any(p.dim() != 2 or p.shape[1] != d for p in parts):
-            raise ValueError(f"{what} sequence has shape {(rows, *parts[0].shape[1:])}, expected {(n, d)}")
-        x = torch.empty((n, d), dtype=torch.float32 if self.cfg.residual_fp32 else torch.bfloat16, device=parts[0].device)
-        first = self.blocks[0] if len(self.blocks) else None      # a subclass or a hook may read its input: it gets it filled
-        if (type(first) is DMBlock and not first._forward_pre_hooks and self.cfg.residual_fp32 and x.is_cuda and d % 8 == 0
-                and all(p.dtype == torch.bfloat16 and p.device == x.device and p.is_contiguous() and p.data_ptr() % 16 == 0
-                        for p in parts)):
-            return x, list(parts)
+    def _stream(self, *parts: torch.Tensor) -> torch.Tensor:
+        """A private, contiguous copy of the joint sequence (its runs, in order) in the dtype the residual stream is kept in:
+        one converting copy per run."""
+        x = torch.empty((sum(p.shape[0] for p in parts), parts[0].shape[1]), device=parts[0].device,
+                        dtype=torch.float32 if self.cfg.residual_fp32 else torch.bfloat16)
         at = 0
         for p in parts:
             x[at:at + p.shape[0]].copy_(p)
             at += p.shape[0]
-        return x, None
+        return x
+
+    def _joined(self, parts: Sequence[torch.Tensor], n: int, what: str):
+        """(stream, sources) of the runs.  Where the first block's norm can join them as it reads them, the stream is not
+        filled yet and ``sources`` are the runs; otherwise it is, and ``sources`` is None."""
+        d = self.cfg.d_model
+        rows = sum(p.shape[0] for p in parts)
+        if rows != n or any(p.dim() != 2 or p.shape[1] != d for p in parts):
+            raise ValueError(f"{what} sequence has shape {(rows, *parts[0].shape[1:])}, expected {(n, d)}")
+        dev = parts[0].device
+        first = self.blocks[0] if len(self.blocks) else None      # a subclass or a hook may read its input: it gets it filled
+        if (type(first) is DMBlock and not first._forward_pre_hooks and self.cfg.residual_fp32 and dev.type == "cuda" and d % 8 == 0
+                and all(p.dtype == torch.bfloat16 and p.device == dev and p.is_contiguous() and p.data_ptr() % 16 == 0 for p in parts)):
+            return torch.empty((n, d), dtype=torch.float32, device=dev), list(parts)
+        return self._stream(*parts), None
 
     def _result(self, x: torch.Tensor, first_video: int, batched: bool, return_dict: bool, joint_only: bool):
         """The video rows of the final stream as bf16 (the transformer's output dtype); "joint" is the stream itself."""
@@ -722,7 +727,7 @@ class DMStack(nn.Module):
             raise ValueError("context cache does not belong to this stack")
         parts = [_as2d(hidden_states)] + self._generator_extras(audio_states, action_states)
         n = c.n_tokens - P
-        x, sources = self._stream(parts, n, "generator")
+        x, sources = self._joined(parts, n, "generator")
         if self._rot_gen is None or self._rot_gen[0].device != x.device:
             cos, sin = self.rotary(x.device)
             self._rot_gen = (cos[P:].contiguous(), sin[P:].contiguous())
