@@ -78,6 +78,9 @@ SIGNATURES = {
     "cdm_grouped_gemm_bf16": (_I32, [_P, _I64, C.POINTER(_P), _I64, C.POINTER(_P), _P, _I64, C.POINTER(_I64),
                                      C.POINTER(_I64), _I32, _I64, _I64, _I32, _P, _I64, C.POINTER(_P), _P, _P, _I64,
                                      _I32, _P]),
+    "cdm_grouped_gemm_scratch_bytes": (_I64, [C.POINTER(_I64), _I32, _I64, _I64, _I32]),
+    "cdm_grouped_gemm_scratch_bf16": (_I32, [_P, _I64, C.POINTER(_P), _I64, _P, _I64, C.POINTER(_I64), C.POINTER(_I64), _I32, _I64,
+                                             _I64, _I32, _P, _I64, C.POINTER(_P), _P, _I64, _P]),
 }
 
 

@@ -803,7 +803,8 @@ int32_t launch(GemmParams& p, TileShape shape, int32_t epilogue, hipStream_t st,
 // variant 0 = the rule of plan_gemm; cross-check build only: 1 = two-stage pipeline, four waves, 32 x 32 MFMAs; 2 = the ring
 // kernel for every size, 3 - 7 = one of the small tiles for every size
 template <bool FP8>
-int32_t run(GemmParams p, const HostSeg* segs, int n_seg, int32_t epilogue, hipStream_t st, const char* who) {
+int32_t run(GemmParams p, const HostSeg* segs, int n_seg, int32_t epilogue, hipStream_t st, const char* who, void* scratch,
+            int64_t scratch_bytes) {
     int i = 0;
     while (i < n_seg) {
         int ns = 0;
@@ -816,8 +817,12 @@ int32_t run(GemmParams p, const HostSeg* segs, int n_seg, int32_t epilogue, hipS
         }
         if (ns == 0) break;
         p.n_seg = ns;
-        const GemmPlan plan = cdm_get_variant(1) == 1 ? GemmPlan{1, -1, {{BM, BN, 4, 2}, {}}} : plan_gemm(p, epilogue, FP8);
+        const GemmPlan plan = cdm_get_variant(1) == 1 ? GemmPlan{1, -1, {{BM, BN, 4, 2}, {}}} : plan_gemm(p, epilogue, FP8, scratch_bytes);
         int32_t rc;
+        if (plan.k_split > 1) {      // several batches of segments use the scratch one after the other: stream order
+            if ((rc = launch_split_k(p, epilogue, plan, scratch, st)) || (rc = cdm_check_launch(who))) return rc;
+            continue;
+        }
         if (plan.parts == 1) {
             if ((rc = launch<FP8>(p, plan.shape[0], epilogue, st, who))) return rc;
             continue;
@@ -846,7 +851,8 @@ int32_t grouped(const char* who, const void* A, int64_t lda, const float* sa, co
                 const int64_t* seg_start, const int64_t* seg_len, int32_t n_seg, int64_t N, int64_t K, int32_t epilogue,
                 const void* R, int64_t ldr, const float* const* gate, const float* cos, const float* sin,
                 int64_t rope_cols, int32_t head_dim, void* stream, const GemmParams* pack = nullptr,
-                const float* k_norm_rows = nullptr, float* row_amax = nullptr, int64_t amax_ld = 0) {
+                const float* k_norm_rows = nullptr, float* row_amax = nullptr, int64_t amax_ld = 0, void* scratch = nullptr,
+                int64_t scratch_bytes = 0) {
     constexpr int esize = FP8 ? 1 : 2;
     CDM_REQUIRE(A && W && C && seg_start && seg_len, CDM_ERR_BAD_ARG, "%s: null pointer", who);
     CDM_REQUIRE((epilogue == CDM_EPI_QKV_PACK) == (pack != nullptr), CDM_ERR_BAD_ARG,
@@ -898,7 +904,7 @@ int32_t grouped(const char* who, const void* A, int64_t lda, const float* sa, co
         p.kp = pack->kp; p.vp = pack->vp; p.kmax = pack->kmax;
         p.d_q = pack->d_q; p.d_kv = pack->d_kv; p.n_key_tiles = pack->n_key_tiles; p.k_eps = pack->k_eps;
     }
-    return run<FP8>(p, segs, n_seg, epilogue, (hipStream_t)stream, who);
+    return run<FP8>(p, segs, n_seg, epilogue, (hipStream_t)stream, who, scratch, scratch ? scratch_bytes : 0);
 }
 
 // QKV projection whose K and V columns leave as the attention kernel's tile images (see the header for the contract)
@@ -1009,6 +1015,34 @@ extern "C" int32_t cdm_grouped_gemm_bf16(const void* A, int64_t lda, const void*
                                          void* stream) {
     return grouped<false>("grouped_gemm_bf16", A, lda, nullptr, W, nullptr, ldw, W2, nullptr, C, ldc, seg_start, seg_len, n_seg,
                           N, K, epilogue, R, ldr, gate, cos, sin, rope_cols, head_dim, stream);
+}
+
+extern "C" int64_t cdm_grouped_gemm_scratch_bytes(const int64_t* seg_len, int32_t n_seg, int64_t N, int64_t K, int32_t epilogue) {
+    if (!seg_len || n_seg < 1 || N <= 0 || K <= 0 || N >= (1ll << 31) || K >= (1ll << 31)) return 0;
+    GemmParams p{};
+    p.N = (int)N; p.K = (int)K;
+    int64_t at = 0;
+    for (int i = 0; i < n_seg; ++i) {
+        if (seg_len[i] < 0 || at + seg_len[i] >= (1ll << 30)) return 0;
+        if (seg_len[i] > 0) {
+            if (p.n_seg == kMaxSeg) return 0;
+            p.seg[p.n_seg].m_start = (int)at; p.seg[p.n_seg++].m_end = (int)(at + seg_len[i]);
+        }
+        at += seg_len[i];
+    }
+    return p.n_seg ? plan_gemm(p, epilogue, false, INT64_MAX).scratch : 0;
+}
+
+extern "C" int32_t cdm_grouped_gemm_scratch_bf16(const void* A, int64_t lda, const void* const* W, int64_t ldw, void* C,
+                                                 int64_t ldc, const int64_t* seg_start, const int64_t* seg_len, int32_t n_seg,
+                                                 int64_t N, int64_t K, int32_t epilogue, const void* R, int64_t ldr,
+                                                 const float* const* gate, void* scratch, int64_t scratch_bytes, void* stream) {
+    const char* who = "grouped_gemm_scratch_bf16";
+    CDM_REQUIRE(epilogue == CDM_EPI_NONE || epilogue == CDM_EPI_GATE_RESIDUAL || epilogue == CDM_EPI_GATE_RESIDUAL_F32, CDM_ERR_UNSUPPORTED,
+                "%s: epilogue %d is never cut along K", who, epilogue);
+    CDM_REQUIRE(cdm_aligned16(scratch) && scratch_bytes >= 0, CDM_ERR_BAD_ALIGN, "%s: scratch must be 16-byte aligned", who);
+    return grouped<false>(who, A, lda, nullptr, W, nullptr, ldw, nullptr, nullptr, C, ldc, seg_start, seg_len, n_seg, N, K, epilogue,
+                          R, ldr, gate, nullptr, nullptr, 0, 0, stream, nullptr, nullptr, nullptr, 0, scratch, scratch_bytes);
 }
 
 extern "C" int32_t cdm_grouped_gemm_fp8(const void* Aq, int64_t lda, const float* sa, const void* const* Wq,

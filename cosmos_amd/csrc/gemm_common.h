@@ -39,6 +39,9 @@ struct GemmParams {
     // CDM_EPI_SWIGLU, optional: [M, amax_ld] fp32, entry (row, c) = largest |output| of the row within output columns
     // 64 c .. 64 c + 63 (as stored): what a per-row quantiser of the output needs, without a pass of its own
     float* row_amax; int64_t amax_ld;
+    // Launches cut along K (gemm_tile.hip): part i of k_split leaves fp32 sums of its k-tiles, [k_split][part_rows][N], row 0 =
+    // token row part_row0
+    float* partial; int k_split, part_rows, part_row0;
     int tiles_n, total_tiles, n_seg;
     GemmSeg seg[kMaxSeg];
 };
@@ -62,11 +65,18 @@ __device__ __forceinline__ T* uniform_ptr(T* ptr) {      // wave-uniform value -
 // tiles, column-major inside the group, so that the 32 tiles an XCD runs at a time share GM A slabs and 32 / GM W slabs
 // in its L2 (256-row tiles: GM = 4 measured best among 2, 3, 4, 6, 8, 16 once the output tiles are stored
 // non-temporally).
-template <int TM, int GM>
+// SPLIT: all tiles once per part of K, part by part (tiles of one part share operand rows, tiles of two parts nothing).
+template <int TM, int GM, bool SPLIT = false>
 __device__ __forceinline__ bool locate_tile(const GemmParams& p, Tile& t) {
-    const int per_xcd = (p.total_tiles + 7) >> 3;
+    const int all = SPLIT ? p.total_tiles * p.k_split : p.total_tiles;
+    const int per_xcd = (all + 7) >> 3;
     int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (logical >= p.total_tiles) return false;
+    if (logical >= all) return false;
+    t.part = 0;
+    if (SPLIT) {
+        t.part = __builtin_amdgcn_readfirstlane(logical / p.total_tiles);
+        logical -= t.part * p.total_tiles;
+    }
     int si = 0;
 #pragma unroll
     for (int i = 0; i < kMaxSeg - 1; ++i) si += (i < p.n_seg - 1 && logical >= p.seg[i].tile_end) ? 1 : 0;
@@ -116,8 +126,12 @@ struct GemmPlan {
     int parts;             // launches: 1, or 2 = the first `row_tiles` 256-row tiles of the segments in shape[0], the rest in shape[1]
     int row_tiles;
     TileShape shape[2];
+    int k_split = 1;       // > 1 (parts == 1): that many ranges of K, and a pass over their sums
+    int64_t scratch = 0;   // bytes that takes
 };
-GemmPlan plan_gemm(const GemmParams& p, int epilogue, bool fp8);
+// scratch_bytes: what the caller brought for a launch cut along K (bf16 operands only)
+GemmPlan plan_gemm(const GemmParams& p, int epilogue, bool fp8, int64_t scratch_bytes);
+int32_t launch_split_k(GemmParams& p, int epilogue, const GemmPlan& plan, void* scratch, hipStream_t st);
 int32_t launch_tile(GemmParams& p, int epilogue, bool fp8, TileShape shape, hipStream_t st);
 
 }  // namespace cdm_gemm

@@ -7,7 +7,8 @@
 // weights in the memory-side cache; a load-only loop over L2-resident rows reaches 110 - 137.  Removing the loads from the
 // 64 x 128 loop takes a third off, removing half of its LDS reads nothing.  So: all the LDS a CU has goes into ring stages
 // (over 100 KB in flight), loads go out one behind every few MFMAs, and the shape is chosen so that every CU has a tile.
-// At M = 512, K = 16384, N = 4096 (bf16, cold weights) the 64 x 128 tile takes 113 us where 32 tiles of 256 x 256 took 287;
+// At M = 512, K = 16384, N = 4096 (bf16, cold weights) the 64 x 128 tile takes 113 us where 32 tiles of 256 x 256 took 287
+// (four ranges of K in 128 x 256 tiles: 82, see best_split);
 // M = 512, N = 12288, K = 4096 (QKV with images): 64 us against 85; M = 64, N = 4096, K = 4096: 14 us against 84.
 //
 // Layout: eight waves (four for the 32 x 32 tile) in a WM x WN grid, v_mfma_f32_16x16x32_bf16 / 16x16x128_f8f6f4, W
@@ -23,6 +24,7 @@ using namespace cdm_gemm;
 namespace {
 
 constexpr int kLds = 160 * 1024;
+constexpr int kMaxSplitK = 8;      // most ranges of K
 
 template <int TM, int TN, int WM, int WN>
 struct Geo {
@@ -158,6 +160,42 @@ __device__ __forceinline__ void pack_piece(const GemmParams& p, const Tile& t, c
     }
 }
 
+constexpr int kPartial = 100;      // "epilogue" of a launch cut along K: the fp32 sums of its k-tiles
+
+// eight finished columns of a row -> C, through the plain or residual epilogues (bf16 epilogues: v is dequantised)
+template <int EPI, bool FP8>
+__device__ __forceinline__ void store8(const GemmParams& p, const float* gate, const float* sw, float sr, int row, int col, float (&v)[8]) {
+    if constexpr (EPI == CDM_EPI_GATE_RESIDUAL_F32) {
+        const float* R = reinterpret_cast<const float*>(p.R) + (int64_t)row * p.ldr + col;
+        float* C = reinterpret_cast<float*>(p.C) + (int64_t)row * p.ldc + col;
+        float r[8], g[8];
+        load8(R, r);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) g[e] = 1.0f;
+        if (gate) load8(gate + col, g);
+        dequant8<FP8>(g, sw, col, sr);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) r[e] = r[e] + g[e] * v[e];
+        *reinterpret_cast<float4*>(C) = make_float4(r[0], r[1], r[2], r[3]);
+        *reinterpret_cast<float4*>(C + 4) = make_float4(r[4], r[5], r[6], r[7]);
+    } else {
+        if constexpr (EPI == CDM_EPI_GATE_RESIDUAL) {
+            const uint4 r4 = *reinterpret_cast<const uint4*>(p.R + (int64_t)row * p.ldr + col);
+            const uint32_t rw[4] = {r4.x, r4.y, r4.z, r4.w};
+            float g[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) g[e] = 1.0f;
+            if (gate) load8(gate + col, g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[2 * e] = bf16lo(rw[e]) + g[2 * e] * v[2 * e];
+                v[2 * e + 1] = bf16hi(rw[e]) + g[2 * e + 1] * v[2 * e + 1];
+            }
+        }
+        *reinterpret_cast<uint4*>(p.C + (int64_t)row * p.ldc + col) = pack8(v);
+    }
+}
+
 template <int EPI, bool FP8, int TM, int TN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tile_kernel(const GemmParams p) {
     using G = Geo<TM, TN, WM, WN>;
@@ -166,7 +204,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
     __shared__ __attribute__((aligned(1024))) char smem[G::SMEM];
 
     Tile tile;
-    if (!locate_tile<TM, 8>(p, tile)) return;
+    if (!locate_tile<TM, 8, EPI == kPartial>(p, tile)) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WN, wn = wave % WN;
@@ -174,6 +212,12 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
     const int n0 = tile.tn * (EPI == CDM_EPI_SWIGLU ? TN / 2 : TN);      // first output column
 
     // ---- load instruction j of this wave covers tile rows 8 (NW j + wave) .. + 7 of [A rows | W rows]
+    int KT = p.K / (FP8 ? 128 : 64), kt0 = 0;
+    if constexpr (EPI == kPartial) {      // this part's k-tiles
+        const int all = KT;
+        kt0 = (int)((int64_t)all * tile.part / p.k_split);
+        KT = (int)((int64_t)all * (tile.part + 1) / p.k_split) - kt0;
+    }
     uint32_t off[L];
     const char* base[L];
 #pragma unroll
@@ -191,7 +235,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
             int bn = EPI == CDM_EPI_SWIGLU ? (wr >> 7) * 64 + (wr & 63) : wr;
             bn = (n0 + bn) < p.N ? bn : p.N - 1 - n0;
             off[j] = (uint32_t)(bn * (int)p.ldw + chunk * 16);
-            base[j] = uniform_ptr(reinterpret_cast<const char*>(up ? tile.W2 : tile.W) + (int64_t)n0 * p.ldw);
+            base[j] = uniform_ptr(reinterpret_cast<const char*>(up ? tile.W2 : tile.W) + (int64_t)n0 * p.ldw + (int64_t)kt0 * 128);
         }
     }
     const uint32_t l0 = lds_addr_of(smem) + wave * 1024;
@@ -259,7 +303,6 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
     // the barrier sits ahead of the step's last k-step: every wave has then read all of tile t (whose slot is refilled with
     // tile t + S) and tile t + 1 has landed, so the fragments the next step starts with are read under this step's last
     // MFMAs.  Loads past the last tile are not issued: the last S steps count the loads still behind them instead.
-    const int KT = p.K / (FP8 ? 128 : 64);
 #pragma unroll
     for (int t = 0; t < S; ++t)
         if (t < KT) {
@@ -401,22 +444,13 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
         }
         float v[8];
         load8(smem + rl * G::PITCH + cl * 4, v);
-        if constexpr (EPI == CDM_EPI_GATE_RESIDUAL_F32) {
-            const float* R = reinterpret_cast<const float*>(p.R) + (int64_t)row * p.ldr + col;
-            float* C = reinterpret_cast<float*>(p.C) + (int64_t)row * p.ldc + col;
-            float r[8], g[8];
-            load8(R, r);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) g[e] = 1.0f;
-            if (tile.gate) load8(tile.gate + col, g);
-            dequant8<FP8>(g, tile.sw, col, sr);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) r[e] = r[e] + g[e] * v[e];
-            *reinterpret_cast<float4*>(C) = make_float4(r[0], r[1], r[2], r[3]);
-            *reinterpret_cast<float4*>(C + 4) = make_float4(r[4], r[5], r[6], r[7]);
+        if constexpr (EPI == kPartial) {
+            float* P = p.partial + ((int64_t)tile.part * p.part_rows + (row - p.part_row0)) * p.N + col;
+            *reinterpret_cast<float4*>(P) = make_float4(v[0], v[1], v[2], v[3]);
+            *reinterpret_cast<float4*>(P + 4) = make_float4(v[4], v[5], v[6], v[7]);
             continue;
         }
-        dequant8<FP8>(v, tile.sw, col, sr);
+        if constexpr (EPI != CDM_EPI_GATE_RESIDUAL_F32) dequant8<FP8>(v, tile.sw, col, sr);
         if constexpr (EPI == CDM_EPI_ROPE_QK) {
             if (col < p.rope_cols) {      // whole heads: tile columns start on head boundaries
                 const int half = p.head_dim >> 1, in_head = col & (p.head_dim - 1), i = in_head & (half - 1);
@@ -434,21 +468,33 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
                 }
             }
         }
-        if constexpr (EPI == CDM_EPI_GATE_RESIDUAL) {
-            const uint4 r4 = *reinterpret_cast<const uint4*>(p.R + (int64_t)row * p.ldr + col);
-            const uint32_t rw[4] = {r4.x, r4.y, r4.z, r4.w};
-            float g[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) g[e] = 1.0f;
-            if (tile.gate) load8(tile.gate + col, g);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                v[2 * e] = bf16lo(rw[e]) + g[2 * e] * v[2 * e];
-                v[2 * e + 1] = bf16hi(rw[e]) + g[2 * e + 1] * v[2 * e + 1];
-            }
-        }
-        *reinterpret_cast<uint4*>(p.C + (int64_t)row * p.ldc + col) = pack8(v);
+        store8<EPI, FP8>(p, tile.gate, tile.sw, sr, row, col, v);
     }
+}
+
+// The sums of a launch cut along K, added part by part, through the epilogue.  Bound by reading them (k_split * 4 bytes per
+// value, most of it from the memory-side cache): one eight-column chunk per thread.
+template <int EPI>
+__global__ __launch_bounds__(256) void finish_split_kernel(const GemmParams p) {
+    const int cpr = p.N >> 3;
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int r = (int)(idx / cpr), col = (int)(idx % cpr) * 8;
+    if (r >= p.part_rows) return;
+    const int row = p.part_row0 + r;
+    const float* gate = nullptr;
+    bool in = false;
+    for (int i = 0; i < p.n_seg; ++i)
+        if (row >= p.seg[i].m_start && row < p.seg[i].m_end) { in = true; gate = p.seg[i].gate; }
+    if (!in) return;
+    float v[8];
+    load8(p.partial + (int64_t)r * p.N + col, v);
+    for (int i = 1; i < p.k_split; ++i) {
+        float w[8];
+        load8(p.partial + ((int64_t)i * p.part_rows + r) * p.N + col, w);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] += w[e];
+    }
+    store8<EPI, false>(p, gate, nullptr, 1.0f, row, col, v);
 }
 
 template <int EPI, bool FP8>
@@ -458,10 +504,10 @@ int32_t launch_epi(const GemmParams& p, TileShape s, int grid, hipStream_t st) {
     CDM_TILE(128, 256, 2, 4)
     CDM_TILE(128, 128, 4, 2)
     CDM_TILE(64, 128, 2, 4)
-    if constexpr (EPI == CDM_EPI_NONE || EPI == CDM_EPI_GATE_RESIDUAL || EPI == CDM_EPI_GATE_RESIDUAL_F32) {
+    if constexpr (EPI == CDM_EPI_NONE || EPI == CDM_EPI_GATE_RESIDUAL || EPI == CDM_EPI_GATE_RESIDUAL_F32 || EPI == kPartial)
         CDM_TILE(64, 64, 2, 4)
+    if constexpr (EPI == CDM_EPI_NONE || EPI == CDM_EPI_GATE_RESIDUAL || EPI == CDM_EPI_GATE_RESIDUAL_F32)
         CDM_TILE(32, 32, 2, 2)
-    }
 #undef CDM_TILE
     CDM_FAIL(CDM_ERR_LAUNCH, "gemm: no kernel for a %d x %d tile", s.tm, s.tn);
 }
@@ -512,16 +558,73 @@ Best best_shape(const int64_t* rows, int n_seg, int64_t N, double kt, int epilog
     return best;
 }
 
+// Launches with few tiles and a long K: every tile once per range of K, fp32 sums in scratch memory and a pass over them
+// (finish_split_kernel: its launch, and the sums written and read at about 8 TB/s).  Whole launch against the cut one, us, fp32
+// residual, weights that no cache holds:
+//     N = 4096, K = 16384:  M = 128  74.8 / 56.2   256  75.0 / 59.7   512  114 / 81.9   768  148 / 125   1024  153 / 135
+//     N = 2048, K = 8192:   M = 64   20.8 / 15.8   256  35.6 / 24.4   512  35.7 / 32.1
+//     N = 4096, K = 4096:   M = 128  22.0 / 19.2;  N = 1024, K = 4096: M = 512 20.0 / 18.5
+// Cut launches stream the weights at 2.4 - 3 TB/s at most (M = 16 and 64 at K = 16384: 55 us against 39 and 46 whole), so such
+// a rate bounds the estimate.  Against 64 bits the sums are closer than uncut ones (K = 16384: 2.8e-7 in four ranges, 5.8e-7).
+struct SplitK { TileShape s; int parts; double us; int64_t bytes; };
+SplitK best_split(const GemmParams& p, const int64_t* rows, double kt, int epilogue) {
+    SplitK best{{}, 1, 1e30, 0};
+    if (epilogue != CDM_EPI_NONE && epilogue != CDM_EPI_GATE_RESIDUAL && epilogue != CDM_EPI_GATE_RESIDUAL_F32) return best;
+    int64_t lo = p.seg[0].m_start, hi = p.seg[0].m_end, filled = 0;
+    for (int i = 0; i < p.n_seg; ++i) {
+        lo = p.seg[i].m_start < lo ? p.seg[i].m_start : lo;
+        hi = p.seg[i].m_end > hi ? p.seg[i].m_end : hi;
+        filled += rows[i];
+    }
+    if (filled != hi - lo) return best;                                     // gaps between the segments
+    for (const ShapeCost& c : kShapes) {
+        if (c.s.tm == 256 || c.s.tm == 32) continue;
+        int64_t n = 0;
+        for (int i = 0; i < p.n_seg; ++i) n += (rows[i] + c.s.tm - 1) / c.s.tm;
+        n *= (p.N + c.s.tn - 1) / c.s.tn;
+        for (int s = 2; s <= kMaxSplitK; ++s) {
+            if (kt < 12.0 * s || n * s > 512) break;
+            const int64_t bytes = (hi - lo) * p.N * 4 * s;
+            const double weights = (double)p.N * kt * 128.0 * p.n_seg / 2.9e6, run = estimate(c, n * s, kt / s);
+            const double us = (run > weights ? run : weights) + 5.5 + 2.0 * (double)bytes / 8e6;
+            if (us < best.us) best = SplitK{c.s, s, us, bytes};
+        }
+    }
+    return best;
+}
+
 }  // namespace
 
 namespace cdm_gemm {
+
+int32_t launch_split_k(GemmParams& p, int epilogue, const GemmPlan& plan, void* scratch, hipStream_t st) {
+    const TileShape s = plan.shape[0];
+    p.partial = (float*)scratch; p.k_split = plan.k_split;
+    p.tiles_n = (p.N + s.tn - 1) / s.tn;
+    int total = 0, lo = p.seg[0].m_start, hi = p.seg[0].m_end;
+    for (int i = 0; i < p.n_seg; ++i) {
+        p.seg[i].tiles_m = (p.seg[i].m_end - p.seg[i].m_start + s.tm - 1) / s.tm;
+        total += p.seg[i].tiles_m * p.tiles_n;
+        p.seg[i].tile_end = total;
+        lo = p.seg[i].m_start < lo ? p.seg[i].m_start : lo;
+        hi = p.seg[i].m_end > hi ? p.seg[i].m_end : hi;
+    }
+    p.total_tiles = total; p.part_row0 = lo; p.part_rows = hi - lo;
+    int32_t rc = launch_epi<kPartial, false>(p, s, (total * p.k_split + 7) / 8 * 8, st);
+    if (rc) return rc;
+    const unsigned grid = (unsigned)(((int64_t)p.part_rows * (p.N / 8) + 255) / 256);
+    if (epilogue == CDM_EPI_NONE) finish_split_kernel<CDM_EPI_NONE><<<grid, 256, 0, st>>>(p);
+    else if (epilogue == CDM_EPI_GATE_RESIDUAL) finish_split_kernel<CDM_EPI_GATE_RESIDUAL><<<grid, 256, 0, st>>>(p);
+    else finish_split_kernel<CDM_EPI_GATE_RESIDUAL_F32><<<grid, 256, 0, st>>>(p);
+    return CDM_OK;
+}
 
 // How a launch is cut: one shape for all of it, or - where 256 x 256 tiles end in a poorly filled round - whole rounds of
 // those tiles and a second launch for the rows behind them in the shape that suits it.  N = 4096, one launch of 256 x 256
 // tiles against the cut: M = 4352 (1.06 rounds) 184 -> 141 us at K = 4096, 667 -> 459 at K = 16384; M = 9000 (2.25) 295 ->
 // 264 and 1043 -> 907; M = 14080 (3.44) 427 -> 414 and 1453 -> 1381; M = 11000 (2.69) keeps one launch.
 // The second launch costs about 5 us of its own (it starts when the first has drained).
-GemmPlan plan_gemm(const GemmParams& p, int epilogue, bool fp8) {
+GemmPlan plan_gemm(const GemmParams& p, int epilogue, bool fp8, int64_t scratch_bytes) {
     const int v = cdm_get_variant(1);
     if (v >= 2) return GemmPlan{1, -1, {kShapes[(v - 2) % 6].s, {}}};      // cross-check build: one shape for everything
     const double kt = p.K / (fp8 ? 128.0 : 64.0);
@@ -533,6 +636,10 @@ GemmPlan plan_gemm(const GemmParams& p, int epilogue, bool fp8) {
     }
     const Best one = best_shape(rows, p.n_seg, p.N, kt, epilogue);
     GemmPlan plan{1, -1, {one.s, {}}};
+    if (scratch_bytes > 0 && !fp8) {
+        const SplitK k = best_split(p, rows, kt, epilogue);
+        if (k.us < 0.93 * one.us && k.bytes <= scratch_bytes) return GemmPlan{1, -1, {k.s, {}}, k.parts, k.bytes};
+    }
     const int64_t cols = epilogue == CDM_EPI_SWIGLU ? 128 : 256, tn = (p.N + cols - 1) / cols;
     const int64_t first = tm * tn / 256 * 256 / tn;                         // row tiles of the whole rounds
     if (first == 0 || first == tm) return plan;

@@ -6,6 +6,7 @@ device pointers, sizes, row strides and the current HIP stream.  There is no fal
 from __future__ import annotations
 
 import ctypes as C
+import functools
 from typing import Optional, Sequence, Tuple
 
 import torch
@@ -14,6 +15,7 @@ from . import _lib
 from ._lib import EPI_GATE_RESIDUAL, EPI_GATE_RESIDUAL_F32, EPI_NONE, EPI_ROPE_QK, EPI_SWIGLU
 
 _EPI = {"none": EPI_NONE, "swiglu": EPI_SWIGLU, "gate_residual": EPI_GATE_RESIDUAL, "rope_qk": EPI_ROPE_QK}
+_MAY_SPLIT_K = (EPI_NONE, EPI_GATE_RESIDUAL, EPI_GATE_RESIDUAL_F32)
 FP8_DTYPE = torch.float8_e4m3fn
 
 
@@ -216,6 +218,14 @@ def _amax_arg(row_amax: Optional[torch.Tensor], rows: int, min_cols: int):
 
 
 # ----------------------------------------------------------------------------- GEMM
+@functools.lru_cache(maxsize=4096)
+def gemm_scratch_bytes(lens: Tuple[int, ...], N: int, K: int, epi: int) -> int:
+    """Scratch for a bf16 GEMM of these segments that is cut along K (few output tiles, long K); 0: it is not cut."""
+    if K < 2048 or sum(lens) * N > 1 << 23:      # too short a K, or enough tiles for the chip
+        return 0
+    return int(_lib.load().cdm_grouped_gemm_scratch_bytes((C.c_int64 * len(lens))(*lens), len(lens), N, K, epi))
+
+
 @_timed("gemm")
 def gemm(a: torch.Tensor, w: torch.Tensor, *, w2: Optional[torch.Tensor] = None, epilogue: str = "none",
          residual: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
@@ -235,6 +245,9 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, w2: Optional[torch.Tensor] = None,
         raise ValueError("w and w2 must share a row stride")
     half = head_dim // 2 if head_dim else 0
     epi, odt = _epilogue(epilogue, out, residual)
+    scratch = gemm_scratch_bytes((M,), N, K, epi) if epi in _MAY_SPLIT_K else 0
+    if scratch:
+        return grouped_gemm(a, [w], [(0, M)], epilogue=epilogue, residual=residual, gates=[gate], out=out)
     rc = lib.cdm_gemm_bf16(_chk(a, "a", torch.bfloat16, 2), a.stride(0), _chk(w, "w", torch.bfloat16, 2), w.stride(0),
                            _chk(w2, "w2", torch.bfloat16, 2), _chk(out, "out", odt, 2), out.stride(0),
                            M, N, K, epi, _chk(residual, "residual", odt, 2),
@@ -298,7 +311,8 @@ def grouped_gemm(a: torch.Tensor, ws: Sequence[torch.Tensor], segments: Sequence
                  w2s: Optional[Sequence[torch.Tensor]] = None, epilogue: str = "none", residual=None,
                  gates: Optional[Sequence[Optional[torch.Tensor]]] = None, cos=None, sin=None, rope_cols: int = 0,
                  head_dim: int = 0, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """MoT routed linear: rows [start, start+len) of ``a`` use ws[g] (w2s[g], gates[g])."""
+    """MoT routed linear: rows [start, start+len) of ``a`` use ws[g] (w2s[g], gates[g]).  ``a`` may be a list of the segments'
+    rows (epilogue "none")."""
     lib = _lib.load()
     M, K = a.shape
     N = ws[0].shape[0]
@@ -317,6 +331,15 @@ def grouped_gemm(a: torch.Tensor, ws: Sequence[torch.Tensor], segments: Sequence
     st, ln = I64(*[int(s) for s, _ in segments]), I64(*[int(l) for _, l in segments])
     half = head_dim // 2 if head_dim else 0
     epi, odt = _epilogue(epilogue, out, residual)
+    scratch = gemm_scratch_bytes(tuple(int(l) for _, l in segments), N, K, epi) if epi in _MAY_SPLIT_K else 0
+    if scratch:
+        buf = torch.empty((scratch,), dtype=torch.uint8, device=a.device)
+        rc = lib.cdm_grouped_gemm_scratch_bf16(_chk(a, "a", torch.bfloat16, 2), a.stride(0), wp, ldw, _chk(out, "out", odt, 2),
+                                               out.stride(0), st, ln, n_seg, N, K, epi, _chk(residual, "residual", odt, 2),
+                                               residual.stride(0) if residual is not None else 0, gp, buf.data_ptr(), scratch,
+                                               _stream())
+        _lib.check(rc, "cdm_grouped_gemm_scratch_bf16")
+        return out
     rc = lib.cdm_grouped_gemm_bf16(_chk(a, "a", torch.bfloat16, 2), a.stride(0), wp, ldw, w2p,
                                    _chk(out, "out", odt, 2), out.stride(0), st, ln, n_seg, N, K,
                                    epi, _chk(residual, "residual", odt, 2),
@@ -376,7 +399,8 @@ def gemm_qkv_pack(a: torch.Tensor, sa: Optional[torch.Tensor], ws: Sequence[torc
     weights when given, then rotated with cos/sin when given) and V go straight into the attention kernel's tile
     images in ``workspace`` (for ``attention_packed``, which takes the same ``qk_norm`` for Q).  ``qk_norm`` =
     (q_weight, k_weight, seg_ends, eps) with one segment per GEMM segment.  e4m3 operands when ``sa`` / ``sws`` are
-    given.  Raises where the fused form does not apply (``qkv_pack_applies`` tells beforehand)."""
+    given.  Raises where the fused form does not apply (``qkv_pack_applies`` tells beforehand).  ``a`` may be a list of the
+    segments' rows (bf16)."""
     lib = _lib.load()
     M, K = a.shape
     n_seg = len(segments)

@@ -333,6 +333,18 @@ int32_t cdm_grouped_gemm_bf16(const void* A, int64_t lda, const void* const* W, 
                               const float* cos, const float* sin, int64_t rope_cols, int32_t head_dim,
                               void* stream);
 
+/*
+ * The same with scratch memory (16-byte aligned) for launches with few output tiles and a long K, epilogues NONE and
+ * GATE_RESIDUAL(_F32): such a launch is cut into ranges of K whose fp32 sums are added behind it, in the order of the ranges.
+ * cdm_grouped_gemm_scratch_bytes says how much that takes for segments that follow each other (0: the launch would not be
+ * cut); with less, the launch is the one above.
+ */
+int64_t cdm_grouped_gemm_scratch_bytes(const int64_t* seg_len, int32_t n_seg, int64_t N, int64_t K, int32_t epilogue);
+int32_t cdm_grouped_gemm_scratch_bf16(const void* A, int64_t lda, const void* const* W, int64_t ldw, void* C, int64_t ldc,
+                                      const int64_t* seg_start, const int64_t* seg_len, int32_t n_seg, int64_t N, int64_t K,
+                                      int32_t epilogue, const void* R, int64_t ldr, const float* const* gate, void* scratch,
+                                      int64_t scratch_bytes, void* stream);
+
 /* The same for e4m3 operands (see cdm_gemm_fp8): sa is the per-token scale of the whole sequence, sw[g] / sw2[g] the
  * per-output-channel scales of segment g's weights. */
 int32_t cdm_grouped_gemm_fp8(const void* Aq, int64_t lda, const float* sa, const void* const* Wq,
