@@ -48,7 +48,7 @@ struct GemmParams {
 
 // what a workgroup works on
 struct Tile {
-    int m0, m_end, tn;
+    int m0, m_end, tn, part;
     const void* W; const void* W2;
     const float* gate; const float* sw; const float* sw2; const float* knw;
 };
