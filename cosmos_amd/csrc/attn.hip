@@ -134,8 +134,10 @@ __device__ __forceinline__ int next_hot_tile(uint32_t hot, int after, int lane) 
 //   at set-up), the row maximum of that tile and the reference update are skipped; where the bound fails - a
 //   tile with an outlier key, un-normalised huge logits - they run in the tail, after block B (one loop body for both
 //   cases: two copies of the loop do not fit the register budget).
-template <int HD, int QB, bool LATE, class Mid>
-__device__ __forceinline__ void pipe_step(Mid&& mid, float late_r, const char* sk_next, const char* sv_cur, const char* sk_next2,
+// STRIDE: from one tile of the wave to its next (2: the waves of a workgroup share the tiles out, see attn_fwd_keys_kernel)
+// slot(i): what else slot i of block A carries (loads of the tiles to come)
+template <int HD, int QB, bool LATE, int STRIDE = 1, class Mid, class Slot>
+__device__ __forceinline__ void pipe_step(Mid&& mid, Slot&& slot, float late_r, const char* sk_next, const char* sv_cur, const char* sk_next2,
                                           const bf16x8 (&qf)[QB][HD / 32], bf16x8 (&kw)[KWIN][KB],
                                           f32x4 (&s_cur)[KB][QB], f32x4 (&s_next)[KB][QB],
                                           f32x4 (&oacc)[HD / 16][QB], f32x4 (&negm)[QB], float (&l_run)[QB], int lane,
@@ -193,6 +195,7 @@ __device__ __forceinline__ void pipe_step(Mid&& mid, float late_r, const char* s
             vw[n_v] = v_frag<HD>(sv_cur, n_v / HB, n_v % HB, lane);
             ++n_v;
         }
+        slot(i);
         __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
@@ -228,7 +231,7 @@ __device__ __forceinline__ void pipe_step(Mid&& mid, float late_r, const char* s
     // tile j + 1 needs row maxima only if it is the wave's next marked tile (one scalar compare on the common path);
     // the tile after it is looked up behind the maxima (need_always: every tile is the next one)
     if (next_tile != next_hot) return;
-    next_hot = need_always ? next_tile + 1 : next_hot_tile(hot, next_tile, lane);
+    next_hot = need_always ? next_tile + STRIDE : next_hot_tile(hot, next_tile, lane);
     float mx[QB];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) mx[qb] = tile_row_max<QB>(s_next, qb);
@@ -311,87 +314,14 @@ constexpr float kSafeLog2 = 60.0f;      // largest excess over the reference tha
 constexpr int kMaxKm = 2048;            // key tiles that get a decision of their own (131,072 keys); longer sequences: one per head
 constexpr int kMaxSplit = 8;            // most key ranges a query block of the last round is split into
 
-// NW = waves per workgroup.  (The bound is given for eight waves also where four are launched: for a 256-thread workgroup
-// the compiler splits the register file and copies accumulators between its halves.)
-template <int HD, int QS, int NW, bool LATE>
-__global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS, 2 / QS))) void attn_fwd_pipe_kernel(
-    const PackedParams p) {
-    constexpr int ROWS = NW * 32 * QS;                 // query rows per workgroup
-    constexpr int QB = 2 * QS;                         // 16-row query blocks per wave
-    constexpr int KS = HD / 32, HB = HD / 16;
-    constexpr int TILE_BYTES = BN * HD * 2;            // same for K and V tiles
-    constexpr int PER_WAVE = TILE_BYTES / 1024 / NW;   // direct-to-LDS instructions per wave per tile
-    // K(t) lives in slot t % 3 and V(t) in slot t % 4.  V is loaded one step further ahead than its first use by
-    // the in-phase waves needs: the out-of-phase waves read the first fragments of V(j) BEFORE barrier j, so V(j)
-    // has to be complete at barrier j - 1
-    constexpr int RING = 3, RING_V = 4;
-    __shared__ __attribute__((aligned(1024))) char sk[RING * TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char sv[RING_V * TILE_BYTES];
-    __shared__ float s_km[kMaxKm];       // largest key norm of every tile of this K / V head, prefix tiles first (set-up only)
-
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+// Q fragments of a wave's rows q0 ..: rotate-half mRoPE (if tables are given) and the factor log2(e)/sqrt(HD), both in fp32 and
+// with ONE rounding to bf16.  The lane holds channels 32ks + 8g .. +7 (g = lane / 16) of its query row for every
+// ks, so the partner of a channel in k-step ks (< KS/2) is the same register element of k-step ks + KS/2.
+// qnorm: the norms of the scaled, rotated, rounded rows.
+template <int HD, int QB>
+__device__ __forceinline__ void load_q(const PackedParams& p, int head, int q0, int lane, bf16x8 (&qf)[QB][HD / 32], float (&qnorm)[QB]) {
+    constexpr int KS = HD / 32;
     const int r16 = lane & 15, g4 = lane >> 4;
-    // XCD-aware placement: workgroup ids are dealt round-robin over the 8 XCDs.  All query blocks of a head go to
-    // ONE XCD, so a head's K / V tile images are fetched into one L2 instead of eight, and an XCD owns a contiguous
-    // range of heads, so the query heads that share a K / V head (grouped-query attention) share an L2 as well.
-    int head, qblk;
-    int unit = -1, part = 0;      // split unit: index into the scratch arrays, and which range of the key tiles
-    {
-        const int nqb = p.n_qblocks, nh = p.n_heads;
-        const int xcd = blockIdx.x & 7;
-        int k = blockIdx.x >> 3;                                  // k-th workgroup of its XCD
-        const int hpx = (nh + 7) >> 3;                            // heads per XCD (the last XCDs may own fewer)
-        if (p.split > 1) {
-            // the last split_tail query blocks of the XCD come `split` times, ordered by key range first: units that run
-            // side by side then stream the same tiles of the same head
-            const int whole = hpx * nqb - p.split_tail;
-            if (k >= whole) {
-                const int u = k - whole;
-                part = u / p.split_tail;
-                k = whole + (u - part * p.split_tail);
-                unit = xcd * p.split_tail * p.split + u;
-            }
-        }
-        const int hi = k / nqb;
-        head = xcd * hpx + hi;
-        qblk = k - hi * nqb;
-        if (hi >= hpx || head >= nh) return;
-    }
-    const int kv_head = head / p.kv_group;
-    const int q0 = qblk * ROWS + wave * (32 * QS);
-
-    // ---- Q fragments: rotate-half mRoPE (if tables are given) and the factor log2(e)/sqrt(HD), both in fp32 and
-    // with ONE rounding to bf16.  The lane holds channels 32ks + 8g .. +7 (g = lane / 16) of its query row for every
-    // ks, so the partner of a channel in k-step ks (< KS/2) is the same register element of k-step ks + KS/2.
-    // An upper bound of every score of a row against a key tile: |q| max_{k in tile} |k| (Cauchy-Schwarz on the very
-    // bf16 values the matrix cores multiply).  The per-tile key norms of this K / V head pass through LDS once: each
-    // wave turns them into one bit per tile ("this tile needs row maxima for my rows"), 32 tiles per lane of one
-    // register, and keeps the index of the next such tile in a scalar register: a step compares its tile index with it
-    // (one scalar instruction) and looks the following one up only after a hit.
-    // A sequence of more than kMaxKm tiles falls back to one bound per head (kmax_all).
-    // A split unit works in a frame of its own: tile 0 is the first tile of its range [t0, t0 + NT), the prefix tiles
-    // are the first NP of that frame (NP <= 0: none left), per-row key limits count from the frame's first key.
-    const int NM = (p.n_tokens + BN - 1) / BN;
-    const int NT_all = p.n_prefix_tiles + NM;
-    const int t0 = unit < 0 ? 0 : (int)((int64_t)NT_all * part / p.split);
-    const int t1 = unit < 0 ? NT_all : (int)((int64_t)NT_all * (part + 1) / p.split);
-    const int NP = p.n_prefix_tiles - t0;
-    const int NT = t1 - t0;
-    const bool per_tile = NT <= kMaxKm;
-    float kmax_all = 0.0f;
-    {
-        const float* km = p.kmax + (int64_t)kv_head * NM - p.n_prefix_tiles + t0;      // indexed by the frame's tile number
-        const float* kmp = p.kmax_prefix + (int64_t)kv_head * p.n_prefix_tiles + t0;
-        if (per_tile) {
-            for (int i = threadIdx.x; i < kMaxKm; i += 64 * NW) s_km[i] = i >= NT ? 0.0f : (i < NP ? kmp[i] : km[i]);
-        } else {
-            for (int i = lane; i < NT; i += 64) kmax_all = fmaxf(kmax_all, i < NP ? kmp[i] : km[i]);
-            kmax_all = wave_max(kmax_all);
-        }
-    }
-    float qnorm[QB];
-    bf16x8 qf[QB][KS];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
         int qrow = q0 + qb * 16 + r16;
@@ -464,6 +394,87 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
             qnorm[qb] = sqrtf(ss);
         }
     }
+}
+
+// NW = waves per workgroup.  (The bound is given for eight waves also where four are launched: for a 256-thread workgroup
+// the compiler splits the register file and copies accumulators between its halves.)
+template <int HD, int QS, int NW, bool LATE>
+__global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS, 2 / QS))) void attn_fwd_pipe_kernel(
+    const PackedParams p) {
+    constexpr int ROWS = NW * 32 * QS;                 // query rows per workgroup
+    constexpr int QB = 2 * QS;                         // 16-row query blocks per wave
+    constexpr int KS = HD / 32, HB = HD / 16;
+    constexpr int TILE_BYTES = BN * HD * 2;            // same for K and V tiles
+    constexpr int PER_WAVE = TILE_BYTES / 1024 / NW;   // direct-to-LDS instructions per wave per tile
+    // K(t) lives in slot t % 3 and V(t) in slot t % 4.  V is loaded one step further ahead than its first use by
+    // the in-phase waves needs: the out-of-phase waves read the first fragments of V(j) BEFORE barrier j, so V(j)
+    // has to be complete at barrier j - 1
+    constexpr int RING = 3, RING_V = 4;
+    __shared__ __attribute__((aligned(1024))) char sk[RING * TILE_BYTES];
+    __shared__ __attribute__((aligned(1024))) char sv[RING_V * TILE_BYTES];
+    __shared__ float s_km[kMaxKm];       // largest key norm of every tile of this K / V head, prefix tiles first (set-up only)
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, g4 = lane >> 4;
+    // XCD-aware placement: workgroup ids are dealt round-robin over the 8 XCDs.  All query blocks of a head go to
+    // ONE XCD, so a head's K / V tile images are fetched into one L2 instead of eight, and an XCD owns a contiguous
+    // range of heads, so the query heads that share a K / V head (grouped-query attention) share an L2 as well.
+    int head, qblk;
+    int unit = -1, part = 0;      // split unit: index into the scratch arrays, and which range of the key tiles
+    {
+        const int nqb = p.n_qblocks, nh = p.n_heads;
+        const int xcd = blockIdx.x & 7;
+        int k = blockIdx.x >> 3;                                  // k-th workgroup of its XCD
+        const int hpx = (nh + 7) >> 3;                            // heads per XCD (the last XCDs may own fewer)
+        if (p.split > 1) {
+            // the last split_tail query blocks of the XCD come `split` times, ordered by key range first: units that run
+            // side by side then stream the same tiles of the same head
+            const int whole = hpx * nqb - p.split_tail;
+            if (k >= whole) {
+                const int u = k - whole;
+                part = u / p.split_tail;
+                k = whole + (u - part * p.split_tail);
+                unit = xcd * p.split_tail * p.split + u;
+            }
+        }
+        const int hi = k / nqb;
+        head = xcd * hpx + hi;
+        qblk = k - hi * nqb;
+        if (hi >= hpx || head >= nh) return;
+    }
+    const int kv_head = head / p.kv_group;
+    const int q0 = qblk * ROWS + wave * (32 * QS);
+
+    // An upper bound of every score of a row against a key tile: |q| max_{k in tile} |k| (Cauchy-Schwarz on the very
+    // bf16 values the matrix cores multiply).  The per-tile key norms of this K / V head pass through LDS once: each
+    // wave turns them into one bit per tile ("this tile needs row maxima for my rows"), 32 tiles per lane of one
+    // register, and keeps the index of the next such tile in a scalar register: a step compares its tile index with it
+    // (one scalar instruction) and looks the following one up only after a hit.
+    // A sequence of more than kMaxKm tiles falls back to one bound per head (kmax_all).
+    // A split unit works in a frame of its own: tile 0 is the first tile of its range [t0, t0 + NT), the prefix tiles
+    // are the first NP of that frame (NP <= 0: none left), per-row key limits count from the frame's first key.
+    const int NM = (p.n_tokens + BN - 1) / BN;
+    const int NT_all = p.n_prefix_tiles + NM;
+    const int t0 = unit < 0 ? 0 : (int)((int64_t)NT_all * part / p.split);
+    const int t1 = unit < 0 ? NT_all : (int)((int64_t)NT_all * (part + 1) / p.split);
+    const int NP = p.n_prefix_tiles - t0;
+    const int NT = t1 - t0;
+    const bool per_tile = NT <= kMaxKm;
+    float kmax_all = 0.0f;
+    {
+        const float* km = p.kmax + (int64_t)kv_head * NM - p.n_prefix_tiles + t0;      // indexed by the frame's tile number
+        const float* kmp = p.kmax_prefix + (int64_t)kv_head * p.n_prefix_tiles + t0;
+        if (per_tile) {
+            for (int i = threadIdx.x; i < kMaxKm; i += 64 * NW) s_km[i] = i >= NT ? 0.0f : (i < NP ? kmp[i] : km[i]);
+        } else {
+            for (int i = lane; i < NT; i += 64) kmax_all = fmaxf(kmax_all, i < NP ? kmp[i] : km[i]);
+            kmax_all = wave_max(kmax_all);
+        }
+    }
+    float qnorm[QB];
+    bf16x8 qf[QB][KS];
+    load_q<HD, QB>(p, head, q0, lane, qf, qnorm);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // Q is in registers: from here on vmcnt counts tile loads only
 
     f32x4 oacc[HB][QB];
@@ -608,7 +619,7 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
         _Pragma("unroll") for (int qb = 0; qb < QB; ++qb)                                                       \
             nvalid[qb] = pre_rag ? p.prefix_last_valid : klim[qb] - (j + 1) * BN;                               \
         /* does tile j + 1 (the scores block A computes) need row maxima?  its bit of the wave's table */      \
-        pipe_step<HD, QB, LATE>([&]() { if (late_sync) { sync(); load_k(); } else load_v(); }, p.late_r,       \
+        pipe_step<HD, QB, LATE>([&]() { if (late_sync) { sync(); load_k(); } else load_v(); }, [](int) {}, p.late_r, \
                           sk + ks_next * TILE_BYTES, sv + v_cur * TILE_BYTES, sk + k_next2 * TILE_BYTES, qf, kw, \
                           SCUR, SNEXT, oacc, negm, l_run, lane, causal_wg || pre_rag || (ragged && j + 2 >= NT), nvalid, \
                           j + 1, next_hot, need_always, hot);     /* tile j + 1: the scores block A computes */ \
@@ -667,6 +678,233 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
         const int rloc = it * RPI + rl;
         const uint4 v = *reinterpret_cast<const uint4*>(stage + rloc * PITCH + ch * 16);
         if (q0 + rloc < p.n_tokens) *reinterpret_cast<uint4*>(orow + rloc * ldo + ch * 8) = v;
+    }
+}
+
+// Small grids (see the launch rule): 128 query rows per workgroup, and two groups of four waves that share the key tiles out -
+// group g takes tiles g, g + 2, ... for all 128 rows - and add up their results at the end.  With one wave per SIMD nothing
+// runs under a wave's exponentials and waits; the second one fills them, and a workgroup makes half the steps.  Every group has
+// a ring of its own, three K and two V tiles (160 KB for both at head_dim 128): a tile is requested one step ahead of its
+// first use.  The partial results stay fp32.
+// Launches in us, 128-row workgroups of four waves against this: 16 heads x 64, 512 keys 12.0 / 11.9, 1024 keys 17.8 / 16.0, 2048
+// keys 28.2 / 24.3; 16 heads x 128, 512 keys 16.9 / 18.1 (32 heads), 1024 keys 23.9 / 22.7, 1637 keys 34.1 / 30.5, 2048 keys 40.7 /
+// 37.9; 8 heads x 128, 4000 keys 70.9 / 62.7.  A step of two tiles takes 1.85 us at head_dim 128 against 2 x 1.03; where the
+// loads stand in it does not matter (one behind every first to fourth MFMA: the same).  A second barrier per step that keeps
+// the groups half a step apart costs more than the overlap brings (2048 keys 39.4).
+template <int HD, bool LATE>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_keys_kernel(const PackedParams p) {
+    constexpr int ROWS = BMQ / 2, QB = 2, KS = HD / 32, HB = HD / 16;
+    constexpr int TILE_BYTES = BN * HD * 2;
+    constexpr int PER_WAVE = TILE_BYTES / 1024 / 4;    // direct-to-LDS instructions per wave per tile
+    constexpr int RING = 3, RING_V = 2, GROUP = (RING + RING_V) * TILE_BYTES;
+    __shared__ __attribute__((aligned(1024))) char smem[2 * GROUP];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int grp = wave >> 2, gw = wave & 3;
+    const int r16 = lane & 15, g4 = lane >> 4;
+    int head, qblk;
+    {      // all query blocks of a head on one XCD, as above
+        const int hpx = (p.n_heads + 7) >> 3, k = blockIdx.x >> 3, hi = k / p.n_qblocks;
+        head = (blockIdx.x & 7) * hpx + hi;
+        qblk = k - hi * p.n_qblocks;
+        if (hi >= hpx || head >= p.n_heads) return;
+    }
+    const int kv_head = head / p.kv_group;
+    const int q0 = qblk * ROWS + gw * 32, b0 = qblk * ROWS;
+    const int NM = (p.n_tokens + BN - 1) / BN, NP = p.n_prefix_tiles, NT = NP + NM;      // 4 <= NT <= kMaxKm, host-checked
+    const char* kbase = p.kp + ((int64_t)kv_head * NM - NP) * TILE_BYTES;
+    const char* vbase = p.vp + ((int64_t)kv_head * NM - NP) * TILE_BYTES;
+    const char* kpre = p.kp_prefix + (int64_t)kv_head * NP * TILE_BYTES;
+    const char* vpre = p.vp_prefix + (int64_t)kv_head * NP * TILE_BYTES;
+    char* sk = smem + grp * GROUP;
+    char* sv = sk + RING * TILE_BYTES;
+    const uint32_t lane_off = (uint32_t)(gw * 1024 + lane * 16);
+    const uint32_t sk_addr = lds_addr_of(sk) + gw * 1024, sv_addr = lds_addr_of(sv) + gw * 1024;
+    // the group's i-th tile (clamped to the last of the sequence) -> ring slot
+    auto issue = [&](const char* base, const char* pre, uint32_t dst_addr, int i, int slot) {
+        const int t = 2 * i + grp, tc = t < NT ? t : NT - 1;
+        const char* src = (tc < NP ? pre : base) + (uint32_t)tc * (uint32_t)TILE_BYTES;
+#pragma unroll
+        for (int l = 0; l < PER_WAVE; ++l) lds_dma16(src + l * 4096, lane_off, dst_addr + slot * TILE_BYTES + l * 4096);
+    };
+    issue(kbase, kpre, sk_addr, 0, 0);
+    issue(kbase, kpre, sk_addr, 1, 1);
+    issue(vbase, vpre, sv_addr, 0, 0);
+    issue(kbase, kpre, sk_addr, 2, 2);
+    const float* km = p.kmax + (int64_t)kv_head * NM - NP;      // indexed by tile
+    const float* kmp = p.kmax_prefix + (int64_t)kv_head * NP;
+    auto tile_norm = [&](int t) { return t < NP ? kmp[t] : t < NT ? km[t] : 0.0f; };
+    const float km0 = tile_norm(lane);
+    float qnorm[QB];
+    bf16x8 qf[QB][KS];
+    load_q<HD, QB>(p, head, q0, lane, qf, qnorm);
+
+    f32x4 oacc[HB][QB], negm[QB];
+    float l_run[QB];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+        l_run[qb] = 0.0f;
+#pragma unroll
+        for (int hb = 0; hb < HB; ++hb) oacc[hb][qb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    const int n_keys = NP * BN + p.n_tokens;
+    const bool ragged = n_keys < NT * BN, causal_wg = b0 < p.causal_prefix;
+    int klim[QB];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+        const int qrow = q0 + qb * 16 + r16;
+        klim[qb] = qrow < p.causal_prefix ? qrow + 1 : n_keys;
+    }
+    const int kmax = (causal_wg && b0 + ROWS <= p.causal_prefix) ? (b0 + ROWS < n_keys ? b0 + ROWS : n_keys) : n_keys;
+    const int NTW = (kmax + BN - 1) / BN;                       // at least 2: both groups have a first tile
+    const int pre_rag_tile = (NP > 0 && p.prefix_last_valid < BN) ? NP - 1 : -1;
+
+    // everything requested so far has landed (Q and the norms included): one wait, one barrier
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    f32x4 s_a[KB][QB], s_b[KB][QB];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) s_a[kb][qb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    scores_tile<HD, QB>(sk, qf, s_a, lane);
+    if (causal_wg || grp == pre_rag_tile) {
+        int nvalid[QB];
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) nvalid[qb] = grp == pre_rag_tile ? p.prefix_last_valid : klim[qb] - grp * BN;
+        mask_scores<QB>(s_a, nvalid, lane);
+    }
+    bool need_always = p.always_max != 0;
+    float t_wave = INFINITY;
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+        float m0 = tile_row_max<QB>(s_a, qb);
+        m0 = m0 == -INFINITY ? 0.0f : m0;      // causal rows that end ahead of this group's first tile: nothing to refer to
+        const float thr = (kSafeLog2 + m0) / (qnorm[qb] * 1.01f);
+        need_always = need_always || __builtin_amdgcn_ballot_w64(thr != thr) != 0;
+        t_wave = fminf(t_wave, thr);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) s_a[kb][qb][e] -= m0;
+            negm[qb][e] = -m0;
+        }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) t_wave = fminf(t_wave, __shfl_xor(t_wave, off, 64));
+    uint32_t hot = 0u;      // bit t in lane l: tile 32 l + t is the group's and needs row maxima for this wave's rows
+    if (!need_always) {
+        for (int c = 0; c * 64 < NT; ++c) {
+            const float v = c == 0 ? km0 : tile_norm(c * 64 + lane);
+            const uint64_t m = __builtin_amdgcn_ballot_w64(!(v <= t_wave) && c * 64 + lane < NT) & (0x5555555555555555ull << grp);
+            if (lane == 2 * c) hot = (uint32_t)m;
+            if (lane == 2 * c + 1) hot = (uint32_t)(m >> 32);
+        }
+    }
+    int next_hot = need_always ? 2 + grp : next_hot_tile(hot, grp, lane);
+    bf16x8 kw[KWIN][KB];
+    preload_k<HD>(sk + TILE_BYTES, kw, lane);
+
+    // step j works on the group's tile j: S(j+1) from K slot (j+1) % 3, P(j) V(j) from V slot j % 2, K(j+2) fragments from
+    // slot (j+2) % 3.  At its barrier everything requested in step j - 1 - K(j+2), V(j) - has landed, and every wave is done
+    // with K(j) and V(j-1), whose slots take K(j+3) and V(j+1).  A group without a tile j (an odd count) only takes the barrier.
+    int ks_next = 1, ks_cur = 0;
+    constexpr int GAP = KS * KB * QB / (4 * PER_WAVE);      // one load behind every GAP-th MFMA of block A's first half
+#define CDM_ATTN_STEP(SCUR, SNEXT)                                                                              \
+    {                                                                                                           \
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");                                           \
+        __builtin_amdgcn_sched_barrier(0);                                                                      \
+        const int k_next2 = ks_next == 2 ? 0 : ks_next + 1, t = 2 * j + grp, tn = t + 2;                        \
+        const int tk = t + 6 < NT ? t + 6 : NT - 1, tv = tn < NT ? tn : NT - 1;      /* K(j+3), V(j+1) */       \
+        const char* ksrc = (tk < NP ? kpre : kbase) + (uint32_t)tk * (uint32_t)TILE_BYTES;                      \
+        const char* vsrc = (tv < NP ? vpre : vbase) + (uint32_t)tv * (uint32_t)TILE_BYTES;                      \
+        const uint32_t kdst = sk_addr + ks_cur * TILE_BYTES, vdst = sv_addr + ((j + 1) & 1) * TILE_BYTES;       \
+        /* one load every few MFMAs: issued back to back they hold a wave for hundreds of cycles */             \
+        auto slot = [&](int i) {                                                                                \
+            const int l = i / GAP;                                                                              \
+            if (i % GAP != GAP - 1 || l >= 2 * PER_WAVE) return;                                                \
+            if (l < PER_WAVE) lds_dma16(vsrc + l * 4096, lane_off, vdst + l * 4096);                            \
+            else lds_dma16(ksrc + (l - PER_WAVE) * 4096, lane_off, kdst + (l - PER_WAVE) * 4096);               \
+        };                                                                                                      \
+        if (t < NTW) {                                                                                          \
+            int nvalid[QB];                                                                                     \
+            const bool pre_rag = tn == pre_rag_tile;                                                            \
+            _Pragma("unroll") for (int qb = 0; qb < QB; ++qb)                                                   \
+                nvalid[qb] = pre_rag ? p.prefix_last_valid : klim[qb] - tn * BN;                                \
+            pipe_step<HD, QB, LATE, 2>([]() {}, slot, p.late_r, sk + ks_next * TILE_BYTES, sv + (j & 1) * TILE_BYTES,  \
+                                       sk + k_next2 * TILE_BYTES, qf, kw, SCUR, SNEXT, oacc, negm, l_run, lane,  \
+                                       causal_wg || pre_rag || (ragged && tn >= NT - 1) || tn >= NT, nvalid, tn, \
+                                       next_hot, need_always, hot);                                             \
+        }                                                                                                       \
+        __builtin_amdgcn_sched_barrier(0);                                                                      \
+        ks_cur = ks_next;                                                                                       \
+        ks_next = k_next2;                                                                                      \
+    }
+    const int steps = (NTW + 1) >> 1;
+    for (int j = 0; j < steps; ++j) {
+        CDM_ATTN_STEP(s_a, s_b)
+        if (++j >= steps) break;
+        CDM_ATTN_STEP(s_b, s_a)
+    }
+#undef CDM_ATTN_STEP
+    // ---- the groups' results: no direct-to-LDS write may outlive the rings, which hold group 1's accumulators, sums and
+    // references from here on, and behind them the output rows that group 0 stages
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    constexpr int EX = (HB * QB + 1) * 1024, PITCH = HD * 2 + 16;
+    static_assert(4 * EX + ROWS * PITCH <= 2 * GROUP, "exchange and staging areas exceed the rings");
+    char* ex = smem + gw * EX + lane * 16;
+    float l_tot[QB], ref[QB];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+        l_tot[qb] = l_run[qb] + __shfl_xor(l_run[qb], 16, 64);
+        l_tot[qb] += __shfl_xor(l_tot[qb], 32, 64);
+        ref[qb] = -negm[qb][0] * (LATE ? p.late_r : 1.0f);
+    }
+    if (grp == 1) {
+#pragma unroll
+        for (int hb = 0; hb < HB; ++hb)
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb) *reinterpret_cast<f32x4*>(ex + (hb * QB + qb) * 1024) = oacc[hb][qb];
+        *reinterpret_cast<f32x4*>(ex + HB * QB * 1024) = f32x4{l_tot[0], l_tot[1], ref[0], ref[1]};
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (grp == 1) return;
+    char* stage = smem + 4 * EX + gw * (32 * PITCH);
+    const f32x4 other = *reinterpret_cast<const f32x4*>(ex + HB * QB * 1024);
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+        // a group whose tiles are all masked for the row has a sum of exactly zero and no say in the common reference
+        const float l1 = other[qb], r0 = l_tot[qb] == 0.0f ? -INFINITY : ref[qb], r1 = l1 == 0.0f ? -INFINITY : other[2 + qb];
+        const float m = fmaxf(r0, r1);
+        const float w0 = l_tot[qb] == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(r0 - m), w1 = l1 == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(r1 - m);
+        const float inv = 1.0f / (l_tot[qb] * w0 + l1 * w1), a0 = w0 * inv, a1 = w1 * inv;
+        float amax = 0.0f;
+#pragma unroll
+        for (int hb = 0; hb < HB; ++hb) {
+            const f32x4 o1 = *reinterpret_cast<const f32x4*>(ex + (hb * QB + qb) * 1024);
+            float o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = oacc[hb][qb][e] * a0 + o1[e] * a1;
+            const uint2 w = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+            *reinterpret_cast<uint2*>(stage + (qb * 16 + r16) * PITCH + (16 * hb + 4 * g4) * 2) = w;
+            amax = fmaxf(fmaxf(amax, fmaxf(fabsf(bf16lo(w.x)), fabsf(bf16hi(w.x)))), fmaxf(fabsf(bf16lo(w.y)), fabsf(bf16hi(w.y))));
+        }
+        if (p.row_amax != nullptr) {
+            amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
+            amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+            const int qrow = q0 + qb * 16 + r16;
+            if (g4 == 0 && qrow < p.n_tokens) p.row_amax[(int64_t)qrow * p.n_heads + head] = amax;
+        }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the wave's own staging writes have landed
+    constexpr int LPR = HD / 8, RPI = 64 / LPR;             // lanes per row, rows per store instruction
+    const int rl = lane / LPR, ch = lane % LPR;
+    bf16_t* orow = p.o + (int64_t)q0 * p.ldo + head * HD;
+#pragma unroll
+    for (int it = 0; it < 32 / RPI; ++it) {
+        const int rloc = it * RPI + rl;
+        const uint4 v = *reinterpret_cast<const uint4*>(stage + rloc * PITCH + ch * 16);
+        if (q0 + rloc < p.n_tokens) *reinterpret_cast<uint4*>(orow + rloc * p.ldo + ch * 8) = v;
     }
 }
 
@@ -998,7 +1236,8 @@ extern "C" int32_t cdm_attn_fwd_packed_bf16(const void* q, int64_t ldq, const fl
     // 1-D grid of 8 x ceil(heads / 8) x query blocks ids: id % 8 = XCD, see the kernel's placement rule
     // variant 0 = 32 query rows per wave (8 waves, two per SIMD), row maxima dropped where the norm bound allows;
     // cross-check build only: 1 = 64 query rows per wave (4 waves), 2 = variant 0 with the row maxima always taken, 3 =
-    // 128-row workgroups and 4 = 256-row workgroups whatever the grid
+    // 128-row workgroups of four waves and 4 = 256-row workgroups whatever the grid, 5 = 128-row workgroups of two groups from
+    // four key tiles on, 6 = those with the row maxima always taken
     const int variant = cdm_get_variant(0);
     // Small grids: 128-row workgroups of four waves (same arithmetic per row, bit-equal).  A wave then has its SIMD to
     // itself and nothing runs under its exponentials, so such a workgroup takes 0.7 of the time of one with twice the
@@ -1006,10 +1245,15 @@ extern "C" int32_t cdm_attn_fwd_packed_bf16(const void* q, int64_t ldq, const fl
     // 256-row against 128-row workgroups: 32 heads x 128, 512 keys 23.2 -> 17.4 us, 1024 keys (16 per XCD) 34.6 -> 27.2, 2048
     // keys (32 per XCD) 64.6 against 84.8; 16 heads x 64, 1024 keys 21.8 -> 17.3, 4096 keys (32 per XCD) equal.
     const int64_t per_xcd = (n_heads + 7) / 8 * ((n_tokens + BMQ - 1) / BMQ);
-    const bool half_blocks = variant == 3 || ((variant == 0 || variant == 2) && per_xcd <= 16);
+    const bool half_blocks = variant == 3 || variant >= 5 || ((variant == 0 || variant == 2) && per_xcd <= 16);
+    // ... with a second group of four waves that takes every other key tile, where the steps saved outweigh the larger rings and
+    // the exchange of the groups' results (attn_fwd_keys_kernel: from 8 tiles on at head_dim 64, 16 at 128)
+    const int64_t key_tiles = p.n_prefix_tiles + pad_tokens(n_tokens) / BN;
+    const int64_t min_tiles = variant >= 5 ? 4 : head_dim == 64 ? 8 : 16;
+    const bool keys = half_blocks && variant != 3 && key_tiles >= min_tiles && key_tiles <= kMaxKm;
     const int rows_wg = half_blocks ? BMQ / 2 : BMQ;
     p.n_qblocks = (int)((n_tokens + rows_wg - 1) / rows_wg);
-    p.always_max = variant == 2;
+    p.always_max = variant == 2 || variant == 6;
     // the last round's query blocks by key range, if the caller brought the scratch memory for it
     p.split = 1; p.split_tail = 0; p.part_o = nullptr; p.part_lse = nullptr;
     const SplitPlan plan = split_plan(n_tokens, n_heads, head_dim, causal_prefix);
@@ -1031,7 +1275,12 @@ extern "C" int32_t cdm_attn_fwd_packed_bf16(const void* q, int64_t ldq, const fl
     if (variant == 1) { CDM_ATTN_LAUNCH(2, 4); }
     else
 #endif
-    if (half_blocks) { CDM_ATTN_LAUNCH(1, 4); }
+    if (keys) {
+        if (head_dim == 128 && late) attn_fwd_keys_kernel<128, true><<<grid, 512, 0, st>>>(p);
+        else if (head_dim == 128) attn_fwd_keys_kernel<128, false><<<grid, 512, 0, st>>>(p);
+        else if (late) attn_fwd_keys_kernel<64, true><<<grid, 512, 0, st>>>(p);
+        else attn_fwd_keys_kernel<64, false><<<grid, 512, 0, st>>>(p);
+    } else if (half_blocks) { CDM_ATTN_LAUNCH(1, 4); }
     else { CDM_ATTN_LAUNCH(1, 8); }
 #undef CDM_ATTN_LAUNCH
     if (p.split > 1) {

@@ -633,8 +633,8 @@ def test_attention_vs_oracle(n, H, hd, variant):
                                                      (1000, 8, 2, 128, 0, 0, True), (385, 16, 16, 64, 64, 0, False),
                                                      (4096, 8, 8, 128, 0, 0, False), (4097, 8, 8, 128, 0, 0, False)])
 def test_attention_128_row_workgroups_equal_the_256_row_ones(n, H, Hkv, hd, P, causal, qkn, request):
-    """Small grids run on workgroups of 128 query rows (the last two sizes lie on either side of the rule): a row's
-    arithmetic does not depend on the workgroup's size, so the bits do not either."""
+    """Workgroups of 128 query rows and four waves: a row's arithmetic does not depend on the workgroup's size, so the bits do
+    not either.  By default short key sequences take that form, and grids beyond the rule of small ones the 256-row one."""
     request.addfinalizer(lambda: ops.set_variant("attn", 0))
     g = gen(n + H)
     q, _ = rand_bf16((n, H * hd), g)
@@ -650,8 +650,77 @@ def test_attention_128_row_workgroups_equal_the_256_row_ones(n, H, Hkv, hd, P, c
         ops.set_variant("attn", variant)
         amax = torch.zeros((n, H), device=dev())
         res[variant] = (ops.attention_packed(q, img, H, hd, None, cos, sin, norm, prefix, causal, Hkv, row_amax=amax), amax)
-    for variant in (3, 0):
+    for variant in (3, 0) if n in (1, 129, 4097) else (3,):
         assert torch.equal(res[variant][0], res[4][0]) and torch.equal(res[variant][1], res[4][1]), f"variant {variant}"
+
+
+@pytest.mark.parametrize("rot", [True, False])
+@pytest.mark.parametrize("n,H,Hkv,hd,P,causal,scale", [
+    (193, 1, 1, 128, 0, 0, 0.2), (256, 2, 1, 64, 0, 0, 0.2), (257, 3, 3, 128, 0, 0, 0.2), (320, 2, 2, 64, 0, 0, 3.0),
+    (130, 2, 2, 128, 70, 0, 0.2), (130, 2, 2, 128, 1, 0, 3.0), (65, 2, 2, 64, 128, 0, 0.2), (500, 3, 3, 64, 0, 190, 0.2),
+    (512, 2, 1, 128, 0, 512, 0.2), (449, 1, 1, 128, 0, 449, 3.0), (300, 2, 2, 128, 0, 1, 0.2), (4000, 4, 1, 128, 500, 0, 0.2),
+    (4090, 4, 4, 64, 0, 0, 6.0)])
+def test_attention_small_grids_share_the_key_tiles(n, H, Hkv, hd, P, causal, scale, rot, request):
+    """The form of small grids with many key tiles, from four on: two groups of waves take every other tile.  Odd and even tile counts, ragged last
+    and prefix tiles, causal rows that see nothing of a group's tiles, more than 64 tiles, logits of a hundred.  Against
+    64 bits no further off than the one-group kernel (the roundings of Q, P and O are the same ones; a quarter for chance)."""
+    request.addfinalizer(lambda: ops.set_variant("attn", 0))
+    g = gen(n + H + P)
+    q, qr = rand_bf16((n, H * hd), g)
+    k, kr = rand_bf16((n, Hkv * hd), g, scale)
+    v, vr = rand_bf16((n, Hkv * hd), g)
+    ang = torch.rand((n, hd // 2), generator=g) * 6.0
+    cos, sin = (ang.cos().to(dev()), ang.sin().to(dev())) if rot else (None, None)
+    img = ops.attention_pack_kv(k, v, Hkv, hd, None, cos, sin)
+    kp, kpr = rand_bf16((max(P, 1), Hkv * hd), g, scale)
+    vp, vpr = rand_bf16((max(P, 1), Hkv * hd), g)
+    prefix = (ops.attention_pack_kv(kp, vp, Hkv, hd), P) if P else None
+    res = {}
+    for variant in (3, 5, 6):
+        ops.set_variant("attn", variant)
+        amax = torch.zeros((n, H), device=dev())
+        o = ops.attention_packed(q, img, H, hd, None, cos, sin, None, prefix, causal, Hkv, row_amax=amax)
+        again = ops.attention_packed(q, img, H, hd, None, cos, sin, None, prefix, causal, Hkv)
+        assert torch.equal(o, again) and torch.equal(amax, o.float().view(n, H, hd).abs().amax(-1))
+        res[variant] = o.double().view(n, H, hd)
+
+    def rotated(x):
+        x = x.double().to(dev()).view(n, -1, hd)
+        if not rot:
+            return x
+        c, s, a, b = cos.double()[:, None], sin.double()[:, None], x[..., :hd // 2], x[..., hd // 2:]
+        return torch.cat([a * c - b * s, b * c + a * s], -1)
+    qd, kd, vd = rotated(qr), rotated(kr).to(torch.bfloat16).double(), vr.double().to(dev()).view(n, Hkv, hd)
+    if P:
+        kd = torch.cat([kpr.double().to(dev()).view(P, Hkv, hd), kd])
+        vd = torch.cat([vpr.double().to(dev()).view(P, Hkv, hd), vd])
+    keep = torch.ones((n, n + P), dtype=torch.bool, device=dev())
+    if causal:
+        keep[:causal] = torch.arange(n, device=dev())[None] <= torch.arange(causal, device=dev())[:, None]
+    want = torch.empty_like(res[3])
+    for h in range(H):
+        sc = qd[:, h] @ kd[:, h // (H // Hkv)].t() * hd ** -0.5
+        want[:, h] = torch.softmax(sc.masked_fill(~keep, -math.inf), -1) @ vd[:, h // (H // Hkv)]
+    rel = lambda a, b: ((a - b).norm() / b.norm()).item()
+    ref = rel(res[3], want)
+    for variant in (5, 6):
+        assert bool(torch.isfinite(res[variant]).all()) and rel(res[variant], want) <= 1.25 * ref + 1e-4, (variant, rel(res[variant], want), ref)
+
+
+@pytest.mark.parametrize("n", [256, 300])
+def test_attention_shared_key_tiles_keep_infinities(n, request):
+    """An infinite value reaches the rows that see it and nothing else, whatever the tile it sits in."""
+    request.addfinalizer(lambda: ops.set_variant("attn", 0))
+    g, hd, H = gen(n), 64, 2
+    q, k, v = (rand_bf16((n, H * hd), g)[0] for _ in range(3))
+    v[n - 1, 5] = math.inf
+    img = ops.attention_pack_kv(k, v, H, hd)
+    ops.set_variant("attn", 5)
+    got = ops.attention_packed(q, img, H, hd)
+    ops.set_variant("attn", 3)
+    want = ops.attention_packed(q, img, H, hd)
+    assert torch.equal(torch.isinf(got), torch.isinf(want)) and torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.isinf(got[:, 5]).all() and bool(torch.isfinite(got[:, 6:]).all())
 
 
 @pytest.mark.parametrize("variant", [0, 1])
