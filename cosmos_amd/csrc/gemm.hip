@@ -480,7 +480,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
         bn = (nb0 + bn) < p.N ? bn : p.N - 1 - nb0;
         ob[i] = (uint32_t)(bn * (int)p.ldw + chunk * 16);
     }
-    const char* abase = reinterpret_cast<const char*>(p.A) + (int64_t)m0 * p.lda;
+    const char* abase = reinterpret_cast<const char*>(tile.A) + (int64_t)m0 * p.lda;
     const char* wbase = reinterpret_cast<const char*>(tile.W) + (int64_t)nb0 * p.ldw;
     const char* w2base = EPI == CDM_EPI_SWIGLU ? reinterpret_cast<const char*>(tile.W2) + (int64_t)nb0 * p.ldw : wbase;
 
@@ -576,7 +576,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         bn = (n0 + bn) < p.N ? bn : p.N - 1 - n0;
         ob[j] = (uint32_t)(bn * (int)p.ldw + chunk * 16);
     }
-    const char* abase = reinterpret_cast<const char*>(p.A) + (int64_t)m0 * p.lda;
+    const char* abase = reinterpret_cast<const char*>(tile.A) + (int64_t)m0 * p.lda;
     const char* wbase = reinterpret_cast<const char*>(tile.W) + (int64_t)n0 * p.ldw;
     const char* w2base = EPI == CDM_EPI_SWIGLU ? reinterpret_cast<const char*>(tile.W2) + (int64_t)n0 * p.ldw : wbase;
     const uint32_t l0 = lds_addr_of(s_ring) + wave * 1024;
@@ -760,7 +760,7 @@ int32_t validate(const char* who, int esize, const void* A, int64_t lda, const v
 // host-side description of one row segment of a (grouped) GEMM
 struct HostSeg {
     int64_t start, len;
-    const void* W; const void* W2;
+    const void* A; const void* W; const void* W2;
     const float* gate; const float* sw; const float* sw2; const float* knw;
 };
 
@@ -812,7 +812,7 @@ int32_t run(GemmParams p, const HostSeg* segs, int n_seg, int32_t epilogue, hipS
             if (segs[i].len == 0) continue;
             GemmSeg& g = p.seg[ns++];
             g.m_start = (int)segs[i].start; g.m_end = (int)(segs[i].start + segs[i].len);
-            g.W = segs[i].W; g.W2 = segs[i].W2; g.gate = segs[i].gate; g.sw = segs[i].sw; g.sw2 = segs[i].sw2;
+            g.A = segs[i].A; g.W = segs[i].W; g.W2 = segs[i].W2; g.gate = segs[i].gate; g.sw = segs[i].sw; g.sw2 = segs[i].sw2;
             g.knw = segs[i].knw;
         }
         if (ns == 0) break;
@@ -852,7 +852,7 @@ int32_t grouped(const char* who, const void* A, int64_t lda, const float* sa, co
                 const void* R, int64_t ldr, const float* const* gate, const float* cos, const float* sin,
                 int64_t rope_cols, int32_t head_dim, void* stream, const GemmParams* pack = nullptr,
                 const float* k_norm_rows = nullptr, float* row_amax = nullptr, int64_t amax_ld = 0, void* scratch = nullptr,
-                int64_t scratch_bytes = 0) {
+                int64_t scratch_bytes = 0, const void* const* runs = nullptr) {
     constexpr int esize = FP8 ? 1 : 2;
     CDM_REQUIRE(A && W && C && seg_start && seg_len, CDM_ERR_BAD_ARG, "%s: null pointer", who);
     CDM_REQUIRE((epilogue == CDM_EPI_QKV_PACK) == (pack != nullptr), CDM_ERR_BAD_ARG,
@@ -873,7 +873,9 @@ int32_t grouped(const char* who, const void* A, int64_t lda, const float* sa, co
     for (int g = 0; g < n_seg; ++g) {
         CDM_REQUIRE(seg_start[g] >= 0 && seg_len[g] >= 0, CDM_ERR_BAD_ARG, "%s: negative segment", who);
         CDM_REQUIRE(W[g], CDM_ERR_BAD_ARG, "%s: null weight for segment %d", who, g);
-        int32_t rc = validate(who, esize, A, lda, W[g], ldw, W2 ? W2[g] : nullptr, C, ldc, seg_len[g], N, K, epilogue, R, ldr,
+        const void* a = runs ? runs[g] : A;
+        CDM_REQUIRE(a || seg_len[g] == 0, CDM_ERR_BAD_ARG, "%s: null rows of segment %d", who, g);
+        int32_t rc = validate(who, esize, a, lda, W[g], ldw, W2 ? W2[g] : nullptr, C, ldc, seg_len[g], N, K, epilogue, R, ldr,
                               cos, sin, rope_cols, head_dim);
         if (rc) return rc;
         const float* gt = gate ? gate[g] : nullptr;
@@ -885,7 +887,8 @@ int32_t grouped(const char* who, const void* A, int64_t lda, const float* sa, co
         for (int h = 0; h < g; ++h)
             CDM_REQUIRE(seg_start[g] >= segs[h].start + segs[h].len || seg_start[g] + seg_len[g] <= segs[h].start,
                         CDM_ERR_BAD_ARG, "%s: segments %d and %d overlap", who, h, g);
-        segs[g] = HostSeg{seg_start[g], seg_len[g], W[g], W2 ? W2[g] : nullptr, gt, FP8 ? sw[g] : nullptr,
+        if (runs) a = (const void*)((uintptr_t)a - (uintptr_t)(seg_start[g] * lda * esize));      // an address, not an object, until rows are added
+        segs[g] = HostSeg{seg_start[g], seg_len[g], a, W[g], W2 ? W2[g] : nullptr, gt, FP8 ? sw[g] : nullptr,
                           (FP8 && sw2) ? sw2[g] : nullptr, k_norm_rows ? k_norm_rows + (int64_t)g * head_dim : nullptr};
         if (seg_start[g] + seg_len[g] > max_end) max_end = seg_start[g] + seg_len[g];
     }
@@ -894,7 +897,7 @@ int32_t grouped(const char* who, const void* A, int64_t lda, const float* sa, co
     int32_t rc = cdm_require_device();
     if (rc) return rc;
     GemmParams p{};
-    p.A = A; p.lda = lda * esize; p.ldw = ldw * esize; p.sa = sa;
+    p.lda = lda * esize; p.ldw = ldw * esize; p.sa = sa;
     p.C = (bf16_t*)C; p.ldc = ldc;
     p.N = (int)N; p.K = (int)K;
     p.R = (const bf16_t*)R; p.ldr = ldr;
@@ -912,7 +915,8 @@ template <bool FP8>
 int32_t qkv_pack(const char* who, const void* A, int64_t lda, const float* sa, const void* const* W, const float* const* sw,
                  int64_t ldw, void* Q, int64_t ldq, const int64_t* seg_start, const int64_t* seg_len, int32_t n_seg,
                  int64_t K, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, const float* cos, const float* sin,
-                 const cdm_qk_norm* qk_norm, void* workspace, int64_t workspace_bytes, void* stream) {
+                 const cdm_qk_norm* qk_norm, void* workspace, int64_t workspace_bytes, void* stream,
+                 const void* const* runs = nullptr) {
     CDM_REQUIRE(seg_start && seg_len && workspace, CDM_ERR_BAD_ARG, "%s: null pointer", who);
     CDM_REQUIRE(head_dim == 128 || head_dim == 64, CDM_ERR_UNSUPPORTED, "%s: head_dim=%d (the fused images need 64 or 128)", who,
                 head_dim);
@@ -958,7 +962,7 @@ int32_t qkv_pack(const char* who, const void* A, int64_t lda, const float* sa, c
     pack.k_eps = qk_norm ? qk_norm->eps : 0.0f;
     int32_t rc = grouped<FP8>(who, A, lda, sa, W, sw, ldw, nullptr, nullptr, Q, ldq, seg_start, seg_len, n_seg, d_q + 2 * d_kv, K,
                               CDM_EPI_QKV_PACK, nullptr, 0, nullptr, cos, sin, d_q, head_dim, stream, &pack,
-                              qk_norm ? qk_norm->k_weight : nullptr);
+                              qk_norm ? qk_norm->k_weight : nullptr, nullptr, 0, nullptr, 0, runs);
     return rc;
 }
 
@@ -982,6 +986,28 @@ extern "C" int32_t cdm_grouped_gemm_qkv_pack_fp8(const void* Aq, int64_t lda, co
                                                  void* workspace, int64_t workspace_bytes, void* stream) {
     return qkv_pack<true>("grouped_gemm_qkv_pack_fp8", Aq, lda, sa, Wq, sw, ldw, Q, ldq, seg_start, seg_len, n_seg, K,
                           n_heads, n_kv_heads, head_dim, cos, sin, qk_norm, workspace, workspace_bytes, stream);
+}
+
+extern "C" int32_t cdm_grouped_gemm_qkv_pack_runs_bf16(const void* const* A, int64_t lda, const void* const* W, int64_t ldw, void* Q,
+                                                       int64_t ldq, const int64_t* seg_start, const int64_t* seg_len,
+                                                       int32_t n_seg, int64_t K, int32_t n_heads, int32_t n_kv_heads,
+                                                       int32_t head_dim, const float* cos, const float* sin,
+                                                       const cdm_qk_norm* qk_norm, void* workspace, int64_t workspace_bytes,
+                                                       void* stream) {
+    const char* who = "grouped_gemm_qkv_pack_runs_bf16";
+    CDM_REQUIRE(A && n_seg >= 1, CDM_ERR_BAD_ARG, "%s: no runs", who);
+    return qkv_pack<false>(who, A[0], lda, nullptr, W, nullptr, ldw, Q, ldq, seg_start, seg_len, n_seg, K, n_heads, n_kv_heads,
+                           head_dim, cos, sin, qk_norm, workspace, workspace_bytes, stream, A);
+}
+
+extern "C" int32_t cdm_grouped_gemm_runs_bf16(const void* const* A, int64_t lda, const void* const* W, int64_t ldw, void* C,
+                                              int64_t ldc, const int64_t* seg_start, const int64_t* seg_len, int32_t n_seg,
+                                              int64_t N, int64_t K, void* stream) {
+    const char* who = "grouped_gemm_runs_bf16";
+    CDM_REQUIRE(A && n_seg >= 1, CDM_ERR_BAD_ARG, "%s: no runs", who);
+    return grouped<false>(who, A[0], lda, nullptr, W, nullptr, ldw, nullptr, nullptr, C, ldc, seg_start, seg_len, n_seg, N, K,
+                          CDM_EPI_NONE, nullptr, 0, nullptr, nullptr, nullptr, 0, 0, stream, nullptr, nullptr, nullptr, 0, nullptr, 0,
+                          A);
 }
 
 extern "C" int32_t cdm_gemm_bf16(const void* A, int64_t lda, const void* W, int64_t ldw, const void* W2, void* C,

@@ -16,6 +16,7 @@ constexpr int kMaxSeg = 8;
 struct GemmSeg {
     int m_start, m_end;                  // token rows [m_start, m_end)
     int tiles_m, tile_end;               // row tiles of the segment; tiles of segments 0..this one
+    const void* A;                       // row 0 of the sequence as this segment's operand rows count (the runs may lie apart)
     const void* W; const void* W2;
     const float* gate;
     const float* sw; const float* sw2;   // fp8 only
@@ -23,8 +24,7 @@ struct GemmSeg {
 };
 
 struct GemmParams {
-    const void* A; int64_t lda;          // operand strides in BYTES
-    int64_t ldw;
+    int64_t lda, ldw;                    // operand strides in BYTES
     const float* sa;                     // fp8 only: per-row scale of A, indexed by the global row
     bf16_t* C; int64_t ldc;              // fp32 storage behind the same pointers for CDM_EPI_GATE_RESIDUAL_F32
     int N, K;
@@ -49,7 +49,7 @@ struct GemmParams {
 // what a workgroup works on
 struct Tile {
     int m0, m_end, tn, part;
-    const void* W; const void* W2;
+    const void* A; const void* W; const void* W2;
     const float* gate; const float* sw; const float* sw2; const float* knw;
 };
 
@@ -91,7 +91,7 @@ __device__ __forceinline__ bool locate_tile(const GemmParams& p, Tile& t) {
     t.m0 = __builtin_amdgcn_readfirstlane(sg.m_start + (first_m + in_group % gsz) * TM);
     t.m_end = __builtin_amdgcn_readfirstlane(sg.m_end);
     t.tn = __builtin_amdgcn_readfirstlane(in_group / gsz);
-    t.W = uniform_ptr(sg.W); t.W2 = uniform_ptr(sg.W2);
+    t.A = uniform_ptr(sg.A); t.W = uniform_ptr(sg.W); t.W2 = uniform_ptr(sg.W2);
     t.gate = uniform_ptr(sg.gate); t.sw = uniform_ptr(sg.sw); t.sw2 = uniform_ptr(sg.sw2); t.knw = uniform_ptr(sg.knw);
     return true;
 }

@@ -227,7 +227,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
         if (r8 < TM) {
             const int am = (m0 + row) < tile.m_end ? row : tile.m_end - 1 - m0;
             off[j] = (uint32_t)(am * (int)p.lda + chunk * 16);
-            base[j] = uniform_ptr(reinterpret_cast<const char*>(p.A) + (int64_t)m0 * p.lda + (int64_t)kt0 * 128);
+            base[j] = uniform_ptr(reinterpret_cast<const char*>(tile.A) + (int64_t)m0 * p.lda + (int64_t)kt0 * 128);
         } else {
             const int wr = row - TM;
             // SWIGLU: 64-row groups of the tile alternate gate / up

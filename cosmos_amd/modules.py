@@ -123,18 +123,25 @@ class DMAttnProcessor:
             raise ValueError("image_rotary_emb=(cos, sin) is required")
         batched = hidden_states.dim() == 3
         x = _as2d(hidden_states)
-        n_enc = 0
+        n_enc, runs = 0, None
         if encoder_hidden_states is not None:
             # diffusers joint-attention convention: context tokens first, then the latent tokens
             if quant_scale is not None or residual is not None:
                 raise NotImplementedError("encoder_hidden_states cannot be combined with fused residual / fp8 input")
             enc = _as2d(encoder_hidden_states)
-            n_enc = enc.shape[0]
-            x = torch.cat([enc, x], dim=0)
+            n_enc, n_lat = enc.shape[0], x.shape[0]
+            # the projection reads the two runs where they lie, if they are laid out alike; otherwise they are joined first
+            if (modality_segments is None and self.rope != "gemm_epilogue" and not attn.fp8 and n_enc > 0 and n_lat > 0
+                    and all(t.is_cuda and t.device == x.device and t.dtype == torch.bfloat16 and t.shape[1] == attn.d_model
+                            and t.stride(1) == 1 and t.stride(0) == x.stride(0) and t.stride(0) >= t.shape[1]
+                            and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (enc, x))):
+                runs = [enc, x]
+            else:
+                x = torch.cat([enc, x], dim=0)
             if modality_segments is None:
                 dm = min(1, attn.n_branches - 1)      # branch 0 serves the context tokens
-                modality_segments = [(0, n_enc, 0, False), (n_enc, x.shape[0] - n_enc, dm, True)]
-        n, d = x.shape[0], attn.d_model
+                modality_segments = [(0, n_enc, 0, False), (n_enc, n_lat, dm, True)]
+        n, d = x.shape[0] + (n_enc if runs is not None else 0), attn.d_model
         if modality_segments is None:
             modality_segments = [(0, n, 0, True)]
         cos, sin = image_rotary_emb
@@ -162,12 +169,12 @@ class DMAttnProcessor:
             if wsb is None:
                 wsb = torch.empty((ops.attn_workspace_total_bytes(n, attn.n_heads, attn.n_kv_heads, attn.head_dim),),
                                   dtype=torch.uint8, device=x.device)
-            attn._qkv_pack(x, quant_scale, modality_segments, qkv, wsb, cos, sin, qkn)
+            attn._qkv_pack(x if runs is None else runs, quant_scale, modality_segments, qkv, wsb, cos, sin, qkn)
             o_amax = ws.o_amax if (attn.fp8 and ws is not None and ws.fp8) else None
             ops.attention_packed(q, wsb, attn.n_heads, attn.head_dim, o, cos, sin, qkn, prefix, causal_prefix,
                                  attn.n_kv_heads, row_amax=o_amax)
         else:
-            attn._linear(x, quant_scale, "qkv", modality_segments, out=qkv, epilogue="none")
+            attn._linear(x if runs is None else runs, quant_scale, "qkv", modality_segments, out=qkv, epilogue="none")
             if self.rope == "streaming":
                 if attn.n_kv_heads == attn.n_heads:
                     ops.mrope_qk_(q, k, cos, sin, attn.n_heads, attn.head_dim)

@@ -306,6 +306,14 @@ def gemm_fp8(aq: torch.Tensor, sa: torch.Tensor, wq: torch.Tensor, sw: torch.Ten
     return out
 
 
+def _run_ptrs(runs: Sequence[torch.Tensor], segments: Sequence[Tuple[int, int]]):
+    """Pointers and row stride of the rows of every segment, kept in tensors of their own."""
+    k, ld = runs[0].shape[1], runs[0].stride(0)
+    if len(runs) != len(segments) or any(r.shape != (int(l), k) or r.stride(0) != ld for r, (_, l) in zip(runs, segments)):
+        raise ValueError("one tensor of rows per segment, all of one width and row stride")
+    return (C.c_void_p * len(runs))(*[_chk(r, "run", torch.bfloat16, 2) for r in runs]), ld
+
+
 @_timed("gemm")
 def grouped_gemm(a: torch.Tensor, ws: Sequence[torch.Tensor], segments: Sequence[Tuple[int, int]], *,
                  w2s: Optional[Sequence[torch.Tensor]] = None, epilogue: str = "none", residual=None,
@@ -314,6 +322,11 @@ def grouped_gemm(a: torch.Tensor, ws: Sequence[torch.Tensor], segments: Sequence
     """MoT routed linear: rows [start, start+len) of ``a`` use ws[g] (w2s[g], gates[g]).  ``a`` may be a list of the segments'
     rows (epilogue "none")."""
     lib = _lib.load()
+    runs = None if isinstance(a, torch.Tensor) else list(a)
+    if runs is not None:
+        if epilogue != "none" or w2s is not None or out is None:
+            raise ValueError("separate runs take the plain epilogue and an output")
+        a = runs[0]
     M, K = a.shape
     N = ws[0].shape[0]
     n_seg = len(segments)
@@ -325,6 +338,16 @@ def grouped_gemm(a: torch.Tensor, ws: Sequence[torch.Tensor], segments: Sequence
             raise ValueError("all segment weights must share shape and row stride")
     PP = C.c_void_p * n_seg
     wp = PP(*[_chk(w, "w", torch.bfloat16, 2) for w in ws])
+    if runs is not None:
+        ap, lda = _run_ptrs(runs, segments)
+        I64 = C.c_int64 * n_seg
+        if out.shape[0] < max(int(s) + int(l) for s, l in segments) or out.shape[1] != N:
+            raise ValueError("out shape mismatch")
+        rc = lib.cdm_grouped_gemm_runs_bf16(ap, lda, wp, ldw, _chk(out, "out", torch.bfloat16, 2), out.stride(0),
+                                            I64(*[int(s) for s, _ in segments]), I64(*[int(l) for _, l in segments]), n_seg, N, K,
+                                            _stream())
+        _lib.check(rc, "cdm_grouped_gemm_runs_bf16")
+        return out
     w2p = PP(*[_chk(w, "w2", torch.bfloat16, 2) for w in w2s]) if w2s is not None else None
     gp = PP(*[(_f32vec(g, "gate", N) or None) for g in gates]) if gates is not None else None
     I64 = C.c_int64 * n_seg
@@ -402,6 +425,8 @@ def gemm_qkv_pack(a: torch.Tensor, sa: Optional[torch.Tensor], ws: Sequence[torc
     given.  Raises where the fused form does not apply (``qkv_pack_applies`` tells beforehand).  ``a`` may be a list of the
     segments' rows (bf16)."""
     lib = _lib.load()
+    runs = None if isinstance(a, torch.Tensor) else list(a)
+    a = a if runs is None else runs[0]
     M, K = a.shape
     n_seg = len(segments)
     ldw = ws[0].stride(0)
@@ -420,9 +445,10 @@ def gemm_qkv_pack(a: torch.Tensor, sa: Optional[torch.Tensor], ws: Sequence[torc
             workspace.numel(), _stream())
     if sa is None:
         wp = PP(*[_chk(w, "w", torch.bfloat16, 2) for w in ws])
-        rc = lib.cdm_grouped_gemm_qkv_pack_bf16(_chk(a, "a", torch.bfloat16, 2), a.stride(0), wp, ldw,
-                                                _chk(q_out, "q_out", torch.bfloat16, 2), q_out.stride(0), st, ln, n_seg, K,
-                                                n_heads, n_kv_heads, head_dim, *tail)
+        fn, given = ((lib.cdm_grouped_gemm_qkv_pack_bf16, (_chk(a, "a", torch.bfloat16, 2), a.stride(0))) if runs is None else
+                     (lib.cdm_grouped_gemm_qkv_pack_runs_bf16, _run_ptrs(runs, segments)))
+        rc = fn(*given, wp, ldw, _chk(q_out, "q_out", torch.bfloat16, 2), q_out.stride(0), st, ln, n_seg, K, n_heads, n_kv_heads,
+                head_dim, *tail)
         _lib.check(rc, "cdm_grouped_gemm_qkv_pack_bf16")
     else:
         N = ws[0].shape[0]

@@ -345,6 +345,19 @@ int32_t cdm_grouped_gemm_scratch_bf16(const void* A, int64_t lda, const void* co
                                       int32_t epilogue, const void* R, int64_t ldr, const float* const* gate, void* scratch,
                                       int64_t scratch_bytes, void* stream);
 
+/*
+ * Epilogue NONE, and the fused QKV projection, on runs that lie apart: A[g] points at the first row of segment g (all runs with
+ * row stride lda); rows of C, the rotary tables and the images keep their place in the joint sequence.
+ */
+int32_t cdm_grouped_gemm_runs_bf16(const void* const* A, int64_t lda, const void* const* W, int64_t ldw, void* C, int64_t ldc,
+                                   const int64_t* seg_start, const int64_t* seg_len, int32_t n_seg, int64_t N, int64_t K,
+                                   void* stream);
+int32_t cdm_grouped_gemm_qkv_pack_runs_bf16(const void* const* A, int64_t lda, const void* const* W, int64_t ldw, void* Q,
+                                            int64_t ldq, const int64_t* seg_start, const int64_t* seg_len, int32_t n_seg,
+                                            int64_t K, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, const float* cos,
+                                            const float* sin, const cdm_qk_norm* qk_norm, void* workspace,
+                                            int64_t workspace_bytes, void* stream);
+
 /* The same for e4m3 operands (see cdm_gemm_fp8): sa is the per-token scale of the whole sequence, sw[g] / sw2[g] the
  * per-output-channel scales of segment g's weights. */
 int32_t cdm_grouped_gemm_fp8(const void* Aq, int64_t lda, const float* sa, const void* const* Wq,

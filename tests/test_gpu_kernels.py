@@ -182,6 +182,31 @@ def test_gemm_cut_along_k(lens, N, K, epi):
         assert bool((err <= tol).all()), (i, err.max().item())
 
 
+@pytest.mark.parametrize("lens", [(77, 1560), (1, 1), (64, 200), (128, 5000)])
+@pytest.mark.parametrize("pitch", [512, 520])
+def test_gemm_of_runs_that_lie_apart(lens, pitch):
+    """Projections of two runs in tensors of their own: the bits of the joined rows, plain and with the fused key images."""
+    g, K, H, hd = gen(sum(lens) + pitch), 512, 4, 128
+    runs = [torch.randn((n, pitch), generator=g).to(dev(), torch.bfloat16)[:, :K] for n in lens]
+    ws = [(torch.randn((3 * H * hd, K), generator=g) * 0.05).to(dev(), torch.bfloat16) for _ in lens]
+    segs, n = [(0, lens[0]), (lens[0], lens[1])], sum(lens)
+    joined = torch.cat(runs)
+    out, ref = (torch.full((n, 3 * H * hd), float("nan"), dtype=torch.bfloat16, device=dev()) for _ in range(2))
+    ops.grouped_gemm(runs, ws, segs, out=out)
+    ops.grouped_gemm(joined, ws, segs, out=ref)
+    assert torch.equal(out, ref)
+    if ops.qkv_pack_applies(segs, hd, H, H):
+        ang = torch.rand((n, hd // 2), generator=g)
+        cos, sin = ang.cos().to(dev()), ang.sin().to(dev())
+        res = []
+        for a in (runs, joined):
+            img = torch.zeros(ops.attn_workspace_bytes(n, H, hd), dtype=torch.uint8, device=dev())
+            q = torch.zeros((n, H * hd), dtype=torch.bfloat16, device=dev())
+            ops.gemm_qkv_pack(a, None, ws, None, segs, H, H, hd, q, img, cos, sin)
+            res.append((q, img))
+        assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
+
+
 @pytest.mark.parametrize("freq,d", [(256, 1024), (4, 4), (260, 68), (256, 4096)])
 def test_timestep_mlp(freq, d):
     """Against the same MLP in 64 bits behind the same sinusoid; fp32 sums of up to 4096 terms: 1e-5."""
