@@ -408,9 +408,11 @@ def _routed_linear(a, sa, weights, qweights, weights2, segments, *, out, epilogu
 
 
 def _plain(lin: nn.Module, device: torch.device, dtype: torch.dtype) -> bool:
-    """An ``nn.Linear`` with bias as it stands - no subclass, wrapper or hook whose forward a kernel on its parameters would
-    pass by - whose parameters such a kernel can read."""
+    """An ``nn.Linear`` with bias as it stands - no subclass, wrapper, replaced forward or hook that a kernel on its parameters
+    would pass by, no gradient asked of it - whose parameters such a kernel can read."""
     return (type(lin) is nn.Linear and lin.bias is not None and not lin._forward_hooks and not lin._forward_pre_hooks
+            and "forward" not in lin.__dict__
+            and not (torch.is_grad_enabled() and (lin.weight.requires_grad or lin.bias.requires_grad))
             and all(p.device == device and p.dtype == dtype and p.is_contiguous() for p in (lin.weight, lin.bias))
             and lin.weight.data_ptr() % 16 == 0 and lin.in_features % 8 == 0 and lin.in_features <= 16384)
 
@@ -421,7 +423,8 @@ def _modulations(blocks: Sequence["DMBlock"], temb: torch.Tensor) -> List[Tuple[
     if not lins:
         return []
     w = lins[0].weight
-    if temb.is_cuda and all(_plain(l, temb.device, torch.bfloat16) and l.weight.shape == w.shape for l in lins):
+    wants_grad = temb.requires_grad and torch.is_grad_enabled()
+    if temb.is_cuda and not wants_grad and all(_plain(l, temb.device, torch.bfloat16) and l.weight.shape == w.shape for l in lins):
         m = ops.adaln_modulation(temb.reshape(-1).to(torch.float32), [l.weight for l in lins], [l.bias for l in lins])
     else:      # other parameter types, wrapped layers: the layer itself
         m = torch.stack([l(torch.nn.functional.silu(temb.reshape(1, -1).to(l.weight.dtype))).float().reshape(-1) for l in lins])
@@ -532,7 +535,7 @@ class TimestepEmbedder(nn.Module):
 
     def sinusoid(self, t: torch.Tensor) -> torch.Tensor:
         half = self.freq_dim // 2
-        if t.is_cuda and self.freq_dim % 2 == 0:
+        if t.is_cuda and self.freq_dim % 2 == 0 and not (t.requires_grad and torch.is_grad_enabled()):
             return ops.timestep_sinusoid(t.reshape(-1).to(torch.float32).contiguous(), self.freq_dim)
         k = torch.arange(half, dtype=torch.float32, device=t.device)
         f = torch.exp(-math.log(10000.0) * k / half)
@@ -700,7 +703,8 @@ class DMStack(nn.Module):
             raise ValueError(f"{what} sequence has shape {(rows, *parts[0].shape[1:])}, expected {(n, d)}")
         dev = parts[0].device
         first = self.blocks[0] if len(self.blocks) else None      # a subclass or a hook may read its input: it gets it filled
-        if (type(first) is DMBlock and not first._forward_pre_hooks and self.cfg.residual_fp32 and dev.type == "cuda" and d % 8 == 0
+        if (type(first) is DMBlock and "forward" not in first.__dict__ and not first._forward_pre_hooks and self.cfg.residual_fp32
+                and dev.type == "cuda" and d % 8 == 0
                 and all(p.dtype == torch.bfloat16 and p.device == dev and p.is_contiguous() and p.data_ptr() % 16 == 0 for p in parts)):
             return torch.empty((n, d), dtype=torch.float32, device=dev), list(parts)
         return self._stream(*parts), None
@@ -905,8 +909,9 @@ class DMTransformer(nn.Module):
                 raise ValueError(f"this configuration expects {name}_states")
             emb[name] = _edge_linear(p_in, _as2d(given[name]).to(dt)) + embed
         # only the stream is read here (a subclass or a hook sees the whole result)
-        kw = {"joint_only": True} if type(self.stack) is DMStack and not self.stack._forward_hooks else {}
-        res = self.stack(tok, timestep, encoder_hidden_states=None if context_cache is not None else encoder_hidden_states,
+        stk = self.stack
+        kw = {"joint_only": True} if type(stk) is DMStack and "forward" not in stk.__dict__ and not stk._forward_hooks else {}
+        res = stk(tok, timestep, encoder_hidden_states=None if context_cache is not None else encoder_hidden_states,
                          action_states=emb.get("action"), return_dict=True, context_cache=context_cache,
                          audio_states=emb.get("audio"), **kw)
         joint = res["joint"]            # with a context cache: the generator tokens only

@@ -233,6 +233,29 @@ def test_conditioning_honours_wrapped_layers():
     assert torch.allclose(hooked, plain + 1.0, rtol=1e-5, atol=1e-5)      # fp32 sums in two orders
 
 
+def test_conditioning_honours_replaced_forwards_and_gradients():
+    """A forward set on the instance is called, and a gradient that is asked for reaches parameters and inputs."""
+    from cosmos_amd import DMBlock, TimestepEmbedder
+    te, t = TimestepEmbedder(64, device=dev()), torch.tensor([3.0], device=dev())
+    blk = DMBlock(64, 1, 64, 128, 1, device=dev())
+    blk.reset_parameters(torch.Generator(device=dev()).manual_seed(1))
+    lin, c = blk.adaLN_modulation, torch.randn((1, 64), generator=gen(2)).to(dev())
+    with torch.no_grad():
+        plain = te(t)
+        inner = te.linear_2.forward
+        te.linear_2.forward = lambda x: inner(x) + 1.0
+        assert torch.allclose(te(t), plain + 1.0, rtol=1e-5, atol=1e-5)      # fp32 sums in two orders
+        shift = blk.modulation(c)[0]
+        del te.linear_2.forward
+    lin.bias.requires_grad_(True)
+    got = blk.modulation(c.requires_grad_(True))[0]
+    assert (got - shift).abs().max() <= 2 ** -7 * shift.abs().max()          # each rounded once to bf16
+    got.sum().backward()
+    assert torch.equal(lin.bias.grad[:64], torch.ones_like(lin.bias[:64])) and c.grad is not None
+    te.sinusoid(t.requires_grad_(True)).sum().backward()
+    assert t.grad is not None
+
+
 @pytest.mark.parametrize("hd,H,sections", [(64, 16, (16, 24, 24)), (128, 4, (32, 48, 48))])
 def test_mrope_standalone(hd, H, sections):
     g = gen(hd)
