@@ -702,6 +702,8 @@ class DMStack(nn.Module):
         if rows != n or any(p.dim() != 2 or p.shape[1] != d for p in parts):
             raise ValueError(f"{what} sequence has shape {(rows, *parts[0].shape[1:])}, expected {(n, d)}")
         dev = parts[0].device
+        if any(p.device != dev for p in parts):
+            raise RuntimeError(f"the runs of the {what} sequence lie on different devices")
         first = self.blocks[0] if len(self.blocks) else None      # a subclass or a hook may read its input: it gets it filled
         if (type(first) is DMBlock and "forward" not in first.__dict__ and not first._forward_pre_hooks and self.cfg.residual_fp32
                 and dev.type == "cuda" and d % 8 == 0

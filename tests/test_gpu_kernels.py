@@ -256,6 +256,14 @@ def test_conditioning_honours_replaced_forwards_and_gradients():
     assert t.grad is not None
 
 
+def test_stack_refuses_runs_on_different_devices():
+    from cosmos_amd import DMConfig, DMStack
+    st = DMStack(DMConfig("t", 256, 2, 128, 512, 1, (2, 4, 9), n_text=37), device=dev())
+    x = torch.zeros((1, 72, 256), device=dev(), dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError):
+        st(x, torch.tensor([5.0], device=dev()), encoder_hidden_states=torch.zeros((1, 37, 256), dtype=torch.bfloat16))
+
+
 @pytest.mark.parametrize("hd,H,sections", [(64, 16, (16, 24, 24)), (128, 4, (32, 48, 48))])
 def test_mrope_standalone(hd, H, sections):
     g = gen(hd)
