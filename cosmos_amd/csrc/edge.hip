@@ -3,6 +3,8 @@
 // dozen elements wide).  Such a layer moves the token rows once - it is bound by HBM, not by the matrix cores - and has
 // K or N far below what the tiled GEMM needs, so it gets a small kernel of its own: 64 token rows per workgroup, all
 // output columns walked in passes, operands staged through LDS in 256-byte row pieces.
+#include <type_traits>
+
 #include "cdm_common.h"
 
 namespace {
@@ -174,6 +176,101 @@ __global__ __launch_bounds__(256) void edge_linear_kernel(const EdgeParams p) {
     }
 }
 
+// Narrow outputs (N <= 64) of wide rows, un-patchify and the action / audio outputs: 16 RB token rows per workgroup, whose eight
+// waves share K out in 64-element steps (wave w: steps w, w + 8, ...), fragments straight from memory - two k-steps of a row at a
+// time, whole 128-byte lines - with the next step's in flight, and add up their fp32 sums through LDS in wave order.
+// The walk over K is a serial chain of loads: 64-row workgroups of the kernel above take 32 chunks of 128 at K = 4096 one after the
+// other, and 3,520 rows are 55 of them on 256 CUs.  Here a wave has K / 512 steps.  What is left is the latency of those steps
+// and every workgroup's read of W from L2.  N = 64, in us, kernel above / RB = 1 / RB = 2:
+//     K = 4096: 256 rows 47.7 / 19.5 / 23.4   3520 60.2 / 22.2 / 27.0   7000 62.8 / 43.9 / 29.9   14080 64.8 / 82.6 / 56.0   28160 73.6 / 144 / 109
+//     K = 1024: 256 rows 11.1 / 6.4 / 7.8     3520 14.0 / 6.8 / 8.0     7000 14.3 / 12.0 / 8.1    14080 17.4 / 24.2 / 16.1
+//     K = 128:  256 rows 7.3 / 3.9 / 4.1      3520 7.5 / 4.0 / 3.9      7000 7.6 / 4.2 / 4.0      28160 7.0 / 12.1 / 9.9
+// RB = 4 spills and is slower than the kernel above wherever that is slower than RB = 2.  Error against 64 bits: the same.
+constexpr int kSplitWaves = 8;
+template <int RB>
+__global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_eu(2, 4))) void edge_narrow_kernel(const EdgeParams p) {
+    constexpr int NB = 4, PITCH = NB * 64 + 16;              // bytes per fp32 row (the pad spreads rows over banks)
+    __shared__ __attribute__((aligned(16))) char smem[kSplitWaves * 16 * PITCH];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, g4 = lane >> 4;
+    const int m0 = blockIdx.x * (16 * RB);
+    const bf16_t* arow[RB];
+    const bf16_t* wrow[NB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+        const int m = m0 + 16 * rb + r16;
+        arow[rb] = p.A + (int64_t)(m < p.M ? m : p.M - 1) * p.lda;
+    }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+        const int n = 16 * nb + r16;
+        wrow[nb] = p.W + (int64_t)(n < p.N ? n : p.N - 1) * p.ldw;
+    }
+    const int steps = (p.K + 63) >> 6;
+    uint4 a[2][RB][2], w[2][NB][2];
+    auto fetch = [&](auto set_c, int s) {
+        constexpr int SET = decltype(set_c)::value;
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) a[SET][rb][h] = load_chunk<true>(arow[rb], s * 64 + h * 32 + g4 * 8, p.K);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) w[SET][nb][h] = load_chunk<true>(wrow[nb], s * 64 + h * 32 + g4 * 8, p.K);
+    };
+    f32x4 acc[RB][NB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) acc[rb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto mma = [&](auto set_c) {
+        constexpr int SET = decltype(set_c)::value;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+                    acc[rb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[SET][nb][h]),
+                                                                          __builtin_bit_cast(bf16x8, a[SET][rb][h]), acc[rb][nb], 0, 0, 0);
+    };
+    using S0 = std::integral_constant<int, 0>;
+    using S1 = std::integral_constant<int, 1>;
+    if (wave < steps) fetch(S0{}, wave);
+    for (int s = wave; s < steps; s += 2 * kSplitWaves) {
+        if (s + kSplitWaves < steps) fetch(S1{}, s + kSplitWaves);
+        mma(S0{});
+        if (s + kSplitWaves >= steps) break;
+        if (s + 2 * kSplitWaves < steps) fetch(S0{}, s + 2 * kSplitWaves);
+        mma(S1{});
+    }
+    // the lane owns token row r16 of a block and columns 16 nb + 4 g4 .. + 3; a thread finishes two columns of a row
+    const int row = tid >> 5, n = (tid & 31) * 2;
+    float b0 = 0.0f, b1 = 0.0f;
+    if (p.bias != nullptr && n < p.N) {                      // N % 8 == 0: two columns are in or out together
+        const uint32_t b = *reinterpret_cast<const uint32_t*>(p.bias + n);
+        b0 = bf16lo(b); b1 = bf16hi(b);
+    }
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+        if (rb) __syncthreads();                             // the sums of the block before have been read
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+            *reinterpret_cast<f32x4*>(smem + (wave * 16 + r16) * PITCH + (16 * nb + 4 * g4) * 4) = acc[rb][nb];
+        __syncthreads();
+        float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kSplitWaves; ++i) {
+            const float2 v = *reinterpret_cast<const float2*>(smem + (i * 16 + row) * PITCH + n * 4);
+            s0 += v.x; s1 += v.y;
+        }
+        const int m = m0 + 16 * rb + row;
+        if (m < p.M && n < p.N) *reinterpret_cast<uint32_t*>(p.C + (int64_t)m * p.ldc + n) = pack_bf16x2(s0 + b0, s1 + b1);
+    }
+}
+
 }  // namespace
 
 extern "C" int32_t cdm_linear_bias_bf16(const void* A, int64_t lda, const void* W, int64_t ldw, const void* bias, void* C,
@@ -194,6 +291,13 @@ extern "C" int32_t cdm_linear_bias_bf16(const void* A, int64_t lda, const void* 
     if (rc) return rc;
     EdgeParams p{(const bf16_t*)A, lda, (const bf16_t*)W, ldw, (const bf16_t*)bias, (bf16_t*)C, ldc, (int)M, (int)N, (int)K, 1};
     hipStream_t st = (hipStream_t)stream;
+    // narrow outputs of few rows: as long as a workgroup of 16, then 32 rows has a CU to itself (see edge_narrow_kernel; at 14,080
+    // rows the two forms are level over the widths, and the 64-row form reads W less often)
+    if (vec && N <= 64 && K > 64 && M <= 32 * 256) {
+        if (M <= 16 * 256) edge_narrow_kernel<1><<<(unsigned)((M + 15) / 16), 64 * kSplitWaves, 0, st>>>(p);
+        else edge_narrow_kernel<2><<<(unsigned)((M + 31) / 32), 64 * kSplitWaves, 0, st>>>(p);
+        return cdm_check_launch("linear_bias");
+    }
     const int64_t gx = (M + EM - 1) / EM;
     const int wr = N <= 64 ? 64 : 128;
     const int64_t passes = (N + wr - 1) / wr;

@@ -508,6 +508,23 @@ def test_linear_bias_at_the_stack_edges(M, N, K, bias):
     assert torch.equal(again, ops.linear_bias(x[:, :K].contiguous(), w, b))
 
 
+@pytest.mark.parametrize("M,N,K,bias", [(1, 8, 72, True), (15, 64, 4096, True), (17, 64, 1024, False), (33, 56, 200, True), (64, 16, 576, True),
+                                        (4100, 64, 2048, True), (8209, 40, 1088, True)])
+def test_linear_bias_narrow_outputs(M, N, K, bias):
+    """Few output columns of wide rows, whose K the waves of a workgroup share out: remainders of rows, columns and k-steps.  fp32
+    sums of exact products (at most K 2^-24 of the sum of their magnitudes) and one rounding to bf16, 2^-8 of the value at most."""
+    g = gen(M + N + K)
+    x, xr = rand_bf16((M, K + 8), g)
+    w, wr = rand_bf16((N, K), g, 0.1)
+    b, br = rand_bf16((N,), g) if bias else (torch.zeros(N), torch.zeros(N))
+    out = torch.full((M + 1, N + 8), 7.0, dtype=torch.bfloat16, device=dev())
+    got = ops.linear_bias(x[:, :K], w, b if bias else None, out=out[:M, :N]).cpu().double()
+    xd, wd = xr[:, :K].double(), wr.double()
+    want, mag = xd @ wd.t() + br.double(), xd.abs() @ wd.abs().t() + br.double().abs()
+    assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -24 * mag).all())
+    assert bool((out[M:] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
+
+
 def test_grouped_gemm_three_segments():
     g = gen(77)
     K, N = 256, 264
