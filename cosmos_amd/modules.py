@@ -407,29 +407,39 @@ def _routed_linear(a, sa, weights, qweights, weights2, segments, *, out, epilogu
                          head_dim=head_dim, out=out, row_amax=row_amax)
 
 
+def _as_is(m: nn.Module, cls: type) -> bool:
+    """Calling ``m`` runs the forward of ``cls`` and nothing else: no subclass, forward set on the instance or hook."""
+    return type(m) is cls and "forward" not in m.__dict__ and not m._forward_hooks and not m._forward_pre_hooks
+
+
 def _plain(lin: nn.Module, device: torch.device, dtype: torch.dtype) -> bool:
     """An ``nn.Linear`` with bias as it stands - no subclass, wrapper, replaced forward or hook that a kernel on its parameters
     would pass by, no gradient asked of it - whose parameters such a kernel can read."""
-    return (type(lin) is nn.Linear and lin.bias is not None and not lin._forward_hooks and not lin._forward_pre_hooks
-            and "forward" not in lin.__dict__
+    return (_as_is(lin, nn.Linear) and lin.bias is not None
             and not (torch.is_grad_enabled() and (lin.weight.requires_grad or lin.bias.requires_grad))
             and all(p.device == device and p.dtype == dtype and p.is_contiguous() for p in (lin.weight, lin.bias))
             and lin.weight.data_ptr() % 16 == 0 and lin.in_features % 8 == 0 and lin.in_features <= 16384)
 
 
-def _modulations(blocks: Sequence["DMBlock"], temb: torch.Tensor) -> List[Tuple[torch.Tensor, ...]]:
-    """(shift1, scale1, gate1, shift2, scale2, gate2), each [d] fp32, of every block: one launch over all of them."""
-    lins = [b.adaLN_modulation for b in blocks]
-    if not lins:
-        return []
-    w = lins[0].weight
+def _modulations(lins: Sequence[nn.Module], temb: torch.Tensor) -> Optional[List[Tuple[torch.Tensor, ...]]]:
+    """(shift1, scale1, gate1, shift2, scale2, gate2), each [d] fp32, of every block from its modulation layer: one launch over
+    all of them.  None where a kernel on their parameters cannot stand in for the layers."""
     wants_grad = temb.requires_grad and torch.is_grad_enabled()
-    if temb.is_cuda and not wants_grad and all(_plain(l, temb.device, torch.bfloat16) and l.weight.shape == w.shape for l in lins):
-        m = ops.adaln_modulation(temb.reshape(-1).to(torch.float32), [l.weight for l in lins], [l.bias for l in lins])
-    else:      # other parameter types, wrapped layers: the layer itself
-        m = torch.stack([l(torch.nn.functional.silu(temb.reshape(1, -1).to(l.weight.dtype))).float().reshape(-1) for l in lins])
+    if not lins or not temb.is_cuda or wants_grad or not all(_plain(l, temb.device, torch.bfloat16) for l in lins):
+        return None
+    if any(l.weight.shape != lins[0].weight.shape for l in lins):
+        return None
+    m = ops.adaln_modulation(temb.reshape(-1).to(torch.float32), [l.weight for l in lins], [l.bias for l in lins])
     rows = m.view(6 * len(lins), -1).unbind(0)
     return [rows[6 * i:6 * i + 6] for i in range(len(lins))]
+
+
+def _bare(blk: Optional[nn.Module]) -> bool:
+    """A block in which only this file's code runs, so that a stack may do parts of its work ahead of its call.  Any other block
+    (a subclass, a wrapper, hooks that change ``temb`` or load weights, a replaced processor) may read, change or ignore what
+    it is called with, and the blocks behind it."""
+    return (_as_is(blk, DMBlock) and "modulation" not in blk.__dict__ and _as_is(blk.attn, DMAttention)
+            and type(blk.attn.processor) is DMAttnProcessor)
 
 
 class DMBlock(nn.Module):
@@ -472,7 +482,13 @@ class DMBlock(nn.Module):
 
     def modulation(self, temb: torch.Tensor) -> Tuple[torch.Tensor, ...]:
         """(shift1, scale1, gate1, shift2, scale2, gate2), each [d] fp32, from the conditioning vector."""
-        return _modulations([self], temb)[0]
+        lin = self.adaLN_modulation
+        mods = _modulations([lin], temb)
+        if mods is not None:
+            return mods[0]
+        # other parameter types, wrapped layers: the layer itself
+        m = lin(torch.nn.functional.silu(temb.reshape(1, -1).to(lin.weight.dtype))).float().reshape(-1)
+        return tuple(t.contiguous() for t in m.chunk(6))
 
     def _norm(self, x, weights, shift, scale, segments, ws, sources=None):
         """Per-branch adaLN-RMSNorm of x (bf16 or fp32) into the workspace: y (bf16), or (e4m3, per-token scale) for
@@ -630,8 +646,9 @@ class DMStack(nn.Module):
         images = []
         for blk in self.blocks:
             img = torch.empty((nbytes,), dtype=torch.uint8, device=x.device)
+            kw = {} if sources is None else {"sources": sources}
             blk(x, None, rot, segs, inplace=True, workspace=ws, modulation=(None,) * 6, causal_prefix=c.n_text,
-                kv_images=img, sources=sources)
+                kv_images=img, **kw)
             sources = None
             images.append(img)
         return ContextCache(images, c.n_text)
@@ -666,10 +683,8 @@ class DMStack(nn.Module):
         temb = self.time_embedder(timestep.reshape(-1)[:1])
         if self._ws is None or not self._ws.fits(c.n_tokens, c.d_model, c.hidden, c.fp8) or self._ws.y.device != x.device:
             self._ws = Workspace(c.n_tokens, c.d_model, c.hidden, c.n_heads, c.head_dim, x.device, c.kv_heads, c.fp8)
-        for blk, mod in zip(self.blocks, _modulations(self.blocks, temb)):
-            blk(x, temb, rot, segs, inplace=True, modulation=mod, workspace=self._ws,
-                causal_prefix=c.n_text if c.hybrid_mask else 0, sources=sources)
-            sources = None
+        kw = {"causal_prefix": c.n_text if c.hybrid_mask else 0}
+        self._run_blocks(x, temb, rot, segs, self._ws, sources, [kw] * len(self.blocks))
         return self._result(x, c.n_text, hidden_states.dim() == 3, return_dict, joint_only)
 
     def capture(self, hidden_states: torch.Tensor, timestep: torch.Tensor,
@@ -705,11 +720,21 @@ class DMStack(nn.Module):
         if any(p.device != dev for p in parts):
             raise RuntimeError(f"the runs of the {what} sequence lie on different devices")
         first = self.blocks[0] if len(self.blocks) else None      # a subclass or a hook may read its input: it gets it filled
-        if (type(first) is DMBlock and "forward" not in first.__dict__ and not first._forward_pre_hooks and self.cfg.residual_fp32
-                and dev.type == "cuda" and d % 8 == 0
+        if (_bare(first) and self.cfg.residual_fp32 and dev.type == "cuda" and d % 8 == 0
                 and all(p.dtype == torch.bfloat16 and p.device == dev and p.is_contiguous() and p.data_ptr() % 16 == 0 for p in parts)):
             return torch.empty((n, d), dtype=torch.float32, device=dev), list(parts)
         return self._stream(*parts), None
+
+    def _run_blocks(self, x: torch.Tensor, temb: torch.Tensor, rot, segs, workspace: Workspace, sources, kws: Sequence[dict]) -> None:
+        """All blocks over the stream x.  Their modulation comes from one launch ahead of the first where all of them are bare;
+        otherwise every block computes its own from the ``temb`` that reaches it, in its own call."""
+        mods = _modulations([b.adaLN_modulation for b in self.blocks], temb) if all(_bare(b) for b in self.blocks) else None
+        for i, (blk, kw) in enumerate(zip(self.blocks, kws)):
+            if mods is not None:
+                kw = {**kw, "modulation": mods[i]}
+            if i == 0 and sources is not None:
+                kw = {**kw, "sources": sources}
+            blk(x, temb, rot, segs, inplace=True, workspace=workspace, **kw)
 
     def _result(self, x: torch.Tensor, first_video: int, batched: bool, return_dict: bool, joint_only: bool):
         """The video rows of the final stream as bf16 (the transformer's output dtype); "joint" is the stream itself."""
@@ -720,7 +745,6 @@ class DMStack(nn.Module):
         if return_dict:
             return {"sample": out, "joint": x}
         return (out,)
-
 
     def _generator_extras(self, audio_states, action_states) -> List[torch.Tensor]:
         """The audio and action runs that follow the video tokens in the joint sequence."""
@@ -748,9 +772,7 @@ class DMStack(nn.Module):
         temb = self.time_embedder(timestep.reshape(-1)[:1])
         if self._ws_gen is None or not self._ws_gen.fits(n, c.d_model, c.hidden, c.fp8) or self._ws_gen.y.device != x.device:
             self._ws_gen = Workspace(n, c.d_model, c.hidden, c.n_heads, c.head_dim, x.device, c.kv_heads, c.fp8)
-        for blk, img, mod in zip(self.blocks, cache.images, _modulations(self.blocks, temb)):
-            blk(x, temb, self._rot_gen, segs, inplace=True, modulation=mod, workspace=self._ws_gen, prefix=(img, P), sources=sources)
-            sources = None
+        self._run_blocks(x, temb, self._rot_gen, segs, self._ws_gen, sources, [{"prefix": (img, P)} for img in cache.images])
         return self._result(x, 0, hidden_states.dim() == 3, return_dict, joint_only)
 
 
@@ -912,7 +934,7 @@ class DMTransformer(nn.Module):
             emb[name] = _edge_linear(p_in, _as2d(given[name]).to(dt)) + embed
         # only the stream is read here (a subclass or a hook sees the whole result)
         stk = self.stack
-        kw = {"joint_only": True} if type(stk) is DMStack and "forward" not in stk.__dict__ and not stk._forward_hooks else {}
+        kw = {"joint_only": True} if _as_is(stk, DMStack) else {}
         res = stk(tok, timestep, encoder_hidden_states=None if context_cache is not None else encoder_hidden_states,
                          action_states=emb.get("action"), return_dict=True, context_cache=context_cache,
                          audio_states=emb.get("audio"), **kw)

@@ -7,6 +7,7 @@ import torch
 import oracle as O
 from cosmos_amd import CONFIGS, DMBlock, DMStack, ops, rotary
 from cosmos_amd.config import DMConfig
+from altered_blocks import ALTERED, alter_block
 from gpu_util import BF16_COS, BF16_REL, FP8_COS, FP8_REL, assert_close, dev, oracle_weights, rand_bf16, record
 
 pytestmark = pytest.mark.gpu
@@ -826,3 +827,29 @@ def test_stack_forward_recorded_as_a_graph():
         graphed(**{**first, "hidden_states": mk(cfg.n_video - 1)})
     with pytest.raises(ValueError):
         graphed(**{**first, "audio_states": None})
+
+
+@pytest.mark.parametrize("kind,i", [("", 0)] + ALTERED)
+def test_stack_of_altered_blocks_equals_the_chain_of_its_blocks(kind, i):
+    """A stack whose block i is not a plain one: the bits of block after block over the joined runs, each with the modulation of the
+    ``temb``, weights and methods that it has when it runs (one launch per block: the sums of the launch over all of them)."""
+    cfg = DMConfig("t", 256, 2, 128, 512, 2, (2, 4, 9), n_text=37)
+    st = DMStack(cfg, device=dev())
+    st.reset_parameters(3)
+    g = torch.Generator().manual_seed(4)
+    ctx, x = rand_bf16((1, 37, 256), g)[0], rand_bf16((1, 72, 256), g)[0]
+    t = torch.tensor([500.0], device=dev())
+    blocks = list(st.blocks)
+    with torch.no_grad():
+        for b in blocks:
+            b.adaLN_modulation.bias.copy_(torch.randn(6 * 256, generator=g))
+    eff = alter_block(kind, st, i)
+    got = st(x, t, encoder_hidden_states=ctx, return_dict=True)["joint"]
+    with torch.no_grad():
+        temb, s = st.time_embedder(t), torch.cat([ctx[0], x[0]]).float()
+        for blk, e in zip(blocks, eff):
+            lin, c = (blk.adaLN_modulation, temb * e) if isinstance(e, float) else (e, temb)
+            w, b = lin.weight.data, lin.bias.data
+            mod = ops.adaln_modulation(c.reshape(-1), [w], [b]).view(6, -1).unbind(0)
+            DMBlock.forward(blk, s, None, st.rotary(dev()), st.segments(), inplace=True, modulation=mod)
+    assert torch.equal(got, s)

@@ -5,6 +5,7 @@ import torch
 import oracle as O
 from cosmos_amd import CONFIGS, rotary
 from cosmos_amd.config import DMConfig
+from altered_blocks import ALTERED, alter_block
 
 
 @pytest.mark.parametrize("n_text,grid,n_action", [(0, (4, 16, 16), 0), (5, (2, 3, 4), 0), (7, (2, 4, 3), 6)])
@@ -92,3 +93,28 @@ def test_unipc_coefficient_rows_on_the_host(monkeypatch, order, corrector, solve
         sampler.UniPCStepper([0.5, 0.7, 0.0])
     with pytest.raises(ValueError):
         sampler.UniPCStepper(sig, solver_order=4)
+
+
+@pytest.mark.parametrize("kind,i", [("", 0)] + ALTERED)
+def test_blocks_compute_their_own_modulation(kind, i, monkeypatch):
+    """The shift vectors that reach the norms of a stack whose block i is not a plain one: those of the ``temb``, weights and
+    methods that the block has when it runs.  The kernels are replaced by stubs."""
+    from cosmos_amd import ops
+    from cosmos_amd.modules import DMStack
+    cfg = DMConfig("t", 128, 2, 64, 256, 2, (2, 4, 4), mrope_sections=(16, 24, 24))
+    st = DMStack(cfg, device="cpu")
+    st.reset_parameters(3)
+    blocks, shifts = list(st.blocks), []
+    monkeypatch.setattr(ops, "adaln_rmsnorm_grouped", lambda x, ws, shift, *rest: shifts.append(shift[0].clone()))
+    for name in ("gemm", "grouped_gemm", "gemm_qkv_pack", "attention_packed", "attention"):
+        monkeypatch.setattr(ops, name, lambda *a, **kw: None)
+    x, t = torch.randn(1, cfg.n_tokens, 128).to(torch.bfloat16), torch.tensor([400.0])
+    eff = alter_block(kind, st, i)
+    st(x, t)
+    assert len(shifts) == 4
+    with torch.no_grad():
+        temb = st.time_embedder(t).to(torch.bfloat16)
+    for b, e in enumerate(eff):
+        lin, c = (blocks[b].adaLN_modulation, temb * e) if isinstance(e, float) else (e, temb)
+        want = torch.nn.functional.linear(torch.nn.functional.silu(c), lin.weight, lin.bias).float().view(6, -1)
+        assert torch.equal(shifts[2 * b], want[0]) and torch.equal(shifts[2 * b + 1], want[3]), f"block {b}"
