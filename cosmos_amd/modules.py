@@ -18,6 +18,7 @@ from typing import List, Optional, Sequence, Tuple
 
 import torch
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook as _any_module_hook
 
 from . import ops, rotary
 from .config import DMConfig
@@ -409,7 +410,8 @@ def _routed_linear(a, sa, weights, qweights, weights2, segments, *, out, epilogu
 
 def _as_is(m: nn.Module, cls: type) -> bool:
     """Calling ``m`` runs the forward of ``cls`` and nothing else: no subclass, forward set on the instance or hook."""
-    return type(m) is cls and "forward" not in m.__dict__ and not m._forward_hooks and not m._forward_pre_hooks
+    return (type(m) is cls and "forward" not in m.__dict__ and not m._forward_hooks and not m._forward_pre_hooks
+            and not _any_module_hook())
 
 
 def _plain(lin: nn.Module, device: torch.device, dtype: torch.dtype) -> bool:

@@ -853,3 +853,25 @@ def test_stack_of_altered_blocks_equals_the_chain_of_its_blocks(kind, i):
             mod = ops.adaln_modulation(c.reshape(-1), [w], [b]).view(6, -1).unbind(0)
             DMBlock.forward(blk, s, None, st.rotary(dev()), st.segments(), inplace=True, modulation=mod)
     assert torch.equal(got, s)
+
+
+def test_stack_under_hooks_of_every_module():
+    """A hook registered for all modules sees the conditioning layers called and the first block's input joined."""
+    cfg = DMConfig("t", 256, 2, 128, 512, 1, (2, 4, 9), n_text=37)
+    st = DMStack(cfg, device=dev())
+    st.reset_parameters(3)
+    g = torch.Generator().manual_seed(4)
+    ctx, x = rand_bf16((1, 37, 256), g)[0], rand_bf16((1, 72, 256), g)[0]
+    t, seen = torch.tensor([500.0], device=dev()), {}
+
+    def note(m, a):
+        seen[m] = a[0].clone()
+
+    hook = torch.nn.modules.module.register_module_forward_pre_hook(note)
+    try:
+        st(x, t, encoder_hidden_states=ctx)
+    finally:
+        hook.remove()
+    te, blk = st.time_embedder, st.blocks[0]
+    assert all(m in seen for m in (te.linear_1, te.linear_2, blk.adaLN_modulation))
+    assert torch.equal(seen[blk], torch.cat([ctx[0], x[0]]).float())
