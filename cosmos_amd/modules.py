@@ -414,6 +414,12 @@ def _as_is(m: nn.Module, cls: type) -> bool:
             and not _any_module_hook())
 
 
+def _eager() -> bool:
+    """No forward-mode derivative or function transform (``torch.func``) is under way, which a kernel that takes pointers would drop
+    or could not read: a tensor that carries a tangent has no mark of its own to ask for."""
+    return torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
+
+
 def _plain(lin: nn.Module, device: torch.device, dtype: torch.dtype) -> bool:
     """An ``nn.Linear`` with bias as it stands - no subclass, wrapper, replaced forward or hook that a kernel on its parameters
     would pass by, no gradient asked of it - whose parameters such a kernel can read."""
@@ -427,7 +433,7 @@ def _modulations(lins: Sequence[nn.Module], temb: torch.Tensor) -> Optional[List
     """(shift1, scale1, gate1, shift2, scale2, gate2), each [d] fp32, of every block from its modulation layer: one launch over
     all of them.  None where a kernel on their parameters cannot stand in for the layers."""
     wants_grad = temb.requires_grad and torch.is_grad_enabled()
-    if not lins or not temb.is_cuda or wants_grad or not all(_plain(l, temb.device, torch.bfloat16) for l in lins):
+    if not lins or not _eager() or not temb.is_cuda or wants_grad or not all(_plain(l, temb.device, torch.bfloat16) for l in lins):
         return None
     if any(l.weight.shape != lins[0].weight.shape for l in lins):
         return None
@@ -553,7 +559,7 @@ class TimestepEmbedder(nn.Module):
 
     def sinusoid(self, t: torch.Tensor) -> torch.Tensor:
         half = self.freq_dim // 2
-        if t.is_cuda and self.freq_dim % 2 == 0 and not (t.requires_grad and torch.is_grad_enabled()):
+        if _eager() and t.is_cuda and self.freq_dim % 2 == 0 and not (t.requires_grad and torch.is_grad_enabled()):
             return ops.timestep_sinusoid(t.reshape(-1).to(torch.float32).contiguous(), self.freq_dim)
         k = torch.arange(half, dtype=torch.float32, device=t.device)
         f = torch.exp(-math.log(10000.0) * k / half)
@@ -562,7 +568,7 @@ class TimestepEmbedder(nn.Module):
 
     def forward(self, t: torch.Tensor) -> torch.Tensor:
         l1, l2 = self.linear_1, self.linear_2
-        if (t.is_cuda and t.numel() == 1 and not torch.is_grad_enabled() and _plain(l1, t.device, torch.float32)
+        if (_eager() and t.is_cuda and t.numel() == 1 and not torch.is_grad_enabled() and _plain(l1, t.device, torch.float32)
                 and _plain(l2, t.device, torch.float32) and l1.in_features == self.freq_dim
                 and l2.weight.shape == (l1.out_features, l1.out_features)):
             return ops.timestep_mlp(t.reshape(-1).to(torch.float32), l1.weight, l1.bias, l2.weight, l2.bias)

@@ -256,6 +256,42 @@ def test_conditioning_honours_replaced_forwards_and_gradients():
     assert t.grad is not None
 
 
+@pytest.mark.parametrize("grad", [True, False])
+def test_conditioning_carries_tangents_and_function_transforms(grad):
+    """Forward-mode derivatives and torch.func transforms of the conditioning layers, against the same layers in 64 bits on the CPU
+    (fp32 embedder 1e-5; the modulation's bf16 layer rounds the activation, its tangent and both results: 2^-6)."""
+    import copy
+    from cosmos_amd import DMBlock, TimestepEmbedder
+    rel = lambda a, b: ((a.double().cpu() - b).norm() / b.norm()).item()
+    te, t = TimestepEmbedder(64, device=dev()), torch.tensor([3.0], device=dev())
+    te64 = copy.deepcopy(te).cpu().double()
+    blk = DMBlock(64, 1, 64, 128, 1, device=dev())
+    blk.reset_parameters(torch.Generator(device=dev()).manual_seed(1))
+    lin, c = copy.deepcopy(blk.adaLN_modulation).cpu().double(), torch.randn((1, 64), generator=gen(2)).to(dev())
+    mod64 = lambda c: lin(torch.nn.functional.silu(c)).reshape(6, -1)[0]
+
+    def embed64(t):
+        a = t.reshape(-1, 1) * torch.exp(-math.log(10000.0) * torch.arange(128, dtype=torch.float64) / 128)
+        return te64.linear_2(torch.nn.functional.silu(te64.linear_1(torch.cat([a.cos(), a.sin()], -1))))
+
+    with torch.set_grad_enabled(grad):
+        one = torch.ones_like(t)
+        want, dwant = torch.func.jvp(embed64, (t.cpu().double(),), (one.cpu().double(),))
+        got, dgot = torch.func.jvp(te, (t,), (one,))
+        assert rel(got.detach(), want.detach()) < 1e-5 and rel(dgot.detach(), dwant.detach()) < 1e-5
+        with torch.autograd.forward_ad.dual_level():
+            dual = te(torch.autograd.forward_ad.make_dual(t, one))
+            tangent = torch.autograd.forward_ad.unpack_dual(dual).tangent
+            assert tangent is not None and rel(tangent.detach(), dwant.detach()) < 1e-5
+        ts = torch.tensor([[3.0], [250.5], [999.0]], device=dev())
+        each = torch.stack([embed64(x.cpu().double()).detach() for x in ts])
+        # (angles of up to 1000 carry a relative error of 2^-24)
+        assert rel(torch.func.vmap(te)(ts).detach(), each) < 1e-4
+        want, dwant = torch.func.jvp(mod64, (c.cpu().double(),), (torch.ones(1, 64, dtype=torch.float64),))
+        got, dgot = torch.func.jvp(lambda c: blk.modulation(c)[0], (c,), (torch.ones_like(c),))
+        assert rel(got.detach(), want.detach()) < 2 ** -6 and rel(dgot.detach(), dwant.detach()) < 2 ** -6
+
+
 def test_stack_refuses_runs_on_different_devices():
     from cosmos_amd import DMConfig, DMStack
     st = DMStack(DMConfig("t", 256, 2, 128, 512, 1, (2, 4, 9), n_text=37), device=dev())
