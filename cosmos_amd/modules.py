@@ -416,8 +416,10 @@ def _as_is(m: nn.Module, cls: type) -> bool:
 
 def _eager() -> bool:
     """No forward-mode derivative or function transform (``torch.func``) is under way, which a kernel that takes pointers would drop
-    or could not read: a tensor that carries a tangent has no mark of its own to ask for."""
-    return torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
+    or could not read (a tensor that carries a tangent has no mark of its own to ask for), and no autocast, which chooses the
+    type a linear layer computes in and returns."""
+    return (torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
+            and not torch.is_autocast_enabled("cuda"))
 
 
 def _plain(lin: nn.Module, device: torch.device, dtype: torch.dtype) -> bool:

@@ -292,6 +292,20 @@ def test_conditioning_carries_tangents_and_function_transforms(grad):
         assert rel(got.detach(), want.detach()) < 2 ** -6 and rel(dgot.detach(), dwant.detach()) < 2 ** -6
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_conditioning_under_autocast(dt):
+    """Autocast decides the type of the embedder's linear layers and the precision of the modulation's."""
+    from cosmos_amd import DMBlock, TimestepEmbedder
+    te, t = TimestepEmbedder(64, device=dev()), torch.tensor([3.0], device=dev())
+    blk = DMBlock(64, 1, 64, 128, 1, device=dev())
+    blk.reset_parameters(torch.Generator(device=dev()).manual_seed(1))
+    lin, c = blk.adaLN_modulation, torch.randn((1, 64), generator=gen(2)).to(dev())
+    with torch.no_grad(), torch.autocast("cuda", dtype=dt):
+        got, shift = te(t), blk.modulation(c)[0]
+        want = lin(torch.nn.functional.silu(c.to(torch.bfloat16))).float()[0, :64]
+    assert got.dtype == dt and torch.equal(shift, want)
+
+
 def test_stack_refuses_runs_on_different_devices():
     from cosmos_amd import DMConfig, DMStack
     st = DMStack(DMConfig("t", 256, 2, 128, 512, 1, (2, 4, 9), n_text=37), device=dev())
