@@ -414,12 +414,16 @@ def _as_is(m: nn.Module, cls: type) -> bool:
             and not _any_module_hook())
 
 
-def _eager() -> bool:
-    """No forward-mode derivative or function transform (``torch.func``) is under way, which a kernel that takes pointers would drop
-    or could not read (a tensor that carries a tangent has no mark of its own to ask for), and no autocast, which chooses the
-    type a linear layer computes in and returns."""
-    return (torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
-            and not torch.is_autocast_enabled("cuda"))
+def _eager(*tensors: torch.Tensor) -> bool:
+    """Plain tensors in plain eager execution, where a kernel that takes their pointers may stand in for torch operators: no
+    compilation, tracing or dispatch mode that has to see the operators, no subclass whose storage is not the value, no
+    forward-mode derivative or function transform (``torch.func``; a tensor that carries a tangent has no mark of its own to ask
+    for), and no autocast, which chooses the type a linear layer computes in and returns."""
+    if torch.compiler.is_compiling():
+        return False
+    return (all(type(t) in (torch.Tensor, nn.Parameter) for t in tensors) and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._get_tracing_state() is None and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0 and not torch.is_autocast_enabled("cuda"))
 
 
 def _plain(lin: nn.Module, device: torch.device, dtype: torch.dtype) -> bool:
@@ -427,7 +431,8 @@ def _plain(lin: nn.Module, device: torch.device, dtype: torch.dtype) -> bool:
     would pass by, no gradient asked of it - whose parameters such a kernel can read."""
     return (_as_is(lin, nn.Linear) and lin.bias is not None
             and not (torch.is_grad_enabled() and (lin.weight.requires_grad or lin.bias.requires_grad))
-            and all(p.device == device and p.dtype == dtype and p.is_contiguous() for p in (lin.weight, lin.bias))
+            and all(type(p) in (torch.Tensor, nn.Parameter) and p.device == device and p.dtype == dtype and p.is_contiguous()
+                    for p in (lin.weight, lin.bias))
             and lin.weight.data_ptr() % 16 == 0 and lin.in_features % 8 == 0 and lin.in_features <= 16384)
 
 
@@ -435,7 +440,7 @@ def _modulations(lins: Sequence[nn.Module], temb: torch.Tensor) -> Optional[List
     """(shift1, scale1, gate1, shift2, scale2, gate2), each [d] fp32, of every block from its modulation layer: one launch over
     all of them.  None where a kernel on their parameters cannot stand in for the layers."""
     wants_grad = temb.requires_grad and torch.is_grad_enabled()
-    if not lins or not _eager() or not temb.is_cuda or wants_grad or not all(_plain(l, temb.device, torch.bfloat16) for l in lins):
+    if not lins or not _eager(temb) or not temb.is_cuda or wants_grad or not all(_plain(l, temb.device, torch.bfloat16) for l in lins):
         return None
     if any(l.weight.shape != lins[0].weight.shape for l in lins):
         return None
@@ -561,7 +566,7 @@ class TimestepEmbedder(nn.Module):
 
     def sinusoid(self, t: torch.Tensor) -> torch.Tensor:
         half = self.freq_dim // 2
-        if _eager() and t.is_cuda and self.freq_dim % 2 == 0 and not (t.requires_grad and torch.is_grad_enabled()):
+        if _eager(t) and t.is_cuda and self.freq_dim % 2 == 0 and not (t.requires_grad and torch.is_grad_enabled()):
             return ops.timestep_sinusoid(t.reshape(-1).to(torch.float32).contiguous(), self.freq_dim)
         k = torch.arange(half, dtype=torch.float32, device=t.device)
         f = torch.exp(-math.log(10000.0) * k / half)
@@ -570,7 +575,7 @@ class TimestepEmbedder(nn.Module):
 
     def forward(self, t: torch.Tensor) -> torch.Tensor:
         l1, l2 = self.linear_1, self.linear_2
-        if (_eager() and t.is_cuda and t.numel() == 1 and not torch.is_grad_enabled() and _plain(l1, t.device, torch.float32)
+        if (_eager(t) and t.is_cuda and t.numel() == 1 and not torch.is_grad_enabled() and _plain(l1, t.device, torch.float32)
                 and _plain(l2, t.device, torch.float32) and l1.in_features == self.freq_dim
                 and l2.weight.shape == (l1.out_features, l1.out_features)):
             return ops.timestep_mlp(t.reshape(-1).to(torch.float32), l1.weight, l1.bias, l2.weight, l2.bias)

@@ -306,6 +306,28 @@ def test_conditioning_under_autocast(dt):
     assert got.dtype == dt and torch.equal(shift, want)
 
 
+@pytest.mark.parametrize("how", ["jit", "fx", "fake", "compile"])
+def test_conditioning_is_traced_as_operators(how):
+    """What records or replaces torch operators sees the embedder's: a recording on one timestep serves another."""
+    from cosmos_amd import TimestepEmbedder
+    te, t, other = TimestepEmbedder(64, device=dev()), torch.tensor([3.0], device=dev()), torch.tensor([700.0], device=dev())
+    with torch.no_grad():
+        want = te(other)
+        if how == "jit":
+            f = torch.jit.trace(te, (t,), check_trace=False)
+        elif how == "fx":
+            from torch.fx.experimental.proxy_tensor import make_fx
+            f = make_fx(te)(t)
+        elif how == "fake":
+            from torch._subclasses.fake_tensor import FakeTensorMode
+            with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+                assert te(mode.from_tensor(t)).shape == (1, 64)
+            return
+        else:
+            f = torch.compile(te, backend="eager", fullgraph=True)
+        assert torch.allclose(f(other), want, rtol=1e-4, atol=1e-5)      # angles of 700 with a relative error of a few 2^-24
+
+
 def test_stack_refuses_runs_on_different_devices():
     from cosmos_amd import DMConfig, DMStack
     st = DMStack(DMConfig("t", 256, 2, 128, 512, 1, (2, 4, 9), n_text=37), device=dev())
