@@ -433,7 +433,7 @@ def _plain(lin: nn.Module, device: torch.device, dtype: torch.dtype) -> bool:
             and not (torch.is_grad_enabled() and (lin.weight.requires_grad or lin.bias.requires_grad))
             and all(type(p) in (torch.Tensor, nn.Parameter) and p.device == device and p.dtype == dtype and p.is_contiguous()
                     for p in (lin.weight, lin.bias))
-            and lin.weight.data_ptr() % 16 == 0 and lin.in_features % 8 == 0 and lin.in_features <= 16384)
+            and lin.weight.data_ptr() % 16 == 0 and lin.in_features % 8 == 0 and 0 < lin.in_features <= 16384)
 
 
 def _modulations(lins: Sequence[nn.Module], temb: torch.Tensor) -> Optional[List[Tuple[torch.Tensor, ...]]]:
@@ -566,7 +566,7 @@ class TimestepEmbedder(nn.Module):
 
     def sinusoid(self, t: torch.Tensor) -> torch.Tensor:
         half = self.freq_dim // 2
-        if _eager(t) and t.is_cuda and self.freq_dim % 2 == 0 and not (t.requires_grad and torch.is_grad_enabled()):
+        if _eager(t) and t.is_cuda and half > 0 and self.freq_dim % 2 == 0 and not (t.requires_grad and torch.is_grad_enabled()):
             return ops.timestep_sinusoid(t.reshape(-1).to(torch.float32).contiguous(), self.freq_dim)
         k = torch.arange(half, dtype=torch.float32, device=t.device)
         f = torch.exp(-math.log(10000.0) * k / half)

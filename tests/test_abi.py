@@ -167,6 +167,14 @@ def test_bad_arguments_are_rejected_on_the_host():
     assert g(epi=5) == _lib.ERR_BAD_ARG and "qkv_pack" in _lib.last_error()
 
 
+def test_conditioning_arguments_are_validated_on_the_host():
+    lib = _lib.load()
+    fake = 0x10000
+    assert lib.cdm_timestep_sinusoid_f32(None, None, 0, 256, None) == _lib.OK          # no timestep: an empty tensor has no address
+    assert lib.cdm_timestep_sinusoid_f32(None, fake, 1, 256, None) == _lib.ERR_BAD_ARG
+    assert lib.cdm_timestep_sinusoid_f32(fake, fake, 1, 255, None) == _lib.ERR_BAD_SHAPE
+
+
 def test_step_arguments_are_validated_on_the_host():
     lib = _lib.load()
     fake = 0x10000

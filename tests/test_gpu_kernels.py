@@ -207,6 +207,17 @@ def test_gemm_of_runs_that_lie_apart(lens, pitch):
         assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
 
 
+def test_empty_conditioning():
+    """No timestep at all, and an embedding without frequencies: what torch's operators give."""
+    from cosmos_amd import TimestepEmbedder
+    none = torch.empty(0, device=dev())
+    te = TimestepEmbedder(64, device=dev())
+    assert te.sinusoid(none).shape == (0, 256) and te(none).shape == (0, 64)
+    flat, t = TimestepEmbedder(64, freq_dim=0, device=dev()), torch.tensor([3.0], device=dev())
+    with torch.no_grad():
+        assert flat.sinusoid(t).shape == (1, 0) and flat(t).shape == (1, 64)
+
+
 @pytest.mark.parametrize("freq,d", [(256, 1024), (4, 4), (260, 68), (256, 4096)])
 def test_timestep_mlp(freq, d):
     """Against the same MLP in 64 bits behind the same sinusoid; fp32 sums of up to 4096 terms: 1e-5."""
