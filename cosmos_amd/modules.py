@@ -652,10 +652,10 @@ class DMStack(nn.Module):
             raise RuntimeError("context reuse needs the hybrid mask (DMConfig.hybrid_mask)")
         if c.n_text == 0:
             raise ValueError("context reuse needs a text run")
-        x, sources = self._joined([_as2d(encoder_hidden_states)], c.n_text, "context")
+        segs = [(0, c.n_text, 0, False)]
+        x, sources = self._joined([_as2d(encoder_hidden_states)], segs, c.n_text, "context")
         cos, sin = self.rotary(x.device)
         rot = (cos[:c.n_text].contiguous(), sin[:c.n_text].contiguous())
-        segs = [(0, c.n_text, 0, False)]
         ws = Workspace(c.n_text, c.d_model, c.hidden, c.n_heads, c.head_dim, x.device, c.kv_heads, c.fp8)
         nbytes = ops.attn_workspace_bytes(c.n_text, c.kv_heads, c.head_dim)
         images = []
@@ -692,9 +692,9 @@ class DMStack(nn.Module):
             parts.append(_as2d(encoder_hidden_states))
         parts.append(_as2d(hidden_states))
         parts += self._generator_extras(audio_states, action_states)
-        x, sources = self._joined(parts, c.n_tokens, "joint")
-        rot = self.rotary(x.device)
         segs = self.segments()
+        x, sources = self._joined(parts, segs, c.n_tokens, "joint")
+        rot = self.rotary(x.device)
         temb = self.time_embedder(timestep.reshape(-1)[:1])
         if self._ws is None or not self._ws.fits(c.n_tokens, c.d_model, c.hidden, c.fp8) or self._ws.y.device != x.device:
             self._ws = Workspace(c.n_tokens, c.d_model, c.hidden, c.n_heads, c.head_dim, x.device, c.kv_heads, c.fp8)
@@ -724,9 +724,9 @@ class DMStack(nn.Module):
             at += p.shape[0]
         return x
 
-    def _joined(self, parts: Sequence[torch.Tensor], n: int, what: str):
-        """(stream, sources) of the runs.  Where the first block's norm can join them as it reads them, the stream is not
-        filled yet and ``sources`` are the runs; otherwise it is, and ``sources`` is None."""
+    def _joined(self, parts: Sequence[torch.Tensor], segs: Sequence[Segment], n: int, what: str):
+        """(stream, sources) of the runs.  Where the first block's norm can join them as it reads them - its segments are the
+        runs -, the stream is not filled yet and ``sources`` are the runs; otherwise it is, and ``sources`` is None."""
         d = self.cfg.d_model
         rows = sum(p.shape[0] for p in parts)
         if rows != n or any(p.dim() != 2 or p.shape[1] != d for p in parts):
@@ -735,7 +735,9 @@ class DMStack(nn.Module):
         if any(p.device != dev for p in parts):
             raise RuntimeError(f"the runs of the {what} sequence lie on different devices")
         first = self.blocks[0] if len(self.blocks) else None      # a subclass or a hook may read its input: it gets it filled
+        starts = [sum(p.shape[0] for p in parts[:i]) for i in range(len(parts))]
         if (_bare(first) and self.cfg.residual_fp32 and dev.type == "cuda" and d % 8 == 0
+                and [(s0, ln) for (s0, ln, _, _) in segs] == [(s0, p.shape[0]) for s0, p in zip(starts, parts)]
                 and all(p.dtype == torch.bfloat16 and p.device == dev and p.is_contiguous() and p.data_ptr() % 16 == 0 for p in parts)):
             return torch.empty((n, d), dtype=torch.float32, device=dev), list(parts)
         return self._stream(*parts), None
@@ -779,11 +781,11 @@ class DMStack(nn.Module):
             raise ValueError("context cache does not belong to this stack")
         parts = [_as2d(hidden_states)] + self._generator_extras(audio_states, action_states)
         n = c.n_tokens - P
-        x, sources = self._joined(parts, n, "generator")
+        segs = [(s0 - P, ln, b, m) for (s0, ln, b, m) in self.segments() if s0 >= P]
+        x, sources = self._joined(parts, segs, n, "generator")
         if self._rot_gen is None or self._rot_gen[0].device != x.device:
             cos, sin = self.rotary(x.device)
             self._rot_gen = (cos[P:].contiguous(), sin[P:].contiguous())
-        segs = [(s0 - P, ln, b, m) for (s0, ln, b, m) in self.segments() if s0 >= P]
         temb = self.time_embedder(timestep.reshape(-1)[:1])
         if self._ws_gen is None or not self._ws_gen.fits(n, c.d_model, c.hidden, c.fp8) or self._ws_gen.y.device != x.device:
             self._ws_gen = Workspace(n, c.d_model, c.hidden, c.n_heads, c.head_dim, x.device, c.kv_heads, c.fp8)

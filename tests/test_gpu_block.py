@@ -875,3 +875,20 @@ def test_stack_under_hooks_of_every_module():
     te, blk = st.time_embedder, st.blocks[0]
     assert all(m in seen for m in (te.linear_1, te.linear_2, blk.adaLN_modulation))
     assert torch.equal(seen[blk], torch.cat([ctx[0], x[0]]).float())
+
+
+def test_stack_whose_segments_are_not_its_runs():
+    """A stack that routes otherwise than its runs are cut (text and the head of the video in one segment): as with fp32 inputs,
+    which are joined first."""
+    class Rerouted(DMStack):
+        def segments(self):
+            return [(0, 64, 0, True), (64, 45, 0, True)]
+
+    cfg = DMConfig("t", 256, 2, 128, 512, 1, (2, 4, 9), n_text=37)
+    st = Rerouted(cfg, device=dev())
+    st.reset_parameters(3)
+    g = torch.Generator().manual_seed(4)
+    ctx, x = rand_bf16((1, 37, 256), g)[0], rand_bf16((1, 72, 256), g)[0]
+    t = torch.tensor([500.0], device=dev())
+    want = st(x.float(), t, encoder_hidden_states=ctx.float())[0]
+    assert torch.equal(st(x, t, encoder_hidden_states=ctx)[0], want)
