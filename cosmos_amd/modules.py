@@ -131,8 +131,10 @@ class DMAttnProcessor:
                 raise NotImplementedError("encoder_hidden_states cannot be combined with fused residual / fp8 input")
             enc = _as2d(encoder_hidden_states)
             n_enc, n_lat = enc.shape[0], x.shape[0]
-            # the projection reads the two runs where they lie, if they are laid out alike; otherwise they are joined first
-            if (modality_segments is None and self.rope != "gemm_epilogue" and not attn.fp8 and n_enc > 0 and n_lat > 0
+            # the projection reads the two runs where they lie, if they are laid out alike; otherwise, and for a subclass's own
+            # projections, they are joined first
+            if (type(attn) in (AdoptedAttention, DMAttention) and modality_segments is None and self.rope != "gemm_epilogue"
+                    and not attn.fp8 and n_enc > 0 and n_lat > 0
                     and all(t.is_cuda and t.device == x.device and t.dtype == torch.bfloat16 and t.shape[1] == attn.d_model
                             and t.stride(1) == 1 and t.stride(0) == x.stride(0) and t.stride(0) >= t.shape[1]
                             and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (enc, x))):

@@ -892,3 +892,27 @@ def test_stack_whose_segments_are_not_its_runs():
     t = torch.tensor([500.0], device=dev())
     want = st(x.float(), t, encoder_hidden_states=ctx.float())[0]
     assert torch.equal(st(x, t, encoder_hidden_states=ctx)[0], want)
+
+
+@pytest.mark.parametrize("n_enc,fuse", [(64, True), (16, True), (64, False)])
+def test_projections_of_an_attention_subclass_get_joined_tokens(n_enc, fuse):
+    """A subclass that works on the rows ahead of its projections, called with a context run: as the plain module on such rows."""
+    from cosmos_amd import DMAttention, DMAttnProcessor
+
+    class Scaled(DMAttention):
+        def _linear(self, a, sa, which, *args, **kw):
+            super()._linear(a * 2.0 if which == "qkv" else a, sa, which, *args, **kw)
+
+        def _qkv_pack(self, a, *args, **kw):
+            super()._qkv_pack(a * 2.0, *args, **kw)
+
+    g = torch.Generator().manual_seed(n_enc)
+    attn = make_block(DMConfig("p", 256, 2, 128, 512, 1, (1, 4, 8), n_text=n_enc, n_branches=2), 21).attn
+    attn.set_processor(DMAttnProcessor(fuse_kv_pack=fuse))
+    e, h = rand_bf16((1, n_enc, 256), g)[0], rand_bf16((1, 32, 256), g)[0]
+    pos, _ = rotary.build_positions(n_enc, (1, 4, 8))
+    rot = rotary.rotary_tables(pos, 128, (32, 48, 48), device=dev())
+    want = attn(h * 2.0, encoder_hidden_states=e * 2.0, image_rotary_emb=rot)
+    attn.__class__ = Scaled
+    got = attn(h, encoder_hidden_states=e, image_rotary_emb=rot)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
