@@ -83,7 +83,7 @@ def _timed(category: str):
 
 def time_ops(enable: bool):
     """Start (True) or stop (False) collecting (category, start, end) HIP event triples around every kernel launcher
-    of this module ("norm", "gemm", "rope", "pack_kv", "quant", "step"; the attention kernel itself is covered by
+    of this module ("norm", "gemm", "edge", "quant", "rope", "pack_kv", "cond", "step"; the attention kernel itself is covered by
     ``time_attention``); stopping returns the list."""
     global _OP_TIMER
     prev, _OP_TIMER = _OP_TIMER, ([] if enable else None)
@@ -226,6 +226,23 @@ def gemm_scratch_bytes(lens: Tuple[int, ...], N: int, K: int, epi: int) -> int:
     return int(_lib.load().cdm_grouped_gemm_scratch_bytes((C.c_int64 * len(lens))(*lens), len(lens), N, K, epi))
 
 
+def _gemm_cut_along_k(a: torch.Tensor, ws: Sequence[torch.Tensor], segments: Sequence[Tuple[int, int]], epi: int, odt: torch.dtype,
+                      residual: Optional[torch.Tensor], gates: Optional[Sequence[Optional[torch.Tensor]]], out: torch.Tensor,
+                      scratch: int) -> torch.Tensor:
+    """A grouped GEMM with the scratch that a cut along K takes (within a timed call of ``gemm`` or ``grouped_gemm``)."""
+    n_seg, (N, K) = len(segments), ws[0].shape
+    PP, I64 = C.c_void_p * n_seg, C.c_int64 * n_seg
+    gp = PP(*[(_f32vec(g, "gate", N) or None) for g in gates]) if gates is not None else None
+    buf = torch.empty((scratch,), dtype=torch.uint8, device=a.device)
+    rc = _lib.load().cdm_grouped_gemm_scratch_bf16(
+        _chk(a, "a", torch.bfloat16, 2), a.stride(0), PP(*[_chk(w, "w", torch.bfloat16, 2) for w in ws]), ws[0].stride(0),
+        _chk(out, "out", odt, 2), out.stride(0), I64(*[int(s) for s, _ in segments]), I64(*[int(l) for _, l in segments]), n_seg, N, K,
+        epi, _chk(residual, "residual", odt, 2), residual.stride(0) if residual is not None else 0, gp, buf.data_ptr(), scratch,
+        _stream())
+    _lib.check(rc, "cdm_grouped_gemm_scratch_bf16")
+    return out
+
+
 @_timed("gemm")
 def gemm(a: torch.Tensor, w: torch.Tensor, *, w2: Optional[torch.Tensor] = None, epilogue: str = "none",
          residual: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
@@ -247,7 +264,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, w2: Optional[torch.Tensor] = None,
     epi, odt = _epilogue(epilogue, out, residual)
     scratch = gemm_scratch_bytes((M,), N, K, epi) if epi in _MAY_SPLIT_K else 0
     if scratch:
-        return grouped_gemm(a, [w], [(0, M)], epilogue=epilogue, residual=residual, gates=[gate], out=out)
+        return _gemm_cut_along_k(a, [w], [(0, M)], epi, odt, residual, [gate], out, scratch)
     rc = lib.cdm_gemm_bf16(_chk(a, "a", torch.bfloat16, 2), a.stride(0), _chk(w, "w", torch.bfloat16, 2), w.stride(0),
                            _chk(w2, "w2", torch.bfloat16, 2), _chk(out, "out", odt, 2), out.stride(0),
                            M, N, K, epi, _chk(residual, "residual", odt, 2),
@@ -356,13 +373,7 @@ def grouped_gemm(a: torch.Tensor, ws: Sequence[torch.Tensor], segments: Sequence
     epi, odt = _epilogue(epilogue, out, residual)
     scratch = gemm_scratch_bytes(tuple(int(l) for _, l in segments), N, K, epi) if epi in _MAY_SPLIT_K else 0
     if scratch:
-        buf = torch.empty((scratch,), dtype=torch.uint8, device=a.device)
-        rc = lib.cdm_grouped_gemm_scratch_bf16(_chk(a, "a", torch.bfloat16, 2), a.stride(0), wp, ldw, _chk(out, "out", odt, 2),
-                                               out.stride(0), st, ln, n_seg, N, K, epi, _chk(residual, "residual", odt, 2),
-                                               residual.stride(0) if residual is not None else 0, gp, buf.data_ptr(), scratch,
-                                               _stream())
-        _lib.check(rc, "cdm_grouped_gemm_scratch_bf16")
-        return out
+        return _gemm_cut_along_k(a, ws, segments, epi, odt, residual, gates, out, scratch)
     rc = lib.cdm_grouped_gemm_bf16(_chk(a, "a", torch.bfloat16, 2), a.stride(0), wp, ldw, w2p,
                                    _chk(out, "out", odt, 2), out.stride(0), st, ln, n_seg, N, K,
                                    epi, _chk(residual, "residual", odt, 2),

@@ -182,6 +182,21 @@ def test_gemm_cut_along_k(lens, N, K, epi):
         assert bool((err <= tol).all()), (i, err.max().item())
 
 
+@pytest.mark.parametrize("grouped", [False, True])
+@pytest.mark.parametrize("M,N,K", [(256, 1024, 8192), (256, 1024, 512)])
+def test_a_gemm_is_timed_once(M, N, K, grouped):
+    """Cut along K or not, a call leaves one entry with the timer."""
+    g = gen(K)
+    a, w = rand_bf16((M, K), g)[0], rand_bf16((N, K), g)[0]
+    assert (ops.gemm_scratch_bytes((M,), N, K, ops.EPI_NONE) > 0) == (K == 8192)
+    ops.time_ops(True)
+    try:
+        ops.grouped_gemm(a, [w], [(0, M)]) if grouped else ops.gemm(a, w)
+    finally:
+        seen = ops.time_ops(False)
+    assert [c for c, _, _ in seen] == ["gemm"]
+
+
 @pytest.mark.parametrize("lens", [(77, 1560), (1, 1), (64, 200), (128, 5000)])
 @pytest.mark.parametrize("pitch", [512, 520])
 def test_gemm_of_runs_that_lie_apart(lens, pitch):
