@@ -262,7 +262,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, w2: Optional[torch.Tensor] = None,
         raise ValueError("w and w2 must share a row stride")
     half = head_dim // 2 if head_dim else 0
     epi, odt = _epilogue(epilogue, out, residual)
-    scratch = gemm_scratch_bytes((M,), N, K, epi) if epi in _MAY_SPLIT_K else 0
+    scratch = gemm_scratch_bytes((M,), N, K, epi) if epi in _MAY_SPLIT_K and w2 is None and cos is None and sin is None else 0
     if scratch:
         return _gemm_cut_along_k(a, [w], [(0, M)], epi, odt, residual, [gate], out, scratch)
     rc = lib.cdm_gemm_bf16(_chk(a, "a", torch.bfloat16, 2), a.stride(0), _chk(w, "w", torch.bfloat16, 2), w.stride(0),
@@ -371,7 +371,9 @@ def grouped_gemm(a: torch.Tensor, ws: Sequence[torch.Tensor], segments: Sequence
     st, ln = I64(*[int(s) for s, _ in segments]), I64(*[int(l) for _, l in segments])
     half = head_dim // 2 if head_dim else 0
     epi, odt = _epilogue(epilogue, out, residual)
-    scratch = gemm_scratch_bytes(tuple(int(l) for _, l in segments), N, K, epi) if epi in _MAY_SPLIT_K else 0
+    # operands that the epilogue does not use are checked below all the same
+    may_split = epi in _MAY_SPLIT_K and w2s is None and cos is None and sin is None
+    scratch = gemm_scratch_bytes(tuple(int(l) for _, l in segments), N, K, epi) if may_split else 0
     if scratch:
         return _gemm_cut_along_k(a, ws, segments, epi, odt, residual, gates, out, scratch)
     rc = lib.cdm_grouped_gemm_bf16(_chk(a, "a", torch.bfloat16, 2), a.stride(0), wp, ldw, w2p,

@@ -182,6 +182,22 @@ def test_gemm_cut_along_k(lens, N, K, epi):
         assert bool((err <= tol).all()), (i, err.max().item())
 
 
+@pytest.mark.parametrize("K", [512, 8192])
+@pytest.mark.parametrize("bad", ["w2 type", "w2 on the host", "cos size", "sin type"])
+@pytest.mark.parametrize("grouped", [False, True])
+def test_gemm_checks_operands_that_its_epilogue_leaves(K, bad, grouped):
+    """Short and long K (the long one may be cut along K) refuse the same calls."""
+    M, N = 256, 1024
+    a, w = (torch.zeros((n, K), dtype=torch.bfloat16, device=dev()) for n in (M, N))
+    kw = {"w2 type": dict(w2=w.float()), "w2 on the host": dict(w2=w.cpu()), "cos size": dict(cos=torch.zeros(3, device=dev()), head_dim=128),
+          "sin type": dict(sin=torch.zeros((M, 64), dtype=torch.float64, device=dev()), head_dim=128)}[bad]
+    with pytest.raises((TypeError, ValueError, RuntimeError)):
+        if grouped:
+            ops.grouped_gemm(a, [w], [(0, M)], **{("w2s" if k == "w2" else k): ([v] if k == "w2" else v) for k, v in kw.items()})
+        else:
+            ops.gemm(a, w, **kw)
+
+
 @pytest.mark.parametrize("grouped", [False, True])
 @pytest.mark.parametrize("M,N,K", [(256, 1024, 8192), (256, 1024, 512)])
 def test_a_gemm_is_timed_once(M, N, K, grouped):
