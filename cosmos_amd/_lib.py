@@ -158,6 +158,10 @@ def set_variant(op: str, variant: int) -> int:
     return prev
 
 
+def selected_variant(op: str) -> int:
+    return _VARIANTS[op]
+
+
 def last_error() -> str:
     return load().cdm_last_error().decode("utf-8", "replace")
 

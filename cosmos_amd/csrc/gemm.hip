@@ -1045,6 +1045,7 @@ extern "C" int32_t cdm_grouped_gemm_bf16(const void* A, int64_t lda, const void*
 
 extern "C" int64_t cdm_grouped_gemm_scratch_bytes(const int64_t* seg_len, int32_t n_seg, int64_t N, int64_t K, int32_t epilogue) {
     if (!seg_len || n_seg < 1 || N <= 0 || K <= 0 || N >= (1ll << 31) || K >= (1ll << 31)) return 0;
+    if (cdm_get_variant(1) == 1) return 0;      // cross-check build: the two-stage kernel is never cut
     GemmParams p{};
     p.N = (int)N; p.K = (int)K;
     int64_t at = 0;

@@ -570,6 +570,7 @@ struct SplitK { TileShape s; int parts; double us; int64_t bytes; };
 SplitK best_split(const GemmParams& p, const int64_t* rows, double kt, int epilogue) {
     SplitK best{{}, 1, 1e30, 0};
     if (epilogue != CDM_EPI_NONE && epilogue != CDM_EPI_GATE_RESIDUAL && epilogue != CDM_EPI_GATE_RESIDUAL_F32) return best;
+    if (kt < 32.0) return best;                                             // K below 2048, where none was measured
     int64_t lo = p.seg[0].m_start, hi = p.seg[0].m_end, filled = 0;
     for (int i = 0; i < p.n_seg; ++i) {
         lo = p.seg[i].m_start < lo ? p.seg[i].m_start : lo;

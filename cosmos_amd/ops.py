@@ -218,11 +218,13 @@ def _amax_arg(row_amax: Optional[torch.Tensor], rows: int, min_cols: int):
 
 
 # ----------------------------------------------------------------------------- GEMM
-@functools.lru_cache(maxsize=4096)
 def gemm_scratch_bytes(lens: Tuple[int, ...], N: int, K: int, epi: int) -> int:
     """Scratch for a bf16 GEMM of these segments that is cut along K (few output tiles, long K); 0: it is not cut."""
-    if K < 2048 or sum(lens) * N > 1 << 23:      # too short a K, or enough tiles for the chip
-        return 0
+    return _gemm_scratch_bytes(lens, N, K, epi, _lib.selected_variant("gemm"))
+
+
+@functools.lru_cache(maxsize=4096)
+def _gemm_scratch_bytes(lens: Tuple[int, ...], N: int, K: int, epi: int, variant: int) -> int:
     return int(_lib.load().cdm_grouped_gemm_scratch_bytes((C.c_int64 * len(lens))(*lens), len(lens), N, K, epi))
 
 

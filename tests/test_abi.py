@@ -175,6 +175,23 @@ def test_conditioning_arguments_are_validated_on_the_host():
     assert lib.cdm_timestep_sinusoid_f32(fake, fake, 1, 255, None) == _lib.ERR_BAD_SHAPE
 
 
+def test_scratch_of_a_cut_along_k_follows_the_selected_kernel():
+    """The library decides from sizes and the selected kernel variant; nothing of a variant's answer is left behind it."""
+    from cosmos_amd import ops
+    ask = lambda M=200, N=4096, K=8192: ops.gemm_scratch_bytes((M,), N, K, _lib.EPI_NONE)
+    try:
+        for variant in (1, 2, 5):
+            ops.set_variant("gemm", variant)
+            assert ask() == 0
+    finally:
+        ops.set_variant("gemm", 0)
+    assert ask() == 200 * 4096 * 4 * 4                   # four ranges
+    lib = _lib.load()
+    for M, N, K in ((200, 4096, 1920), (200, 4096, 2048), (4096, 4096, 8192)):      # short K; enough tiles
+        assert lib.cdm_grouped_gemm_scratch_bytes((C.c_int64 * 1)(M), 1, N, K, _lib.EPI_NONE) == ask(M, N, K)
+        assert K >= 2048 or ask(M, N, K) == 0
+
+
 def test_step_arguments_are_validated_on_the_host():
     lib = _lib.load()
     fake = 0x10000
