@@ -854,7 +854,7 @@ int32_t grouped(const char* who, const void* A, int64_t lda, const float* sa, co
                 const float* k_norm_rows = nullptr, float* row_amax = nullptr, int64_t amax_ld = 0, void* scratch = nullptr,
                 int64_t scratch_bytes = 0, const void* const* runs = nullptr) {
     constexpr int esize = FP8 ? 1 : 2;
-    CDM_REQUIRE(A && W && C && seg_start && seg_len, CDM_ERR_BAD_ARG, "%s: null pointer", who);
+    CDM_REQUIRE((A || runs) && W && C && seg_start && seg_len, CDM_ERR_BAD_ARG, "%s: null pointer", who);
     CDM_REQUIRE((epilogue == CDM_EPI_QKV_PACK) == (pack != nullptr), CDM_ERR_BAD_ARG,
                 "%s: the QKV_PACK epilogue belongs to the qkv_pack entry points", who);
     CDM_REQUIRE(n_seg >= 0 && n_seg <= 64, CDM_ERR_BAD_ARG, "%s: n_seg=%d out of range", who, n_seg);
@@ -873,8 +873,8 @@ int32_t grouped(const char* who, const void* A, int64_t lda, const float* sa, co
     for (int g = 0; g < n_seg; ++g) {
         CDM_REQUIRE(seg_start[g] >= 0 && seg_len[g] >= 0, CDM_ERR_BAD_ARG, "%s: negative segment", who);
         CDM_REQUIRE(W[g], CDM_ERR_BAD_ARG, "%s: null weight for segment %d", who, g);
-        const void* a = runs ? runs[g] : A;
-        CDM_REQUIRE(a || seg_len[g] == 0, CDM_ERR_BAD_ARG, "%s: null rows of segment %d", who, g);
+        const void* a = !runs ? A : seg_len[g] > 0 ? runs[g] : W[g];      // an empty run may be null: nothing reads its rows
+        CDM_REQUIRE(a, CDM_ERR_BAD_ARG, "%s: null rows of segment %d", who, g);
         int32_t rc = validate(who, esize, a, lda, W[g], ldw, W2 ? W2[g] : nullptr, C, ldc, seg_len[g], N, K, epilogue, R, ldr,
                               cos, sin, rope_cols, head_dim);
         if (rc) return rc;
@@ -996,7 +996,7 @@ extern "C" int32_t cdm_grouped_gemm_qkv_pack_runs_bf16(const void* const* A, int
                                                        void* stream) {
     const char* who = "grouped_gemm_qkv_pack_runs_bf16";
     CDM_REQUIRE(A && n_seg >= 1, CDM_ERR_BAD_ARG, "%s: no runs", who);
-    return qkv_pack<false>(who, A[0], lda, nullptr, W, nullptr, ldw, Q, ldq, seg_start, seg_len, n_seg, K, n_heads, n_kv_heads,
+    return qkv_pack<false>(who, nullptr, lda, nullptr, W, nullptr, ldw, Q, ldq, seg_start, seg_len, n_seg, K, n_heads, n_kv_heads,
                            head_dim, cos, sin, qk_norm, workspace, workspace_bytes, stream, A);
 }
 
@@ -1005,7 +1005,7 @@ extern "C" int32_t cdm_grouped_gemm_runs_bf16(const void* const* A, int64_t lda,
                                               int64_t N, int64_t K, void* stream) {
     const char* who = "grouped_gemm_runs_bf16";
     CDM_REQUIRE(A && n_seg >= 1, CDM_ERR_BAD_ARG, "%s: no runs", who);
-    return grouped<false>(who, A[0], lda, nullptr, W, nullptr, ldw, nullptr, nullptr, C, ldc, seg_start, seg_len, n_seg, N, K,
+    return grouped<false>(who, nullptr, lda, nullptr, W, nullptr, ldw, nullptr, nullptr, C, ldc, seg_start, seg_len, n_seg, N, K,
                           CDM_EPI_NONE, nullptr, 0, nullptr, nullptr, nullptr, 0, 0, stream, nullptr, nullptr, nullptr, 0, nullptr, 0,
                           A);
 }

@@ -326,9 +326,9 @@ def gemm_fp8(aq: torch.Tensor, sa: torch.Tensor, wq: torch.Tensor, sw: torch.Ten
 
 
 def _run_ptrs(runs: Sequence[torch.Tensor], segments: Sequence[Tuple[int, int]]):
-    """Pointers and row stride of the rows of every segment, kept in tensors of their own."""
-    k, ld = runs[0].shape[1], runs[0].stride(0)
-    if len(runs) != len(segments) or any(r.shape != (int(l), k) or r.stride(0) != ld for r, (_, l) in zip(runs, segments)):
+    """Pointers and row stride of the rows of every segment, kept in tensors of their own (empty ones for empty segments)."""
+    k, ld = runs[0].shape[1], next((r.stride(0) for r in runs if r.shape[0]), runs[0].stride(0))
+    if len(runs) != len(segments) or any(r.shape != (int(l), k) or (r.shape[0] and r.stride(0) != ld) for r, (_, l) in zip(runs, segments)):
         raise ValueError("one tensor of rows per segment, all of one width and row stride")
     return (C.c_void_p * len(runs))(*[_chk(r, "run", torch.bfloat16, 2) for r in runs]), ld
 

@@ -347,7 +347,7 @@ int32_t cdm_grouped_gemm_scratch_bf16(const void* A, int64_t lda, const void* co
 
 /*
  * Epilogue NONE, and the fused QKV projection, on runs that lie apart: A[g] points at the first row of segment g (all runs with
- * row stride lda); rows of C, the rotary tables and the images keep their place in the joint sequence.
+ * row stride lda; null for an empty segment); rows of C, the rotary tables and the images keep their place in the joint sequence.
  */
 int32_t cdm_grouped_gemm_runs_bf16(const void* const* A, int64_t lda, const void* const* W, int64_t ldw, void* C, int64_t ldc,
                                    const int64_t* seg_start, const int64_t* seg_len, int32_t n_seg, int64_t N, int64_t K,

@@ -175,6 +175,32 @@ def test_conditioning_arguments_are_validated_on_the_host():
     assert lib.cdm_timestep_sinusoid_f32(fake, fake, 1, 255, None) == _lib.ERR_BAD_SHAPE
 
 
+def test_runs_that_lie_apart_are_validated_on_the_host():
+    lib = _lib.load()
+    fake = 0x10000
+    accepted = (_lib.OK, _lib.ERR_NO_DEVICE) if not HAS_GPU else ()      # (these addresses are for hosts without a device)
+    W = (C.c_void_p * 2)(fake, fake)
+
+    def plain(rows, lens, lda=256, n_seg=2, starts=None):
+        st, ln = (C.c_int64 * 2)(*(starts or (0, lens[0]))), (C.c_int64 * 2)(*lens)
+        return lib.cdm_grouped_gemm_runs_bf16((C.c_void_p * 2)(*rows) if rows else None, lda, W, 256, fake, 512, st, ln, n_seg, 512, 256, None)
+
+    def pack(rows, lens, lda=256, n_seg=2, starts=None):
+        st, ln = (C.c_int64 * 2)(*(starts or (0, lens[0]))), (C.c_int64 * 2)(*lens)
+        return lib.cdm_grouped_gemm_qkv_pack_runs_bf16((C.c_void_p * 2)(*rows) if rows else None, lda, W, 256, fake, 128, st, ln, n_seg, 256, 1, 1,
+                                                       128, None, None, None, fake, 1 << 24, None)
+    for call in (plain, pack):
+        assert call(None, (64, 64)) == _lib.ERR_BAD_ARG
+        assert call((fake, fake), (64, 64), n_seg=0) == _lib.ERR_BAD_ARG
+        assert call((fake, None), (64, 64)) == _lib.ERR_BAD_ARG and "null rows of segment 1" in _lib.last_error()
+        assert call((fake, fake + 8), (64, 64)) == _lib.ERR_BAD_ALIGN
+        assert call((fake, fake), (64, 64), lda=128) == _lib.ERR_BAD_ARG
+        if accepted:      # an empty run has no rows: its address may be null
+            assert call((None, fake), (0, 64)) in accepted and call((fake, None), (64, 0)) in accepted
+    assert plain((fake, fake), (64, 64), starts=(0, 63)) == _lib.ERR_BAD_ARG and "overlap" in _lib.last_error()
+    assert pack((fake, fake), (64, 64), starts=(0, 128)) == _lib.ERR_UNSUPPORTED
+
+
 def test_scratch_of_a_cut_along_k_follows_the_selected_kernel():
     """The library decides from sizes and the selected kernel variant; nothing of a variant's answer is left behind it."""
     from cosmos_amd import ops

@@ -213,7 +213,7 @@ def test_a_gemm_is_timed_once(M, N, K, grouped):
     assert [c for c, _, _ in seen] == ["gemm"]
 
 
-@pytest.mark.parametrize("lens", [(77, 1560), (1, 1), (64, 200), (128, 5000)])
+@pytest.mark.parametrize("lens", [(77, 1560), (1, 1), (64, 200), (128, 5000), (0, 300), (192, 0)])
 @pytest.mark.parametrize("pitch", [512, 520])
 def test_gemm_of_runs_that_lie_apart(lens, pitch):
     """Projections of two runs in tensors of their own: the bits of the joined rows, plain and with the fused key images."""
