@@ -25,6 +25,7 @@ namespace {
 
 constexpr int kLds = 160 * 1024;
 constexpr int kMaxSplitK = 8;      // most ranges of K
+constexpr int kKeyNorms = 64 / 8 * 2;      // what pack_piece leaves of a piece's 64 keys: a float per eight keys and head (up to two)
 
 template <int TM, int TN, int WM, int WN>
 struct Geo {
@@ -33,11 +34,12 @@ struct Geo {
     static constexpr int STAGE = (TM + TN) * 128;                 // bytes of one k-tile of both operands
     static constexpr int LPW = (TM + TN) / 8 / (WM * WN);         // direct-to-LDS instructions (8 rows each) per wave and k-tile
     static constexpr int PITCH = TN * 4 + 16;                     // bytes of a staged fp32 row (the pad spreads rows over banks)
-    static constexpr int KSQ = TM / 8 * 4;                        // QKV_PACK: one float per eight keys
+    static constexpr int KSQ = kKeyNorms * 4;                     // QKV_PACK: behind the staged rows
     static constexpr int MAXS = (TM + TN) >= 256 ? 5 : 8;
     static constexpr int S = kLds / STAGE < MAXS ? kLds / STAGE : MAXS;      // ring stages
     static constexpr int SMEM = S * STAGE > TM * PITCH + KSQ ? S * STAGE : TM * PITCH + KSQ;
     static_assert((TM + TN) / 8 % (WM * WN) == 0 && S >= 3 && S <= 8 && SMEM <= kLds, "tile shape");
+    static_assert(KSQ >= kKeyNorms * 4, "key norms of a piece exceed their reserve");
 };
 
 __device__ __forceinline__ void unpack4(const float4& v, float* f) { f[0] = v.x; f[1] = v.y; f[2] = v.z; f[3] = v.w; }
