@@ -235,12 +235,15 @@ def _gemm_cut_along_k(a: torch.Tensor, ws: Sequence[torch.Tensor], segments: Seq
     n_seg, (N, K) = len(segments), ws[0].shape
     PP, I64 = C.c_void_p * n_seg, C.c_int64 * n_seg
     gp = PP(*[(_f32vec(g, "gate", N) or None) for g in gates]) if gates is not None else None
-    buf = torch.empty((scratch,), dtype=torch.uint8, device=a.device)
+    try:
+        buf = torch.empty((scratch,), dtype=torch.uint8, device=a.device)
+    except torch.OutOfMemoryError:      # without scratch the launch is the uncut one, which takes no memory
+        buf, scratch = None, 0
     rc = _lib.load().cdm_grouped_gemm_scratch_bf16(
         _chk(a, "a", torch.bfloat16, 2), a.stride(0), PP(*[_chk(w, "w", torch.bfloat16, 2) for w in ws]), ws[0].stride(0),
         _chk(out, "out", odt, 2), out.stride(0), I64(*[int(s) for s, _ in segments]), I64(*[int(l) for _, l in segments]), n_seg, N, K,
-        epi, _chk(residual, "residual", odt, 2), residual.stride(0) if residual is not None else 0, gp, buf.data_ptr(), scratch,
-        _stream())
+        epi, _chk(residual, "residual", odt, 2), residual.stride(0) if residual is not None else 0, gp,
+        buf.data_ptr() if buf is not None else None, scratch, _stream())
     _lib.check(rc, "cdm_grouped_gemm_scratch_bf16")
     return out
 

@@ -182,6 +182,26 @@ def test_gemm_cut_along_k(lens, N, K, epi):
         assert bool((err <= tol).all()), (i, err.max().item())
 
 
+@pytest.mark.parametrize("grouped", [False, True])
+def test_gemm_without_room_for_scratch(grouped, monkeypatch):
+    """Where the scratch of a cut along K cannot be had, the launch is the uncut one (the same bits)."""
+    g, M, N, K = gen(5), 256, 1024, 8192
+    a, w = rand_bf16((M, K), g)[0], rand_bf16((N, K), g, 0.02)[0]
+    assert ops.gemm_scratch_bytes((M,), N, K, ops.EPI_NONE) > 0
+    tables = torch.zeros((M, 64), device=dev())
+    want = ops.gemm(a, w, cos=tables, sin=tables, head_dim=128)      # a call that brings unused operands is not cut
+    empty = torch.empty
+
+    def no_bytes(*size, **kw):
+        if kw.get("dtype") == torch.uint8:
+            raise torch.OutOfMemoryError("no room")
+        return empty(*size, **kw)
+
+    monkeypatch.setattr(torch, "empty", no_bytes)
+    got = ops.grouped_gemm(a, [w], [(0, M)]) if grouped else ops.gemm(a, w)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("K", [512, 8192])
 @pytest.mark.parametrize("bad", ["w2 type", "w2 on the host", "cos size", "sin type"])
 @pytest.mark.parametrize("grouped", [False, True])
