@@ -232,7 +232,7 @@ def _gemm_cut_along_k(a: torch.Tensor, ws: Sequence[torch.Tensor], segments: Seq
                       residual: Optional[torch.Tensor], gates: Optional[Sequence[Optional[torch.Tensor]]], out: torch.Tensor,
                       scratch: int) -> torch.Tensor:
     """A grouped GEMM with the scratch that a cut along K takes (within a timed call of ``gemm`` or ``grouped_gemm``)."""
-    n_seg, (N, K) = len(segments), ws[0].shape
+    n_seg, N, K = len(segments), ws[0].shape[0], a.shape[1]
     PP, I64 = C.c_void_p * n_seg, C.c_int64 * n_seg
     gp = PP(*[(_f32vec(g, "gate", N) or None) for g in gates]) if gates is not None else None
     try:

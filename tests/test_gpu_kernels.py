@@ -182,6 +182,14 @@ def test_gemm_cut_along_k(lens, N, K, epi):
         assert bool((err <= tol).all()), (i, err.max().item())
 
 
+@pytest.mark.parametrize("K", [512, 8192])
+def test_grouped_gemm_of_wider_weights(K):
+    """Weights with more columns than the rows have: their first K columns, cut along K or not."""
+    g = gen(K)
+    a, w = rand_bf16((256, K), g)[0], rand_bf16((1024, K + 1024), g, 0.02)[0]
+    assert torch.equal(ops.grouped_gemm(a, [w], [(0, 256)]), ops.grouped_gemm(a, [w[:, :K].contiguous()], [(0, 256)]))
+
+
 @pytest.mark.parametrize("grouped", [False, True])
 def test_gemm_without_room_for_scratch(grouped, monkeypatch):
     """Where the scratch of a cut along K cannot be had, the launch is the uncut one (the same bits)."""
