@@ -155,6 +155,8 @@ def adaln_rmsnorm_grouped(x: torch.Tensor, ws: Sequence[torch.Tensor], shifts: S
     if any(s < 0 or l < 0 or s + l > n for s, l in segments):
         raise ValueError("token run outside x")
     k = len(segments)
+    if not len(ws) == len(shifts) == len(scales) == k or any(w.shape != (d,) for w in ws):
+        raise ValueError("every token run needs its weights [d] and an entry of shifts and scales")
     PP, I64 = C.c_void_p * k, C.c_int64 * k
     if sources is None:
         fn, given = lib.cdm_adaln_rmsnorm_grouped, (_chk(x, "x", x.dtype if f32 else torch.bfloat16, 2), int(f32))

@@ -250,3 +250,17 @@ def test_ops_refuse_cpu_tensors():
     x = torch.zeros(4, 64, dtype=torch.bfloat16)
     with pytest.raises(RuntimeError, match="GPU"):
         ops.adaln_rmsnorm(x, torch.ones(64, dtype=torch.bfloat16))
+
+
+def test_grouped_norm_refuses_weights_that_do_not_fit():
+    """Refused ahead of any launch: the kernel reads d weights of every run."""
+    from cosmos_amd import ops
+    x, y, w = torch.zeros(4, 64), torch.zeros(4, 64, dtype=torch.bfloat16), torch.ones(64, dtype=torch.bfloat16)
+    none = [None, None]
+    with pytest.raises(RuntimeError, match="GPU"):      # in order but for the device
+        ops.adaln_rmsnorm_grouped(x, [w, w], none, none, [(0, 2), (2, 2)], 1e-6, y)
+    for ws, shifts, scales, segs in (([w, w[:32]], none, none, [(0, 2), (2, 2)]), ([w], none, none, [(0, 2), (2, 2)]),
+                                     ([w, w], [None], none, [(0, 2), (2, 2)]), ([w, w], none, [None], [(0, 2), (2, 2)]),
+                                     ([w, w], none, none, [(0, 2), (2, 3)]), ([w, w], none, none, [(-1, 2), (2, 2)])):
+        with pytest.raises(ValueError):
+            ops.adaln_rmsnorm_grouped(x, ws, shifts, scales, segs, 1e-6, y)
