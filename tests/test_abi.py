@@ -174,6 +174,62 @@ def test_conditioning_arguments_are_validated_on_the_host():
     assert lib.cdm_timestep_sinusoid_f32(None, fake, 1, 256, None) == _lib.ERR_BAD_ARG
     assert lib.cdm_timestep_sinusoid_f32(fake, fake, 1, 255, None) == _lib.ERR_BAD_SHAPE
 
+    def mlp(t=fake, w1=fake, b1=fake, w2=fake, b2=fake, hidden=fake, out=fake, freq=256, d=64):
+        return lib.cdm_timestep_mlp_f32(t, w1, b1, w2, b2, hidden, out, freq, d, None)
+    for name in ("t", "w1", "b1", "w2", "b2", "hidden", "out"):
+        assert mlp(**{name: None}) == _lib.ERR_BAD_ARG
+    for name in ("w1", "w2", "hidden"):
+        assert mlp(**{name: fake + 4}) == _lib.ERR_BAD_ALIGN
+    for sizes in (dict(freq=0), dict(freq=258), dict(freq=16388), dict(d=0), dict(d=66), dict(d=16388)):
+        assert mlp(**sizes) == _lib.ERR_BAD_SHAPE
+
+    def mod(c=fake, w=(fake, fake), b=(fake, fake), n=2, out=fake, d=64, n_out=384):
+        P = C.c_void_p * 2
+        return lib.cdm_adaln_modulation_bf16(c, P(*w) if w else None, P(*b) if b else None, n, out, d, n_out, None)
+    assert mod(c=None) == mod(w=None) == mod(b=None) == mod(out=None) == mod(n=-1) == mod(n_out=0) == _lib.ERR_BAD_ARG
+    assert mod(w=(fake, None)) == mod(w=(fake, fake + 2)) == mod(b=(None, fake)) == _lib.ERR_BAD_ARG and "block 0" in _lib.last_error()
+    assert mod(d=60) == mod(d=16392) == mod(n_out=1 << 24) == _lib.ERR_BAD_SHAPE
+    assert mod(n=0) == _lib.OK
+
+
+def test_grouped_norms_are_validated_on_the_host():
+    lib = _lib.load()
+    fake = 0x10000
+    P, I = C.c_void_p * 2, C.c_int64 * 2
+
+    def norm(x=fake, w=(fake, fake), shift=(None, None), scale=(None, None), start=(0, 4), length=(4, 4), n=2, y=fake, d=64, src=None):
+        args = (P(*w) if w else None, P(*shift), P(*scale), I(*start) if start else None, I(*length), n, y, None, d, 1e-6, None)
+        return lib.cdm_adaln_rmsnorm_grouped(x, 0, *args) if src is None else lib.cdm_adaln_rmsnorm_join(P(*src) if src else None, x, *args)
+    for kw in ({}, {"src": (fake, fake)}):
+        assert norm(x=None, **kw) == norm(w=None, **kw) == norm(w=(fake, None), **kw) == norm(y=None, **kw) == _lib.ERR_BAD_ARG
+        assert norm(start=None, **kw) == norm(n=-1, **kw) == norm(n=65, **kw) == norm(start=(0, -1), **kw) == _lib.ERR_BAD_ARG
+        assert norm(length=(4, -4), **kw) == norm(start=(0, 1 << 31), **kw) == _lib.ERR_BAD_ARG
+        assert norm(d=60, **kw) == norm(d=8200, **kw) == _lib.ERR_BAD_SHAPE
+        assert norm(x=fake + 8, **kw) == norm(w=(fake, fake + 8), **kw) == norm(shift=(None, fake + 4), **kw) == _lib.ERR_BAD_ALIGN
+    assert norm(src=()) == _lib.ERR_BAD_ARG
+    assert norm(src=(fake, None)) == norm(src=(fake + 8, fake)) == _lib.ERR_BAD_ALIGN
+
+
+def test_gemm_with_scratch_is_validated_on_the_host():
+    lib = _lib.load()
+    fake = 0x10000
+
+    def call(epi=_lib.EPI_NONE, scratch=fake, n=1 << 20, K=8192, R=None, gate=None, A=fake):
+        one = lambda v: (C.c_void_p * 1)(v)
+        return lib.cdm_grouped_gemm_scratch_bf16(A, K, one(fake), K, fake, 512, (C.c_int64 * 1)(0), (C.c_int64 * 1)(64), 1, 512, K, epi, R, 512,
+                                                 one(gate) if gate else None, scratch, n, None)
+    for epi in (_lib.EPI_SWIGLU, _lib.EPI_ROPE_QK, 5):
+        assert call(epi=epi) == _lib.ERR_UNSUPPORTED
+    assert call(scratch=fake + 8) == call(n=-1) == call(A=fake + 8) == _lib.ERR_BAD_ALIGN
+    assert call(A=None) == call(epi=_lib.EPI_GATE_RESIDUAL_F32) == _lib.ERR_BAD_ARG                      # residual missing
+    assert call(epi=_lib.EPI_GATE_RESIDUAL_F32, R=fake, gate=fake + 4) == _lib.ERR_BAD_ALIGN
+    assert call(K=8200) == _lib.ERR_BAD_SHAPE
+    # refused or none: no scratch to bring
+    ask = lambda lens, N=512, K=8192, epi=_lib.EPI_NONE: lib.cdm_grouped_gemm_scratch_bytes((C.c_int64 * len(lens))(*lens), len(lens), N, K, epi)
+    assert ask([64]) > 0 and ask([32, 0, 32]) > 0
+    assert ask([0]) == ask([-1]) == ask([64], N=0) == ask([64], K=0) == ask([64], epi=_lib.EPI_SWIGLU) == ask([8] * 9) == 0
+    assert lib.cdm_grouped_gemm_scratch_bytes(None, 1, 512, 8192, 0) == 0
+
 
 def test_runs_that_lie_apart_are_validated_on_the_host():
     lib = _lib.load()

@@ -155,7 +155,8 @@ def test_adaln_rmsnorm_closed_form():
 @pytest.mark.parametrize("epi", ["none", "gate_residual", "gate_residual_f32"])
 def test_gemm_cut_along_k(lens, N, K, epi):
     """Launches with few tiles and a long K run in ranges of K.  Ragged rows and columns, several segments, a k-tile count that
-    the ranges do not divide.  Against 64 bits: fp32 sums within 1e-6 of the product's scale, bf16 outputs half a unit more."""
+    the ranges do not divide.  Against 64 bits: fp32 sums within 1e-5 (of the scale of one, rounded K / 32 = 512 times at most, by
+    chance sqrt(512) 2^-24 = 1.4e-6, times gates of up to four), bf16 outputs half a unit more."""
     g = gen(N + K + sum(lens))
     M, f32 = sum(lens), epi == "gate_residual_f32"
     at = [sum(lens[:i]) for i in range(len(lens))]
@@ -849,7 +850,8 @@ def test_attention_vs_oracle(n, H, hd, variant):
                                                      (4096, 8, 8, 128, 0, 0, False), (4097, 8, 8, 128, 0, 0, False)])
 def test_attention_128_row_workgroups_equal_the_256_row_ones(n, H, Hkv, hd, P, causal, qkn, request):
     """Workgroups of 128 query rows and four waves: a row's arithmetic does not depend on the workgroup's size, so the bits do
-    not either.  By default short key sequences take that form, and grids beyond the rule of small ones the 256-row one."""
+    not either.  By default short key sequences take that form, grids beyond the rule of small ones the 256-row one, and small
+    grids with many key tiles the one whose two groups of waves share the tiles out."""
     request.addfinalizer(lambda: ops.set_variant("attn", 0))
     g = gen(n + H)
     q, _ = rand_bf16((n, H * hd), g)
@@ -861,12 +863,13 @@ def test_attention_128_row_workgroups_equal_the_256_row_ones(n, H, Hkv, hd, P, c
     img = ops.attention_pack_kv(k, v, Hkv, hd, None, cos, sin, norm)
     prefix = (ops.attention_pack_kv(k[:P].contiguous(), v[:P].contiguous(), Hkv, hd), P) if P else None
     res = {}
-    for variant in (4, 3, 0):
+    for variant in (4, 3, 0, 5):
         ops.set_variant("attn", variant)
         amax = torch.zeros((n, H), device=dev())
         res[variant] = (ops.attention_packed(q, img, H, hd, None, cos, sin, norm, prefix, causal, Hkv, row_amax=amax), amax)
-    for variant in (3, 0) if n in (1, 129, 4097) else (3,):
-        assert torch.equal(res[variant][0], res[4][0]) and torch.equal(res[variant][1], res[4][1]), f"variant {variant}"
+    for variant, like in ((3, 4), (0, 4 if n in (1, 129, 4097) else 5)):
+        assert torch.equal(res[variant][0], res[like][0]) and torch.equal(res[variant][1], res[like][1]), f"variant {variant}"
+    assert n in (1, 129, 4097) or not torch.equal(res[5][0], res[4][0])      # the forms' sums are in another order
 
 
 @pytest.mark.parametrize("rot", [True, False])
