@@ -13,6 +13,7 @@ Per-branch ("Mixture-of-Transformers") weights: branch b of a layer owns
 """
 from __future__ import annotations
 
+import itertools
 import math
 from typing import List, Optional, Sequence, Tuple
 
@@ -416,33 +417,41 @@ def _as_is(m: nn.Module, cls: type) -> bool:
             and not _any_module_hook())
 
 
-def _eager(*tensors: torch.Tensor) -> bool:
-    """Plain tensors in plain eager execution, where a kernel that takes their pointers may stand in for torch operators: no
+_TENSORS = (torch.Tensor, nn.Parameter)
+
+
+def _eager(t: torch.Tensor) -> bool:
+    """A plain tensor in plain eager execution, where a kernel that takes pointers may stand in for torch operators: no
     compilation, tracing or dispatch mode that has to see the operators, no subclass whose storage is not the value, no
     forward-mode derivative or function transform (``torch.func``; a tensor that carries a tangent has no mark of its own to ask
     for), and no autocast, which chooses the type a linear layer computes in and returns."""
     if torch.compiler.is_compiling():
         return False
-    return (all(type(t) in (torch.Tensor, nn.Parameter) for t in tensors) and torch._C._len_torch_dispatch_stack() == 0
-            and torch._C._get_tracing_state() is None and torch._C._functorch.peek_interpreter_stack() is None
-            and torch.autograd.forward_ad._current_level < 0 and not torch.is_autocast_enabled("cuda"))
+    return (type(t) in _TENSORS and torch._C._len_torch_dispatch_stack() == 0 and torch._C._get_tracing_state() is None
+            and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
+            and not torch.is_autocast_enabled("cuda"))
 
 
 def _plain(lin: nn.Module, device: torch.device, dtype: torch.dtype) -> bool:
     """An ``nn.Linear`` with bias as it stands - no subclass, wrapper, replaced forward or hook that a kernel on its parameters
     would pass by, no gradient asked of it - whose parameters such a kernel can read."""
-    return (_as_is(lin, nn.Linear) and lin.bias is not None
-            and not (torch.is_grad_enabled() and (lin.weight.requires_grad or lin.bias.requires_grad))
-            and all(type(p) in (torch.Tensor, nn.Parameter) and p.device == device and p.dtype == dtype and p.is_contiguous()
-                    for p in (lin.weight, lin.bias))
-            and lin.weight.data_ptr() % 16 == 0 and lin.in_features % 8 == 0 and 0 < lin.in_features <= 16384)
+    if not _as_is(lin, nn.Linear):
+        return False
+    w, b, k = lin.weight, lin.bias, lin.in_features
+    for p in (w, b):
+        if type(p) not in _TENSORS or p.dtype != dtype or p.device != device or not p.is_contiguous():      # (a missing bias: None)
+            return False
+    if torch.is_grad_enabled() and (w.requires_grad or b.requires_grad):
+        return False
+    return w.data_ptr() % 16 == 0 and k % 8 == 0 and 0 < k <= 16384
 
 
 def _modulations(lins: Sequence[nn.Module], temb: torch.Tensor) -> Optional[List[Tuple[torch.Tensor, ...]]]:
     """(shift1, scale1, gate1, shift2, scale2, gate2), each [d] fp32, of every block from its modulation layer: one launch over
     all of them.  None where a kernel on their parameters cannot stand in for the layers."""
     wants_grad = temb.requires_grad and torch.is_grad_enabled()
-    if not lins or not _eager(temb) or not temb.is_cuda or wants_grad or not all(_plain(l, temb.device, torch.bfloat16) for l in lins):
+    device = temb.device
+    if not lins or not _eager(temb) or device.type != "cuda" or wants_grad or not all(_plain(l, device, torch.bfloat16) for l in lins):
         return None
     if any(l.weight.shape != lins[0].weight.shape for l in lins):
         return None
@@ -451,12 +460,14 @@ def _modulations(lins: Sequence[nn.Module], temb: torch.Tensor) -> Optional[List
     return [rows[6 * i:6 * i + 6] for i in range(len(lins))]
 
 
-def _bare(blk: Optional[nn.Module]) -> bool:
+def _bare(blk: nn.Module) -> bool:
     """A block in which only this file's code runs, so that a stack may do parts of its work ahead of its call.  Any other block
     (a subclass, a wrapper, hooks that change ``temb`` or load weights, a replaced processor) may read, change or ignore what
     it is called with, and the blocks behind it."""
-    return (_as_is(blk, DMBlock) and "modulation" not in blk.__dict__ and _as_is(blk.attn, DMAttention)
-            and type(blk.attn.processor) is DMAttnProcessor)
+    if not _as_is(blk, DMBlock) or "modulation" in blk.__dict__:
+        return False
+    attn = blk.attn
+    return _as_is(attn, DMAttention) and type(attn.processor) is DMAttnProcessor
 
 
 class DMBlock(nn.Module):
@@ -655,7 +666,7 @@ class DMStack(nn.Module):
         if c.n_text == 0:
             raise ValueError("context reuse needs a text run")
         segs = [(0, c.n_text, 0, False)]
-        x, sources = self._joined([_as2d(encoder_hidden_states)], segs, c.n_text, "context")
+        x, sources = self._joined([_as2d(encoder_hidden_states)], segs, c.n_text, "context", len(self.blocks) > 0 and _bare(self.blocks[0]))
         cos, sin = self.rotary(x.device)
         rot = (cos[:c.n_text].contiguous(), sin[:c.n_text].contiguous())
         ws = Workspace(c.n_text, c.d_model, c.hidden, c.n_heads, c.head_dim, x.device, c.kv_heads, c.fp8)
@@ -695,13 +706,14 @@ class DMStack(nn.Module):
         parts.append(_as2d(hidden_states))
         parts += self._generator_extras(audio_states, action_states)
         segs = self.segments()
-        x, sources = self._joined(parts, segs, c.n_tokens, "joint")
+        bare = [_bare(b) for b in self.blocks]
+        x, sources = self._joined(parts, segs, c.n_tokens, "joint", bare[:1] == [True])
         rot = self.rotary(x.device)
         temb = self.time_embedder(timestep.reshape(-1)[:1])
         if self._ws is None or not self._ws.fits(c.n_tokens, c.d_model, c.hidden, c.fp8) or self._ws.y.device != x.device:
             self._ws = Workspace(c.n_tokens, c.d_model, c.hidden, c.n_heads, c.head_dim, x.device, c.kv_heads, c.fp8)
         kw = {"causal_prefix": c.n_text if c.hybrid_mask else 0}
-        self._run_blocks(x, temb, rot, segs, self._ws, sources, [kw] * len(self.blocks))
+        self._run_blocks(x, temb, rot, segs, self._ws, sources, all(bare), [kw] * len(bare))
         return self._result(x, c.n_text, hidden_states.dim() == 3, return_dict, joint_only)
 
     def capture(self, hidden_states: torch.Tensor, timestep: torch.Tensor,
@@ -726,9 +738,10 @@ class DMStack(nn.Module):
             at += p.shape[0]
         return x
 
-    def _joined(self, parts: Sequence[torch.Tensor], segs: Sequence[Segment], n: int, what: str):
-        """(stream, sources) of the runs.  Where the first block's norm can join them as it reads them - its segments are the
-        runs -, the stream is not filled yet and ``sources`` are the runs; otherwise it is, and ``sources`` is None."""
+    def _joined(self, parts: Sequence[torch.Tensor], segs: Sequence[Segment], n: int, what: str, first_bare: bool):
+        """(stream, sources) of the runs.  Where the first block's norm can join them as it reads them - the block is a bare one
+        (others may read their input) and its segments are the runs -, the stream is not filled yet and ``sources`` are the runs;
+        otherwise it is, and ``sources`` is None."""
         d = self.cfg.d_model
         rows = sum(p.shape[0] for p in parts)
         if rows != n or any(p.dim() != 2 or p.shape[1] != d for p in parts):
@@ -736,18 +749,18 @@ class DMStack(nn.Module):
         dev = parts[0].device
         if any(p.device != dev for p in parts):
             raise RuntimeError(f"the runs of the {what} sequence lie on different devices")
-        first = self.blocks[0] if len(self.blocks) else None      # a subclass or a hook may read its input: it gets it filled
-        starts = [sum(p.shape[0] for p in parts[:i]) for i in range(len(parts))]
-        if (_bare(first) and self.cfg.residual_fp32 and dev.type == "cuda" and d % 8 == 0
-                and [(s0, ln) for (s0, ln, _, _) in segs] == [(s0, p.shape[0]) for s0, p in zip(starts, parts)]
-                and all(p.dtype == torch.bfloat16 and p.device == dev and p.is_contiguous() and p.data_ptr() % 16 == 0 for p in parts)):
+        lens = [p.shape[0] for p in parts]
+        if (first_bare and self.cfg.residual_fp32 and dev.type == "cuda" and d % 8 == 0
+                and [(s0, ln) for (s0, ln, _, _) in segs] == list(zip(itertools.accumulate(lens, initial=0), lens))
+                and all(p.dtype == torch.bfloat16 and p.is_contiguous() and p.data_ptr() % 16 == 0 for p in parts)):
             return torch.empty((n, d), dtype=torch.float32, device=dev), list(parts)
         return self._stream(*parts), None
 
-    def _run_blocks(self, x: torch.Tensor, temb: torch.Tensor, rot, segs, workspace: Workspace, sources, kws: Sequence[dict]) -> None:
+    def _run_blocks(self, x: torch.Tensor, temb: torch.Tensor, rot, segs, workspace: Workspace, sources, bare: bool,
+                    kws: Sequence[dict]) -> None:
         """All blocks over the stream x.  Their modulation comes from one launch ahead of the first where all of them are bare;
         otherwise every block computes its own from the ``temb`` that reaches it, in its own call."""
-        mods = _modulations([b.adaLN_modulation for b in self.blocks], temb) if all(_bare(b) for b in self.blocks) else None
+        mods = _modulations([b.adaLN_modulation for b in self.blocks], temb) if bare else None
         for i, (blk, kw) in enumerate(zip(self.blocks, kws)):
             if mods is not None:
                 kw = {**kw, "modulation": mods[i]}
@@ -784,14 +797,15 @@ class DMStack(nn.Module):
         parts = [_as2d(hidden_states)] + self._generator_extras(audio_states, action_states)
         n = c.n_tokens - P
         segs = [(s0 - P, ln, b, m) for (s0, ln, b, m) in self.segments() if s0 >= P]
-        x, sources = self._joined(parts, segs, n, "generator")
+        bare = [_bare(b) for b in self.blocks]
+        x, sources = self._joined(parts, segs, n, "generator", bare[:1] == [True])
         if self._rot_gen is None or self._rot_gen[0].device != x.device:
             cos, sin = self.rotary(x.device)
             self._rot_gen = (cos[P:].contiguous(), sin[P:].contiguous())
         temb = self.time_embedder(timestep.reshape(-1)[:1])
         if self._ws_gen is None or not self._ws_gen.fits(n, c.d_model, c.hidden, c.fp8) or self._ws_gen.y.device != x.device:
             self._ws_gen = Workspace(n, c.d_model, c.hidden, c.n_heads, c.head_dim, x.device, c.kv_heads, c.fp8)
-        self._run_blocks(x, temb, self._rot_gen, segs, self._ws_gen, sources, [{"prefix": (img, P)} for img in cache.images])
+        self._run_blocks(x, temb, self._rot_gen, segs, self._ws_gen, sources, all(bare), [{"prefix": (img, P)} for img in cache.images])
         return self._result(x, 0, hidden_states.dim() == 3, return_dict, joint_only)
 
 
