@@ -1,6 +1,8 @@
 // The "NT" GEMM C[M,N] = A[M,K] . W[N,K]^T for launches that 256 x 256 tiles (gemm.hip) leave the chip idle for: a text
 // run, an action run, one image, small models.  Same operands, same order of every sum (a row of C comes out bit for bit
-// the same whatever the tile), same epilogues; smaller output tiles.
+// the same whatever the tile), same epilogues; smaller output tiles.  The exception are launches cut along K (best_split: bf16,
+// plain and residual epilogues): their ranges' sums are added last, and as the number of rows decides about the cut, the last
+// bits of a row depend on how many rows share the call.
 //
 // What bounds it: the feed of one CU.  With weights that no cache holds (every weight of a prompt is read exactly once) a CU
 // takes 57 - 72 bytes per ns into its LDS whatever the tile (0.40 us per k-tile at 64 x 128, 0.53 at 128 x 128), 78 with the
