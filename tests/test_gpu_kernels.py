@@ -399,6 +399,32 @@ def test_conditioning_is_traced_as_operators(how):
         assert torch.allclose(f(other), want, rtol=1e-4, atol=1e-5)      # angles of 700 with a relative error of a few 2^-24
 
 
+def test_conditioning_under_function_modes():
+    """A mode that sees or replaces torch functions gets the conditioning layers' own; ``torch.device`` as a context does neither."""
+    from torch.overrides import TorchFunctionMode
+    from cosmos_amd import DMBlock, TimestepEmbedder
+    te, t = TimestepEmbedder(64, device=dev()), torch.tensor([3.0], device=dev())
+    blk = DMBlock(64, 1, 64, 128, 1, device=dev())
+    blk.reset_parameters(torch.Generator(device=dev()).manual_seed(1))
+    c, seen = torch.randn((1, 64), generator=gen(2)).to(dev()), []
+
+    class Note(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with torch.no_grad():
+        with Note(), torch.device("cuda"):
+            te(t), blk.modulation(c), te.sinusoid(t)
+        assert seen.count(torch.nn.functional.linear) == 3 and seen.count(torch.cat) == 2
+        ops.time_ops(True)
+        try:
+            with torch.device("cuda"):
+                te(t), blk.modulation(c), te.sinusoid(t)
+        finally:
+            assert [n for n, _, _ in ops.time_ops(False)] == ["cond"] * 3
+
+
 def test_stack_refuses_runs_on_different_devices():
     from cosmos_amd import DMConfig, DMStack
     st = DMStack(DMConfig("t", 256, 2, 128, 512, 1, (2, 4, 9), n_text=37), device=dev())
