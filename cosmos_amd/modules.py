@@ -412,10 +412,14 @@ def _routed_linear(a, sa, weights, qweights, weights2, segments, *, out, epilogu
                          head_dim=head_dim, out=out, row_amax=row_amax)
 
 
+# the forwards as written (those of this file's classes: below DMStack); one may be replaced for the whole class later
+_FORWARD = {nn.Linear: nn.Linear.forward}
+
+
 def _as_is(m: nn.Module, cls: type) -> bool:
-    """Calling ``m`` runs the forward of ``cls`` and nothing else: no subclass, forward set on the instance or hook."""
-    return (type(m) is cls and "forward" not in m.__dict__ and not m._forward_hooks and not m._forward_pre_hooks
-            and not _any_module_hook())
+    """Calling ``m`` runs the forward of ``cls`` and nothing else: no subclass, forward set on the instance or class, or hook."""
+    return (type(m) is cls and "forward" not in m.__dict__ and cls.forward is _FORWARD[cls] and not m._forward_hooks
+            and not m._forward_pre_hooks and not _any_module_hook())
 
 
 _TENSORS = (torch.Tensor, nn.Parameter)
@@ -471,7 +475,7 @@ def _bare(blk: nn.Module) -> bool:
     """A block in which only this file's code runs, so that a stack may do parts of its work ahead of its call.  Any other block
     (a subclass, a wrapper, hooks that change ``temb`` or load weights, a replaced processor) may read, change or ignore what
     it is called with, and the blocks behind it."""
-    if not _as_is(blk, DMBlock) or "modulation" in blk.__dict__:
+    if not _as_is(blk, DMBlock) or "modulation" in blk.__dict__ or DMBlock.modulation is not _MODULATION:
         return False
     attn = blk.attn
     return _as_is(attn, DMAttention) and type(attn.processor) is DMAttnProcessor
@@ -814,6 +818,10 @@ class DMStack(nn.Module):
             self._ws_gen = Workspace(n, c.d_model, c.hidden, c.n_heads, c.head_dim, x.device, c.kv_heads, c.fp8)
         self._run_blocks(x, temb, self._rot_gen, segs, self._ws_gen, sources, all(bare), [{"prefix": (img, P)} for img in cache.images])
         return self._result(x, 0, hidden_states.dim() == 3, return_dict, joint_only)
+
+
+_FORWARD.update({cls: cls.forward for cls in (DMAttention, DMBlock, DMStack)})
+_MODULATION = DMBlock.modulation
 
 
 class GraphedStack:

@@ -916,3 +916,34 @@ def test_projections_of_an_attention_subclass_get_joined_tokens(n_enc, fuse):
     attn.__class__ = Scaled
     got = attn(h, encoder_hidden_states=e, image_rotary_emb=rot)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+def test_stack_under_methods_replaced_on_a_class(monkeypatch):
+    """Methods that are replaced for a whole class are called like those of one block or layer."""
+    cfg = DMConfig("t", 256, 2, 128, 512, 2, (2, 4, 9), n_text=37)
+    st = DMStack(cfg, device=dev())
+    st.reset_parameters(3)
+    g = torch.Generator().manual_seed(4)
+    ctx, x = rand_bf16((1, 37, 256), g)[0], rand_bf16((1, 72, 256), g)[0]
+    t, te = torch.tensor([500.0], device=dev()), st.time_embedder
+    own = DMBlock.modulation
+    run = lambda: st(x, t, encoder_hidden_states=ctx, return_dict=True)["joint"]
+    with monkeypatch.context() as m:
+        m.setattr(DMBlock, "modulation", lambda self, temb: own(self, temb * 2.0))
+        got = run()
+    for i in range(2):
+        alter_block("modulation set on the instance", st, i)
+    assert torch.equal(got, run())
+    for b in st.blocks:
+        del b.modulation
+    linear, block, seen = torch.nn.Linear.forward, DMBlock.forward, []
+    with monkeypatch.context() as m:
+        m.setattr(torch.nn.Linear, "forward", lambda self, v: linear(self, v) * 2.0)
+        got = te(t)
+    with torch.no_grad():
+        want = linear(te.linear_2, torch.nn.functional.silu(linear(te.linear_1, te.sinusoid(t)) * 2.0)) * 2.0
+    assert torch.equal(got, want)
+    with monkeypatch.context() as m:
+        m.setattr(DMBlock, "forward", lambda self, v, *a, **kw: (seen.append(v.clone()), block(self, v, *a, **kw))[1])
+        run()
+    assert torch.equal(seen[0], torch.cat([ctx[0], x[0]]).float())
