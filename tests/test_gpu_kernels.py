@@ -425,6 +425,24 @@ def test_conditioning_under_function_modes():
             assert [n for n, _, _ in ops.time_ops(False)] == ["cond"] * 3
 
 
+@pytest.mark.parametrize("how", ["subclass", "instance", "class"])
+def test_embedder_takes_another_sinusoid(how, monkeypatch):
+    """An embedding that is overridden feeds the two layers."""
+    from cosmos_amd import TimestepEmbedder
+    te, t = TimestepEmbedder(64, device=dev()), torch.tensor([3.0], device=dev())
+    own = te.sinusoid
+    with torch.no_grad():
+        want = te.linear_2(torch.nn.functional.silu(te.linear_1(own(t) * 2.0)))
+        if how == "subclass":
+            te.__class__ = type("Doubled", (TimestepEmbedder,), {"sinusoid": lambda self, t: own(t) * 2.0})
+        elif how == "instance":
+            te.sinusoid = lambda t: own(t) * 2.0
+        else:
+            first = TimestepEmbedder.sinusoid
+            monkeypatch.setattr(TimestepEmbedder, "sinusoid", lambda self, t: first(self, t) * 2.0)
+        assert torch.equal(te(t), want)
+
+
 def test_stack_refuses_runs_on_different_devices():
     from cosmos_amd import DMConfig, DMStack
     st = DMStack(DMConfig("t", 256, 2, 128, 512, 1, (2, 4, 9), n_text=37), device=dev())
