@@ -600,7 +600,7 @@ class TimestepEmbedder(nn.Module):
     def forward(self, t: torch.Tensor) -> torch.Tensor:
         l1, l2 = self.linear_1, self.linear_2
         if (_eager(t) and t.is_cuda and t.numel() == 1 and not torch.is_grad_enabled() and _plain(l1, t.device, torch.float32)
-                and _plain(l2, t.device, torch.float32) and l1.in_features == self.freq_dim
+                and _plain(l2, t.device, torch.float32) and l1.weight.shape[1] == self.freq_dim
                 and l2.weight.shape == (l1.out_features, l1.out_features)
                 and getattr(self.sinusoid, "__func__", None) is _SINUSOID):      # the MLP's kernel builds this file's own
             return ops.timestep_mlp(t.reshape(-1).to(torch.float32), l1.weight, l1.bias, l2.weight, l2.bias)

@@ -443,6 +443,15 @@ def test_embedder_takes_another_sinusoid(how, monkeypatch):
         assert torch.equal(te(t), want)
 
 
+def test_embedder_refuses_weights_of_another_width():
+    """The first layer's weights and the sinusoid have to agree, as torch's product asks."""
+    from cosmos_amd import TimestepEmbedder
+    te, t = TimestepEmbedder(64, device=dev()), torch.tensor([3.0], device=dev())
+    te.linear_1.weight = torch.nn.Parameter(torch.zeros(64, 128, device=dev()))
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        te(t)
+
+
 def test_stack_refuses_runs_on_different_devices():
     from cosmos_amd import DMConfig, DMStack
     st = DMStack(DMConfig("t", 256, 2, 128, 512, 1, (2, 4, 9), n_text=37), device=dev())
