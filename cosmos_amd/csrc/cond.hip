@@ -109,7 +109,8 @@ __global__ __launch_bounds__(64 * kWaves) void modulation_kernel(const ModParams
 
 extern "C" int32_t cdm_timestep_sinusoid_f32(const float* t, float* out, int64_t n, int64_t freq_dim, void* stream) {
     CDM_REQUIRE((t && out) || n == 0, CDM_ERR_BAD_ARG, "timestep_sinusoid: null pointer");
-    CDM_REQUIRE(n >= 0 && n < (1ll << 31) && freq_dim >= 2 && freq_dim % 2 == 0 && freq_dim < (1ll << 24), CDM_ERR_BAD_SHAPE,
+    // (a workgroup of 256 threads per timestep: fewer than 2^32 threads)
+    CDM_REQUIRE(n >= 0 && n < (1ll << 24) && freq_dim >= 2 && freq_dim % 2 == 0 && freq_dim < (1ll << 24), CDM_ERR_BAD_SHAPE,
                 "timestep_sinusoid: n=%lld, freq_dim=%lld (even)", (long long)n, (long long)freq_dim);
     if (n == 0) return CDM_OK;
     int32_t rc = cdm_require_device();

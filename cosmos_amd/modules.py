@@ -590,7 +590,8 @@ class TimestepEmbedder(nn.Module):
 
     def sinusoid(self, t: torch.Tensor) -> torch.Tensor:
         half = self.freq_dim // 2
-        if _eager(t) and t.is_cuda and half > 0 and self.freq_dim % 2 == 0 and not (t.requires_grad and torch.is_grad_enabled()):
+        if (_eager(t) and t.is_cuda and 0 < half < 1 << 23 and self.freq_dim % 2 == 0 and t.numel() < 1 << 24      # (the launch's limits)
+                and not (t.requires_grad and torch.is_grad_enabled())):
             return ops.timestep_sinusoid(t.reshape(-1).to(torch.float32).contiguous(), self.freq_dim)
         k = torch.arange(half, dtype=torch.float32, device=t.device)
         f = torch.exp(-math.log(10000.0) * k / half)

@@ -296,7 +296,7 @@ int32_t cdm_linear_bias_bf16(const void* A, int64_t lda, const void* W, int64_t 
 /*
  * Sinusoidal embedding ahead of the time_embedder's MLP (parameter names: transformers
  * models/cosmos3_omni/modeling_cosmos3_omni.py:50): out[i] = [cos | sin](t[i] f_k), f_k = 10000^(-k / (freq_dim / 2)).
- * t: [n] fp32; out: [n, freq_dim] fp32.
+ * t: [n] fp32; out: [n, freq_dim] fp32; n and freq_dim below 2^24.
  */
 int32_t cdm_timestep_sinusoid_f32(const float* t, float* out, int64_t n, int64_t freq_dim, void* stream);
 

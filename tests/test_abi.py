@@ -210,6 +210,13 @@ def test_grouped_norms_are_validated_on_the_host():
     assert norm(src=(fake, None)) == norm(src=(fake + 8, fake)) == _lib.ERR_BAD_ALIGN
 
 
+def test_sinusoid_refuses_what_its_launch_does_not_hold():
+    """A workgroup of 256 threads per timestep, fewer than 2^32 threads."""
+    lib = _lib.load()
+    assert lib.cdm_timestep_sinusoid_f32(0x10000, 0x10000, 1 << 24, 2, None) == _lib.ERR_BAD_SHAPE
+    assert lib.cdm_timestep_sinusoid_f32(0x10000, 0x10000, 1, 1 << 24, None) == _lib.ERR_BAD_SHAPE
+
+
 def test_gemm_with_scratch_is_validated_on_the_host():
     lib = _lib.load()
     fake = 0x10000

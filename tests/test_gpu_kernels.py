@@ -452,6 +452,20 @@ def test_embedder_refuses_weights_of_another_width():
         te(t)
 
 
+@pytest.mark.parametrize("n,freq", [(1 << 24, 2), ((1 << 24) - 1, 2), (1, 1 << 24), (1, (1 << 24) - 2)])
+def test_sinusoid_at_the_ends_of_its_launch(n, freq):
+    """Timesteps or frequencies beyond one launch go through torch.  Angles below 1: 1e-6."""
+    from cosmos_amd import TimestepEmbedder
+    te = TimestepEmbedder(1, freq_dim=freq, device=dev())
+    t = torch.linspace(0.0, 1.0, n, device=dev())
+    e = te.sinusoid(t)
+    assert e.shape == (n, freq)
+    half = freq // 2
+    for i in (0, n // 2, n - 1):
+        a = t[i].double() * torch.exp(-math.log(10000.0) * torch.arange(half, dtype=torch.float64, device=dev()) / half)
+        assert (e[i].double() - torch.cat([a.cos(), a.sin()])).abs().max().item() < 1e-6
+
+
 def test_stack_refuses_runs_on_different_devices():
     from cosmos_amd import DMConfig, DMStack
     st = DMStack(DMConfig("t", 256, 2, 128, 512, 1, (2, 4, 9), n_text=37), device=dev())
