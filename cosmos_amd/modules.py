@@ -139,7 +139,7 @@ class DMAttnProcessor:
                     and not attn.fp8 and n_enc > 0 and n_lat > 0
                     and all(t.is_cuda and t.device == x.device and t.dtype == torch.bfloat16 and t.shape[1] == attn.d_model
                             and t.stride(1) == 1 and t.stride(0) == x.stride(0) and t.stride(0) >= t.shape[1]
-                            and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (enc, x))):
+                            and t.stride(0) % 8 == 0 and t.stride(0) < 1 << 22 and t.data_ptr() % 16 == 0 for t in (enc, x))):
                 runs = [enc, x]
             else:
                 x = torch.cat([enc, x], dim=0)

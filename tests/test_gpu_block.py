@@ -947,3 +947,21 @@ def test_stack_under_methods_replaced_on_a_class(monkeypatch):
         m.setattr(DMBlock, "forward", lambda self, v, *a, **kw: (seen.append(v.clone()), block(self, v, *a, **kw))[1])
         run()
     assert torch.equal(seen[0], torch.cat([ctx[0], x[0]]).float())
+
+
+@pytest.mark.parametrize("fuse", [True, False])
+def test_context_and_latent_rows_far_apart(fuse):
+    """Rows further apart than the GEMM's strides reach are joined ahead of it."""
+    from cosmos_amd import DMAttnProcessor
+    g = torch.Generator().manual_seed(8)
+    attn = make_block(DMConfig("p", 256, 2, 128, 512, 1, (1, 2, 4), n_text=64, n_branches=2), 21).attn
+    attn.set_processor(DMAttnProcessor(fuse_kv_pack=fuse))
+    rows = rand_bf16((64, 512), g)[0]
+    pos, _ = rotary.build_positions(64, (1, 8, 8))
+    rot = rotary.rotary_tables(pos, 128, (32, 48, 48), device=dev())
+    want = attn(rows[None, :, 256:], encoder_hidden_states=rows[None, :, :256], image_rotary_emb=rot)
+    for stride in ((1 << 22) - 8, 1 << 22):
+        far = torch.empty((63 * stride + 512,), dtype=torch.bfloat16, device=dev()).as_strided((64, 512), (stride, 1))
+        far.copy_(rows)
+        got = attn(far[None, :, 256:], encoder_hidden_states=far[None, :, :256], image_rotary_emb=rot)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
