@@ -328,7 +328,6 @@ int32_t norm_runs(const void* const* src, const void* x, NormInput in, const voi
         if (rc) return rc;
         CDM_REQUIRE(in != kJoin || len[i] == 0 || (src[i] && cdm_aligned16(src[i])), CDM_ERR_BAD_ALIGN,
                     "adaln_rmsnorm_join: rows of run %d null or misaligned", i);
-        CDM_REQUIRE(start[i] >= 0 && start[i] + len[i] < (1ll << 31), CDM_ERR_BAD_ARG, "adaln_rmsnorm: bad token run %d", i);
     }
     int32_t rc = cdm_require_device();
     if (rc) return rc;
@@ -347,6 +346,14 @@ int32_t norm_runs(const void* const* src, const void* x, NormInput in, const voi
         else rc = s_tok == nullptr ? launch_norm<false, kBf16>(p, st) : launch_norm<true, kBf16>(p, st);
         if (rc) return rc;
     }
+    return CDM_OK;
+}
+
+// several runs of one sequence; a single one (start 0) has as many rows as its memory holds
+int32_t check_runs(const int64_t* start, const int64_t* len, int32_t n_seg) {
+    for (int i = 0; i < n_seg; ++i)
+        CDM_REQUIRE(start[i] >= 0 && len[i] >= 0 && start[i] < (1ll << 31) && len[i] < (1ll << 31) - start[i], CDM_ERR_BAD_ARG,
+                    "adaln_rmsnorm: bad token run %d", i);
     return CDM_OK;
 }
 
@@ -384,6 +391,8 @@ extern "C" int32_t cdm_adaln_rmsnorm_grouped(const void* x, int32_t x_is_f32, co
                                              const float* const* scale, const int64_t* seg_start, const int64_t* seg_len,
                                              int32_t n_seg, void* y, float* s_tok, int64_t d, float eps, void* stream) {
     CDM_REQUIRE(w && seg_start && seg_len && n_seg >= 0 && n_seg <= 64, CDM_ERR_BAD_ARG, "adaln_rmsnorm_grouped: bad token runs");
+    int32_t rc = check_runs(seg_start, seg_len, n_seg);
+    if (rc) return rc;
     return norm_runs(nullptr, x, x_is_f32 != 0 ? kF32 : kBf16, w, shift, scale, seg_start, seg_len, n_seg, y, s_tok, d, eps, stream);
 }
 
@@ -391,6 +400,8 @@ extern "C" int32_t cdm_adaln_rmsnorm_join(const void* const* src, float* x, cons
                                           const float* const* scale, const int64_t* seg_start, const int64_t* seg_len,
                                           int32_t n_seg, void* y, float* s_tok, int64_t d, float eps, void* stream) {
     CDM_REQUIRE(src && w && seg_start && seg_len && n_seg >= 0 && n_seg <= 64, CDM_ERR_BAD_ARG, "adaln_rmsnorm_join: bad token runs");
+    int32_t rc = check_runs(seg_start, seg_len, n_seg);
+    if (rc) return rc;
     return norm_runs(src, x, kJoin, w, shift, scale, seg_start, seg_len, n_seg, y, s_tok, d, eps, stream);
 }
 

@@ -217,6 +217,17 @@ def test_sinusoid_refuses_what_its_launch_does_not_hold():
     assert lib.cdm_timestep_sinusoid_f32(0x10000, 0x10000, 1, 1 << 24, None) == _lib.ERR_BAD_SHAPE
 
 
+@pytest.mark.skipif(HAS_GPU, reason="the addresses are for hosts without a device")
+def test_norms_of_one_run_take_any_number_of_rows():
+    """2^31 rows of eight channels are 34 GB."""
+    lib = _lib.load()
+    fake, rows = 0x10000, 1 << 31
+    for fn in (lib.cdm_adaln_rmsnorm_bf16, lib.cdm_adaln_rmsnorm_f32):
+        assert fn(fake, fake, None, None, fake, rows, 8, 1e-6, None) == _lib.ERR_NO_DEVICE
+    for fn in (lib.cdm_adaln_rmsnorm_quant_e4m3, lib.cdm_adaln_rmsnorm_f32_quant_e4m3):
+        assert fn(fake, fake, None, None, fake, fake, rows, 8, 1e-6, None) == _lib.ERR_NO_DEVICE
+
+
 def test_gemm_with_scratch_is_validated_on_the_host():
     lib = _lib.load()
     fake = 0x10000
