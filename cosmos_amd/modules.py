@@ -443,18 +443,18 @@ def _eager(t: torch.Tensor) -> bool:
             and not torch.is_autocast_enabled("cuda") and not _function_modes())
 
 
-def _plain(lin: nn.Module, device: torch.device, dtype: torch.dtype) -> bool:
-    """An ``nn.Linear`` with bias as it stands - no subclass, wrapper, replaced forward or hook that a kernel on its parameters
-    would pass by, no gradient asked of it - whose parameters such a kernel can read."""
+def _plain(lin: nn.Module, device: torch.device, dtype: torch.dtype) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+    """(weight, bias) of an ``nn.Linear`` with bias as it stands - no subclass, wrapper, replaced forward or hook that a kernel on
+    its parameters would pass by, no gradient asked of it - whose parameters such a kernel can read; None for any other."""
     if not _as_is(lin, nn.Linear):
-        return False
+        return None
     w, b, k = lin.weight, lin.bias, lin.in_features
     for p in (w, b):
         if type(p) not in _TENSORS or p.dtype != dtype or p.device != device or not p.is_contiguous():      # (a missing bias: None)
-            return False
+            return None
     if torch.is_grad_enabled() and (w.requires_grad or b.requires_grad):
-        return False
-    return w.data_ptr() % 16 == 0 and k % 8 == 0 and 0 < k <= 16384
+        return None
+    return (w, b) if w.data_ptr() % 16 == 0 and k % 8 == 0 and 0 < k <= 16384 else None
 
 
 def _modulations(lins: Sequence[nn.Module], temb: torch.Tensor) -> Optional[List[Tuple[torch.Tensor, ...]]]:
@@ -462,11 +462,15 @@ def _modulations(lins: Sequence[nn.Module], temb: torch.Tensor) -> Optional[List
     all of them.  None where a kernel on their parameters cannot stand in for the layers."""
     wants_grad = temb.requires_grad and torch.is_grad_enabled()
     device = temb.device
-    if not lins or not _eager(temb) or device.type != "cuda" or wants_grad or not all(_plain(l, device, torch.bfloat16) for l in lins):
+    if not lins or not _eager(temb) or device.type != "cuda" or wants_grad:
         return None
-    if any(l.weight.shape != lins[0].weight.shape for l in lins):
-        return None
-    m = ops.adaln_modulation(temb.reshape(-1).to(torch.float32), [l.weight for l in lins], [l.bias for l in lins])
+    ws, bs = [], []
+    for lin in lins:
+        wb = _plain(lin, device, torch.bfloat16)
+        if wb is None or (ws and wb[0].shape != ws[0].shape):
+            return None
+        ws.append(wb[0]); bs.append(wb[1])
+    m = ops.adaln_modulation(temb.reshape(-1).to(torch.float32), ws, bs)
     rows = m.view(6 * len(lins), -1).unbind(0)
     return [rows[6 * i:6 * i + 6] for i in range(len(lins))]
 
@@ -600,13 +604,13 @@ class TimestepEmbedder(nn.Module):
 
     def forward(self, t: torch.Tensor) -> torch.Tensor:
         l1, l2 = self.linear_1, self.linear_2
-        if (_eager(t) and t.is_cuda and t.numel() == 1 and not torch.is_grad_enabled() and _plain(l1, t.device, torch.float32)
-                and _plain(l2, t.device, torch.float32) and l1.weight.shape[1] == self.freq_dim
-                and l2.weight.shape == (l1.out_features, l1.out_features)
+        if (_eager(t) and t.is_cuda and t.numel() == 1 and not torch.is_grad_enabled()
                 and getattr(self.sinusoid, "__func__", None) is _SINUSOID):      # the MLP's kernel builds this file's own
-            return ops.timestep_mlp(t.reshape(-1).to(torch.float32), l1.weight, l1.bias, l2.weight, l2.bias)
-        e = self.sinusoid(t).to(self.linear_1.weight.dtype)
-        return self.linear_2(torch.nn.functional.silu(self.linear_1(e)))
+            p1, p2 = _plain(l1, t.device, torch.float32), _plain(l2, t.device, torch.float32)
+            if p1 and p2 and p1[0].shape[1] == self.freq_dim and p2[0].shape == (l1.out_features, l1.out_features):
+                return ops.timestep_mlp(t.reshape(-1).to(torch.float32), *p1, *p2)
+        e = self.sinusoid(t).to(l1.weight.dtype)
+        return l2(torch.nn.functional.silu(l1(e)))
 
 
 _SINUSOID = TimestepEmbedder.sinusoid
