@@ -14,6 +14,7 @@
 // Rotate-half mRoPE (and the QK-RMSNorm ahead of it) is applied in registers: to K while it is re-tiled for the
 // kernel, to Q when the kernel loads its Q fragments (both members of a rotary pair sit in the same lane).
 #include <mutex>
+#include <type_traits>
 
 #include "cdm_common.h"
 
@@ -95,6 +96,38 @@ __device__ __forceinline__ void mask_scores(f32x4 (&s)[KB][QB], const int (&keys
     }
 }
 
+// op(x, x of the lane 16 or 32 further: lane ^ 16, lane ^ 32), one instruction each instead of a round trip through the LDS unit:
+// with both operands x, v_permlane16_swap leaves the even rows of 16 lanes in one result and the odd ones in the other (32: halves)
+template <class Op>
+__device__ __forceinline__ float with_xor16(float x, Op op) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+template <class Op>
+__device__ __forceinline__ float with_xor32(float x, Op op) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// over the four quarter-waves: the lanes that hold a query row between them
+__device__ __forceinline__ float quarters_sum(float x) {
+    const auto add = [](float a, float b) { return a + b; };
+    return with_xor32(with_xor16(x, add), add);
+}
+__device__ __forceinline__ float quarters_max(float x) {
+    const auto max = [](float a, float b) { return __builtin_fmaxf(a, b); };
+    return with_xor32(with_xor16(x, max), max);
+}
+// smallest value among the 16 lanes of a row (quad exchanges, then mirrored halves and rows)
+__device__ __forceinline__ float row16_min(float x) {
+#define CDM_DPP_MIN(CTRL) x = __builtin_fminf(x, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true)))
+    CDM_DPP_MIN(0xb1);       // quad_perm [1, 0, 3, 2]
+    CDM_DPP_MIN(0x4e);       // quad_perm [2, 3, 0, 1]
+    CDM_DPP_MIN(0x141);      // row_half_mirror
+    CDM_DPP_MIN(0x140);      // row_mirror
+#undef CDM_DPP_MIN
+    return x;
+}
+
 template <int QB>
 __device__ __forceinline__ float tile_row_max(const f32x4 (&s)[KB][QB], int qb) {
     float mx = __builtin_fmaxf(s[0][qb][0], s[0][qb][1]);
@@ -102,8 +135,7 @@ __device__ __forceinline__ float tile_row_max(const f32x4 (&s)[KB][QB], int qb) 
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
         for (int e = (kb == 0 ? 2 : 0); e < 4; e += 2) mx = __builtin_fmaxf(__builtin_fmaxf(mx, s[kb][qb][e]), s[kb][qb][e + 1]);   // v_max3_f32
-    mx = __builtin_fmaxf(mx, __shfl_xor(mx, 16, 64));
-    return __builtin_fmaxf(mx, __shfl_xor(mx, 32, 64));
+    return quarters_max(mx);
 }
 
 // Index of the first tile after `after` whose bit is set in the wave's table (bit t of lane l = tile 32 l + t), or a
@@ -289,7 +321,7 @@ struct PackedParams {
     const float* cos; const float* sin;   // optional rotary tables [n_tokens, HD/2] applied to Q at load
     QkNormDev qn;                          // optional per-head RMSNorm of Q, applied before the rotation
     int n_tokens, n_heads, n_qblocks;
-    int kv_group;                // query heads per K / V head (1 = multi-head attention)
+    uint64_t kv_magic;           // ceil(2^32 / query heads per K / V head): head * kv_magic >> 32 is the K / V head (heads < 2^16)
     int always_max;              // cross-check: take the row maxima of every tile whatever the norm bound says
     float scale_log2e;           // factor on Q ahead of its rounding to bf16: log2(e)/sqrt(HD), or only its power of two
     float late_r;                // ... with the rest of it (in [1, 2)) applied to the fp32 scores (LATE kernels)
@@ -297,6 +329,7 @@ struct PackedParams {
     // are replaced by `split` units each, which cover consecutive ranges of the key tiles and leave a normalised partial
     // output and the row's log-sum in scratch memory for merge_split_kernel.  split = 1: no split.
     int split, split_tail;
+    __device__ __forceinline__ int kv_head_of(int head) const { return (int)((uint64_t)(uint32_t)head * kv_magic >> 32); }
     bf16_t* part_o;              // [8 * split_tail * split][256][HD]
     float* part_lse;             // [8 * split_tail * split][256]   log2 of the unit's sum of exponentials, reference added
 };
@@ -314,12 +347,22 @@ constexpr float kSafeLog2 = 60.0f;      // largest excess over the reference tha
 constexpr int kMaxKm = 2048;            // key tiles that get a decision of their own (131,072 keys); longer sequences: one per head
 constexpr int kMaxSplit = 8;            // most key ranges a query block of the last round is split into
 
-// Q fragments of a wave's rows q0 ..: rotate-half mRoPE (if tables are given) and the factor log2(e)/sqrt(HD), both in fp32 and
-// with ONE rounding to bf16.  The lane holds channels 32ks + 8g .. +7 (g = lane / 16) of its query row for every
-// ks, so the partner of a channel in k-step ks (< KS/2) is the same register element of k-step ks + KS/2.
-// qnorm: the norms of the scaled, rotated, rounded rows.
+// What a lane needs for the Q fragments of its rows, as it lies in memory: channels 32ks + 8g .. +7 (g = lane / 16) of every
+// k-step, the rotary factors of the first half of the k-steps (the partner of a channel in k-step ks < KS/2 is the same
+// register element of k-step ks + KS/2) and the norm's weights.  All of it is requested before anything is used, one round trip
+// to memory instead of one per row block and kind.  What bounds the set-up of a workgroup from there on is moving it into
+// the CU (256 rows of 128 channels: 64 KB of Q and 128 KB of tables, next to 48 - 96 KB of tiles) and the instructions
+// of finish_rows (an instruction per pair of values is 0.06 us with two waves per SIMD): 7.6 us at 256 rows of 128 channels,
+// 4.9 at 128, 3.9 at 64.
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));      // norm weights: rows of any 4-byte alignment
 template <int HD, int QB>
-__device__ __forceinline__ void load_q(const PackedParams& p, int head, int q0, int lane, bf16x8 (&qf)[QB][HD / 32], float (&qnorm)[QB]) {
+struct QRows {
+    u32x4 raw[QB][HD / 32];
+    f32x4 c[QB][HD / 64][2], s[QB][HD / 64][2], w[QB][HD / 32][2];
+};
+
+template <int HD, int QB>
+__device__ __forceinline__ void request_q(const PackedParams& p, int head, int q0, int lane, QRows<HD, QB>& r) {
     constexpr int KS = HD / 32;
     const int r16 = lane & 15, g4 = lane >> 4;
 #pragma unroll
@@ -327,72 +370,124 @@ __device__ __forceinline__ void load_q(const PackedParams& p, int head, int q0, 
         int qrow = q0 + qb * 16 + r16;
         qrow = qrow < p.n_tokens ? qrow : p.n_tokens - 1;
         const bf16_t* qp = p.q + (int64_t)qrow * p.ldq + head * HD + 8 * g4;
-        uint4 raw[KS];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) raw[ks] = *reinterpret_cast<const uint4*>(qp + 32 * ks);
+        for (int ks = 0; ks < KS; ++ks) r.raw[qb][ks] = *reinterpret_cast<const u32x4*>(qp + 32 * ks);
+    }
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+        int qrow = q0 + qb * 16 + r16;
+        qrow = qrow < p.n_tokens ? qrow : p.n_tokens - 1;
+        if (p.cos != nullptr) {
+            const f32x4* cp = reinterpret_cast<const f32x4*>(p.cos + (int64_t)qrow * (HD / 2) + 8 * g4);
+            const f32x4* sp = reinterpret_cast<const f32x4*>(p.sin + (int64_t)qrow * (HD / 2) + 8 * g4);
+#pragma unroll
+            for (int ks = 0; ks < KS / 2; ++ks)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) { r.c[qb][ks][h] = cp[8 * ks + h]; r.s[qb][ks][h] = sp[8 * ks + h]; }
+        } else {
+#pragma unroll
+            for (int ks = 0; ks < KS / 2; ++ks)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) { r.c[qb][ks][h] = f32x4{1.f, 1.f, 1.f, 1.f}; r.s[qb][ks][h] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+        }
+        if (p.qn.w != nullptr) {
+            const f32x4_any* nw = reinterpret_cast<const f32x4_any*>(p.qn.row(qrow, HD) + 8 * g4);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) { r.w[qb][ks][0] = nw[8 * ks]; r.w[qb][ks][1] = nw[8 * ks + 1]; }
+        }
+    }
+    asm volatile("" ::: "memory");      // the requests stay ahead of whatever follows
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// What was requested has arrived: the compiler's wait for it stands here, ahead of loads that are issued behind this point
+template <int HD, int QB>
+__device__ __forceinline__ void arrived(const PackedParams& p, QRows<HD, QB>& r) {
+    constexpr int KS = HD / 32;
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(r.raw[qb][ks]));
+#pragma unroll
+        for (int i = 0; i < KS; ++i) asm volatile("" : "+v"(r.c[qb][i / 2][i % 2]), "+v"(r.s[qb][i / 2][i % 2]));
+        if (p.qn.w != nullptr)
+#pragma unroll
+            for (int i = 0; i < 2 * KS; ++i) asm volatile("" : "+v"(r.w[qb][i / 2][i % 2]));
+    }
+}
+
+__device__ __forceinline__ void unpack8(const f32x4 (&v)[2], float (&f)[8]) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = v[e / 4][e % 4];
+}
+
+// Q fragments of a wave's rows: per-head RMSNorm (NORM), rotate-half mRoPE (factors 1 and 0 without tables) and the factor
+// log2(e)/sqrt(HD), all in fp32 and with ONE rounding to bf16.
+template <int HD, int QB, bool NORM>
+__device__ __forceinline__ void finish_rows(const PackedParams& p, const QRows<HD, QB>& r, bf16x8 (&qf)[QB][HD / 32]) {
+    constexpr int KS = HD / 32;
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+        const u32x4 (&raw)[KS] = r.raw[qb];
         // per-head RMSNorm: the lane holds 8 channels per k-step, the other three quarter-waves the rest of the row
         float rnorm = 1.0f;
-        const float* nw = nullptr;
-        if (p.qn.w != nullptr) {
+        if constexpr (NORM) {
             float ss = 0.0f;
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                const uint32_t w[4] = {raw[ks].x, raw[ks].y, raw[ks].z, raw[ks].w};
+            for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) { const float a = bf16lo(w[j]), b = bf16hi(w[j]); ss += a * a + b * b; }
-            }
-            ss += __shfl_xor(ss, 16, 64);
-            ss += __shfl_xor(ss, 32, 64);
-            rnorm = rsqrtf(ss * (1.0f / HD) + p.qn.eps);
-            nw = p.qn.row(qrow, HD) + 8 * g4;
+                for (int j = 0; j < 4; ++j) { const float a = bf16lo(raw[ks][j]), b = bf16hi(raw[ks][j]); ss += a * a + b * b; }
+            rnorm = rsqrtf(quarters_sum(ss) * (1.0f / HD) + p.qn.eps);
         }
 #pragma unroll
         for (int ks = 0; ks < KS / 2; ++ks) {
-            const uint32_t w1[4] = {raw[ks].x, raw[ks].y, raw[ks].z, raw[ks].w};
-            const uint32_t w2[4] = {raw[ks + KS / 2].x, raw[ks + KS / 2].y, raw[ks + KS / 2].z, raw[ks + KS / 2].w};
-            float n1[8], n2[8];      // norm factors of the channels of k-step ks and of its rotary partners
+            const u32x4 w1 = raw[ks], w2 = raw[ks + KS / 2];
+            float c[8], sn[8], n1[8], n2[8];      // rotary factors; norm factors of the channels of k-step ks and of their partners
+            unpack8(r.c[qb][ks], c);
+            unpack8(r.s[qb][ks], sn);
+            if constexpr (NORM) {
+                unpack8(r.w[qb][ks], n1);
+                unpack8(r.w[qb][ks + KS / 2], n2);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                n1[e] = nw ? rnorm * nw[32 * ks + e] : 1.0f;
-                n2[e] = nw ? rnorm * nw[32 * (ks + KS / 2) + e] : 1.0f;
+                for (int e = 0; e < 8; ++e) { n1[e] *= rnorm; n2[e] *= rnorm; }
             }
-            float c[8], sn[8];
-            if (p.cos != nullptr) {
-                const float4* cp = reinterpret_cast<const float4*>(p.cos + (int64_t)qrow * (HD / 2) + 32 * ks + 8 * g4);
-                const float4* sp = reinterpret_cast<const float4*>(p.sin + (int64_t)qrow * (HD / 2) + 32 * ks + 8 * g4);
-                const float4 c0 = cp[0], c1 = cp[1], s0 = sp[0], s1 = sp[1];
-                c[0] = c0.x; c[1] = c0.y; c[2] = c0.z; c[3] = c0.w; c[4] = c1.x; c[5] = c1.y; c[6] = c1.z; c[7] = c1.w;
-                sn[0] = s0.x; sn[1] = s0.y; sn[2] = s0.z; sn[3] = s0.w; sn[4] = s1.x; sn[5] = s1.y; sn[6] = s1.z; sn[7] = s1.w;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) { c[e] = 1.0f; sn[e] = 0.0f; }
-            }
-            uint32_t o1[4], o2[4];
+            u32x4 o1, o2;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const float a0 = bf16lo(w1[j]) * n1[2 * j], a1 = bf16hi(w1[j]) * n1[2 * j + 1];
-                const float b0 = bf16lo(w2[j]) * n2[2 * j], b1 = bf16hi(w2[j]) * n2[2 * j + 1];
+                float a0 = bf16lo(w1[j]), a1 = bf16hi(w1[j]), b0 = bf16lo(w2[j]), b1 = bf16hi(w2[j]);
+                if constexpr (NORM) { a0 *= n1[2 * j]; a1 *= n1[2 * j + 1]; b0 *= n2[2 * j]; b1 *= n2[2 * j + 1]; }
                 o1[j] = pack_bf16x2((a0 * c[2 * j] - b0 * sn[2 * j]) * p.scale_log2e,
                                     (a1 * c[2 * j + 1] - b1 * sn[2 * j + 1]) * p.scale_log2e);
                 o2[j] = pack_bf16x2((b0 * c[2 * j] + a0 * sn[2 * j]) * p.scale_log2e,
                                     (b1 * c[2 * j + 1] + a1 * sn[2 * j + 1]) * p.scale_log2e);
             }
-            qf[qb][ks] = __builtin_bit_cast(bf16x8, make_uint4(o1[0], o1[1], o1[2], o1[3]));
-            qf[qb][ks + KS / 2] = __builtin_bit_cast(bf16x8, make_uint4(o2[0], o2[1], o2[2], o2[3]));
+            qf[qb][ks] = __builtin_bit_cast(bf16x8, o1);
+            qf[qb][ks + KS / 2] = __builtin_bit_cast(bf16x8, o2);
         }
-        {      // norm of the scaled, rotated, rounded query row (a quarter of it in each quarter-wave)
-            float ss = 0.0f;
+    }
+}
+template <int HD, int QB>
+__device__ __forceinline__ void finish_q(const PackedParams& p, const QRows<HD, QB>& r, bf16x8 (&qf)[QB][HD / 32]) {
+    if (p.qn.w != nullptr) finish_rows<HD, QB, true>(p, r, qf);
+    else finish_rows<HD, QB, false>(p, r, qf);
+}
+
+// The norms of the scaled, rotated, rounded rows: for a bound with 1 % slack, so two products per instruction
+template <int HD, int QB>
+__device__ __forceinline__ void frag_norms(const bf16x8 (&qf)[QB][HD / 32], float (&qnorm)[QB]) {
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                const uint4 u = __builtin_bit_cast(uint4, qf[qb][ks]);
-                const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+    for (int qb = 0; qb < QB; ++qb) {
+        float qq = 0.0f;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) { const float a = bf16lo(w[j]), b = bf16hi(w[j]); ss += a * a + b * b; }
+        for (int ks = 0; ks < HD / 32; ++ks) {
+            const u32x4 u = __builtin_bit_cast(u32x4, qf[qb][ks]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const bf16x2 v = __builtin_bit_cast(bf16x2, u[j]);
+                qq = __builtin_amdgcn_fdot2_f32_bf16(v, v, qq, false);
             }
-            ss += __shfl_xor(ss, 16, 64);
-            ss += __shfl_xor(ss, 32, 64);
-            qnorm[qb] = sqrtf(ss);
         }
+        qnorm[qb] = sqrtf(quarters_sum(qq));
     }
 }
 
@@ -423,27 +518,27 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
     int head, qblk;
     int unit = -1, part = 0;      // split unit: index into the scratch arrays, and which range of the key tiles
     {
-        const int nqb = p.n_qblocks, nh = p.n_heads;
-        const int xcd = blockIdx.x & 7;
-        int k = blockIdx.x >> 3;                                  // k-th workgroup of its XCD
-        const int hpx = (nh + 7) >> 3;                            // heads per XCD (the last XCDs may own fewer)
+        const int nh = p.n_heads, xcd = blockIdx.x & 7, hpx = (nh + 7) >> 3;      // heads per XCD (the last XCDs may own fewer)
+        int hi = blockIdx.z;                                      // grid (8, query blocks, heads per XCD): no division
+        qblk = blockIdx.y;
         if (p.split > 1) {
-            // the last split_tail query blocks of the XCD come `split` times, ordered by key range first: units that run
-            // side by side then stream the same tiles of the same head
-            const int whole = hpx * nqb - p.split_tail;
+            // 1-D grid: the last split_tail query blocks of the XCD come `split` times, ordered by key range first: units that
+            // run side by side then stream the same tiles of the same head
+            int k = blockIdx.x >> 3;                              // k-th workgroup of its XCD
+            const int whole = hpx * p.n_qblocks - p.split_tail;
             if (k >= whole) {
                 const int u = k - whole;
                 part = u / p.split_tail;
                 k = whole + (u - part * p.split_tail);
                 unit = xcd * p.split_tail * p.split + u;
             }
+            hi = k / p.n_qblocks;
+            qblk = k - hi * p.n_qblocks;
         }
-        const int hi = k / nqb;
         head = xcd * hpx + hi;
-        qblk = k - hi * nqb;
         if (hi >= hpx || head >= nh) return;
     }
-    const int kv_head = head / p.kv_group;
+    const int kv_head = p.kv_head_of(head);
     const int q0 = qblk * ROWS + wave * (32 * QS);
 
     // An upper bound of every score of a row against a key tile: |q| max_{k in tile} |k| (Cauchy-Schwarz on the very
@@ -461,21 +556,63 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
     const int NP = p.n_prefix_tiles - t0;
     const int NT = t1 - t0;
     const bool per_tile = NT <= kMaxKm;
-    float kmax_all = 0.0f;
-    {
-        const float* km = p.kmax + (int64_t)kv_head * NM - p.n_prefix_tiles + t0;      // indexed by the frame's tile number
-        const float* kmp = p.kmax_prefix + (int64_t)kv_head * p.n_prefix_tiles + t0;
-        if (per_tile) {
-            for (int i = threadIdx.x; i < kMaxKm; i += 64 * NW) s_km[i] = i >= NT ? 0.0f : (i < NP ? kmp[i] : km[i]);
-        } else {
-            for (int i = lane; i < NT; i += 64) kmax_all = fmaxf(kmax_all, i < NP ? kmp[i] : km[i]);
-            kmax_all = wave_max(kmax_all);
+    const uint32_t lane_off = (uint32_t)(wave * 1024 + lane * 16);
+    // tile t of the key sequence [prefix tiles | main tiles] lives at pre + t * TILE_BYTES (t < NP) or at
+    // base + t * TILE_BYTES with base shifted back by the prefix length: one 32-bit offset serves both
+    const char* kbase = p.kp + ((int64_t)kv_head * NM - NP) * TILE_BYTES;
+    const char* vbase = p.vp + ((int64_t)kv_head * NM - NP) * TILE_BYTES;
+    const char* kpre = p.kp_prefix + ((int64_t)kv_head * p.n_prefix_tiles + t0) * TILE_BYTES;
+    const char* vpre = p.vp_prefix + ((int64_t)kv_head * p.n_prefix_tiles + t0) * TILE_BYTES;
+    const uint32_t sk_addr = lds_addr_of(sk) + wave * 1024, sv_addr = lds_addr_of(sv) + wave * 1024;
+
+    // tile `t` (clamped to the last tile, so that every step issues the same number of loads and the
+    // vmcnt arithmetic below stays valid at the end of the sequence) -> ring slot `slot`
+    auto issue = [&](const char* base, const char* pre, uint32_t dst_addr, int t, int slot) {
+        const int tc = t < NT ? t : NT - 1;
+        const char* src = (tc < NP ? pre : base) + (uint32_t)tc * (uint32_t)TILE_BYTES;      // images stay below 4 GB per head
+#pragma unroll
+        for (int i = 0; i < PER_WAVE; ++i)
+            lds_dma16(src + i * (NW * 1024), lane_off, dst_addr + slot * TILE_BYTES + i * (NW * 1024));
+    };
+
+    // ---- prologue: K(0) | K(1), V(0) and what Q and the key norms take, in ONE round trip to memory; then K(2), V(1) | V(2)
+    // under the arithmetic on Q
+    issue(kbase, kpre, sk_addr, 0, 0);
+    issue(kbase, kpre, sk_addr, 1, 1);
+    issue(vbase, vpre, sv_addr, 0, 0);
+    const float* km = p.kmax + (int64_t)kv_head * NM - p.n_prefix_tiles + t0;      // indexed by the frame's tile number
+    const float* kmp = p.kmax_prefix + (int64_t)kv_head * p.n_prefix_tiles + t0;
+    constexpr int KMV = kMaxKm / (64 * NW);
+    float kmv[KMV];
+#pragma unroll
+    for (int u = 0; u < KMV; ++u) {
+        kmv[u] = 0.0f;
+        if (per_tile && u * (64 * NW) < NT) {      // (loads nothing waits for inside the branch)
+            const int i = u * (64 * NW) + (int)threadIdx.x, ic = i < NT ? i : NT - 1;
+            kmv[u] = (ic < NP ? kmp : km)[ic];
         }
     }
+    QRows<HD, QB> qr;
+    request_q<HD, QB>(p, head, q0, lane, qr);
+    arrived<HD, QB>(p, qr);      // ... and with it everything requested ahead of it: from here on vmcnt counts tile loads only
+    issue(kbase, kpre, sk_addr, 2, 2);
+    issue(vbase, vpre, sv_addr, 1, 1);
+    issue(vbase, vpre, sv_addr, 2, 2);
     float qnorm[QB];
     bf16x8 qf[QB][KS];
-    load_q<HD, QB>(p, head, q0, lane, qf, qnorm);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // Q is in registers: from here on vmcnt counts tile loads only
+    finish_q<HD, QB>(p, qr, qf);
+    frag_norms<HD, QB>(qf, qnorm);
+    float kmax_all = 0.0f;
+    if (per_tile) {
+#pragma unroll
+        for (int u = 0; u < KMV; ++u) {
+            const int i = u * (64 * NW) + (int)threadIdx.x;
+            s_km[i] = i < NT ? kmv[u] : 0.0f;
+        }
+    } else {
+        for (int i = lane; i < NT; i += 64) kmax_all = fmaxf(kmax_all, i < NP ? kmp[i] : km[i]);
+        kmax_all = wave_max(kmax_all);
+    }
 
     f32x4 oacc[HB][QB];
     // negm = minus the softmax reference of the lane's query row (log2 units), replicated over a 4-register
@@ -508,32 +645,6 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
     }
     const int kmax = (causal_wg && b0 + ROWS <= p.causal_prefix) ? (b0 + ROWS < n_keys ? b0 + ROWS : n_keys) : n_keys;
     const int NTW = (kmax + BN - 1) / BN;
-    const uint32_t lane_off = (uint32_t)(wave * 1024 + lane * 16);
-    // tile t of the key sequence [prefix tiles | main tiles] lives at pre + t * TILE_BYTES (t < NP) or at
-    // base + t * TILE_BYTES with base shifted back by the prefix length: one 32-bit offset serves both
-    const char* kbase = p.kp + ((int64_t)kv_head * NM - NP) * TILE_BYTES;
-    const char* vbase = p.vp + ((int64_t)kv_head * NM - NP) * TILE_BYTES;
-    const char* kpre = p.kp_prefix + ((int64_t)kv_head * p.n_prefix_tiles + t0) * TILE_BYTES;
-    const char* vpre = p.vp_prefix + ((int64_t)kv_head * p.n_prefix_tiles + t0) * TILE_BYTES;
-    const uint32_t sk_addr = lds_addr_of(sk) + wave * 1024, sv_addr = lds_addr_of(sv) + wave * 1024;
-
-    // tile `t` (clamped to the last tile, so that every step issues the same number of loads and the
-    // vmcnt arithmetic below stays valid at the end of the sequence) -> ring slot `slot`
-    auto issue = [&](const char* base, const char* pre, uint32_t dst_addr, int t, int slot) {
-        const int tc = t < NT ? t : NT - 1;
-        const char* src = (tc < NP ? pre : base) + (uint32_t)tc * (uint32_t)TILE_BYTES;      // images stay below 4 GB per head
-#pragma unroll
-        for (int i = 0; i < PER_WAVE; ++i)
-            lds_dma16(src + i * (NW * 1024), lane_off, dst_addr + slot * TILE_BYTES + i * (NW * 1024));
-    };
-
-    // ---- prologue: K(0) | K(1), V(0) | K(2), V(1) | V(2); scores of tile 0 with an exact first reference
-    issue(kbase, kpre, sk_addr, 0, 0);
-    issue(kbase, kpre, sk_addr, 1, 1);
-    issue(vbase, vpre, sv_addr, 0, 0);
-    issue(kbase, kpre, sk_addr, 2, 2);
-    issue(vbase, vpre, sv_addr, 1, 1);
-    issue(vbase, vpre, sv_addr, 2, 2);
     // K(0), K(1), V(0) have landed, and every wave's share of the key-norm table is in LDS
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(3 * PER_WAVE) : "memory");
     f32x4 s_a[KB][QB], s_b[KB][QB];      // score tiles ping-pong between the two halves of the unrolled loop
@@ -569,9 +680,7 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
             negm[qb][e] = -m0;
         }
     }
-    float t_wave = t_lane;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) t_wave = fminf(t_wave, __shfl_xor(t_wave, off, 64));
+    const float t_wave = row16_min(t_lane);      // (the quarter-waves hold the same rows)
     if (!per_tile) need_always = need_always || !(kmax_all <= t_wave);
     uint32_t hot = 0u;      // bit t in lane l: tile 32 l + t needs row maxima for this wave's rows
     if (per_tile && !need_always) {
@@ -643,8 +752,7 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
     char* stage = (wave < NW / 2 ? sk : sv) + (wave % (NW / 2)) * (32 * QS * PITCH);     // half the waves per ring
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
-        float l_tot = l_run[qb] + __shfl_xor(l_run[qb], 16, 64);
-        l_tot += __shfl_xor(l_tot, 32, 64);
+        const float l_tot = quarters_sum(l_run[qb]);
         const float inv = 1.0f / l_tot;
         float amax = 0.0f;
 #pragma unroll
@@ -661,8 +769,7 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
                 p.part_lse[(int64_t)unit * BMQ + wave * (32 * QS) + qb * 16 + r16] =
                     __log2f(l_tot) - negm[qb][0] * (LATE ? p.late_r : 1.0f);
         } else if (p.row_amax != nullptr) {      // the row's channels of this head are spread over the four quarter-waves
-            amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-            amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+            amax = quarters_max(amax);
             const int qrow = q0 + qb * 16 + r16;
             if (g4 == 0 && qrow < p.n_tokens) p.row_amax[(int64_t)qrow * p.n_heads + head] = amax;
         }
@@ -681,38 +788,39 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
     }
 }
 
-// Small grids (see the launch rule): 128 query rows per workgroup, and two groups of four waves that share the key tiles out -
-// group g takes tiles g, g + 2, ... for all 128 rows - and add up their results at the end.  With one wave per SIMD nothing
-// runs under a wave's exponentials and waits; the second one fills them, and a workgroup makes half the steps.  Every group has
-// a ring of its own, three K and two V tiles (160 KB for both at head_dim 128): a tile is requested one step ahead of its
-// first use.  The partial results stay fp32.
-// Launches in us, 128-row workgroups of four waves against this: 16 heads x 64, 512 keys 12.0 / 11.9, 1024 keys 17.8 / 16.0, 2048
-// keys 28.2 / 24.3; 16 heads x 128, 512 keys 16.9 / 18.1 (32 heads), 1024 keys 23.9 / 22.7, 1637 keys 34.1 / 30.5, 2048 keys 40.7 /
-// 37.9; 8 heads x 128, 4000 keys 70.9 / 62.7.  A step of two tiles takes 1.85 us at head_dim 128 against 2 x 1.03; where the
-// loads stand in it does not matter (one behind every first to fourth MFMA: the same).  A second barrier per step that keeps
-// the groups half a step apart costs more than the overlap brings (2048 keys 39.4).
-template <int HD, bool LATE>
+// Small grids (see the launch rule): NG groups of GW waves share the key tiles out - group g takes tiles g, g + NG, ... for all
+// 32 GW query rows of the workgroup - and add up their results at the end.  With one wave per SIMD nothing runs under a
+// wave's exponentials and waits; waves of other groups fill them, and a workgroup makes 1 / NG of the steps.  Every group has a ring of
+// its own, three K and two V tiles: a tile is requested one step ahead of its first use.  The partial results stay fp32.
+// What leads up to the first MFMA is shared as well: groups 0 and 1 turn 16 of a wave's 32 rows each into Q fragments and leave
+// them in the ring's second V slot for everybody, and at the end they merge and store the same 16 rows each.
+// Where the set-up is shared counts: a wave per group that prepared all of its rows itself took 7.4 us ahead of its first
+// step at head_dim 128, 5.3 now.  A step of two tiles takes 1.85 us with two groups of four waves at head_dim 128 against 2 x 1.03
+// of one group; where the loads stand in it does not matter.  A second barrier per step that keeps the groups half a step
+// apart costs more than the overlap brings.
+// Launches in us: one group of four waves (128 rows) / two groups of four (128 rows) / of two (64 rows) / four groups of two:
+//   16 heads x 64    256 keys  9.1 / 8.6 / 6.8 / 7.6    512  11.6 / 10.4 / 8.3 / 8.6    1024  18.8 / 16.5 / - / 12.6    2048  30.1 / 24.9
+//   16 heads x 128   256 keys 12.6 / 12.2 / 9.2         512  16.4 / 15.0 / 11.2         1024  26.4 / 22.6 / 18.3        1637  36.3 / 30.4
+//   32 heads x 128   256 keys 12.7 / 12.3 / 9.2         512  16.6 / 15.3 / 11.5         1024  27.3 / 24.5
+template <int HD, bool LATE, int GW, int NG>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_keys_kernel(const PackedParams p) {
-    constexpr int ROWS = BMQ / 2, QB = 2, KS = HD / 32, HB = HD / 16;
+    constexpr int ROWS = 32 * GW, QB = 2, KS = HD / 32, HB = HD / 16;
     constexpr int TILE_BYTES = BN * HD * 2;
-    constexpr int PER_WAVE = TILE_BYTES / 1024 / 4;    // direct-to-LDS instructions per wave per tile
+    constexpr int PER_WAVE = TILE_BYTES / 1024 / GW;   // direct-to-LDS instructions per wave per tile
     constexpr int RING = 3, RING_V = 2, GROUP = (RING + RING_V) * TILE_BYTES;
-    __shared__ __attribute__((aligned(1024))) char smem[2 * GROUP];
+    static_assert(NG * GROUP <= 160 * 1024 && (NG == 1 || NG == 2 || NG == 4) && GW * KS * 1024 <= TILE_BYTES, "rings exceed the LDS");
+    __shared__ __attribute__((aligned(1024))) char smem[NG * GROUP];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int grp = wave >> 2, gw = wave & 3;
+    const int grp = wave / GW, gw = wave % GW;
     const int r16 = lane & 15, g4 = lane >> 4;
-    int head, qblk;
-    {      // all query blocks of a head on one XCD, as above
-        const int hpx = (p.n_heads + 7) >> 3, k = blockIdx.x >> 3, hi = k / p.n_qblocks;
-        head = (blockIdx.x & 7) * hpx + hi;
-        qblk = k - hi * p.n_qblocks;
-        if (hi >= hpx || head >= p.n_heads) return;
-    }
-    const int kv_head = head / p.kv_group;
+    // all query blocks of a head on one XCD, as above
+    const int head = (blockIdx.x & 7) * ((p.n_heads + 7) >> 3) + blockIdx.z, qblk = blockIdx.y;
+    if (head >= p.n_heads) return;
+    const int kv_head = p.kv_head_of(head);
     const int q0 = qblk * ROWS + gw * 32, b0 = qblk * ROWS;
-    const int NM = (p.n_tokens + BN - 1) / BN, NP = p.n_prefix_tiles, NT = NP + NM;      // 4 <= NT <= kMaxKm, host-checked
+    const int NM = (p.n_tokens + BN - 1) / BN, NP = p.n_prefix_tiles, NT = NP + NM;      // NT <= kMaxKm, host-checked
     const char* kbase = p.kp + ((int64_t)kv_head * NM - NP) * TILE_BYTES;
     const char* vbase = p.vp + ((int64_t)kv_head * NM - NP) * TILE_BYTES;
     const char* kpre = p.kp_prefix + (int64_t)kv_head * NP * TILE_BYTES;
@@ -723,22 +831,43 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const uint32_t sk_addr = lds_addr_of(sk) + gw * 1024, sv_addr = lds_addr_of(sv) + gw * 1024;
     // the group's i-th tile (clamped to the last of the sequence) -> ring slot
     auto issue = [&](const char* base, const char* pre, uint32_t dst_addr, int i, int slot) {
-        const int t = 2 * i + grp, tc = t < NT ? t : NT - 1;
+        const int t = NG * i + grp, tc = t < NT ? t : NT - 1;
         const char* src = (tc < NP ? pre : base) + (uint32_t)tc * (uint32_t)TILE_BYTES;
 #pragma unroll
-        for (int l = 0; l < PER_WAVE; ++l) lds_dma16(src + l * 4096, lane_off, dst_addr + slot * TILE_BYTES + l * 4096);
+        for (int l = 0; l < PER_WAVE; ++l) lds_dma16(src + l * (GW * 1024), lane_off, dst_addr + slot * TILE_BYTES + l * (GW * 1024));
     };
     issue(kbase, kpre, sk_addr, 0, 0);
-    issue(kbase, kpre, sk_addr, 1, 1);
-    issue(vbase, vpre, sv_addr, 0, 0);
-    issue(kbase, kpre, sk_addr, 2, 2);
     const float* km = p.kmax + (int64_t)kv_head * NM - NP;      // indexed by tile
     const float* kmp = p.kmax_prefix + (int64_t)kv_head * NP;
-    auto tile_norm = [&](int t) { return t < NP ? kmp[t] : t < NT ? km[t] : 0.0f; };
+    auto tile_norm = [&](int t) {
+        const int tc = t < NT ? t : NT - 1;
+        return (tc < NP ? kmp : km)[tc];
+    };
     const float km0 = tile_norm(lane);
-    float qnorm[QB];
+    auto rest = [&]() {
+        issue(kbase, kpre, sk_addr, 1, 1);
+        issue(vbase, vpre, sv_addr, 0, 0);
+        issue(kbase, kpre, sk_addr, 2, 2);
+    };
+    constexpr int MINE = NG == 1 ? QB : 1;      // 16-row blocks that a wave turns into fragments
     bf16x8 qf[QB][KS];
-    load_q<HD, QB>(p, head, q0, lane, qf, qnorm);
+    if (grp < QB) {
+        QRows<HD, MINE> qr;
+        request_q<HD, MINE>(p, head, q0 + grp * 16, lane, qr);
+        arrived<HD, MINE>(p, qr);      // ... and with it K(0) and the norms
+        rest();
+        if constexpr (NG == 1) {
+            finish_q<HD, QB>(p, qr, qf);
+        } else {
+            bf16x8 mine[1][KS];
+            finish_q<HD, 1>(p, qr, mine);
+            char* to = smem + grp * GROUP + (RING + 1) * TILE_BYTES + gw * (KS * 1024) + lane * 16;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) *reinterpret_cast<bf16x8*>(to + ks * 1024) = mine[0][ks];
+        }
+    } else {
+        rest();
+    }
 
     f32x4 oacc[HB][QB], negm[QB];
     float l_run[QB];
@@ -757,18 +886,29 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         klim[qb] = qrow < p.causal_prefix ? qrow + 1 : n_keys;
     }
     const int kmax = (causal_wg && b0 + ROWS <= p.causal_prefix) ? (b0 + ROWS < n_keys ? b0 + ROWS : n_keys) : n_keys;
-    const int NTW = (kmax + BN - 1) / BN;                       // at least 2: both groups have a first tile
+    const int NTW = (kmax + BN - 1) / BN;
     const int pre_rag_tile = (NP > 0 && p.prefix_last_valid < BN) ? NP - 1 : -1;
 
-    // everything requested so far has landed (Q and the norms included): one wait, one barrier
+    // everything requested so far has landed and the Q fragments are in LDS: one wait, one barrier
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    float qnorm[QB];
+    if constexpr (NG > 1) {
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) {
+            const char* from = smem + qb * GROUP + (RING + 1) * TILE_BYTES + gw * (KS * 1024) + lane * 16;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) qf[qb][ks] = *reinterpret_cast<const bf16x8*>(from + ks * 1024);
+        }
+    }
+    frag_norms<HD, QB>(qf, qnorm);
     f32x4 s_a[KB][QB], s_b[KB][QB];
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) s_a[kb][qb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     scores_tile<HD, QB>(sk, qf, s_a, lane);
-    if (causal_wg || grp == pre_rag_tile) {
+    // (a group without a first tile masks all of its copy of the last one)
+    if (causal_wg || grp == pre_rag_tile || grp >= NT || (ragged && grp == NT - 1)) {
         int nvalid[QB];
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) nvalid[qb] = grp == pre_rag_tile ? p.prefix_last_valid : klim[qb] - grp * BN;
@@ -779,7 +919,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
         float m0 = tile_row_max<QB>(s_a, qb);
-        m0 = m0 == -INFINITY ? 0.0f : m0;      // causal rows that end ahead of this group's first tile: nothing to refer to
+        m0 = m0 == -INFINITY ? 0.0f : m0;      // rows that see nothing of this group's first tile: nothing to refer to
         const float thr = (kSafeLog2 + m0) / (qnorm[qb] * 1.01f);
         need_always = need_always || __builtin_amdgcn_ballot_w64(thr != thr) != 0;
         t_wave = fminf(t_wave, thr);
@@ -790,32 +930,35 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             negm[qb][e] = -m0;
         }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) t_wave = fminf(t_wave, __shfl_xor(t_wave, off, 64));
+    t_wave = row16_min(t_wave);      // (the quarter-waves hold the same rows)
     uint32_t hot = 0u;      // bit t in lane l: tile 32 l + t is the group's and needs row maxima for this wave's rows
     if (!need_always) {
+        constexpr uint64_t kOwn = NG == 1 ? ~0ull : NG == 2 ? 0x5555555555555555ull : 0x1111111111111111ull;
         for (int c = 0; c * 64 < NT; ++c) {
             const float v = c == 0 ? km0 : tile_norm(c * 64 + lane);
-            const uint64_t m = __builtin_amdgcn_ballot_w64(!(v <= t_wave) && c * 64 + lane < NT) & (0x5555555555555555ull << grp);
+            const uint64_t m = __builtin_amdgcn_ballot_w64(!(v <= t_wave) && c * 64 + lane < NT) & (kOwn << grp);
             if (lane == 2 * c) hot = (uint32_t)m;
             if (lane == 2 * c + 1) hot = (uint32_t)(m >> 32);
         }
     }
-    int next_hot = need_always ? 2 + grp : next_hot_tile(hot, grp, lane);
+    int next_hot = need_always ? NG + grp : next_hot_tile(hot, grp, lane);
     bf16x8 kw[KWIN][KB];
     preload_k<HD>(sk + TILE_BYTES, kw, lane);
 
     // step j works on the group's tile j: S(j+1) from K slot (j+1) % 3, P(j) V(j) from V slot j % 2, K(j+2) fragments from
     // slot (j+2) % 3.  At its barrier everything requested in step j - 1 - K(j+2), V(j) - has landed, and every wave is done
-    // with K(j) and V(j-1), whose slots take K(j+3) and V(j+1).  A group without a tile j (an odd count) only takes the barrier.
+    // with K(j) and V(j-1), whose slots take K(j+3) and V(j+1).  (What V's second slot held of Q is in registers by step 0's
+    // barrier.)  A group without a tile j only takes the barrier.
     int ks_next = 1, ks_cur = 0;
-    constexpr int GAP = KS * KB * QB / (4 * PER_WAVE);      // one load behind every GAP-th MFMA of block A's first half
+    constexpr int NA = KS * KB * QB;                               // MFMAs of block A
+    constexpr int GAP = NA / (GW * PER_WAVE);                      // one load behind every GAP-th of them
+    static_assert(2 * PER_WAVE * GAP <= NA, "block A has too few slots for the loads");
 #define CDM_ATTN_STEP(SCUR, SNEXT)                                                                              \
     {                                                                                                           \
         asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");                                           \
         __builtin_amdgcn_sched_barrier(0);                                                                      \
-        const int k_next2 = ks_next == 2 ? 0 : ks_next + 1, t = 2 * j + grp, tn = t + 2;                        \
-        const int tk = t + 6 < NT ? t + 6 : NT - 1, tv = tn < NT ? tn : NT - 1;      /* K(j+3), V(j+1) */       \
+        const int k_next2 = ks_next == 2 ? 0 : ks_next + 1, t = NG * j + grp, tn = t + NG;                      \
+        const int tk = t + 3 * NG < NT ? t + 3 * NG : NT - 1, tv = tn < NT ? tn : NT - 1;      /* K(j+3), V(j+1) */ \
         const char* ksrc = (tk < NP ? kpre : kbase) + (uint32_t)tk * (uint32_t)TILE_BYTES;                      \
         const char* vsrc = (tv < NP ? vpre : vbase) + (uint32_t)tv * (uint32_t)TILE_BYTES;                      \
         const uint32_t kdst = sk_addr + ks_cur * TILE_BYTES, vdst = sv_addr + ((j + 1) & 1) * TILE_BYTES;       \
@@ -823,15 +966,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         auto slot = [&](int i) {                                                                                \
             const int l = i / GAP;                                                                              \
             if (i % GAP != GAP - 1 || l >= 2 * PER_WAVE) return;                                                \
-            if (l < PER_WAVE) lds_dma16(vsrc + l * 4096, lane_off, vdst + l * 4096);                            \
-            else lds_dma16(ksrc + (l - PER_WAVE) * 4096, lane_off, kdst + (l - PER_WAVE) * 4096);               \
+            if (l < PER_WAVE) lds_dma16(vsrc + l * (GW * 1024), lane_off, vdst + l * (GW * 1024));              \
+            else lds_dma16(ksrc + (l - PER_WAVE) * (GW * 1024), lane_off, kdst + (l - PER_WAVE) * (GW * 1024)); \
         };                                                                                                      \
         if (t < NTW) {                                                                                          \
             int nvalid[QB];                                                                                     \
             const bool pre_rag = tn == pre_rag_tile;                                                            \
             _Pragma("unroll") for (int qb = 0; qb < QB; ++qb)                                                   \
                 nvalid[qb] = pre_rag ? p.prefix_last_valid : klim[qb] - tn * BN;                                \
-            pipe_step<HD, QB, LATE, 2>([]() {}, slot, p.late_r, sk + ks_next * TILE_BYTES, sv + (j & 1) * TILE_BYTES,  \
+            pipe_step<HD, QB, LATE, NG>([]() {}, slot, p.late_r, sk + ks_next * TILE_BYTES, sv + (j & 1) * TILE_BYTES,  \
                                        sk + k_next2 * TILE_BYTES, qf, kw, SCUR, SNEXT, oacc, negm, l_run, lane,  \
                                        causal_wg || pre_rag || (ragged && tn >= NT - 1) || tn >= NT, nvalid, tn, \
                                        next_hot, need_always, hot);                                             \
@@ -840,72 +983,85 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         ks_cur = ks_next;                                                                                       \
         ks_next = k_next2;                                                                                      \
     }
-    const int steps = (NTW + 1) >> 1;
+    const int steps = (NTW + NG - 1) / NG;
     for (int j = 0; j < steps; ++j) {
         CDM_ATTN_STEP(s_a, s_b)
         if (++j >= steps) break;
         CDM_ATTN_STEP(s_b, s_a)
     }
 #undef CDM_ATTN_STEP
-    // ---- the groups' results: no direct-to-LDS write may outlive the rings, which hold group 1's accumulators, sums and
-    // references from here on, and behind them the output rows that group 0 stages
+    // ---- the groups' results: no direct-to-LDS write may outlive the rings, which from here on hold, per 16-row block, the
+    // accumulators, sums and references of the groups that do not merge it, and behind them the output rows
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    constexpr int EX = (HB * QB + 1) * 1024, PITCH = HD * 2 + 16;
-    static_assert(4 * EX + ROWS * PITCH <= 2 * GROUP, "exchange and staging areas exceed the rings");
-    char* ex = smem + gw * EX + lane * 16;
+    constexpr int EX = HB * 1024 + 512, PITCH = HD * 2 + 16;
+    static_assert(QB * (NG - 1) * GW * EX + ROWS * PITCH <= NG * GROUP, "exchange and staging areas exceed the rings");
+    // block qb as group g left it for group qb, which merges it
+    auto left = [&](int qb, int g) { return smem + ((qb * (NG - 1) + (g < qb ? g : g - 1)) * GW + gw) * EX; };
     float l_tot[QB], ref[QB];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
-        l_tot[qb] = l_run[qb] + __shfl_xor(l_run[qb], 16, 64);
-        l_tot[qb] += __shfl_xor(l_tot[qb], 32, 64);
+        l_tot[qb] = quarters_sum(l_run[qb]);
         ref[qb] = -negm[qb][0] * (LATE ? p.late_r : 1.0f);
-    }
-    if (grp == 1) {
+        if (NG == 1 || grp == qb) continue;
+        char* ex = left(qb, grp);
 #pragma unroll
-        for (int hb = 0; hb < HB; ++hb)
-#pragma unroll
-            for (int qb = 0; qb < QB; ++qb) *reinterpret_cast<f32x4*>(ex + (hb * QB + qb) * 1024) = oacc[hb][qb];
-        *reinterpret_cast<f32x4*>(ex + HB * QB * 1024) = f32x4{l_tot[0], l_tot[1], ref[0], ref[1]};
+        for (int hb = 0; hb < HB; ++hb) *reinterpret_cast<f32x4*>(ex + hb * 1024 + lane * 16) = oacc[hb][qb];
+        *reinterpret_cast<float2*>(ex + HB * 1024 + lane * 8) = make_float2(l_tot[qb], ref[qb]);
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (grp == 1) return;
-    char* stage = smem + 4 * EX + gw * (32 * PITCH);
-    const f32x4 other = *reinterpret_cast<const f32x4*>(ex + HB * QB * 1024);
+    if (grp >= QB) return;
+    auto merge = [&](auto qb_c) {
+        constexpr int qb = decltype(qb_c)::value;
+        float l[NG], r[NG], w[NG], m = -INFINITY, sum = 0.0f;
 #pragma unroll
-    for (int qb = 0; qb < QB; ++qb) {
-        // a group whose tiles are all masked for the row has a sum of exactly zero and no say in the common reference
-        const float l1 = other[qb], r0 = l_tot[qb] == 0.0f ? -INFINITY : ref[qb], r1 = l1 == 0.0f ? -INFINITY : other[2 + qb];
-        const float m = fmaxf(r0, r1);
-        const float w0 = l_tot[qb] == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(r0 - m), w1 = l1 == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(r1 - m);
-        const float inv = 1.0f / (l_tot[qb] * w0 + l1 * w1), a0 = w0 * inv, a1 = w1 * inv;
+        for (int g = 0; g < NG; ++g) {
+            float2 lr = make_float2(l_tot[qb], ref[qb]);
+            if (NG > 1 && g != qb) lr = *reinterpret_cast<const float2*>(left(qb, g) + HB * 1024 + lane * 8);
+            l[g] = lr.x;
+            // a group whose tiles are all masked for the row has a sum of exactly zero and no say in the common reference
+            r[g] = lr.x == 0.0f ? -INFINITY : lr.y;
+            m = fmaxf(m, r[g]);
+        }
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            w[g] = l[g] == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(r[g] - m);
+            sum += l[g] * w[g];
+        }
+        const float inv = 1.0f / sum;
+        char* stage = smem + QB * (NG - 1) * GW * EX + (gw * 32 + qb * 16) * PITCH;
         float amax = 0.0f;
 #pragma unroll
         for (int hb = 0; hb < HB; ++hb) {
-            const f32x4 o1 = *reinterpret_cast<const f32x4*>(ex + (hb * QB + qb) * 1024);
-            float o[4];
+            float o[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = oacc[hb][qb][e] * a0 + o1[e] * a1;
-            const uint2 w = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
-            *reinterpret_cast<uint2*>(stage + (qb * 16 + r16) * PITCH + (16 * hb + 4 * g4) * 2) = w;
-            amax = fmaxf(fmaxf(amax, fmaxf(fabsf(bf16lo(w.x)), fabsf(bf16hi(w.x)))), fmaxf(fabsf(bf16lo(w.y)), fabsf(bf16hi(w.y))));
+            for (int g = 0; g < NG; ++g) {
+                f32x4 og = oacc[hb][qb];
+                if (NG > 1 && g != qb) og = *reinterpret_cast<const f32x4*>(left(qb, g) + hb * 1024 + lane * 16);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] += og[e] * (w[g] * inv);
+            }
+            const uint2 u = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+            *reinterpret_cast<uint2*>(stage + r16 * PITCH + (16 * hb + 4 * g4) * 2) = u;
+            amax = fmaxf(fmaxf(amax, fmaxf(fabsf(bf16lo(u.x)), fabsf(bf16hi(u.x)))), fmaxf(fabsf(bf16lo(u.y)), fabsf(bf16hi(u.y))));
         }
+        const int row = q0 + qb * 16;      // first of the block's rows
         if (p.row_amax != nullptr) {
-            amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-            amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-            const int qrow = q0 + qb * 16 + r16;
-            if (g4 == 0 && qrow < p.n_tokens) p.row_amax[(int64_t)qrow * p.n_heads + head] = amax;
+            amax = quarters_max(amax);
+            if (g4 == 0 && row + r16 < p.n_tokens) p.row_amax[(int64_t)(row + r16) * p.n_heads + head] = amax;
         }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the wave's own staging writes have landed
-    constexpr int LPR = HD / 8, RPI = 64 / LPR;             // lanes per row, rows per store instruction
-    const int rl = lane / LPR, ch = lane % LPR;
-    bf16_t* orow = p.o + (int64_t)q0 * p.ldo + head * HD;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the wave's own staging writes have landed
+        constexpr int LPR = HD / 8, RPI = 64 / LPR;             // lanes per row, rows per store instruction
+        const int rl = lane / LPR, ch = lane % LPR;
+        bf16_t* orow = p.o + (int64_t)row * p.ldo + head * HD;
 #pragma unroll
-    for (int it = 0; it < 32 / RPI; ++it) {
-        const int rloc = it * RPI + rl;
-        const uint4 v = *reinterpret_cast<const uint4*>(stage + rloc * PITCH + ch * 16);
-        if (q0 + rloc < p.n_tokens) *reinterpret_cast<uint4*>(orow + rloc * p.ldo + ch * 8) = v;
-    }
+        for (int it = 0; it < 16 / RPI; ++it) {
+            const int rloc = it * RPI + rl;
+            const uint4 v = *reinterpret_cast<const uint4*>(stage + rloc * PITCH + ch * 16);
+            if (row + rloc < p.n_tokens) *reinterpret_cast<uint4*>(orow + rloc * p.ldo + ch * 8) = v;
+        }
+    };
+    if (grp == 0) merge(std::integral_constant<int, 0>{});
+    if (NG == 1 || grp == 1) merge(std::integral_constant<int, 1>{});
 }
 
 // Merge of the split units' partial results: one workgroup per query block of the split tail.  Part i of a row holds
@@ -1225,7 +1381,9 @@ extern "C" int32_t cdm_attn_fwd_packed_bf16(const void* q, int64_t ldq, const fl
     p.row_amax = row_amax;
     p.cos = cos; p.sin = sin;
     p.qn = qn;
-    p.n_tokens = (int)n_tokens; p.n_heads = n_heads; p.kv_group = n_heads / n_kv_heads;
+    p.n_tokens = (int)n_tokens; p.n_heads = n_heads;
+    const uint64_t group = (uint64_t)(n_heads / n_kv_heads);
+    p.kv_magic = ((1ull << 32) + group - 1) / group;
     // Q untouched by rotation and norm: only the power-of-two part of the factor goes into Q (see LATE above)
     const bool late = cos == nullptr && qk_norm == nullptr;
     const float full = 1.4426950408889634f / sqrtf((float)head_dim);
@@ -1233,38 +1391,44 @@ extern "C" int32_t cdm_attn_fwd_packed_bf16(const void* q, int64_t ldq, const fl
     const float mant = frexpf(full, &ex);                 // full = mant * 2^ex, mant in [0.5, 1)
     p.scale_log2e = late ? ldexpf(1.0f, ex - 1) : full;
     p.late_r = late ? 2.0f * mant : 1.0f;
-    // 1-D grid of 8 x ceil(heads / 8) x query blocks ids: id % 8 = XCD, see the kernel's placement rule
+    // grid of 8 x query blocks x ceil(heads / 8): linear id % 8 = XCD, see the kernel's placement rule
     // variant 0 = 32 query rows per wave (8 waves, two per SIMD), row maxima dropped where the norm bound allows;
     // cross-check build only: 1 = 64 query rows per wave (4 waves), 2 = variant 0 with the row maxima always taken, 3 =
     // 128-row workgroups of four waves and 4 = 256-row workgroups whatever the grid, 5 = 128-row workgroups of two groups from
-    // four key tiles on, 6 = those with the row maxima always taken
+    // four key tiles on, 6 = those with the row maxima always taken, 7, 8 and 9 = 64-row workgroups of one, two and (head_dim 64)
+    // four groups
     const int variant = cdm_get_variant(0);
     // Small grids: 128-row workgroups of four waves (same arithmetic per row, bit-equal).  A wave then has its SIMD to
     // itself and nothing runs under its exponentials, so such a workgroup takes 0.7 of the time of one with twice the
     // rows; it pays where the larger ones would leave half of an XCD's 32 CUs idle, i.e. up to 16 per XCD.  Measured,
-    // 256-row against 128-row workgroups: 32 heads x 128, 512 keys 23.2 -> 17.4 us, 1024 keys (16 per XCD) 34.6 -> 27.2, 2048
-    // keys (32 per XCD) 64.6 against 84.8; 16 heads x 64, 1024 keys 21.8 -> 17.3, 4096 keys (32 per XCD) equal.
-    const int64_t per_xcd = (n_heads + 7) / 8 * ((n_tokens + BMQ - 1) / BMQ);
-    const bool half_blocks = variant == 3 || variant >= 5 || ((variant == 0 || variant == 2) && per_xcd <= 16);
+    // 256-row against 128-row workgroups: 32 heads x 128, 1024 keys (16 per XCD) 34.6 -> 27.2 us, 2048 keys (32 per XCD) 64.6
+    // against 84.8; 16 heads x 64, 1024 keys 21.8 -> 17.3, 4096 keys (32 per XCD) equal.
+    const int64_t hpx = (n_heads + 7) / 8, per_xcd = hpx * ((n_tokens + BMQ - 1) / BMQ);
+    const bool half_blocks = variant == 3 || variant == 5 || variant == 6 || ((variant == 0 || variant == 2) && per_xcd <= 16);
     // ... with a second group of four waves that takes every other key tile, where the steps saved outweigh the larger rings and
     // the exchange of the groups' results (attn_fwd_keys_kernel: from 8 tiles on at head_dim 64, 16 at 128)
     const int64_t key_tiles = p.n_prefix_tiles + pad_tokens(n_tokens) / BN;
     const int64_t min_tiles = variant >= 5 ? 4 : head_dim == 64 ? 8 : 16;
-    const bool keys = half_blocks && variant != 3 && key_tiles >= min_tiles && key_tiles <= kMaxKm;
-    const int rows_wg = half_blocks ? BMQ / 2 : BMQ;
+    // ... and 64-row workgroups (groups of two waves) where even those all find a CU of their own: half the set-up per workgroup
+    // and half the steps (figures at the kernel).  One group, bit-equal to the forms above, below 6 tiles; four at
+    // head_dim 64, whose rings are half as large, from 12 on (three tiles each: 1024 keys 12.6 us against 14.5 with two).
+    const bool quarter = key_tiles <= kMaxKm && ((variant >= 7 && variant <= 9) || (variant == 0 && half_blocks && hpx * ((n_tokens + 63) / 64) <= 32));
+    const int groups = variant >= 7 ? (variant == 9 ? (head_dim == 64 ? 4 : 2) : variant - 6) : key_tiles < 6 ? 1 : head_dim == 64 && key_tiles >= 12 ? 4 : 2;
+    const bool keys = !quarter && half_blocks && variant != 3 && key_tiles >= min_tiles && key_tiles <= kMaxKm;
+    const int rows_wg = quarter ? BMQ / 4 : half_blocks ? BMQ / 2 : BMQ;
     p.n_qblocks = (int)((n_tokens + rows_wg - 1) / rows_wg);
     p.always_max = variant == 2 || variant == 6;
     // the last round's query blocks by key range, if the caller brought the scratch memory for it
     p.split = 1; p.split_tail = 0; p.part_o = nullptr; p.part_lse = nullptr;
     const SplitPlan plan = split_plan(n_tokens, n_heads, head_dim, causal_prefix);
-    if (split_scratch != nullptr && plan.split > 1 && split_scratch_bytes >= plan.bytes && variant != 1 && !half_blocks) {
+    if (split_scratch != nullptr && plan.split > 1 && split_scratch_bytes >= plan.bytes && variant != 1 && !half_blocks && !quarter) {
         p.split = plan.split; p.split_tail = plan.tail;
         p.part_o = (bf16_t*)split_scratch;
         p.part_lse = (float*)((char*)split_scratch + 8ll * plan.tail * plan.split * BMQ * head_dim * 2);
     }
-    const int64_t nwg = 8ll * ((n_heads + 7) / 8) * p.n_qblocks + 8ll * p.split_tail * (p.split - 1);
+    const int64_t nwg = 8ll * hpx * p.n_qblocks + 8ll * p.split_tail * (p.split - 1);
     CDM_REQUIRE(nwg < (1ll << 31), CDM_ERR_BAD_SHAPE, "attn_fwd_packed: grid too large");
-    dim3 grid((unsigned)nwg);
+    const dim3 grid = p.split > 1 ? dim3((unsigned)nwg) : dim3(8, (unsigned)p.n_qblocks, (unsigned)hpx);      // at most 65,535 x 8,192
     hipStream_t st = (hipStream_t)stream;
 #define CDM_ATTN_LAUNCH(QS_, NW_)                                                                                     \
     if (head_dim == 128 && late) attn_fwd_pipe_kernel<128, QS_, NW_, true><<<grid, 64 * NW_, 0, st>>>(p);            \
@@ -1275,13 +1439,22 @@ extern "C" int32_t cdm_attn_fwd_packed_bf16(const void* q, int64_t ldq, const fl
     if (variant == 1) { CDM_ATTN_LAUNCH(2, 4); }
     else
 #endif
-    if (keys) {
-        if (head_dim == 128 && late) attn_fwd_keys_kernel<128, true><<<grid, 512, 0, st>>>(p);
-        else if (head_dim == 128) attn_fwd_keys_kernel<128, false><<<grid, 512, 0, st>>>(p);
-        else if (late) attn_fwd_keys_kernel<64, true><<<grid, 512, 0, st>>>(p);
-        else attn_fwd_keys_kernel<64, false><<<grid, 512, 0, st>>>(p);
-    } else if (half_blocks) { CDM_ATTN_LAUNCH(1, 4); }
+#define CDM_KEYS_LAUNCH(HD_, GW_, NG_)                                                                     \
+    if (late) attn_fwd_keys_kernel<HD_, true, GW_, NG_><<<grid, 64 * GW_ * NG_, 0, st>>>(p);              \
+    else attn_fwd_keys_kernel<HD_, false, GW_, NG_><<<grid, 64 * GW_ * NG_, 0, st>>>(p)
+    if (quarter && head_dim == 64) {
+        if (groups == 4) { CDM_KEYS_LAUNCH(64, 2, 4); }
+        else if (groups == 2) { CDM_KEYS_LAUNCH(64, 2, 2); }
+        else { CDM_KEYS_LAUNCH(64, 2, 1); }
+    } else if (quarter) {
+        if (groups == 2) { CDM_KEYS_LAUNCH(128, 2, 2); }
+        else { CDM_KEYS_LAUNCH(128, 2, 1); }
+    }
+    else if (keys && head_dim == 64) { CDM_KEYS_LAUNCH(64, 4, 2); }
+    else if (keys) { CDM_KEYS_LAUNCH(128, 4, 2); }
+    else if (half_blocks) { CDM_ATTN_LAUNCH(1, 4); }
     else { CDM_ATTN_LAUNCH(1, 8); }
+#undef CDM_KEYS_LAUNCH
 #undef CDM_ATTN_LAUNCH
     if (p.split > 1) {
         if ((rc = cdm_check_launch("attn_fwd_packed"))) return rc;

@@ -992,6 +992,64 @@ def test_attention_small_grids_share_the_key_tiles(n, H, Hkv, hd, P, causal, sca
         assert bool(torch.isfinite(res[variant]).all()) and rel(res[variant], want) <= 1.25 * ref + 1e-4, (variant, rel(res[variant], want), ref)
 
 
+@pytest.mark.parametrize("n,H,Hkv,hd,P,causal,qkn", [
+    (1, 8, 8, 64, 0, 0, False), (64, 3, 1, 128, 0, 0, True), (65, 2, 2, 64, 0, 0, False), (129, 2, 1, 128, 70, 0, True), (320, 8, 2, 128, 0, 0, False),
+    (321, 9, 3, 128, 0, 0, False), (384, 16, 16, 64, 0, 0, True), (130, 2, 2, 128, 300, 0, False), (500, 3, 3, 64, 0, 190, False),
+    (703, 4, 4, 64, 0, 0, True), (705, 4, 2, 64, 1, 0, False), (449, 8, 8, 128, 0, 449, False), (1024, 16, 4, 64, 77, 0, True),
+    (1000, 8, 8, 64, 0, 70, False), (2048, 8, 8, 64, 0, 0, False)])
+def test_attention_64_row_workgroups(n, H, Hkv, hd, P, causal, qkn, request):
+    """64-row workgroups of one, two and four groups of two waves: one group's bits are those of the 256-row form, two groups' those of
+    the 128-row form with two groups, and the default is one of them where 64-row blocks of an XCD's heads all find a CU.
+    Groups without a tile, a ragged first tile, masked prefix tiles, causal rows that see nothing of a group's tiles.  Against
+    64 bits no further off than one group (the roundings of Q, P and O are the same ones; a quarter for chance)."""
+    request.addfinalizer(lambda: ops.set_variant("attn", 0))
+    g = gen(n + H + P)
+    q, qr = rand_bf16((n, H * hd), g)
+    k, kr = rand_bf16((n, Hkv * hd), g, 0.4)
+    v, vr = rand_bf16((n, Hkv * hd), g)
+    kp, kpr = rand_bf16((max(P, 1), Hkv * hd), g, 0.4)
+    vp, vpr = rand_bf16((max(P, 1), Hkv * hd), g)
+    ang = torch.rand((n, hd // 2), generator=g) * 6.0
+    cos, sin = ang.cos().to(dev()), ang.sin().to(dev())
+    w = (1.0 + 0.2 * torch.randn((1, hd), generator=g)).to(dev())
+    norm = (w, w, (n,), 1e-6) if qkn else None
+    img = ops.attention_pack_kv(k, v, Hkv, hd, None, cos, sin, norm)
+    prefix = (ops.attention_pack_kv(kp, vp, Hkv, hd), P) if P else None
+    res = {}
+    for variant in (0, 4, 5, 7, 8, 9):
+        ops.set_variant("attn", variant)
+        amax = torch.zeros((n, H), device=dev())
+        res[variant] = ops.attention_packed(q, img, H, hd, None, cos, sin, norm, prefix, causal, Hkv, row_amax=amax)
+        assert torch.equal(amax, res[variant].float().view(n, H, hd).abs().amax(-1)), variant
+    assert torch.equal(res[7], res[4])
+    tiles = -(-P // 64) + -(-n // 64)
+    if tiles >= 4:
+        assert torch.equal(res[8], res[5])
+    if -(-H // 8) * -(-n // 64) <= 32:
+        assert torch.equal(res[0], res[7 if tiles < 6 else 9 if hd == 64 and tiles >= 12 else 8])
+
+    def rotated(x):
+        x = x.double().to(dev()).view(n, -1, hd)
+        if qkn:
+            x = x * torch.rsqrt((x * x).mean(-1, keepdim=True) + 1e-6) * w.double()
+        c, s, a, b = cos.double()[:, None], sin.double()[:, None], x[..., :hd // 2], x[..., hd // 2:]
+        return torch.cat([a * c - b * s, b * c + a * s], -1)
+    qd, kd, vd = rotated(qr), rotated(kr).to(torch.bfloat16).double(), vr.double().to(dev()).view(n, Hkv, hd)
+    if P:
+        kd = torch.cat([kpr.double().to(dev()).view(P, Hkv, hd), kd])
+        vd = torch.cat([vpr.double().to(dev()).view(P, Hkv, hd), vd])
+    keep = torch.ones((n, n + P), dtype=torch.bool, device=dev())
+    if causal:
+        keep[:causal] = torch.arange(n, device=dev())[None] <= torch.arange(causal, device=dev())[:, None]
+    want = torch.empty((n, H, hd), dtype=torch.float64, device=dev())
+    for h in range(H):
+        sc = qd[:, h] @ kd[:, h // (H // Hkv)].t() * hd ** -0.5
+        want[:, h] = torch.softmax(sc.masked_fill(~keep, -math.inf), -1) @ vd[:, h // (H // Hkv)]
+    rel = lambda variant: ((res[variant].double().view(n, H, hd) - want).norm() / want.norm()).item()
+    for variant in (8, 9):
+        assert rel(variant) <= 1.25 * rel(7) + 1e-4, (variant, rel(variant), rel(7))
+
+
 @pytest.mark.parametrize("n", [256, 300])
 def test_attention_shared_key_tiles_keep_infinities(n, request):
     """An infinite value reaches the rows that see it and nothing else, whatever the tile it sits in."""
