@@ -330,7 +330,8 @@ struct PackedParams {
     // output and the row's log-sum in scratch memory for merge_split_kernel.  split = 1: no split.
     int split, split_tail;
     __device__ __forceinline__ int kv_head_of(int head) const { return (int)((uint64_t)(uint32_t)head * kv_magic >> 32); }
-    bf16_t* part_o;              // [8 * split_tail * split][256][HD]
+    void* part_o;                // [8 * split_tail * split][256][HD], fp32 where part_f32, bf16 otherwise
+    int part_f32;
     float* part_lse;             // [8 * split_tail * split][256]   log2 of the unit's sum of exponentials, reference added
 };
 
@@ -755,6 +756,11 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
         const float l_tot = quarters_sum(l_run[qb]);
         const float inv = 1.0f / l_tot;
         float amax = 0.0f;
+        if (unit >= 0 && p.part_f32) {
+            float* orow = (float*)p.part_o + ((int64_t)unit * BMQ + wave * (32 * QS) + qb * 16 + r16) * HD + 4 * g4;
+#pragma unroll
+            for (int hb = 0; hb < HB; ++hb) *reinterpret_cast<f32x4*>(orow + 16 * hb) = oacc[hb][qb] * inv;
+        }
 #pragma unroll
         for (int hb = 0; hb < HB; ++hb) {
             uint2 w;
@@ -774,11 +780,12 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
             if (g4 == 0 && qrow < p.n_tokens) p.row_amax[(int64_t)qrow * p.n_heads + head] = amax;
         }
     }
+    if (unit >= 0 && p.part_f32) return;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the wave's own staging writes have landed
     constexpr int LPR = HD / 8, RPI = 64 / LPR;             // lanes per row, rows per store instruction
     const int rl = lane / LPR, ch = lane % LPR;
     bf16_t* orow = unit < 0 ? p.o + (int64_t)q0 * p.ldo + head * HD
-                            : p.part_o + ((int64_t)unit * BMQ + wave * (32 * QS)) * HD;      // row of the wave's first query
+                            : (bf16_t*)p.part_o + ((int64_t)unit * BMQ + wave * (32 * QS)) * HD;      // row of the wave's first query
     const int64_t ldo = unit < 0 ? p.ldo : HD;
 #pragma unroll
     for (int it = 0; it < 32 * QS / RPI; ++it) {
@@ -1064,18 +1071,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (NG == 1 || grp == 1) merge(std::integral_constant<int, 1>{});
 }
 
-// Merge of the split units' partial results: one workgroup per query block of the split tail.  Part i of a row holds
+// Merge of the split units' partial results: 32 rows of a query block of the split tail per workgroup.  Part i of a row holds
 // o_i = (sum_k p_k v_k) / l_i over its key range and lse_i = log2(l_i) + m_i; the row of the whole range is
 // sum_i w_i o_i / sum_i w_i with w_i = 2^(lse_i - max_i lse_i).
-template <int HD>
+template <int HD, bool F32>
 __global__ __launch_bounds__(256) void merge_split_kernel(const PackedParams p) {
-    constexpr int LPR = HD / 8;                       // lanes per row: 16 bytes each
+    constexpr int LPR = HD / 8, ROWS = 32;            // lanes per row: eight channels each
     const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;      // j-th query block of the XCD's tail
     const int nqb = p.n_qblocks, hpx = (p.n_heads + 7) >> 3;
     const int k = hpx * nqb - p.split_tail + j;
     const int hi = k / nqb, head = xcd * hpx + hi, qblk = k - hi * nqb;
-    for (int idx = threadIdx.x; idx < BMQ * LPR; idx += 256) {
-        const int r = idx / LPR, ch = idx % LPR;
+#pragma unroll
+    for (int idx = threadIdx.x; idx < ROWS * LPR; idx += 256) {
+        const int r = blockIdx.y * ROWS + idx / LPR, ch = idx % LPR;
         const int qrow = qblk * BMQ + r;
         float lse[kMaxSplit], mx = -INFINITY;
 #pragma unroll
@@ -1089,11 +1097,18 @@ __global__ __launch_bounds__(256) void merge_split_kernel(const PackedParams p) 
             if (i >= p.split) break;
             const float w = exp2f(lse[i] - mx);
             den += w;
-            const uint4 u = *reinterpret_cast<const uint4*>(
-                p.part_o + (((int64_t)xcd * p.split_tail * p.split + i * p.split_tail + j) * BMQ + r) * HD + ch * 8);
-            const uint32_t q[4] = {u.x, u.y, u.z, u.w};
+            const int64_t at = (((int64_t)xcd * p.split_tail * p.split + i * p.split_tail + j) * BMQ + r) * HD + ch * 8;
+            if constexpr (F32) {
+                const f32x4 lo = *reinterpret_cast<const f32x4*>((const float*)p.part_o + at);
+                const f32x4 hi4 = *reinterpret_cast<const f32x4*>((const float*)p.part_o + at + 4);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) { acc[2 * e] += w * bf16lo(q[e]); acc[2 * e + 1] += w * bf16hi(q[e]); }
+                for (int e = 0; e < 4; ++e) { acc[e] += w * lo[e]; acc[4 + e] += w * hi4[e]; }
+            } else {
+                const uint4 u = *reinterpret_cast<const uint4*>((const bf16_t*)p.part_o + at);
+                const uint32_t q[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { acc[2 * e] += w * bf16lo(q[e]); acc[2 * e + 1] += w * bf16hi(q[e]); }
+            }
         }
         const float inv = 1.0f / den;
         uint4 o;
@@ -1231,31 +1246,39 @@ inline int64_t kmax_bytes(int64_t n_tokens, int n_heads) {      // one float per
 
 // The last, partial round of workgroups.  An XCD owns heads/8 x query blocks workgroups and runs 32 at a time (one per
 // CU: the K / V rings fill the LDS), so a launch takes ceil(workgroups / 32) rounds of equal length however few
-// workgroups the last round holds.  The plan cuts each query block of that last round into `split` units by key range
-// (the smallest of 2, 4, 8 that minimises ceil(tail * split / 32) / split rounds), which the merge kernel puts together.
-// Only where it pays: the chip is power-limited, so a round that leaves CUs idle already runs faster than a full one,
-// and every unit repeats the set-up; measured at 56 k tokens x 32 heads, a plan that ends in half a round or less gains
-// 1 - 3 % and one that ends in three quarters gains nothing.  So: the split round must take at most half a round, and
-// there must be at least two whole rounds, heads a multiple of 8, at least 8 key tiles per unit, and no causal rows in
+// workgroups the last round holds.  The plan cuts each query block of that last round into `split` units by key range,
+// which the merge kernel puts together.  Needs heads a multiple of 8, at least 8 key tiles per unit, and no causal rows in
 // the tail's query blocks.
-struct SplitPlan { int split, tail; int64_t bytes; };
+// Behind two or more whole rounds: the smallest of 2, 4, 8 that minimises ceil(tail * split / 32) / split rounds, bf16 partial
+// results, and only where it pays: the chip is power-limited, so a round that leaves CUs idle already runs faster than a
+// full one, and every unit repeats the set-up; measured at 56 k tokens x 32 heads, a plan that ends in half a round or less
+// gains 1 - 3 % and one that ends in three quarters gains nothing.
+// Behind one whole round the last one is up to half of the launch.  There the set-up (8 us) and the merge count, so the split is
+// the cheapest by their estimate, and the partial results are fp32 (such launches had no partial results before).  One pass
+// against the split, us: 32 heads x 128, 2304 tokens (32 + 4 workgroups per XCD) 120 / 98.6, 2560 (32 + 8) 131 / 111, 3072 (32 + 16)
+// 152 / 144; 16 heads x 128, 4352 (32 + 2) 204 / 148, 5000 (32 + 8) 234 / 183, 6144 (32 + 16) 279 / 250; 16 x 64, 4352 132 / 91.6,
+// 6144 180 / 153.  20 or more left over (32 x 128, 3328 tokens: 163 / 199), or no whole round at all, lose.
+struct SplitPlan { int split, tail; int64_t bytes; int f32; };
 inline SplitPlan split_plan(int64_t n_tokens, int n_heads, int head_dim, int64_t causal_prefix) {
-    SplitPlan none{1, 0, 0};
+    SplitPlan none{1, 0, 0, 0};
     const int64_t nqb = (n_tokens + BMQ - 1) / BMQ, per_xcd = (n_heads / 8) * nqb;
-    if (n_heads % 8 != 0 || per_xcd < 64) return none;
+    if (n_heads % 8 != 0 || per_xcd < 32) return none;
     const int tail = (int)(per_xcd % 32);
     if (tail == 0) return none;
     if (causal_prefix > 0 && (tail >= nqb || (nqb - tail) * BMQ < causal_prefix)) return none;
     const int64_t nm = (n_tokens + BN - 1) / BN;
+    const bool f32 = per_xcd < 64;
+    const double tile = head_dim == 128 ? 1.4 : 0.8, setup = 8.0, whole = f32 ? setup + tile * (double)nm : 1.0;
     int best = 1;
-    double best_cost = 1.0;
+    double best_cost = f32 ? 0.8 * whole : 0.5 + 1e-9;
     for (int s = 2; s <= kMaxSplit && nm / s >= 8; s *= 2) {
-        const double cost = (double)((tail * s + 31) / 32) / s;
-        if (cost < best_cost - 1e-9) { best_cost = cost; best = s; }
+        const int rounds = (tail * s + 31) / 32;
+        const double merge = 5.0 + 2.0 * 8.0 * tail * s * BMQ * head_dim * 4.0 / 8e6;
+        const double cost = f32 ? rounds * (setup + tile * (double)nm / s) + merge : (double)rounds / s;
+        if (cost < best_cost - (best > 1 ? 1e-9 : 0.0)) { best_cost = cost; best = s; }
     }
-    if (best == 1 || best_cost > 0.5 + 1e-9) return none;
-    const int64_t units = 8ll * tail * best;
-    return SplitPlan{best, tail, units * BMQ * ((int64_t)head_dim * 2 + 4)};
+    if (best == 1) return none;
+    return SplitPlan{best, tail, 8ll * tail * best * BMQ * ((int64_t)head_dim * (f32 ? 4 : 2) + 4), f32};
 }
 
 // host view of the optional QK-norm argument -> kernel descriptor (which = 0: q weights, 1: k weights)
@@ -1419,12 +1442,12 @@ extern "C" int32_t cdm_attn_fwd_packed_bf16(const void* q, int64_t ldq, const fl
     p.n_qblocks = (int)((n_tokens + rows_wg - 1) / rows_wg);
     p.always_max = variant == 2 || variant == 6;
     // the last round's query blocks by key range, if the caller brought the scratch memory for it
-    p.split = 1; p.split_tail = 0; p.part_o = nullptr; p.part_lse = nullptr;
+    p.split = 1; p.split_tail = 0; p.part_o = nullptr; p.part_lse = nullptr; p.part_f32 = 0;
     const SplitPlan plan = split_plan(n_tokens, n_heads, head_dim, causal_prefix);
     if (split_scratch != nullptr && plan.split > 1 && split_scratch_bytes >= plan.bytes && variant != 1 && !half_blocks && !quarter) {
         p.split = plan.split; p.split_tail = plan.tail;
-        p.part_o = (bf16_t*)split_scratch;
-        p.part_lse = (float*)((char*)split_scratch + 8ll * plan.tail * plan.split * BMQ * head_dim * 2);
+        p.part_o = split_scratch; p.part_f32 = plan.f32;
+        p.part_lse = (float*)((char*)split_scratch + 8ll * plan.tail * plan.split * BMQ * head_dim * (plan.f32 ? 4 : 2));
     }
     const int64_t nwg = 8ll * hpx * p.n_qblocks + 8ll * p.split_tail * (p.split - 1);
     CDM_REQUIRE(nwg < (1ll << 31), CDM_ERR_BAD_SHAPE, "attn_fwd_packed: grid too large");
@@ -1458,8 +1481,11 @@ extern "C" int32_t cdm_attn_fwd_packed_bf16(const void* q, int64_t ldq, const fl
 #undef CDM_ATTN_LAUNCH
     if (p.split > 1) {
         if ((rc = cdm_check_launch("attn_fwd_packed"))) return rc;
-        if (head_dim == 128) merge_split_kernel<128><<<dim3(8u * p.split_tail), 256, 0, st>>>(p);
-        else merge_split_kernel<64><<<dim3(8u * p.split_tail), 256, 0, st>>>(p);
+        const dim3 mg(8u * p.split_tail, BMQ / 32);
+        if (head_dim == 128 && p.part_f32) merge_split_kernel<128, true><<<mg, 256, 0, st>>>(p);
+        else if (head_dim == 128) merge_split_kernel<128, false><<<mg, 256, 0, st>>>(p);
+        else if (p.part_f32) merge_split_kernel<64, true><<<mg, 256, 0, st>>>(p);
+        else merge_split_kernel<64, false><<<mg, 256, 0, st>>>(p);
     }
     return cdm_check_launch("attn_fwd_packed");
 }

@@ -251,9 +251,11 @@ int32_t cdm_attn_fwd_packed_bf16(const void* q, int64_t ldq, const float* cos, c
  * and takes ceil(n_heads / 8 * ceil(n_tokens / 256) / 32) rounds however few workgroups the last one holds.  Given
  * `split_scratch` of at least this many bytes, cdm_attn_fwd_packed_bf16 cuts the query blocks of that last round into
  * 2, 4 or 8 units by key range and merges their results with a second, small kernel (same operator; the output
- * differs from the single-pass one by the rounding of the partial results to bf16).  0 = nothing to split for this
- * shape (fewer than two whole rounds, heads not a multiple of 8, a whole number of rounds, or no split that ends in
- * half a round or less - a round with idle CUs runs faster on this power-limited chip, so less does not pay); a launch whose causal
+ * differs from the single-pass one by the rounding of the partial results to bf16 - behind a single whole round, where they
+ * are fp32, by the order of fp32 sums).  0 = nothing to split for this
+ * shape (no whole round, heads not a multiple of 8, a whole number of rounds, or no split that pays: behind two rounds or more one
+ * that ends in half a round or less - a round with idle CUs runs faster on this power-limited chip -, behind one round one
+ * that takes less than 0.8 of it with set-up and merge); a launch whose causal
  * prefix reaches into the last round's query blocks is never split.  n_heads counts query heads.
  * cdm_attn_fwd_bf16 uses what its workspace holds beyond cdm_attn_workspace_bytes (rounded up to 256) for this.
  */
