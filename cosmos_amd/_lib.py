@@ -120,6 +120,8 @@ def load():
     global _LIB
     if _XLIB is not None and any(_VARIANTS.values()):
         return _XLIB
+    if _LIB is not None:      # (once set it stays)
+        return _LIB
     with _LOCK:
         if _LIB is not None:
             return _LIB

@@ -159,7 +159,8 @@ class DMAttnProcessor:
 
         wsb = kv_images if kv_images is not None else (ws.attn_ws if ws is not None else None)
         mask_kw = dict(causal_prefix=causal_prefix, prefix=prefix, n_kv_heads=attn.n_kv_heads)
-        q, k, v = qkv[:, :d], qkv[:, d:d + dkv], qkv[:, d + dkv:]
+        q = qkv[:, :d]
+        keys_values = lambda: (qkv[:, d:d + dkv], qkv[:, d + dkv:])
         qkn = attn.qk_norm_args(modality_segments)
         o_amax = None      # per-head maxima of the attention output rows, where the attention kernel leaves them
         if qkn is not None and self.rope != "in_attention":
@@ -167,7 +168,7 @@ class DMAttnProcessor:
         if self.rope == "gemm_epilogue":
             attn._linear(x, quant_scale, "qkv", modality_segments, out=qkv, epilogue="rope_qk", cos=cos, sin=sin,
                          rope_cols=d + dkv, head_dim=attn.head_dim)
-            ops.attention(q, k, v, attn.n_heads, attn.head_dim, out=o, workspace=wsb, **mask_kw)
+            ops.attention(q, *keys_values(), attn.n_heads, attn.head_dim, out=o, workspace=wsb, **mask_kw)
         elif (self.rope == "in_attention" and self.fuse_kv_pack
               and ops.qkv_pack_applies([(s0, ln) for (s0, ln, _, _) in modality_segments], attn.head_dim, attn.n_heads,
                                        attn.n_kv_heads)):
@@ -180,6 +181,7 @@ class DMAttnProcessor:
                                  attn.n_kv_heads, row_amax=o_amax)
         else:
             attn._linear(x if runs is None else runs, quant_scale, "qkv", modality_segments, out=qkv, epilogue="none")
+            k, v = keys_values()
             if self.rope == "streaming":
                 if attn.n_kv_heads == attn.n_heads:
                     ops.mrope_qk_(q, k, cos, sin, attn.n_heads, attn.head_dim)
@@ -256,13 +258,20 @@ class _AttentionCore:
             qw = self._q["qkv"]
             ws, sws = [qw[b][0] for (_, _, b, _) in segments], [qw[b][1] for (_, _, b, _) in segments]
         else:
-            ws, sws = [_data(self.qkv_weight[b]) for (_, _, b, _) in segments], None
+            weights = self.qkv_weight
+            ws, sws = [_data(_entry(weights, b)) for (_, _, b, _) in segments], None
         ops.gemm_qkv_pack(a, sa if self.fp8 else None, ws, sws, segl, self.n_heads, self.n_kv_heads, self.head_dim,
                           qkv[:, :self.d_model], images, cos, sin, qk_norm)
 
 
 def _data(t):
     return t.data if isinstance(t, nn.Parameter) else t
+
+
+def _entry(weights, b: int):
+    """``weights[b]``; of a parameter list past the name look-ups of its subscript, which cost as much as an argument check."""
+    p = weights._parameters.get(str(b)) if type(weights) is nn.ParameterList else None
+    return weights[b] if p is None else p
 
 
 class AdoptedAttention(_AttentionCore):
@@ -390,18 +399,17 @@ class DMAttention(nn.Module, _AttentionCore):
 def _routed_linear(a, sa, weights, qweights, weights2, segments, *, out, epilogue, residual=None, gates=None, cos=None,
                    sin=None, rope_cols=0, head_dim=0, qweights2=None, row_amax=None) -> None:
     """Per-modality linear over contiguous token segments: one grouped launch over all segments."""
+    if qweights is None and len(segments) == 1:
+        (s0, ln, b, _), = segments
+        rows = lambda t: t if t is None or (s0 == 0 and t.shape[0] == ln) else t[s0:s0 + ln]
+        ops.gemm(rows(a), _entry(weights, b), w2=_entry(weights2, b) if weights2 is not None else None, epilogue=epilogue, residual=rows(residual),
+                 gate=gates[0] if gates is not None else None, cos=rows(cos), sin=rows(sin), rope_cols=rope_cols, head_dim=head_dim,
+                 out=rows(out))
+        return
     segl = [(s, l) for (s, l, _, _) in segments]
     if qweights is None:
-        if len(segments) == 1:
-            (s0, ln, b, _), = segments
-            sl = slice(s0, s0 + ln)
-            ops.gemm(a[sl], weights[b], w2=weights2[b] if weights2 is not None else None, epilogue=epilogue,
-                     residual=residual[sl] if residual is not None else None, gate=gates[0] if gates is not None else None,
-                     cos=cos[sl] if cos is not None else None, sin=sin[sl] if sin is not None else None,
-                     rope_cols=rope_cols, head_dim=head_dim, out=out[sl])
-            return
-        ops.grouped_gemm(a, [weights[b] for (_, _, b, _) in segments], segl,
-                         w2s=[weights2[b] for (_, _, b, _) in segments] if weights2 is not None else None,
+        ops.grouped_gemm(a, [_entry(weights, b) for (_, _, b, _) in segments], segl,
+                         w2s=[_entry(weights2, b) for (_, _, b, _) in segments] if weights2 is not None else None,
                          epilogue=epilogue, residual=residual, gates=gates, cos=cos, sin=sin, rope_cols=rope_cols,
                          head_dim=head_dim, out=out)
         return
@@ -537,7 +545,7 @@ class DMBlock(nn.Module):
         """Per-branch adaLN-RMSNorm of x (bf16 or fp32) into the workspace: y (bf16), or (e4m3, per-token scale) for
         the fp8 variant.  ``sources``: x is still to be joined from these runs, in the same pass."""
         y, st = (ws.yq, ws.ys) if self.fp8 else (ws.y, None)
-        ops.adaln_rmsnorm_grouped(x, [weights[b] for (_, _, b, _) in segments], [shift if m else None for (_, _, _, m) in segments],
+        ops.adaln_rmsnorm_grouped(x, [_entry(weights, b) for (_, _, b, _) in segments], [shift if m else None for (_, _, _, m) in segments],
                                   [scale if m else None for (_, _, _, m) in segments], [(s0, ln) for (s0, ln, _, _) in segments],
                                   self.eps, y, st, sources)
         return y, st

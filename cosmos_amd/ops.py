@@ -42,9 +42,10 @@ def _chk(t: Optional[torch.Tensor], name: str, dtype=None, ndim: Optional[int] =
         raise RuntimeError(f"{name} must live on the GPU (the HIP path has no CPU fallback)")
     if dtype is not None and t.dtype != dtype:
         raise TypeError(f"{name} must be {dtype}, got {t.dtype}")
-    if ndim is not None and t.dim() != ndim:
+    st = t.stride()      # (as long as the shape)
+    if ndim is not None and len(st) != ndim:
         raise ValueError(f"{name} must be {ndim}-D, got shape {tuple(t.shape)}")
-    if t.dim() and t.stride(-1) != 1:
+    if st and st[-1] != 1:
         raise ValueError(f"{name} must be contiguous along its last dimension")
     return t.data_ptr()
 
@@ -56,7 +57,9 @@ def _f32vec(t: Optional[torch.Tensor], name: str, n: int) -> int:
         raise ValueError(f"{name} must have {n} elements, got {t.numel()}")
     if t.dtype != torch.float32 or not t.is_contiguous():
         raise TypeError(f"{name} must be a contiguous fp32 tensor")
-    return _chk(t.reshape(-1), name)
+    if not t.is_cuda:
+        raise RuntimeError(f"{name} must live on the GPU (the HIP path has no CPU fallback)")
+    return t.data_ptr()
 
 
 _OP_TIMER = None     # None, or the list that collects (category, start event, end event) while timing is on
