@@ -1429,6 +1429,21 @@ def test_quant_rows_exact(rows, cols):
     assert torch.equal(q.float().cpu(), wq)
 
 
+@pytest.mark.parametrize("exponent", [-126, -100, -72, -71, -70, -1, 0, 40, 88, 89, 100])
+def test_quantiser_quotients_are_divisions(exponent):
+    """The quantisers divide by product, remainder and correction where the scale leaves room for it (2^-80 .. 2^80, i.e. row
+    maxima from 2^-71 to 2^88) and by the division beyond: the codes of fp32 division everywhere."""
+    g = gen(exponent + 200)
+    a = (torch.randn((16, 4096), generator=g) * 2.0 ** exponent).to(torch.bfloat16)
+    a[:, 0] = 2.0 ** exponent * 1.9921875      # the maximum: the random values are folded below it
+    a = torch.where(a.abs().float() > 2.0 ** exponent * 1.9921875, (a.float() * 0.25).to(torch.bfloat16), a)
+    amax = a.float().abs().amax(-1)
+    s = amax / 448.0
+    want = (a.float() / s[:, None]).clamp(-448.0, 448.0).to(torch.float8_e4m3fn)
+    for q, sc in (ops.quant_rows(a.to(dev())), ops.quant_rows_from_parts(a.to(dev()), a.float().abs().view(16, 64, 64).amax(-1).to(dev()))):
+        assert torch.equal(sc.cpu(), s) and torch.equal(q.view(torch.uint8).cpu(), want.view(torch.uint8))
+
+
 @pytest.mark.parametrize("n,H,Hkv,hd", [(300, 4, 2, 128), (1000, 2, 2, 128), (130, 3, 3, 64)])
 def test_quant_from_attention_row_maxima(n, H, Hkv, hd):
     """The attention kernel leaves the largest |o| of every output row within every head; the quantiser that starts from
