@@ -69,32 +69,45 @@ struct ModParams {
 
 // out[l] = W_l silu(c) + b_l for every block l.  The vector is rounded to bf16 ahead of the activation and behind it, and the
 // result to bf16, as the bf16 linear layer it stands for does; sums are fp32.
+// PRE: how many chunks of 64 x 16 bytes of its rows a wave requests ahead of the activation (d >= 512 PRE)
+template <int PRE>
 __global__ __launch_bounds__(64 * kWaves) void modulation_kernel(const ModParams p) {
     extern __shared__ float s[];         // silu(c), d values
+    const int blk = blockIdx.x / p.per_block;
+    const int lane = threadIdx.x & 63, n8 = p.d >> 3;
+    const int row0 = ((blockIdx.x - blk * p.per_block) * kWaves + (threadIdx.x >> 6)) * kRows;
+    const bf16_t* w = p.w[blk];
+    const uint4* wr[kRows];
+    uint4 pre[PRE > 0 ? PRE : 1][kRows];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) wr[r] = reinterpret_cast<const uint4*>(w + (int64_t)(row0 + r < p.n_out ? row0 + r : p.n_out - 1) * p.d);
+#pragma unroll
+    for (int k = 0; k < PRE; ++k)
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) pre[k][r] = wr[r][lane + 64 * k];
+    asm volatile("" ::: "memory");
     for (int i = threadIdx.x; i < p.d; i += 64 * kWaves) {
         const float c = bf16lo(pack_bf16x2(p.c[i], 0.0f));
         s[i] = bf16lo(pack_bf16x2(silu_exact(c), 0.0f));
     }
     __syncthreads();
-    const int blk = blockIdx.x / p.per_block;
-    const int lane = threadIdx.x & 63;
-    const int row0 = ((blockIdx.x - blk * p.per_block) * kWaves + (threadIdx.x >> 6)) * kRows;
     if (row0 >= p.n_out) return;
-    const bf16_t* w = p.w[blk];
-    const uint4* wr[kRows];
-#pragma unroll
-    for (int r = 0; r < kRows; ++r) wr[r] = reinterpret_cast<const uint4*>(w + (int64_t)(row0 + r < p.n_out ? row0 + r : p.n_out - 1) * p.d);
-    const int n8 = p.d >> 3;
     float acc[kRows] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-    for (int i = lane; i < n8; i += 64) {
+    auto add = [&](const uint4 (&v)[kRows], int i) {
         const float4 s0 = reinterpret_cast<const float4*>(s)[2 * i], s1 = reinterpret_cast<const float4*>(s)[2 * i + 1];
 #pragma unroll
-        for (int r = 0; r < kRows; ++r) {
-            const uint4 v = wr[r][i];
-            acc[r] += bf16lo(v.x) * s0.x + bf16hi(v.x) * s0.y + bf16lo(v.y) * s0.z + bf16hi(v.y) * s0.w + bf16lo(v.z) * s1.x +
-                      bf16hi(v.z) * s1.y + bf16lo(v.w) * s1.z + bf16hi(v.w) * s1.w;
-        }
+        for (int r = 0; r < kRows; ++r)
+            acc[r] += bf16lo(v[r].x) * s0.x + bf16hi(v[r].x) * s0.y + bf16lo(v[r].y) * s0.z + bf16hi(v[r].y) * s0.w + bf16lo(v[r].z) * s1.x +
+                      bf16hi(v[r].z) * s1.y + bf16lo(v[r].w) * s1.z + bf16hi(v[r].w) * s1.w;
+    };
+#pragma unroll
+    for (int k = 0; k < PRE; ++k) add(pre[k], lane + 64 * k);
+#pragma unroll 4
+    for (int i = lane + 64 * PRE; i < n8; i += 64) {
+        uint4 v[kRows];
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) v[r] = wr[r][i];
+        add(v, i);
     }
 #pragma unroll
     for (int r = 0; r < kRows; ++r) {
@@ -153,7 +166,11 @@ extern "C" int32_t cdm_adaln_modulation_bf16(const float* c, const void* const* 
         const int nb = n_blocks - at < kMaxBlocks ? n_blocks - at : kMaxBlocks;
         for (int i = 0; i < nb; ++i) { p.w[i] = (const bf16_t*)w[at + i]; p.b[i] = (const bf16_t*)b[at + i]; }
         p.out = out + (int64_t)at * n_out;
-        modulation_kernel<<<(unsigned)(nb * p.per_block), 64 * kWaves, (size_t)d * 4, (hipStream_t)stream>>>(p);
+        // from d = 4096 on (16 activations per thread) the first weights travel under the activation; at smaller widths the
+        // registers that takes cost more waves than it hides.  Two / four / eight blocks, us without and with it: d = 4096 86.7 / 155 /
+        // 293 and 77.9 / 144 / 268 (6.0 TB/s), d = 2048 24.9 / 42.7 / 76.1 and 28.0 / 48.8 / 86.9
+        if (d >= 4096) modulation_kernel<4><<<(unsigned)(nb * p.per_block), 64 * kWaves, (size_t)d * 4, (hipStream_t)stream>>>(p);
+        else modulation_kernel<0><<<(unsigned)(nb * p.per_block), 64 * kWaves, (size_t)d * 4, (hipStream_t)stream>>>(p);
         if ((rc = cdm_check_launch("adaln_modulation"))) return rc;
     }
     return CDM_OK;
