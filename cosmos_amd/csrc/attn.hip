@@ -1147,74 +1147,91 @@ __global__ __launch_bounds__(256) void pack_kv_kernel(const bf16_t* __restrict__
     const int t0 = tile_idx * 64;
     char* kt = kp + ((int64_t)head * n_tiles + tile_idx) * TILE_BYTES;
     char* vt = vp + ((int64_t)head * n_tiles + tile_idx) * TILE_BYTES;
-    // one thread handles the chunk pair (ch, ch + CPR/2) of one token: the two halves of 8 rotary pairs
-    for (int idx = threadIdx.x; idx < 64 * (CPR / 2); idx += 256) {
-        const int r = idx / (CPR / 2), ch = idx % (CPR / 2);
-        uint4 k1 = make_uint4(0, 0, 0, 0), k2 = k1, v1 = k1, v2 = k1;
-        if (t0 + r < n_tokens) {
-            const bf16_t* kr = k + (int64_t)(t0 + r) * ldk + head * HD + ch * 8;
-            const bf16_t* vr = v + (int64_t)(t0 + r) * ldv + head * HD + ch * 8;
-            k1 = *reinterpret_cast<const uint4*>(kr);
-            k2 = *reinterpret_cast<const uint4*>(kr + HALF);
-            v1 = *reinterpret_cast<const uint4*>(vr);
-            v2 = *reinterpret_cast<const uint4*>(vr + HALF);
-            if (cos != nullptr || kn.w != nullptr) {
-                float c[8], sn[8], n1[8], n2[8];
+    // one thread handles the chunk pair (ch, ch + CPR/2) of one token (at head_dim 128 of two tokens): the two halves of 8 rotary
+    // pairs.  Everything it needs is requested before anything is used, one round trip to memory instead of four (8 heads x 128
+    // with norm, 1637 tokens 6.45 us, now 5.95; 32 x 128, 56,320 tokens 383, now 367).  Rows past the end are the last token's.
+    constexpr int ITER = 64 * (CPR / 2) / 256;
+    u32x4 kr[ITER][2], vr[ITER][2];
+    f32x4 cr[ITER][2], sr[ITER][2], wr[ITER][2][2];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) { c[e] = 1.0f; sn[e] = 0.0f; n1[e] = 1.0f; n2[e] = 1.0f; }
-                const uint32_t w1[4] = {k1.x, k1.y, k1.z, k1.w}, w2[4] = {k2.x, k2.y, k2.z, k2.w};
-                if (kn.w != nullptr) {
-                    // per-head RMSNorm: the CPR/2 consecutive threads of a token hold its HD channels
-                    float ss = 0.0f;
+    for (int it = 0; it < ITER; ++it) {
+        const int idx = it * 256 + threadIdx.x, r = idx / (CPR / 2), ch = idx % (CPR / 2);
+        const int row = t0 + r < n_tokens ? t0 + r : n_tokens - 1;
+        const bf16_t* kp_ = k + (int64_t)row * ldk + head * HD + ch * 8;
+        const bf16_t* vp_ = v + (int64_t)row * ldv + head * HD + ch * 8;
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const float a0 = bf16lo(w1[j]), a1 = bf16hi(w1[j]), b0 = bf16lo(w2[j]), b1 = bf16hi(w2[j]);
-                        ss += a0 * a0 + a1 * a1 + b0 * b0 + b1 * b1;
-                    }
+        for (int h = 0; h < 2; ++h) {
+            kr[it][h] = *reinterpret_cast<const u32x4*>(kp_ + h * HALF);
+            vr[it][h] = *reinterpret_cast<const u32x4*>(vp_ + h * HALF);
+            cr[it][h] = f32x4{1.f, 1.f, 1.f, 1.f}; sr[it][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        if (cos != nullptr)
 #pragma unroll
-                    for (int off = 1; off < CPR / 2; off <<= 1) ss += __shfl_xor(ss, off, 64);
-                    const float rn = rsqrtf(ss * (1.0f / HD) + kn.eps);
-                    const float* nw = kn.row(t0 + r, HD) + ch * 8;
+            for (int h = 0; h < 2; ++h) {
+                cr[it][h] = reinterpret_cast<const f32x4*>(cos + (int64_t)row * HALF + ch * 8)[h];
+                sr[it][h] = reinterpret_cast<const f32x4*>(sin + (int64_t)row * HALF + ch * 8)[h];
+            }
+        if (kn.w != nullptr) {
+            const float* nw = kn.row(row, HD) + ch * 8;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) { n1[e] = rn * nw[e]; n2[e] = rn * nw[HALF + e]; }
-                }
-                if (cos != nullptr) {
-                    const float4* cp = reinterpret_cast<const float4*>(cos + (int64_t)(t0 + r) * HALF + ch * 8);
-                    const float4* sp = reinterpret_cast<const float4*>(sin + (int64_t)(t0 + r) * HALF + ch * 8);
-                    const float4 c0 = cp[0], c1 = cp[1], s0 = sp[0], s1 = sp[1];
-                    c[0] = c0.x; c[1] = c0.y; c[2] = c0.z; c[3] = c0.w; c[4] = c1.x; c[5] = c1.y; c[6] = c1.z; c[7] = c1.w;
-                    sn[0] = s0.x; sn[1] = s0.y; sn[2] = s0.z; sn[3] = s0.w; sn[4] = s1.x; sn[5] = s1.y; sn[6] = s1.z; sn[7] = s1.w;
-                }
-                uint32_t o1[4], o2[4];
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) wr[it][h][j] = reinterpret_cast<const f32x4_any*>(nw + h * HALF)[j];
+        }
+    }
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int it = 0; it < ITER; ++it) {
+        const int idx = it * 256 + threadIdx.x, r = idx / (CPR / 2), ch = idx % (CPR / 2);
+        u32x4 k1 = kr[it][0], k2 = kr[it][1], v1 = vr[it][0], v2 = vr[it][1];
+        if (cos != nullptr || kn.w != nullptr) {
+            float c[8], sn[8], n1[8], n2[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { n1[e] = 1.0f; n2[e] = 1.0f; c[e] = cr[it][e / 4][e % 4]; sn[e] = sr[it][e / 4][e % 4]; }
+            if (kn.w != nullptr) {
+                // per-head RMSNorm: the CPR/2 consecutive threads of a token hold its HD channels
+                float ss = 0.0f;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const float a0 = bf16lo(w1[j]) * n1[2 * j], a1 = bf16hi(w1[j]) * n1[2 * j + 1];
-                    const float b0 = bf16lo(w2[j]) * n2[2 * j], b1 = bf16hi(w2[j]) * n2[2 * j + 1];
-                    o1[j] = pack_bf16x2(a0 * c[2 * j] - b0 * sn[2 * j], a1 * c[2 * j + 1] - b1 * sn[2 * j + 1]);
-                    o2[j] = pack_bf16x2(b0 * c[2 * j] + a0 * sn[2 * j], b1 * c[2 * j + 1] + a1 * sn[2 * j + 1]);
+                    const float a0 = bf16lo(k1[j]), a1 = bf16hi(k1[j]), b0 = bf16lo(k2[j]), b1 = bf16hi(k2[j]);
+                    ss += a0 * a0 + a1 * a1 + b0 * b0 + b1 * b1;
                 }
-                k1 = make_uint4(o1[0], o1[1], o1[2], o1[3]);
-                k2 = make_uint4(o2[0], o2[1], o2[2], o2[3]);
+#pragma unroll
+                for (int off = 1; off < CPR / 2; off <<= 1) ss += __shfl_xor(ss, off, 64);
+                const float rn = rsqrtf(ss * (1.0f / HD) + kn.eps);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) { n1[e] = rn * wr[it][0][e / 4][e % 4]; n2[e] = rn * wr[it][1][e / 4][e % 4]; }
             }
+            u32x4 o1, o2;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float a0 = bf16lo(k1[j]) * n1[2 * j], a1 = bf16hi(k1[j]) * n1[2 * j + 1];
+                const float b0 = bf16lo(k2[j]) * n2[2 * j], b1 = bf16hi(k2[j]) * n2[2 * j + 1];
+                o1[j] = pack_bf16x2(a0 * c[2 * j] - b0 * sn[2 * j], a1 * c[2 * j + 1] - b1 * sn[2 * j + 1]);
+                o2[j] = pack_bf16x2(b0 * c[2 * j] + a0 * sn[2 * j], b1 * c[2 * j + 1] + a1 * sn[2 * j + 1]);
+            }
+            k1 = o1;
+            k2 = o2;
         }
+        if (t0 + r >= n_tokens) k1 = k2 = v1 = v2 = u32x4{0u, 0u, 0u, 0u};      // padding keys of a ragged last tile
         {   // squared norm of the key as stored (rounded to bf16): the CPR/2 consecutive threads of a token hold it
-            const uint32_t w1[4] = {k1.x, k1.y, k1.z, k1.w}, w2[4] = {k2.x, k2.y, k2.z, k2.w};
             float ss = 0.0f;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const float a0 = bf16lo(w1[j]), a1 = bf16hi(w1[j]), b0 = bf16lo(w2[j]), b1 = bf16hi(w2[j]);
+                const float a0 = bf16lo(k1[j]), a1 = bf16hi(k1[j]), b0 = bf16lo(k2[j]), b1 = bf16hi(k2[j]);
                 ss += a0 * a0 + a1 * a1 + b0 * b0 + b1 * b1;
             }
 #pragma unroll
             for (int off = 1; off < CPR / 2; off <<= 1) ss += __shfl_xor(ss, off, 64);
             ksq_max = fmaxf(ksq_max, ss);
         }
-        *reinterpret_cast<uint4*>(kt + (ch * 64 + r) * 16) = k1;                  // chunk-major K image
-        *reinterpret_cast<uint4*>(kt + ((ch + CPR / 2) * 64 + r) * 16) = k2;
+        *reinterpret_cast<u32x4*>(kt + (ch * 64 + r) * 16) = k1;                  // chunk-major K image
+        *reinterpret_cast<u32x4*>(kt + ((ch + CPR / 2) * 64 + r) * 16) = k2;
         uint32_t* d1 = reinterpret_cast<uint32_t*>(&tile[r][ch * 8]);
         uint32_t* d2 = reinterpret_cast<uint32_t*>(&tile[r][HALF + ch * 8]);
-        d1[0] = v1.x; d1[1] = v1.y; d1[2] = v1.z; d1[3] = v1.w;
-        d2[0] = v2.x; d2[1] = v2.y; d2[2] = v2.z; d2[3] = v2.w;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) { d1[j] = v1[j]; d2[j] = v2[j]; }
     }
     ksq_max = wave_max(ksq_max);
     if ((threadIdx.x & 63) == 0) wave_kmax[threadIdx.x >> 6] = ksq_max;
