@@ -22,10 +22,12 @@ struct StepParams {
 
 __device__ __forceinline__ float combine(float c, float u, float g, bool guided) { return guided ? u + g * (c - u) : c; }
 
-// 4 elements per thread per iteration: 8-byte loads of the bf16 predictions, 16-byte loads/stores of the fp32 tensors.
+// 4 elements per thread per iteration: 8-byte loads of the bf16 predictions, 16-byte loads/stores of the fp32 tensors.  The number
+// of kept tensors is a template argument: all loads of a thread are then in flight at once, without branches between them.
 // Every input element is read before any output element of the same index is written and elements are independent,
 // so an output may be the very tensor of an input (the latents in place, a history slot being recycled).
-__global__ __launch_bounds__(256) void cfg_step_kernel(const StepParams p) {
+template <int NH>
+__global__ __launch_bounds__(1024) void cfg_step_kernel(const StepParams p) {
     const bool guided = p.vu != nullptr;
     const int64_t n4 = p.n >> 2;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (int64_t)gridDim.x * blockDim.x) {
@@ -36,13 +38,12 @@ __global__ __launch_bounds__(256) void cfg_step_kernel(const StepParams p) {
         const float x[4] = {x4.x, x4.y, x4.z, x4.w};
         const float v[4] = {combine(bf16lo(c2.x), bf16lo(u2.x), p.guidance, guided), combine(bf16hi(c2.x), bf16hi(u2.x), p.guidance, guided),
                             combine(bf16lo(c2.y), bf16lo(u2.y), p.guidance, guided), combine(bf16hi(c2.y), bf16hi(u2.y), p.guidance, guided)};
-        float h[kMaxHist][4];
+        float h[NH > 0 ? NH : 1][4];
 #pragma unroll
-        for (int k = 0; k < kMaxHist; ++k)
-            if (k < p.n_hist) {
-                const float4 h4 = reinterpret_cast<const float4*>(p.hist[k])[i];
-                h[k][0] = h4.x; h[k][1] = h4.y; h[k][2] = h4.z; h[k][3] = h4.w;
-            }
+        for (int k = 0; k < NH; ++k) {
+            const float4 h4 = reinterpret_cast<const float4*>(p.hist[k])[i];
+            h[k][0] = h4.x; h[k][1] = h4.y; h[k][2] = h4.z; h[k][3] = h4.w;
+        }
 #pragma unroll
         for (int j = 0; j < kMaxOut; ++j)
             if (j < p.n_out) {
@@ -50,11 +51,9 @@ __global__ __launch_bounds__(256) void cfg_step_kernel(const StepParams p) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) o[e] = p.c[j][0] * x[e] + p.c[j][1] * v[e];
 #pragma unroll
-                for (int k = 0; k < kMaxHist; ++k)
-                    if (k < p.n_hist) {
+                for (int k = 0; k < NH; ++k)
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) o[e] += p.c[j][2 + k] * h[k][e];
-                    }
+                    for (int e = 0; e < 4; ++e) o[e] += p.c[j][2 + k] * h[k][e];
                 reinterpret_cast<float4*>(p.out[j])[i] = make_float4(o[0], o[1], o[2], o[3]);
             }
     }
@@ -65,11 +64,13 @@ __global__ __launch_bounds__(256) void cfg_step_kernel(const StepParams p) {
         const float u = guided ? bf16_bits_to_f32(p.vu[t]) : c;
         const float v = combine(c, u, p.guidance, guided);
         const float x = p.x[t];
-        float h[kMaxHist];
-        for (int k = 0; k < p.n_hist; ++k) h[k] = p.hist[k][t];
+        float h[NH > 0 ? NH : 1];
+#pragma unroll
+        for (int k = 0; k < NH; ++k) h[k] = p.hist[k][t];
         for (int j = 0; j < p.n_out; ++j) {
             float o = p.c[j][0] * x + p.c[j][1] * v;
-            for (int k = 0; k < p.n_hist; ++k) o += p.c[j][2 + k] * h[k];
+#pragma unroll
+            for (int k = 0; k < NH; ++k) o += p.c[j][2 + k] * h[k];
             p.out[j][t] = o;
         }
     }
@@ -103,10 +104,14 @@ extern "C" int32_t cdm_cfg_step_f32(const float* x, const void* v_cond, const vo
     if (n == 0) return CDM_OK;
     int32_t rc = cdm_require_device();
     if (rc) return rc;
+    // one pass of three kept tensors and three outputs, workgroups of 256 / 512 / 1024 threads: 3.6 M values 18.6 / 18.4 / 18.0 us, 1.8 M
+    // 8.6 / 8.6 / 8.3 (6.9 TB/s), 0.38 M 3.4 / 3.3 / 3.9 (with the number of kept tensors at run time and 256 threads 19.1, 8.8, 3.6)
+    const int threads = n >= 1 << 20 ? 1024 : 512;
     const int64_t work = (n + 3) / 4;
-    int64_t blocks = (work + 255) / 256;
-    if (blocks > 256 * 256) blocks = 256 * 256;      // measured on the update of 2^26 values: 4096 workgroups 5.0 - 5.1 TB/s, 16384 5.2 - 5.3, 65536 5.5 - 5.7
-    if (blocks < 1) blocks = 1;
-    cfg_step_kernel<<<(unsigned)blocks, 256, 0, (hipStream_t)stream>>>(p);
+    int64_t blocks = (work + threads - 1) / threads;
+    if (blocks > (1 << 24) / threads) blocks = (1 << 24) / threads;      // measured on the update of 2^26 values: 2^20 threads 5.0 - 5.1 TB/s, 2^22 5.2 - 5.3, 2^24 5.5 - 5.7
+    const auto kernel = n_hist == 0 ? cfg_step_kernel<0> : n_hist == 1 ? cfg_step_kernel<1> : n_hist == 2 ? cfg_step_kernel<2>
+                        : n_hist == 3 ? cfg_step_kernel<3> : cfg_step_kernel<4>;
+    kernel<<<(unsigned)blocks, threads, 0, (hipStream_t)stream>>>(p);
     return cdm_check_launch("cfg_step");
 }
