@@ -66,26 +66,36 @@ __device__ __forceinline__ T* uniform_ptr(T* ptr) {      // wave-uniform value -
 // in its L2 (256-row tiles: GM = 4 measured best among 2, 3, 4, 6, 8, 16 once the output tiles are stored
 // non-temporally).
 // SPLIT: all tiles once per part of K, part by part (tiles of one part share operand rows, tiles of two parts nothing).
+// What a launch of one segment needs is requested from the kernel's arguments at once; launches of several read their segment's
+// entry behind that.  Left to itself the compiler asks for it where it is used, in six dependent steps: 1.2 us until the
+// first operand load, 0.5 now (M = 1024, N = K = 1024: 7.8 -> 7.4 us; M = 1024, K = 1024, SwiGLU to 4096: 20.9 -> 19.9; M = 512, N = K = 2048 11.7 ->
+// 10.9; M = 512, QKV of K = 2048 21.6 -> 20.3).
 template <int TM, int GM, bool SPLIT = false>
 __device__ __forceinline__ bool locate_tile(const GemmParams& p, Tile& t) {
-    const int all = SPLIT ? p.total_tiles * p.k_split : p.total_tiles;
+    const int total = p.total_tiles, tiles_n = p.tiles_n, n_seg = p.n_seg;
+    GemmSeg sg = p.seg[0];
+    asm volatile("" ::"s"(total), "s"(tiles_n), "s"(n_seg), "s"(p.lda), "s"(p.ldw), "s"(p.N), "s"(p.K), "s"(sg.m_start), "s"(sg.m_end),
+                 "s"(sg.tiles_m), "s"(sg.A), "s"(sg.W), "s"(sg.W2));
+    const int all = SPLIT ? total * p.k_split : total;
     const int per_xcd = (all + 7) >> 3;
     int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if (logical >= all) return false;
     t.part = 0;
     if (SPLIT) {
-        t.part = __builtin_amdgcn_readfirstlane(logical / p.total_tiles);
-        logical -= t.part * p.total_tiles;
+        t.part = __builtin_amdgcn_readfirstlane(logical / total);
+        logical -= t.part * total;
     }
-    int si = 0;
+    if (n_seg > 1) {
+        int si = 0;
 #pragma unroll
-    for (int i = 0; i < kMaxSeg - 1; ++i) si += (i < p.n_seg - 1 && logical >= p.seg[i].tile_end) ? 1 : 0;
-    const GemmSeg& sg = p.seg[si];
-    logical -= si ? p.seg[si - 1].tile_end : 0;
-    const int group = logical / (GM * p.tiles_n);
+        for (int i = 0; i < kMaxSeg - 1; ++i) si += (i < n_seg - 1 && logical >= p.seg[i].tile_end) ? 1 : 0;
+        sg = p.seg[si];
+        logical -= si ? p.seg[si - 1].tile_end : 0;
+    }
+    const int group = logical / (GM * tiles_n);
     const int first_m = group * GM;
     const int gsz = (sg.tiles_m - first_m) < GM ? (sg.tiles_m - first_m) : GM;
-    const int in_group = logical - group * GM * p.tiles_n;
+    const int in_group = logical - group * GM * tiles_n;
     // everything here is a function of blockIdx: pin it to scalar registers (the segment table is indexed
     // dynamically, which the compiler would otherwise treat as a per-lane value)
     t.m0 = __builtin_amdgcn_readfirstlane(sg.m_start + (first_m + in_group % gsz) * TM);
