@@ -35,8 +35,8 @@ __device__ __forceinline__ void quotient8(float (&f)[8], float s, float inv) {
     if (s >= 0x1p-80f && s <= 0x1p80f) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const float q = f[i] * inv;
-            f[i] = __builtin_fmaf(__builtin_fmaf(-q, s, f[i]), inv, q);
+            const float q = f[i] * inv, over = __builtin_fmaf(q, s, -f[i]);      // (this sign: the correction of a -0 is -0)
+            f[i] = __builtin_fmaf(-over, inv, q);
         }
     } else {
 #pragma unroll

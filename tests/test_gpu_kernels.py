@@ -1444,6 +1444,21 @@ def test_quantiser_quotients_are_divisions(exponent):
         assert torch.equal(sc.cpu(), s) and torch.equal(q.view(torch.uint8).cpu(), want.view(torch.uint8))
 
 
+@pytest.mark.parametrize("top", [0.0, 2.0 ** -100, 1.0, 2.0 ** 100])
+def test_quantisers_keep_signed_zeros(top):
+    """Zeros keep their sign in the codes, as under a division, whatever the row's scale; so do values that round to zero."""
+    a = torch.zeros((4, 512), dtype=torch.bfloat16)
+    a[:, 1::2] = -0.0
+    a[:, 2::8], a[:, 5::8] = top * 2.0 ** -24, -top * 2.0 ** -24
+    a[:, 0] = top
+    a[:, 7] = -top
+    s = a.float().abs().amax(-1) / 448.0
+    want = (a.float() / torch.where(s == 0, 1.0, s)[:, None]).to(torch.float8_e4m3fn).view(torch.uint8)
+    assert int((want == 0x80).sum()) >= 4 * 255
+    for q, _ in (ops.quant_rows(a.to(dev())), ops.quant_rows_from_parts(a.to(dev()), a.float().abs().view(4, 8, 64).amax(-1).to(dev()))):
+        assert torch.equal(q.view(torch.uint8).cpu(), want)
+
+
 @pytest.mark.parametrize("n,H,Hkv,hd", [(300, 4, 2, 128), (1000, 2, 2, 128), (130, 3, 3, 64)])
 def test_quant_from_attention_row_maxima(n, H, Hkv, hd):
     """The attention kernel leaves the largest |o| of every output row within every head; the quantiser that starts from
