@@ -217,10 +217,10 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
 
     // ---- load instruction j of this wave covers tile rows 8 (NW j + wave) .. + 7 of [A rows | W rows]
     int KT = p.K / (FP8 ? 128 : 64), kt0 = 0;
-    if constexpr (EPI == kPartial) {      // this part's k-tiles
-        const int all = KT;
-        kt0 = (int)((int64_t)all * tile.part / p.k_split);
-        KT = (int)((int64_t)all * (tile.part + 1) / p.k_split) - kt0;
+    if constexpr (EPI == kPartial) {      // this part's k-tiles: an even number, as a whole K's is
+        const int pairs = KT >> 1;
+        kt0 = (int)((int64_t)pairs * tile.part / p.k_split) * 2;
+        KT = (int)((int64_t)pairs * (tile.part + 1) / p.k_split) * 2 - kt0;
     }
     uint32_t off[L];
     const char* base[L];
@@ -269,44 +269,47 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
     for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
         for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
-    T a[2][MI], b[2][NI];      // fragments of the k-step at hand and of the next one
+    T a[2][KS][MI], b[2][KS][NI];      // fragments of the k-tile at hand and of the next one
     auto read = [&](int slot, int ks, int set) {
         const uint32_t s0 = slot * G::STAGE;
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi) a[set][mi] = rd(fa[ks] + s0 + mi * 2048);
+        for (int mi = 0; mi < MI; ++mi) a[set][ks][mi] = rd(fa[ks] + s0 + mi * 2048);
 #pragma unroll
-        for (int ni = 0; ni < NI; ++ni) b[set][ni] = rd(fb[ks] + s0 + ni * 2048);
+        for (int ni = 0; ni < NI; ++ni) b[set][ks][ni] = rd(fb[ks] + s0 + ni * 2048);
         __builtin_amdgcn_sched_barrier(0);      // the reads go out ahead of the MFMAs they run under
     };
-    // the MFMAs of one k-step; LOADS: the refill of slot `slot` with tile t, one load behind every few MFMAs (a wave that
-    // issues its loads back to back sits in the vector-memory issue queue with the matrix pipe idle)
-    auto mma = [&](int set, auto loads_c, int t, int slot) {
+    // the MFMAs of k-step ks; LOADS: its share of the refill of slot `slot` with tile t, one load behind every few MFMAs (a wave
+    // that issues its loads back to back sits in the vector-memory issue queue with the matrix pipe idle)
+    auto mma = [&](int set, auto ks_c, auto loads_c, int t, int slot) {
         constexpr bool LOADS = decltype(loads_c)::value;
-        constexpr int NM = MI * NI, GAP = NM / L > 0 ? NM / L : 1;
-        int nl = 0;
+        constexpr int ks = decltype(ks_c)::value, NM = MI * NI, GAP = KS * NM / L > 0 ? KS * NM / L : 1;
+        int nl = ks * NM / GAP < L ? ks * NM / GAP : L;
 #pragma unroll
         for (int i = 0; i < NM; ++i) {
             const int ni = i / MI, mi = i % MI;
             if constexpr (FP8)
-                acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b[set][ni], a[set][mi], acc[mi][ni], 0 /*A: e4m3*/,
+                acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b[set][ks][ni], a[set][ks][mi], acc[mi][ni], 0 /*A: e4m3*/,
                                                                                0 /*B: e4m3*/, 0, 0, 0, 0);
             else
-                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[set][ni], a[set][mi], acc[mi][ni], 0, 0, 0);
-            if (LOADS && i % GAP == GAP - 1 && nl < L) {
+                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[set][ks][ni], a[set][ks][mi], acc[mi][ni], 0, 0, 0);
+            if (LOADS && (ks * NM + i) % GAP == GAP - 1 && nl < L) {
                 lds_dma16(base[nl] + t * 128, off[nl], l0 + slot * G::STAGE + nl * (NW * 1024));
                 ++nl;
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (LOADS)
+        if (LOADS && ks == KS - 1)
             for (; nl < L; ++nl) lds_dma16(base[nl] + t * 128, off[nl], l0 + slot * G::STAGE + nl * (NW * 1024));
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    // ---- k-tiles.  Tile t lives in slot t % S.  A wave enters step t with the fragments of its first k-step in registers;
-    // the barrier sits ahead of the step's last k-step: every wave has then read all of tile t (whose slot is refilled with
-    // tile t + S) and tile t + 1 has landed, so the fragments the next step starts with are read under this step's last
-    // MFMAs.  Loads past the last tile are not issued: the last S steps count the loads still behind them instead.
+    // ---- k-tiles.  Tile t lives in slot t % S.  A wave enters step t with all fragments of tile t in registers (set t % 2);
+    // at the step's barrier every wave has read tile t, whose slot is refilled with tile t + S, and tile t + 1 has landed,
+    // whose fragments are read under the MFMAs of tile t: one barrier and one read latency per k-tile, both under a
+    // whole tile's MFMAs.  With one k-step's fragments at a time a small tile's step was a chain of two read latencies and a
+    // barrier.  us, before and now: M = 64, N = K = 4096 11.5 / 10.4; M = 256, N = K = 1024 4.3 / 3.8; M = 1024, N = 1024, K = 4096 17.3 /
+    // 16.4; M = 512, N = 12288, K = 4096 59.7 / 58.0; where the feed is the bound (M = 512, N = K = 4096: 28.4 / 28.6) nothing changes,
+    // and a wave more that requests W's lines ahead into the L2 costs there (38.3): it is requests, not their latency.  Loads past the last tile are not issued: the last S steps count the loads still behind them instead.
 #pragma unroll
     for (int t = 0; t < S; ++t)
         if (t < KT) {
@@ -315,43 +318,41 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
         }
     using std::false_type;
     using std::true_type;
+    using C0 = std::integral_constant<int, 0>;
+    using C1 = std::integral_constant<int, 1>;
+    constexpr bool BURST = KS * (MI + NI) <= 15;      // more reads than the counter of outstanding ones holds go out in two parts
     int slot = 0;
-    // SET: fragment set of the tile's first (e4m3: only) k-step - bf16 always 0, e4m3 alternating
+    // SET: fragment set of the tile at hand
     auto step = [&](auto behind_c, auto refill_c, auto set_c, int t) {
         constexpr int BEHIND = decltype(behind_c)::value;      // tiles that may still be in flight behind tile t + 1
         constexpr int SET = decltype(set_c)::value;
         const int next = slot == S - 1 ? 0 : slot + 1;
-        if constexpr (!FP8) {
-            read(slot, 1, 1);
-            mma(0, false_type{}, 0, 0);
-        }
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(BEHIND * L) : "memory");
         __builtin_amdgcn_sched_barrier(0);
-        read(next, 0, FP8 ? 1 - SET : 0);
-        mma(FP8 ? SET : 1, refill_c, t + S, slot);
+        read(next, 0, 1 - SET);
+        if constexpr (KS == 2 && BURST) read(next, 1, 1 - SET);
+        mma(SET, C0{}, refill_c, t + S, slot);
+        if constexpr (KS == 2) {
+            if constexpr (!BURST) read(next, 1, 1 - SET);
+            mma(SET, C1{}, refill_c, t + S, slot);
+        }
         slot = next;
     };
-    using C0 = std::integral_constant<int, 0>;
-    using C1 = std::integral_constant<int, FP8 ? 1 : 0>;
     using Deep = std::integral_constant<int, S - 2>;
     // tile 0 has landed everywhere
     if (KT >= S) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * L) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    read(0, 0, 0);
-    int t = 0;
-    if constexpr (FP8) {
-        for (; t + S < KT; t += 2) {
-            step(Deep{}, true_type{}, C0{}, t);
-            if (S % 2 == 0 || t + 1 + S < KT) step(Deep{}, true_type{}, C1{}, t + 1);      // KT is even
-        }
-    } else {
-        for (; t + S < KT; ++t) step(Deep{}, true_type{}, C0{}, t);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) read(0, ks, 0);
+    for (int t = 0; t + S < KT; t += 2) {
+        step(Deep{}, true_type{}, C0{}, t);
+        if (S % 2 == 0 || t + 1 + S < KT) step(Deep{}, true_type{}, C1{}, t + 1);      // KT is even
     }
     auto tail = [&](auto rem_c) {      // REM tiles behind this one; its index KT - 1 - REM has the parity of REM + 1
         constexpr int REM = decltype(rem_c)::value;
         if constexpr (REM > 0 && REM < S) {
             if (KT > REM)
-                step(std::integral_constant<int, REM - 1>{}, false_type{}, std::integral_constant<int, FP8 ? (REM + 1) % 2 : 0>{}, 0);
+                step(std::integral_constant<int, REM - 1>{}, false_type{}, std::integral_constant<int, (REM + 1) % 2>{}, 0);
         }
     };
     tail(std::integral_constant<int, 7>{});
@@ -361,11 +362,8 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
     tail(std::integral_constant<int, 3>{});
     tail(std::integral_constant<int, 2>{});
     tail(std::integral_constant<int, 1>{});
-    if constexpr (!FP8) {
-        read(slot, 1, 1);
-        mma(0, false_type{}, 0, 0);
-    }
-    mma(1, false_type{}, 0, 0);      // the last tile: an odd index
+    mma(1, C0{}, false_type{}, 0, 0);      // the last tile: an odd index
+    if constexpr (KS == 2) mma(1, C1{}, false_type{}, 0, 0);
 
     // ---- accumulators -> fp32 rows in LDS (every wave is done with the ring)
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
