@@ -872,6 +872,7 @@ class GraphedStack:
                  audio_states: Optional[torch.Tensor] = None) -> dict:
         given = dict(hidden_states=hidden_states, timestep=timestep, encoder_hidden_states=encoder_hidden_states,
                      action_states=action_states, audio_states=audio_states)
+        runs = []
         for k, v in given.items():
             dst = self.static[k]
             if (v is None) != (dst is None):
@@ -879,7 +880,8 @@ class GraphedStack:
             if v is not None:
                 if tuple(v.shape) != tuple(dst.shape):
                     raise ValueError(f"{k}: shape {tuple(v.shape)} differs from the recorded {tuple(dst.shape)}")
-                dst.copy_(v)
+                runs.append((dst, v))
+        ops.copy_runs(*zip(*runs))
         self.graph.replay()
         return self.out
 

@@ -746,6 +746,34 @@ def cfg_step(x: torch.Tensor, v_cond: torch.Tensor, v_uncond: Optional[torch.Ten
     return out
 
 
+def copy_runs(dsts: Sequence[torch.Tensor], srcs: Sequence[torch.Tensor]) -> None:
+    """``dst.copy_(src)`` for every pair, in order.  Contiguous GPU tensors of one type, up to 16 MB each, take one launch between
+    them; whatever else ``copy_`` accepts goes through it.  Tokens and a timestep, two copies against one launch: 2 MB 4.1 / 2.2 us,
+    16 MB 5.9 / 4.9, 32 MB 12.0 / 11.6."""
+    todo = []
+    for d, s in zip(dsts, srcs):
+        if (type(s) is torch.Tensor and type(d) is torch.Tensor and s.is_cuda and s.device == d.device and s.dtype == d.dtype
+                and s.shape == d.shape and s.is_contiguous() and d.is_contiguous() and not (s.requires_grad or d.requires_grad)
+                and not (s.is_neg() or s.is_conj()) and s.nbytes <= 1 << 24 and d.device.index == torch.cuda.current_device()):
+            todo.append((s.data_ptr(), d.data_ptr(), s.nbytes))
+            if len(todo) == 8:
+                _copy_runs(todo)
+                todo = []
+            continue
+        _copy_runs(todo)
+        todo = []
+        d.copy_(s)
+    _copy_runs(todo)
+
+
+def _copy_runs(todo) -> None:
+    n = len(todo)
+    if n:
+        rc = _lib.load().cdm_copy_runs((C.c_void_p * n)(*[s for s, _, _ in todo]), (C.c_void_p * n)(*[d for _, d, _ in todo]),
+                                       (C.c_int64 * n)(*[b for _, _, b in todo]), n, _stream())
+        _lib.check(rc, "cdm_copy_runs")
+
+
 _ATTN_TIMER = None
 
 

@@ -433,6 +433,12 @@ int32_t cdm_cfg_step_f32(const float* x, const void* v_cond, const void* v_uncon
                          const float* const* hist, int32_t n_hist, const float* coef, float* const* outs,
                          int32_t n_out, int64_t n, void* stream);
 
+/* Copies of up to 8 contiguous buffers in one launch: dst[i][0 .. bytes[i]) = src[i][0 .. bytes[i]), in the order of the runs (a run
+ * that touches what an earlier one writes, or writes what one reads, runs in a launch behind it).  src, dst, bytes: HOST arrays
+ * of n entries; device pointers of any alignment.  A run may be its own target; one that overlaps it otherwise is refused.
+ */
+int32_t cdm_copy_runs(const void* const* src, void* const* dst, const int64_t* bytes, int32_t n, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

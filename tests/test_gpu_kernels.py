@@ -1698,3 +1698,37 @@ def test_grouped_gemm_sweep(case):
                 want[s0:s0 + ln] = rr[s0:s0 + ln] + (1.0 if gates[i] is None else gates[i]) * (ar[s0:s0 + ln] @ ws[i][1].t())
     assert torch.equal(out, ref), f"grouped != per-segment launches ({n_seg} segments, {epi})"
     assert_close(out, want, 0.9999, 1e-2, f"grouped sweep {n_seg} segments {M}x{N}x{K} {epi}")
+
+
+@pytest.mark.parametrize("sizes", [(1,), (0, 3), (4096, 1, 17), (2 ** 20 + 5, 1), (7,) * 9, (2 ** 23 + 8, 33)])
+@pytest.mark.parametrize("shift", [0, 1, 3])
+def test_copy_runs(sizes, shift):
+    """Several buffers in one launch: whole and partial 16-byte groups, either end off its alignment, more runs than a launch takes, one
+    above the limit; nothing beside the targets is written."""
+    src = [torch.randint(-30000, 30000, (n + 16,), dtype=torch.int16, device=dev()) for n in sizes]
+    dst = [torch.full((n + 16,), 7, dtype=torch.int16, device=dev()) for n in sizes]
+    ops.copy_runs([d[8:8 + n] for d, n in zip(dst, sizes)], [s[shift:shift + n] for s, n in zip(src, sizes)])
+    for s, d, n in zip(src, dst, sizes):
+        assert torch.equal(d[8:8 + n], s[shift:shift + n]) and bool((d[:8] == 7).all()) and bool((d[8 + n:] == 7).all())
+
+
+def test_copy_runs_keeps_the_order_and_what_copies_do():
+    """A run that reads an earlier run's target, one that overwrites an earlier one's source, a run onto itself, and everything that
+    torch's copy takes besides: another type, strides, host memory, sizes that broadcast.  A run that overlaps its own target is
+    refused, as by torch."""
+    buf = torch.arange(4096, dtype=torch.float32, device=dev())
+    want = buf.clone()
+    a, b, c = slice(0, 1000), slice(1000, 2000), slice(2000, 3000)
+    pairs = [(b, a), (c, b), (a, c), (b, b)]
+    for d, s in pairs:
+        want[d].copy_(want[s].clone())
+    ops.copy_runs([buf[d] for d, _ in pairs], [buf[s] for _, s in pairs])
+    assert torch.equal(buf, want)
+    out = [torch.zeros(6, 4, device=dev()) for _ in range(5)]
+    x = torch.randn(6, 4, device=dev())
+    ops.copy_runs(out, [x.bfloat16(), x.t().contiguous().t(), x.cpu(), x[:1], x])
+    assert torch.equal(out[0], x.bfloat16().float()) and torch.equal(out[3], x[:1].expand(6, 4))
+    assert all(torch.equal(out[i], x) for i in (1, 2, 4))
+    with pytest.raises(RuntimeError):
+        ops.copy_runs([buf[8:108]], [buf[:100]])
+    ops.copy_runs([], [])
