@@ -83,6 +83,8 @@ SIGNATURES = {
                                           _I64, _I64, _P]),
     "cdm_grouped_gemm_qkv_pack_runs_bf16": (_I32, [C.POINTER(_P), _I64, C.POINTER(_P), _I64, _P, _I64, C.POINTER(_I64),
                                                    C.POINTER(_I64), _I32, _I64, _I32, _I32, _I32, _P, _P, _P, _P, _I64, _P]),
+    "cdm_grouped_gemm_residual_bf16": (_I32, [_P, _I64, C.POINTER(_P), _I64, _P, _I64, C.POINTER(_I64), C.POINTER(_I64), _I32, _I64, _I64,
+                                              _P, _I64, C.POINTER(_P), _P, _I64, _I64, _I64, _P, _I64, _P]),
     "cdm_grouped_gemm_scratch_bytes": (_I64, [C.POINTER(_I64), _I32, _I64, _I64, _I32]),
     "cdm_grouped_gemm_scratch_bf16": (_I32, [_P, _I64, C.POINTER(_P), _I64, _P, _I64, C.POINTER(_I64), C.POINTER(_I64), _I32, _I64,
                                              _I64, _I32, _P, _I64, C.POINTER(_P), _P, _I64, _P]),

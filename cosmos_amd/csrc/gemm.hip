@@ -757,6 +757,18 @@ int32_t validate(const char* who, int esize, const void* A, int64_t lda, const v
     return CDM_OK;
 }
 
+// rows of an fp32 result as bf16: eight columns per thread (what the 256 x 256 kernel leaves to a launch of its own: its waves
+// hold four columns of a row each, and at its sizes the launch is nothing beside the product)
+__global__ __launch_bounds__(256) void rows_to_bf16_kernel(const float* __restrict__ x, int64_t ldx, bf16_t* __restrict__ y, int64_t ldy, int rows,
+                                                           int cols) {
+    const int cpr = cols >> 3;
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x, r = idx / cpr;
+    if (r >= rows) return;
+    const int c = (int)(idx - r * cpr) * 8;
+    const float4 a = *reinterpret_cast<const float4*>(x + r * ldx + c), b = *reinterpret_cast<const float4*>(x + r * ldx + c + 4);
+    *reinterpret_cast<uint4*>(y + r * ldy + c) = make_uint4(pack_bf16x2(a.x, a.y), pack_bf16x2(a.z, a.w), pack_bf16x2(b.x, b.y), pack_bf16x2(b.z, b.w));
+}
+
 // host-side description of one row segment of a (grouped) GEMM
 struct HostSeg {
     int64_t start, len;
@@ -796,6 +808,14 @@ int32_t launch(GemmParams& p, TileShape shape, int32_t epilogue, hipStream_t st,
         default: CDM_LAUNCH(CDM_EPI_ROPE_QK); break;
     }
 #undef CDM_LAUNCH
+    for (int k = 0; p.C16 != nullptr && k < p.n_seg; ++k) {
+        const int lo = p.seg[k].m_start > p.c16_row0 ? p.seg[k].m_start : p.c16_row0, end = p.c16_row0 + p.c16_rows;
+        const int rows = (p.seg[k].m_end < end ? p.seg[k].m_end : end) - lo;
+        if (rows <= 0) continue;
+        const unsigned blocks = (unsigned)(((int64_t)rows * (p.N / 8) + 255) / 256);
+        rows_to_bf16_kernel<<<blocks, 256, 0, st>>>(reinterpret_cast<const float*>(p.C) + (int64_t)lo * p.ldc, p.ldc,
+                                                    p.C16 + (int64_t)(lo - p.c16_row0) * p.ldc16, p.ldc16, rows, p.N);
+    }
     return cdm_check_launch(who);
 }
 
@@ -852,7 +872,8 @@ int32_t grouped(const char* who, const void* A, int64_t lda, const float* sa, co
                 const void* R, int64_t ldr, const float* const* gate, const float* cos, const float* sin,
                 int64_t rope_cols, int32_t head_dim, void* stream, const GemmParams* pack = nullptr,
                 const float* k_norm_rows = nullptr, float* row_amax = nullptr, int64_t amax_ld = 0, void* scratch = nullptr,
-                int64_t scratch_bytes = 0, const void* const* runs = nullptr) {
+                int64_t scratch_bytes = 0, const void* const* runs = nullptr, void* c16 = nullptr, int64_t ldc16 = 0, int64_t c16_row0 = 0,
+                int64_t c16_rows = 0) {
     constexpr int esize = FP8 ? 1 : 2;
     CDM_REQUIRE((A || runs) && W && C && seg_start && seg_len, CDM_ERR_BAD_ARG, "%s: null pointer", who);
     CDM_REQUIRE((epilogue == CDM_EPI_QKV_PACK) == (pack != nullptr), CDM_ERR_BAD_ARG,
@@ -897,6 +918,7 @@ int32_t grouped(const char* who, const void* A, int64_t lda, const float* sa, co
     int32_t rc = cdm_require_device();
     if (rc) return rc;
     GemmParams p{};
+    p.C16 = (bf16_t*)c16; p.ldc16 = ldc16; p.c16_row0 = (int)c16_row0; p.c16_rows = (int)c16_rows;
     p.lda = lda * esize; p.ldw = ldw * esize; p.sa = sa;
     p.C = (bf16_t*)C; p.ldc = ldc;
     p.N = (int)N; p.K = (int)K;
@@ -1070,6 +1092,20 @@ extern "C" int32_t cdm_grouped_gemm_scratch_bf16(const void* A, int64_t lda, con
     CDM_REQUIRE(cdm_aligned16(scratch) && scratch_bytes >= 0, CDM_ERR_BAD_ALIGN, "%s: scratch must be 16-byte aligned", who);
     return grouped<false>(who, A, lda, nullptr, W, nullptr, ldw, nullptr, nullptr, C, ldc, seg_start, seg_len, n_seg, N, K, epilogue,
                           R, ldr, gate, nullptr, nullptr, 0, 0, stream, nullptr, nullptr, nullptr, 0, scratch, scratch_bytes);
+}
+
+extern "C" int32_t cdm_grouped_gemm_residual_bf16(const void* A, int64_t lda, const void* const* W, int64_t ldw, float* C, int64_t ldc,
+                                                  const int64_t* seg_start, const int64_t* seg_len, int32_t n_seg, int64_t N, int64_t K,
+                                                  const float* R, int64_t ldr, const float* const* gate, void* C16, int64_t ldc16,
+                                                  int64_t c16_row0, int64_t c16_rows, void* scratch, int64_t scratch_bytes, void* stream) {
+    const char* who = "grouped_gemm_residual_bf16";
+    if (c16_rows == 0) C16 = nullptr;
+    CDM_REQUIRE(c16_rows <= 0 || (C16 && cdm_aligned16(C16) && ldc16 % 8 == 0 && ldc16 >= N), CDM_ERR_BAD_ALIGN, "%s: C16 rows must be 16-byte aligned and hold N columns", who);
+    CDM_REQUIRE(c16_row0 >= 0 && c16_rows >= 0 && c16_row0 + c16_rows < (1ll << 31) - 512, CDM_ERR_BAD_ARG, "%s: rows of C16 out of range", who);
+    CDM_REQUIRE(cdm_aligned16(scratch) && scratch_bytes >= 0, CDM_ERR_BAD_ALIGN, "%s: scratch must be 16-byte aligned", who);
+    return grouped<false>(who, A, lda, nullptr, W, nullptr, ldw, nullptr, nullptr, C, ldc, seg_start, seg_len, n_seg, N, K,
+                          CDM_EPI_GATE_RESIDUAL_F32, R, ldr, gate, nullptr, nullptr, 0, 0, stream, nullptr, nullptr, nullptr, 0,
+                          scratch, scratch ? scratch_bytes : 0, nullptr, C16, ldc16, c16_row0, c16_rows);
 }
 
 extern "C" int32_t cdm_grouped_gemm_fp8(const void* Aq, int64_t lda, const float* sa, const void* const* Wq,

@@ -42,6 +42,8 @@ struct GemmParams {
     // Launches cut along K (gemm_tile.hip): part i of k_split leaves fp32 sums of its k-tiles, [k_split][part_rows][N], row 0 =
     // token row part_row0
     float* partial; int k_split, part_rows, part_row0;
+    // CDM_EPI_GATE_RESIDUAL_F32, optional: rows c16_row0 .. + c16_rows - 1 of the result as bf16 too, from row 0 of C16 on
+    bf16_t* C16; int64_t ldc16; int c16_row0, c16_rows;
     int tiles_n, total_tiles, n_seg;
     GemmSeg seg[kMaxSeg];
 };

@@ -228,6 +228,8 @@ __device__ __forceinline__ void store8(const GemmParams& p, const float (&gate)[
         for (int e = 0; e < 8; ++e) r[e] = r[e] + g[e] * v[e];
         *reinterpret_cast<float4*>(C) = make_float4(r[0], r[1], r[2], r[3]);
         *reinterpret_cast<float4*>(C + 4) = make_float4(r[4], r[5], r[6], r[7]);
+        if (p.C16 != nullptr && (unsigned)(row - p.c16_row0) < (unsigned)p.c16_rows)
+            *reinterpret_cast<uint4*>(p.C16 + (int64_t)(row - p.c16_row0) * p.ldc16 + col) = pack8(r);
     } else {
         if constexpr (EPI == CDM_EPI_GATE_RESIDUAL)
 #pragma unroll

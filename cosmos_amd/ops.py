@@ -254,6 +254,30 @@ def _gemm_cut_along_k(a: torch.Tensor, ws: Sequence[torch.Tensor], segments: Seq
 
 
 @_timed("gemm")
+def residual_gemm_(x: torch.Tensor, a: torch.Tensor, ws: Sequence[torch.Tensor], segments: Sequence[Tuple[int, int]],
+                   gates: Sequence[Optional[torch.Tensor]], rows16: torch.Tensor, first: int) -> None:
+    """x += gate * (a @ w^T) per segment on fp32 rows, with the new rows ``first`` .. of x left in ``rows16`` as bf16 too."""
+    n_seg, (M, N), K = len(segments), x.shape, a.shape[1]
+    if a.shape[0] != M or any(w.shape != (N, K) or w.stride(0) != ws[0].stride(0) for w in ws):
+        raise ValueError("shape mismatch")
+    if rows16.shape[1] != N or first < 0 or first + rows16.shape[0] > M or any(s < 0 or l < 0 or s + l > M for s, l in segments):
+        raise ValueError("rows out of range")
+    scratch, buf = gemm_scratch_bytes(tuple(int(l) for _, l in segments), N, K, EPI_GATE_RESIDUAL_F32), None
+    if scratch:
+        try:
+            buf = torch.empty((scratch,), dtype=torch.uint8, device=a.device)
+        except torch.OutOfMemoryError:      # without scratch the launch is the uncut one, which takes no memory
+            scratch = 0
+    PP, I64 = C.c_void_p * n_seg, C.c_int64 * n_seg
+    rc = _lib.load().cdm_grouped_gemm_residual_bf16(
+        _chk(a, "a", torch.bfloat16, 2), a.stride(0), PP(*[_chk(w, "w", torch.bfloat16, 2) for w in ws]), ws[0].stride(0),
+        _chk(x, "x", torch.float32, 2), x.stride(0), I64(*[int(s) for s, _ in segments]), I64(*[int(l) for _, l in segments]), n_seg, N, K,
+        x.data_ptr(), x.stride(0), PP(*[(_f32vec(g, "gate", N) or None) for g in gates]), _chk(rows16, "rows16", torch.bfloat16, 2),
+        rows16.stride(0), first, rows16.shape[0], buf.data_ptr() if buf is not None else None, scratch, _stream())
+    _lib.check(rc, "cdm_grouped_gemm_residual_bf16")
+
+
+@_timed("gemm")
 def gemm(a: torch.Tensor, w: torch.Tensor, *, w2: Optional[torch.Tensor] = None, epilogue: str = "none",
          residual: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
          cos: Optional[torch.Tensor] = None, sin: Optional[torch.Tensor] = None, rope_cols: int = 0,

@@ -347,6 +347,14 @@ int32_t cdm_grouped_gemm_scratch_bf16(const void* A, int64_t lda, const void* co
                                       int32_t epilogue, const void* R, int64_t ldr, const float* const* gate, void* scratch,
                                       int64_t scratch_bytes, void* stream);
 
+/* cdm_grouped_gemm_scratch_bf16 with CDM_EPI_GATE_RESIDUAL_F32 that also leaves rows c16_row0 .. c16_row0 + c16_rows - 1 of C rounded to
+ * bf16 in C16, row c16_row0 in its row 0: the end of a stack whose caller wants bf16 rows.  Rows in no segment are not written.
+ * scratch may be null. */
+int32_t cdm_grouped_gemm_residual_bf16(const void* A, int64_t lda, const void* const* W, int64_t ldw, float* C, int64_t ldc,
+                                       const int64_t* seg_start, const int64_t* seg_len, int32_t n_seg, int64_t N, int64_t K,
+                                       const float* R, int64_t ldr, const float* const* gate, void* C16, int64_t ldc16,
+                                       int64_t c16_row0, int64_t c16_rows, void* scratch, int64_t scratch_bytes, void* stream);
+
 /*
  * Epilogue NONE, and the fused QKV projection, on runs that lie apart: A[g] points at the first row of segment g (all runs with
  * row stride lda; null for an empty segment); rows of C, the rotary tables and the images keep their place in the joint sequence.

@@ -1732,3 +1732,58 @@ def test_copy_runs_keeps_the_order_and_what_copies_do():
     with pytest.raises(RuntimeError):
         ops.copy_runs([buf[8:108]], [buf[:100]])
     ops.copy_runs([], [])
+
+
+@pytest.mark.parametrize("variant", [0, 1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("n,N,K,segs,first,rows", [
+    (1, 8, 128, [(0, 1)], 0, 1), (70, 264, 256, [(0, 37), (37, 33)], 37, 33), (300, 512, 384, [(0, 100), (120, 180)], 90, 100),
+    (512, 1024, 4096, [(0, 512)], 0, 512), (64, 2048, 8192, [(0, 64)], 5, 59), (2500, 4096, 128, [(0, 77), (77, 2423)], 77, 2400), (130, 264, 128, [(0, 130)], 130, 0)])
+def test_residual_gemm_leaves_bf16_rows(n, N, K, segs, first, rows, variant, request):
+    """The gated fp32 residual that also leaves some of its rows as bf16: the stream's bits are those of the plain form, the rows those of
+    a conversion behind it, whatever tile, cut or range of K the launch takes; rows outside the segments are not written."""
+    request.addfinalizer(lambda: ops.set_variant("gemm", 0))
+    g = gen(n + N + K)
+    a, _ = rand_bf16((n, K), g)
+    ws = [rand_bf16((N, K), g, 0.05)[0] for _ in segs]
+    gates = [None if i else torch.randn((N,), generator=g).to(dev()) for i in range(len(segs))]
+    x = torch.randn((n, N), generator=g).to(dev())
+    ops.set_variant("gemm", variant)
+    want, got = x.clone(), x.clone()
+    ops.grouped_gemm(a, ws, segs, epilogue="gate_residual", residual=want, gates=gates, out=want)
+    rows16 = torch.full((rows, N), 7.0, dtype=torch.bfloat16, device=dev())
+    ops.residual_gemm_(got, a, ws, segs, gates, rows16, first)
+    assert torch.equal(got, want)
+    inside = torch.zeros(n, dtype=torch.bool, device=dev())
+    for s, l in segs:
+        inside[s:s + l] = True
+    inside = inside[first:first + rows, None]
+    assert torch.equal(rows16, torch.where(inside, want[first:first + rows].to(torch.bfloat16), torch.full_like(rows16, 7.0)))
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(n_text=37), dict(n_text=64, n_action=6, n_branches=3)])
+def test_stack_video_rows_are_the_streams(kw):
+    """A stack's video rows - a recorded one's are left by its last product - are the rows of the stream it returns, rounded; so are those
+    of a stack whose tail is somebody else's, recorded or not."""
+    from cosmos_amd import DMConfig, DMStack
+
+    cfg = DMConfig("v", 256, 2, 128, 512, 2, (2, 4, 9), **kw)
+    st = DMStack(cfg, device=dev())
+    st.reset_parameters(5)
+    g = gen(5)
+    mk = lambda n: rand_bf16((1, n, 256), g)[0] if n else None
+    args = (mk(cfg.n_video), torch.tensor([300.0], device=dev()), mk(cfg.n_text), mk(cfg.n_action))
+    res = st(*args, return_dict=True)
+    want = res["joint"][cfg.n_text:cfg.n_text + cfg.n_video].to(torch.bfloat16)
+    assert res["sample"].shape == (1, cfg.n_video, 256) and torch.equal(res["sample"][0], want) and torch.equal(st(*args)[0][0], want)
+    names = ("hidden_states", "timestep", "encoder_hidden_states", "action_states")
+    given = {k: v for k, v in zip(names, args) if v is not None}
+    seen = []
+    for tail in (None, lambda x, *a: seen.append(x) or DMStack._result(st, x, *a)):
+        if tail is not None:
+            st._result = tail
+        graph = st.capture(**given)
+        for _ in range(2):
+            got = graph(**given)
+            torch.cuda.synchronize()
+            assert torch.equal(got["sample"][0], want) and torch.equal(got["joint"], res["joint"])
+    assert len(seen) == 3 and torch.equal(st(*args)[0][0], want)
