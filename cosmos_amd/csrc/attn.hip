@@ -457,10 +457,10 @@ __device__ __forceinline__ void finish_rows(const PackedParams& p, const QRows<H
             for (int j = 0; j < 4; ++j) {
                 float a0 = bf16lo(w1[j]), a1 = bf16hi(w1[j]), b0 = bf16lo(w2[j]), b1 = bf16hi(w2[j]);
                 if constexpr (NORM) { a0 *= n1[2 * j]; a1 *= n1[2 * j + 1]; b0 *= n2[2 * j]; b1 *= n2[2 * j + 1]; }
-                o1[j] = pack_bf16x2((a0 * c[2 * j] - b0 * sn[2 * j]) * p.scale_log2e,
-                                    (a1 * c[2 * j + 1] - b1 * sn[2 * j + 1]) * p.scale_log2e);
-                o2[j] = pack_bf16x2((b0 * c[2 * j] + a0 * sn[2 * j]) * p.scale_log2e,
-                                    (b1 * c[2 * j + 1] + a1 * sn[2 * j + 1]) * p.scale_log2e);
+                rotate_pair(a0, b0, c[2 * j], sn[2 * j]);
+                rotate_pair(a1, b1, c[2 * j + 1], sn[2 * j + 1]);
+                o1[j] = pack_bf16x2(a0 * p.scale_log2e, a1 * p.scale_log2e);
+                o2[j] = pack_bf16x2(b0 * p.scale_log2e, b1 * p.scale_log2e);
             }
             qf[qb][ks] = __builtin_bit_cast(bf16x8, o1);
             qf[qb][ks + KS / 2] = __builtin_bit_cast(bf16x8, o2);
@@ -1206,10 +1206,11 @@ __global__ __launch_bounds__(256) void pack_kv_kernel(const bf16_t* __restrict__
             u32x4 o1, o2;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
+                // roundings written out; the second member fuses its other product than rotate_pair's does (kept images stay the same)
                 const float a0 = bf16lo(k1[j]) * n1[2 * j], a1 = bf16hi(k1[j]) * n1[2 * j + 1];
                 const float b0 = bf16lo(k2[j]) * n2[2 * j], b1 = bf16hi(k2[j]) * n2[2 * j + 1];
-                o1[j] = pack_bf16x2(a0 * c[2 * j] - b0 * sn[2 * j], a1 * c[2 * j + 1] - b1 * sn[2 * j + 1]);
-                o2[j] = pack_bf16x2(b0 * c[2 * j] + a0 * sn[2 * j], b1 * c[2 * j + 1] + a1 * sn[2 * j + 1]);
+                o1[j] = pack_bf16x2(__builtin_fmaf(a0, c[2 * j], -(b0 * sn[2 * j])), __builtin_fmaf(a1, c[2 * j + 1], -(b1 * sn[2 * j + 1])));
+                o2[j] = pack_bf16x2(__builtin_fmaf(b0, c[2 * j], a0 * sn[2 * j]), __builtin_fmaf(b1, c[2 * j + 1], a1 * sn[2 * j + 1]));
             }
             k1 = o1;
             k2 = o2;

@@ -60,6 +60,14 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
     return __builtin_bit_cast(uint32_t, p);
 }
 
+// rotate-half pair, (x1, x2) -> (x1 c - x2 s, x2 c + x1 s), with its roundings written out: kernels whose compiler-chosen
+// contractions differ would put rows one bf16 rounding apart
+__device__ __forceinline__ void rotate_pair(float& x1, float& x2, float c, float s) {
+    const float a = x1, b = x2;
+    x1 = __builtin_fmaf(c, a, -(s * b));
+    x2 = __builtin_fmaf(s, a, c * b);
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);

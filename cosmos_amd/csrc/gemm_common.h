@@ -119,14 +119,6 @@ __device__ __forceinline__ float silu_f(float g) {
     return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g));
 }
 
-// rotate-half pair, (x1, x2) -> (x1 c - x2 s, x2 c + x1 s), with its roundings written out: kernels whose compiler-chosen
-// contractions differ would put K rows one bf16 rounding apart
-__device__ __forceinline__ void rotate_pair(float& x1, float& x2, float c, float s) {
-    const float a = x1, b = x2;
-    x1 = __builtin_fmaf(c, a, -(s * b));
-    x2 = __builtin_fmaf(s, a, c * b);
-}
-
 __device__ __forceinline__ uint2 pack4_bf16(float a, float b, float c, float d) {
     return make_uint2(pack_bf16x2(a, b), pack_bf16x2(c, d));
 }

@@ -1050,6 +1050,43 @@ def test_attention_64_row_workgroups(n, H, Hkv, hd, P, causal, qkn, request):
         assert rel(variant) <= 1.25 * rel(7) + 1e-4, (variant, rel(variant), rel(7))
 
 
+@pytest.mark.parametrize("variant,n,H,hd", [(0, 4200, 8, 64), (0, 2304, 16, 128)] + [(v, 130, 2, hd) for v in (1, 3, 4, 5, 7, 8, 9) for hd in (64, 128)])
+def test_rotations_round_as_written(variant, n, H, hd, request):
+    """Which product of (x1 c - x2 s, x2 c + x1 s) is rounded ahead of the sum and which is fused into it: x2's in both sums in every form
+    of the attention kernel, x1's in the second sum of the re-tiled K.  With x2 = -x1 and equal factors the second value is nothing
+    but that rounding's error, and the other choice gives its negative.  Scores from these values alone, of a few units either way."""
+    request.addfinalizer(lambda: ops.set_variant("attn", 0))
+    g = gen(n + hd)
+    half = hd // 2
+    a = torch.randn((n, H, half), generator=g).to(torch.bfloat16)
+    x = torch.cat([a, -a], -1)
+    c = torch.rand((n, half), generator=g) * 0.5 + 0.5
+    cb = c[:, None] * -a.float()                            # fp32, rounded
+    e = (c[:, None].double() * a.double() + cb.double()).float()
+    x1 = (c[:, None].double() * a.double() - cb.double()).float()
+    rotated = torch.cat([x1, e], -1)
+    tables = c.to(dev()), c.to(dev())
+    flat = x.reshape(n, H * hd).to(dev())
+    # K as stored: chunk-major images [heads, tiles, hd / 8, 64 keys, 8]
+    img = ops.attention_pack_kv(flat, flat, H, hd, None, *tables)
+    nt = -(-n // 64)
+    kimg = img[:H * nt * hd * 128].view(torch.bfloat16).view(H, nt, hd // 8, 64, 8).permute(1, 3, 0, 2, 4).reshape(nt * 64, H, hd)[:n]
+    assert torch.equal(kimg.cpu(), torch.cat([x1, -e], -1).to(torch.bfloat16))
+    # key j: 2^25 in one channel of the second half
+    k = torch.zeros((n, H, hd))
+    k[torch.arange(n), :, half + torch.arange(n) % half] = 2.0 ** 25
+    v, vr = rand_bf16((n, H * hd), g)
+    img = ops.attention_pack_kv(k.reshape(n, H * hd).to(torch.bfloat16).to(dev()), v, H, hd)
+    ops.set_variant("attn", variant)
+    got = ops.attention_packed(flat, img, H, hd, None, *tables)
+    scale = torch.tensor(1.4426950408889634) / torch.tensor(float(hd)).sqrt()
+    q = (rotated * scale).to(torch.bfloat16).double().to(dev())
+    want = torch.empty((n, H, hd), dtype=torch.float64, device=dev())
+    for h in range(H):
+        want[:, h] = torch.softmax(q[:, h] @ k[:, h].double().to(dev()).t() * math.log(2.0), -1) @ vr.view(n, H, hd)[:, h].double().to(dev())
+    assert_close(got, want.reshape(n, H * hd), 0.999, 2e-2, f"rotation roundings variant {variant} hd {hd}")
+
+
 @pytest.mark.parametrize("n", [256, 300])
 def test_attention_shared_key_tiles_keep_infinities(n, request):
     """An infinite value reaches the rows that see it and nothing else, whatever the tile it sits in."""
