@@ -347,6 +347,7 @@ constexpr float kSafeLog2 = 60.0f;      // largest excess over the reference tha
 // and fold the whole factor into that rounding.
 constexpr int kMaxKm = 2048;            // key tiles that get a decision of their own (131,072 keys); longer sequences: one per head
 constexpr int kMaxSplit = 8;            // most key ranges a query block of the last round is split into
+constexpr float kLostNorm = 0x1p-70f;   // a norm whose squares vanish in fp32 (below 2^-149 each) is this much too small at most
 
 // What a lane needs for the Q fragments of its rows, as it lies in memory: channels 32ks + 8g .. +7 (g = lane / 16) of every
 // k-step, the rotary factors of the first half of the k-steps (the partner of a channel in k-step ks < KS/2 is the same
@@ -488,7 +489,7 @@ __device__ __forceinline__ void frag_norms(const bf16x8 (&qf)[QB][HD / 32], floa
                 qq = __builtin_amdgcn_fdot2_f32_bf16(v, v, qq, false);
             }
         }
-        qnorm[qb] = sqrtf(quarters_sum(qq));
+        qnorm[qb] = sqrtf(quarters_sum(qq)) + kLostNorm;
     }
 }
 
@@ -671,7 +672,7 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
         // a tile whose largest key norm is at most thr cannot raise any score of this row more than 2^kSafeLog2 above its
         // reference (1 % slack for the fp32 accumulation of the dot products and of the norms); a reference that is not
         // a number asks for the maxima everywhere
-        const float thr = (kSafeLog2 + m0) / (qnorm[qb] * 1.01f);
+        const float thr = (kSafeLog2 + m0) / (qnorm[qb] * 1.01f) - kLostNorm;
         need_always = need_always || __builtin_amdgcn_ballot_w64(thr != thr) != 0;
         t_lane = fminf(t_lane, thr);
 #pragma unroll
@@ -927,7 +928,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int qb = 0; qb < QB; ++qb) {
         float m0 = tile_row_max<QB>(s_a, qb);
         m0 = m0 == -INFINITY ? 0.0f : m0;      // rows that see nothing of this group's first tile: nothing to refer to
-        const float thr = (kSafeLog2 + m0) / (qnorm[qb] * 1.01f);
+        const float thr = (kSafeLog2 + m0) / (qnorm[qb] * 1.01f) - kLostNorm;
         need_always = need_always || __builtin_amdgcn_ballot_w64(thr != thr) != 0;
         t_wave = fminf(t_wave, thr);
 #pragma unroll

@@ -1087,6 +1087,24 @@ def test_rotations_round_as_written(variant, n, H, hd, request):
     assert_close(got, want.reshape(n, H * hd), 0.999, 2e-2, f"rotation roundings variant {variant} hd {hd}")
 
 
+@pytest.mark.parametrize("variant", [0, 1, 2, 3, 4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("query,key", [(1e-20, 1e30), (1e-22, 1e30), (1e-30, 1e38), (1e38, 1e-22), (1e38, 1e-30)])
+def test_attention_bounds_hold_where_squares_vanish(variant, hd, query, key, request):
+    """The bound that spares tiles their row maxima is |q| |k|.  The squares of one of them leave the range of fp32, but a key makes
+    scores of 10^7 and more: it must still be seen, and its value be the output of every row."""
+    request.addfinalizer(lambda: ops.set_variant("attn", 0))
+    n, H = 330, 2
+    g = gen(hd)
+    q = torch.full((n, H * hd), query, dtype=torch.bfloat16, device=dev())
+    k = torch.zeros((n, H * hd), dtype=torch.bfloat16, device=dev())
+    v, _ = rand_bf16((n, H * hd), g)
+    k[250] = key
+    img = ops.attention_pack_kv(k, v, H, hd)
+    ops.set_variant("attn", variant)
+    assert torch.equal(ops.attention_packed(q, img, H, hd), v[250].expand(n, -1))
+
+
 @pytest.mark.parametrize("n", [256, 300])
 def test_attention_shared_key_tiles_keep_infinities(n, request):
     """An infinite value reaches the rows that see it and nothing else, whatever the tile it sits in."""
