@@ -14,11 +14,8 @@ __device__ __forceinline__ void unpack8(const uint4& u, float* f) {
     f[4] = bf16lo(u.z); f[5] = bf16hi(u.z); f[6] = bf16lo(u.w); f[7] = bf16hi(u.w);
 }
 
-// 8 floats (|v| <= 448 after clamping) -> 8 e4m3 bytes
-__device__ __forceinline__ uint2 pack_e4m3x8(const float* f) {
-    float c[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) c[i] = fminf(fmaxf(f[i], -kE4M3Max), kE4M3Max);
+// 8 floats that round to at most 448 in size -> 8 e4m3 bytes
+__device__ __forceinline__ uint2 pack_e4m3x8(const float* c) {
     int lo = 0, hi = 0;
     lo = __builtin_amdgcn_cvt_pk_fp8_f32(c[0], c[1], lo, false);
     lo = __builtin_amdgcn_cvt_pk_fp8_f32(c[2], c[3], lo, true);
@@ -27,20 +24,22 @@ __device__ __forceinline__ uint2 pack_e4m3x8(const float* f) {
     return make_uint2((uint32_t)lo, (uint32_t)hi);
 }
 
-// f[i] / s to the last bit, for |f[i]| up to about 448 s: with inv the correctly rounded 1 / s, a product, its exact remainder and one
-// correction give the correctly rounded quotient (Markstein); three instructions per value instead of the ten of a division,
-// which at 16384 columns were half of a quantiser's time where its rows come from the memory-side cache.  Scales for which a
-// remainder could leave the normal range (or that are not finite) divide.
+// f[i] / s to the last bit, bounded as the codes are (values beyond the maxima that a caller brought come out as +-448): with inv
+// the correctly rounded 1 / s, a product, its exact remainder and one correction give the correctly rounded quotient (Markstein); three
+// instructions per value instead of the ten of a division, which at 16384 columns were half of a quantiser's time where its rows
+// come from the memory-side cache.  The bound, 449 s, stands ahead of the product, which must not overflow: the remainder of an
+// infinity is not a number.  Scales for which a remainder could leave the normal range (or that are not finite) divide.
 __device__ __forceinline__ void quotient8(float (&f)[8], float s, float inv) {
     if (s >= 0x1p-80f && s <= 0x1p80f) {
+        const float most = (kE4M3Max + 1.0f) * s;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const float q = f[i] * inv, over = __builtin_fmaf(q, s, -f[i]);      // (this sign: the correction of a -0 is -0)
+            const float v = __builtin_amdgcn_fmed3f(f[i], -most, most), q = v * inv, over = __builtin_fmaf(q, s, -v);      // (this sign: the correction of a -0 is -0)
             f[i] = __builtin_fmaf(-over, inv, q);
         }
     } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) f[i] = f[i] / s;
+        for (int i = 0; i < 8; ++i) f[i] = fminf(fmaxf(f[i] / s, -kE4M3Max), kE4M3Max);
     }
 }
 

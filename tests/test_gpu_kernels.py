@@ -1499,6 +1499,20 @@ def test_quantiser_quotients_are_divisions(exponent):
         assert torch.equal(sc.cpu(), s) and torch.equal(q.view(torch.uint8).cpu(), want.view(torch.uint8))
 
 
+@pytest.mark.parametrize("part", [2.0 ** -100, 2.0 ** -60, 0.25, 2.0 ** 60])
+def test_quantiser_bounds_values_beyond_the_given_maxima(part):
+    """Maxima a caller brings may lie below the row's (values are then clipped): +-448, infinities and values whose quotient overflows too."""
+    g = gen(3)
+    a = torch.randn((16, 4096), generator=g).to(torch.bfloat16)
+    a[:, 5], a[:, 6] = math.inf, -math.inf
+    a[:, 7], a[:, 8] = 3e38, -3e38
+    parts = torch.full((16, 4), part)
+    s = parts[:, 0] / 448.0
+    want = (a.float() / s[:, None]).clamp(-448.0, 448.0).to(torch.float8_e4m3fn).view(torch.uint8)
+    q, sc = ops.quant_rows_from_parts(a.to(dev()), parts.to(dev()))
+    assert torch.equal(sc.cpu(), s) and torch.equal(q.view(torch.uint8).cpu(), want)
+
+
 @pytest.mark.parametrize("top", [0.0, 2.0 ** -100, 1.0, 2.0 ** 100])
 def test_quantisers_keep_signed_zeros(top):
     """Zeros keep their sign in the codes, as under a division, whatever the row's scale; so do values that round to zero."""
