@@ -20,7 +20,6 @@ from typing import List, Optional, Sequence, Tuple
 import torch
 from torch import nn
 from torch.nn.modules.module import _has_any_global_hook as _any_module_hook
-from torch.utils._device import DeviceContext
 
 from . import ops, rotary
 from .config import DMConfig
@@ -433,22 +432,10 @@ def _as_is(m: nn.Module, cls: type) -> bool:
 _TENSORS = (torch.Tensor, nn.Parameter)
 
 
-def _function_modes() -> bool:
-    """A mode that sees or replaces calls of torch functions is on (``torch.device`` as a context only changes where they create)."""
-    n = torch._C._len_torch_function_stack()
-    return n > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(n))
-
-
 def _eager(t: torch.Tensor) -> bool:
-    """A plain tensor in plain eager execution, where a kernel that takes pointers may stand in for torch operators: no
-    compilation, tracing, function or dispatch mode that has to see the operators, no subclass whose storage is not the value, no
-    forward-mode derivative or function transform (``torch.func``; a tensor that carries a tangent has no mark of its own to ask
-    for), and no autocast, which chooses the type a linear layer computes in and returns."""
-    if torch.compiler.is_compiling():
-        return False
-    return (type(t) in _TENSORS and torch._C._len_torch_dispatch_stack() == 0 and torch._C._get_tracing_state() is None
-            and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
-            and not torch.is_autocast_enabled("cuda") and not _function_modes())
+    """A plain tensor in plain eager execution, where a kernel that takes pointers may stand in for torch operators: no subclass
+    whose storage is not the value, and no autocast, which chooses the type a linear layer computes in and returns."""
+    return ops.operators_unseen() and type(t) in _TENSORS and not torch.is_autocast_enabled("cuda")
 
 
 def _plain(lin: nn.Module, device: torch.device, dtype: torch.dtype) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:

@@ -10,6 +10,7 @@ import functools
 from typing import Optional, Sequence, Tuple
 
 import torch
+from torch.utils._device import DeviceContext
 
 from . import _lib
 from ._lib import EPI_GATE_RESIDUAL, EPI_GATE_RESIDUAL_F32, EPI_NONE, EPI_ROPE_QK, EPI_SWIGLU
@@ -60,6 +61,22 @@ def _f32vec(t: Optional[torch.Tensor], name: str, n: int) -> int:
     if not t.is_cuda:
         raise RuntimeError(f"{name} must live on the GPU (the HIP path has no CPU fallback)")
     return t.data_ptr()
+
+
+def _function_modes() -> bool:
+    """A mode that sees or replaces calls of torch functions is on (``torch.device`` as a context only changes where they create)."""
+    n = torch._C._len_torch_function_stack()
+    return n > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(n))
+
+
+def operators_unseen() -> bool:
+    """Nothing but torch itself would see an operator called now: no compilation, tracing, function or dispatch mode, and no
+    forward-mode derivative or function transform (``torch.func``; a tensor that carries a tangent has no mark of its own to ask for)."""
+    if torch.compiler.is_compiling():
+        return False
+    return (torch._C._len_torch_dispatch_stack() == 0 and torch._C._get_tracing_state() is None
+            and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
+            and not _function_modes())
 
 
 _OP_TIMER = None     # None, or the list that collects (category, start event, end event) while timing is on
@@ -772,14 +789,15 @@ def cfg_step(x: torch.Tensor, v_cond: torch.Tensor, v_uncond: Optional[torch.Ten
 
 def copy_runs(dsts: Sequence[torch.Tensor], srcs: Sequence[torch.Tensor]) -> None:
     """``dst.copy_(src)`` for every pair, in order.  Contiguous GPU tensors of one type, up to 16 MB each, take one launch between
-    them; whatever else ``copy_`` accepts goes through it.  Tokens and a timestep, two copies against one launch: 2 MB 4.1 / 2.2 us,
-    16 MB 5.9 / 4.9, 32 MB 12.0 / 11.6."""
-    todo = []
+    them; whatever else ``copy_`` accepts goes through it, and everything where somebody would see it.  Tokens and a timestep, two
+    copies against one launch: 2 MB 4.1 / 2.2 us, 16 MB 5.9 / 4.9, 32 MB 12.0 / 11.6."""
+    todo, plain = [], operators_unseen()
     for d, s in zip(dsts, srcs):
-        if (type(s) is torch.Tensor and type(d) is torch.Tensor and s.is_cuda and s.device == d.device and s.dtype == d.dtype
+        if (plain and type(s) is torch.Tensor and type(d) is torch.Tensor and s.is_cuda and s.device == d.device and s.dtype == d.dtype
                 and s.shape == d.shape and s.is_contiguous() and d.is_contiguous() and not (s.requires_grad or d.requires_grad)
-                and not (s.is_neg() or s.is_conj()) and s.nbytes <= 1 << 24 and d.device.index == torch.cuda.current_device()):
-            todo.append((s.data_ptr(), d.data_ptr(), s.nbytes))
+                and not (s.is_neg() or s.is_conj() or d.is_inference()) and s.nbytes <= 1 << 24
+                and d.device.index == torch.cuda.current_device()):
+            todo.append((s, d))
             if len(todo) == 8:
                 _copy_runs(todo)
                 todo = []
@@ -793,9 +811,10 @@ def copy_runs(dsts: Sequence[torch.Tensor], srcs: Sequence[torch.Tensor]) -> Non
 def _copy_runs(todo) -> None:
     n = len(todo)
     if n:
-        rc = _lib.load().cdm_copy_runs((C.c_void_p * n)(*[s for s, _, _ in todo]), (C.c_void_p * n)(*[d for _, d, _ in todo]),
-                                       (C.c_int64 * n)(*[b for _, _, b in todo]), n, _stream())
+        rc = _lib.load().cdm_copy_runs((C.c_void_p * n)(*[s.data_ptr() for s, _ in todo]), (C.c_void_p * n)(*[d.data_ptr() for _, d in todo]),
+                                       (C.c_int64 * n)(*[s.nbytes for s, _ in todo]), n, _stream())
         _lib.check(rc, "cdm_copy_runs")
+        torch.autograd.graph.increment_version([d for _, d in todo])
 
 
 _ATTN_TIMER = None

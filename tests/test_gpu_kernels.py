@@ -1803,6 +1803,43 @@ def test_copy_runs_keeps_the_order_and_what_copies_do():
     ops.copy_runs([], [])
 
 
+def test_copy_runs_is_seen_where_copies_are():
+    """Modes see ``copy_``, a tangent goes along, the targets' version counters rise, and what may not be written stays refused."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    src, dst = [torch.randn(64, device=dev()) for _ in range(2)], [torch.zeros(64, device=dev()) for _ in range(2)]
+    seen = []
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func.overloadpacket.__name__)
+            return func(*args, **(kwargs or {}))
+
+    for mode in (Functions, Dispatch):
+        with mode():
+            ops.copy_runs(dst, src)
+        assert seen.count("copy_") == 2
+        seen.clear()
+    before = [d._version for d in dst]
+    ops.copy_runs(dst, src)
+    assert [d._version for d in dst] == [v + 1 for v in before] and all(torch.equal(d, s) for d, s in zip(dst, src))
+    with torch.autograd.forward_ad.dual_level():
+        out = torch.zeros(64, device=dev())
+        ops.copy_runs([out], [torch.autograd.forward_ad.make_dual(src[0], src[1])])
+        assert torch.equal(torch.autograd.forward_ad.unpack_dual(out).tangent, src[1])
+    with torch.inference_mode():
+        kept = torch.zeros(64, device=dev())
+        ops.copy_runs([kept], src[:1])
+    with pytest.raises(RuntimeError):
+        ops.copy_runs([kept], src[1:])
+
+
 @pytest.mark.parametrize("variant", [0, 1, 2, 3, 4, 5, 6, 7])
 @pytest.mark.parametrize("n,N,K,segs,first,rows", [
     (1, 8, 128, [(0, 1)], 0, 1), (70, 264, 256, [(0, 37), (37, 33)], 37, 33), (300, 512, 384, [(0, 100), (120, 180)], 90, 100),
