@@ -1781,6 +1781,19 @@ def test_copy_runs(sizes, shift):
         assert torch.equal(d[8:8 + n], s[shift:shift + n]) and bool((d[:8] == 7).all()) and bool((d[8 + n:] == 7).all())
 
 
+def test_copy_runs_leaves_long_misaligned_runs_to_copies(monkeypatch):
+    """A run off its 16-byte alignment goes by single bytes: above 4 MB it is torch's, an aligned one from 16 MB on."""
+    launched = []
+    inner = ops._copy_runs
+    monkeypatch.setattr(ops, "_copy_runs", lambda todo: launched.extend(r[2] for r in todo) or inner(todo))
+    for shift, n, own in ((0, 1 << 23, True), (0, (1 << 23) + 8, False), (1, 1 << 21, True), (1, (1 << 21) + 1, False), (4, 1 << 23, False)):
+        src = torch.randint(-30000, 30000, (n + 8,), dtype=torch.int16, device=dev())[shift:shift + n]
+        for d, s in ((torch.zeros(n, dtype=torch.int16, device=dev()), src), (torch.zeros(n + 8, dtype=torch.int16, device=dev())[shift:shift + n], src.clone())):
+            launched.clear()
+            ops.copy_runs([d], [s])
+            assert launched == ([2 * n] if own else []) and torch.equal(d, s), (shift, n)
+
+
 def test_copy_runs_keeps_the_order_and_what_copies_do():
     """A run that reads an earlier run's target, one that overwrites an earlier one's source, a run onto itself, and everything that
     torch's copy takes besides: another type, strides, host memory, sizes that broadcast.  A run that overlaps its own target is
