@@ -668,7 +668,8 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
     if (pre_rag_tile == 0) mask_scores<QB>(s_a, pre_valid, lane);
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
-        const float m0 = tile_row_max<QB>(s_a, qb);      // exact first reference: every row has at least one finite score
+        float m0 = tile_row_max<QB>(s_a, qb);            // exact first reference
+        m0 = m0 == -INFINITY ? 0.0f : m0;                // (a first tile, or a key range's, of infinite keys: nothing to refer to)
         // a tile whose largest key norm is at most thr cannot raise any score of this row more than 2^kSafeLog2 above its
         // reference (1 % slack for the fp32 accumulation of the dot products and of the norms); a reference that is not
         // a number asks for the maxima everywhere
@@ -755,7 +756,7 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
         const float l_tot = quarters_sum(l_run[qb]);
-        const float inv = 1.0f / l_tot;
+        const float inv = unit >= 0 && l_tot == 0.0f ? 0.0f : 1.0f / l_tot;      // (a range of infinite keys has no say in the row)
         float amax = 0.0f;
         if (unit >= 0 && p.part_f32) {
             float* orow = (float*)p.part_o + ((int64_t)unit * BMQ + wave * (32 * QS) + qb * 16 + r16) * HD + 4 * g4;

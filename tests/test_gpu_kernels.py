@@ -1121,6 +1121,88 @@ def test_attention_shared_key_tiles_keep_infinities(n, request):
     assert torch.isinf(got[:, 5]).all() and bool(torch.isfinite(got[:, 6:]).all())
 
 
+def _softmax64(q, k, v, H, hd):
+    """Attention in 64 bits by products and sums alone, so that infinities and NaN go where arithmetic sends them: [n, H * hd]."""
+    n = q.shape[0]
+    q, k, v = (t.double().view(-1, H, hd) for t in (q, k, v))
+    out = torch.empty((n, H, hd), dtype=torch.float64, device=q.device)
+    for h in range(H):
+        for r in range(0, n, 64):
+            p = torch.softmax((q[r:r + 64, None, h] * k[None, :, h]).sum(-1) * hd ** -0.5, -1)
+            out[r:r + 64, h] = (p[:, :, None] * v[None, :, h]).sum(1)
+    return out.reshape(n, H * hd)
+
+
+def _assert_same_specials(got, want, what):
+    got = got.double()
+    for pred in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(pred(got), pred(want)), (what, pred.__name__, int(pred(got).sum()), int(pred(want).sum()))
+    m = torch.isfinite(want)
+    assert bool(m.any()) and ((got - want)[m].abs().max() <= 1e-2 * want[m].abs().max()), what
+
+
+@pytest.mark.parametrize("variant", [0, 1, 2, 3, 4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("n,hd", [(300, 64), (300, 128), (830, 64), (830, 128)])
+def test_attention_forms_keep_infinities_and_nans(variant, n, hd, request):
+    """Values, single keys, a whole tile of keys and query rows that hold infinities or NaN, at places that fall to different groups of
+    waves: every form leaves what the arithmetic in 64 bits does, and the other rows as they are.  (Logits of a few units: the
+    roundings of Q, P and O stay within 1e-2 of the largest value.)"""
+    request.addfinalizer(lambda: ops.set_variant("attn", 0))
+    g, H = gen(n + hd), 2
+    q0, k0, v0 = (rand_bf16((n, H * hd), g)[0] for _ in range(3))
+    q0 = torch.where(q0 == 0, torch.ones_like(q0), q0)      # (an infinite key makes infinities of every row, not NaN)
+    def case(what):
+        q, k, v = q0.clone(), k0.clone(), v0.clone()
+        if what == "values":
+            v[n - 1, 5], v[70, 9], v[3, 11], v[200, hd + 2] = math.inf, -math.inf, math.nan, math.inf
+        elif what == "key":
+            k[150, 3], k[n - 1, hd + 1] = math.inf, -math.inf
+        elif what == "query":
+            q[7, 2], q[100, hd], q[n - 1, 4] = math.nan, math.inf, -math.inf
+        else:
+            k[64 * what:64 * what + 64, 0] = math.inf
+        return q, k, v
+    for what in ("values", "key", "query", 0, 1, 2, 3):
+        q, k, v = case(what)
+        img = ops.attention_pack_kv(k, v, H, hd)
+        ops.set_variant("attn", variant)
+        got = ops.attention_packed(q, img, H, hd)
+        ops.set_variant("attn", 0)
+        _assert_same_specials(got, _softmax64(q, k, v, H, hd), (variant, what))
+
+
+@pytest.mark.parametrize("n,H,Hkv,hd", [(2305, 32, 8, 128), (4225, 16, 16, 64), (9372, 16, 4, 128)])
+def test_attention_split_keeps_infinities_and_nans(n, H, Hkv, hd):
+    """The same where the last round's blocks are cut by key range (fp32 partial results; bf16 ones in the last shape): rows of the
+    tail, with infinite values, keys, whole first tiles of a range and whole ranges."""
+    g = gen(n)
+    q0, k0, v0 = (rand_bf16((n, h * hd), g, s)[0] for h, s in ((H, 1.0), (Hkv, 0.5), (Hkv, 1.0)))
+    q0 = torch.where(q0 == 0, torch.ones_like(q0), q0)
+    scratch = torch.empty((ops.attn_split_scratch_bytes(n, H, hd),), dtype=torch.uint8, device=dev())
+    assert scratch.numel() > 0
+    rows, h = slice(n - 60, n), H - 1                       # (the last query block of the last head is in every XCD's tail)
+    kv = h // (H // Hkv)
+    cols = slice(kv * hd, kv * hd + hd)
+    nt = -(-n // 64)
+    for what in ("values", "key", "query", "range", nt // 2, nt // 4, 0):
+        q, k, v = q0.clone(), k0.clone(), v0.clone()
+        if what == "values":
+            v[n - 1, kv * hd + 5], v[70, kv * hd + 9], v[n // 2, kv * hd + 11] = math.inf, -math.inf, math.nan
+        elif what == "key":
+            k[n // 3, kv * hd + 3] = math.inf
+        elif what == "query":
+            q[n - 7, h * hd + 2], q[n - 3, h * hd] = math.nan, math.inf
+        elif what == "range":
+            k[nt // 2 * 64:, kv * hd] = math.inf
+        else:
+            k[64 * what:64 * what + 64, kv * hd] = math.inf
+        img = ops.attention_pack_kv(k, v, Hkv, hd)[:ops.attn_workspace_bytes(n, Hkv, hd)]
+        want = _softmax64(q[rows, h * hd:h * hd + hd], k[:, cols], v[:, cols], 1, hd)
+        for scr in (None, scratch):
+            got = ops.attention_packed(q, img, H, hd, n_kv_heads=Hkv, split_scratch=scr)
+            _assert_same_specials(got[rows, h * hd:h * hd + hd], want, (what, scr is not None))
+
+
 @pytest.mark.parametrize("variant", [0, 1])
 @pytest.mark.parametrize("n,H,hd,sections", [(300, 2, 128, (32, 48, 48)), (130, 3, 64, (16, 24, 24))])
 def test_attention_with_rope_in_registers(n, H, hd, sections, variant):
