@@ -275,7 +275,7 @@ def residual_gemm_(x: torch.Tensor, a: torch.Tensor, ws: Sequence[torch.Tensor],
                    gates: Sequence[Optional[torch.Tensor]], rows16: torch.Tensor, first: int) -> None:
     """x += gate * (a @ w^T) per segment on fp32 rows, with the new rows ``first`` .. of x left in ``rows16`` as bf16 too."""
     n_seg, (M, N), K = len(segments), x.shape, a.shape[1]
-    if a.shape[0] != M or any(w.shape != (N, K) or w.stride(0) != ws[0].stride(0) for w in ws):
+    if a.shape[0] != M or ws[0].shape[0] != N or ws[0].shape[1] < K or any(w.shape != ws[0].shape or w.stride(0) != ws[0].stride(0) for w in ws):
         raise ValueError("shape mismatch")
     if rows16.shape[1] != N or first < 0 or first + rows16.shape[0] > M or any(s < 0 or l < 0 or s + l > M for s, l in segments):
         raise ValueError("rows out of range")

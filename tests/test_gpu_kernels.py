@@ -1961,6 +1961,17 @@ def test_residual_gemm_leaves_bf16_rows(n, N, K, segs, first, rows, variant, req
     assert torch.equal(rows16, torch.where(inside, want[first:first + rows].to(torch.bfloat16), torch.full_like(rows16, 7.0)))
 
 
+def test_residual_gemm_of_wider_weights():
+    """Weights with more columns than the rows have: their first K columns, as a grouped linear takes them."""
+    g = gen(9)
+    a, w, x = rand_bf16((200, 512), g)[0], [rand_bf16((256, 640), g, 0.05)[0] for _ in range(2)], torch.randn((200, 256), generator=g).to(dev())
+    segs, gates, want = [(0, 70), (70, 130)], [None, None], x.clone()
+    ops.grouped_gemm(a, w, segs, epilogue="gate_residual", residual=want, gates=gates, out=want)
+    rows16 = torch.empty((130, 256), dtype=torch.bfloat16, device=dev())
+    ops.residual_gemm_(x, a, w, segs, gates, rows16, 70)
+    assert torch.equal(x, want) and torch.equal(rows16, want[70:].to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("kw", [dict(), dict(n_text=37), dict(n_text=64, n_action=6, n_branches=3)])
 def test_stack_video_rows_are_the_streams(kw):
     """A stack's video rows - a recorded one's are left by its last product - are the rows of the stream it returns, rounded; so are those
