@@ -183,6 +183,27 @@ def test_gemm_cut_along_k(lens, N, K, epi):
         assert bool((err <= tol).all()), (i, err.max().item())
 
 
+@pytest.mark.parametrize("M,parts", [(333, 5), (528, 3)])
+def test_gemm_in_an_odd_number_of_ranges(M, parts):
+    """Five and three ranges of 256 k-tiles, cut between pairs of tiles.  Sums of a range are shorter than a whole row's, so that
+    against 64 bits they are no further off than the uncut launch's (2-norm over 10^6 values; what chance moves it by is in the
+    fourth digit)."""
+    g, N, K = gen(M), 4096, 16384
+    a = torch.randn((M, K), generator=g).to(dev(), torch.bfloat16)
+    w = (torch.randn((N, K), generator=g) * K ** -0.5).to(dev(), torch.bfloat16)
+    r = torch.randn((M, N), generator=g).to(dev())
+    assert ops.gemm_scratch_bytes((M,), N, K, ops.EPI_GATE_RESIDUAL_F32) == parts * M * N * 4
+    want = a.double() @ w.double().t() + r.double()
+    cut = ops.gemm(a, w, epilogue="gate_residual", residual=r, out=torch.empty_like(r))
+    prev = ops.set_variant("gemm", 5)                       # one shape for the whole of K
+    try:
+        whole = ops.gemm(a, w, epilogue="gate_residual", residual=r, out=torch.empty_like(r))
+    finally:
+        ops.set_variant("gemm", prev)
+    err = lambda o: ((o.double() - want).norm() / want.norm()).item()
+    assert not torch.equal(cut, whole) and err(cut) <= 1.01 * err(whole), (err(cut), err(whole))
+
+
 @pytest.mark.parametrize("K", [512, 8192])
 def test_grouped_gemm_of_wider_weights(K):
     """Weights with more columns than the rows have: their first K columns, cut along K or not."""
