@@ -474,7 +474,8 @@ __device__ __forceinline__ void finish_q(const PackedParams& p, const QRows<HD, 
     else finish_rows<HD, QB, false>(p, r, qf);
 }
 
-// The norms of the scaled, rotated, rounded rows: for a bound with 1 % slack, so two products per instruction
+// The norms of the scaled, rotated, rounded rows.  Sums of fp32 products, as the bits of a launch hang on them where a tile's bound
+// comes close to the limit (with v_dot2_f32_bf16, half the instructions, two blocks over 56,832 tokens moved by 2.5e-5)
 template <int HD, int QB>
 __device__ __forceinline__ void frag_norms(const bf16x8 (&qf)[QB][HD / 32], float (&qnorm)[QB]) {
 #pragma unroll
@@ -484,10 +485,7 @@ __device__ __forceinline__ void frag_norms(const bf16x8 (&qf)[QB][HD / 32], floa
         for (int ks = 0; ks < HD / 32; ++ks) {
             const u32x4 u = __builtin_bit_cast(u32x4, qf[qb][ks]);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const bf16x2 v = __builtin_bit_cast(bf16x2, u[j]);
-                qq = __builtin_amdgcn_fdot2_f32_bf16(v, v, qq, false);
-            }
+            for (int j = 0; j < 4; ++j) { const float x = bf16lo(u[j]), y = bf16hi(u[j]); qq += x * x + y * y; }
         }
         qnorm[qb] = sqrtf(quarters_sum(qq)) + kLostNorm;
     }
