@@ -1275,7 +1275,8 @@ inline int64_t kmax_bytes(int64_t n_tokens, int n_heads) {      // one float per
 // the cheapest by their estimate, and the partial results are fp32 (such launches had no partial results before).  One pass
 // against the split, us: 32 heads x 128, 2304 tokens (32 + 4 workgroups per XCD) 120 / 98.6, 2560 (32 + 8) 131 / 111, 3072 (32 + 16)
 // 152 / 144; 16 heads x 128, 4352 (32 + 2) 204 / 148, 5000 (32 + 8) 234 / 183, 6144 (32 + 16) 279 / 250; 16 x 64, 4352 132 / 91.6,
-// 6144 180 / 153.  20 or more left over (32 x 128, 3328 tokens: 163 / 199), or no whole round at all, lose.
+// 6144 180 / 153.  More than 16 left over are never cut (two parts of each fill two rounds, finer ones miss the bound; 20, at 32 x
+// 128, 3328 tokens: 163 / 199), nor is a launch without a whole round.
 struct SplitPlan { int split, tail; int64_t bytes; int f32; };
 inline SplitPlan split_plan(int64_t n_tokens, int n_heads, int head_dim, int64_t causal_prefix) {
     SplitPlan none{1, 0, 0, 0};

@@ -1,17 +1,17 @@
 // The "NT" GEMM C[M,N] = A[M,K] . W[N,K]^T for launches that 256 x 256 tiles (gemm.hip) leave the chip idle for: a text
 // run, an action run, one image, small models.  Same operands, same order of every sum (a row of C comes out bit for bit
 // the same whatever the tile), same epilogues; smaller output tiles.  The exception are launches cut along K (best_split: bf16,
-// plain and residual epilogues): their ranges' sums are added last, and as the number of rows decides about the cut, the last
-// bits of a row depend on how many rows share the call.
+// plain and residual epilogues, between pairs of k-tiles): their ranges' sums are added last, and as the number of rows decides
+// about the cut, the last bits of a row depend on how many rows share the call.
 //
 // What bounds it: the feed of one CU.  With weights that no cache holds (every weight of a prompt is read exactly once) a CU
 // takes 57 - 72 bytes per ns into its LDS whatever the tile (0.40 us per k-tile at 64 x 128, 0.53 at 128 x 128), 78 with the
 // weights in the memory-side cache; a load-only loop over L2-resident rows reaches 110 - 137.  Removing the loads from the
 // 64 x 128 loop takes a third off, removing half of its LDS reads nothing.  So: all the LDS a CU has goes into ring stages
 // (over 100 KB in flight), loads go out one behind every few MFMAs, and the shape is chosen so that every CU has a tile.
-// At M = 512, K = 16384, N = 4096 (bf16, cold weights) the 64 x 128 tile takes 113 us where 32 tiles of 256 x 256 took 287
-// (four ranges of K in 128 x 256 tiles: 82, see best_split);
-// M = 512, N = 12288, K = 4096 (QKV with images): 64 us against 85; M = 64, N = 4096, K = 4096: 14 us against 84.
+// At M = 512, K = 16384, N = 4096 (bf16, cold weights) the 64 x 128 tile takes 111 us where 32 tiles of 256 x 256 take 285
+// (four ranges of K in 128 x 256 tiles: 79, see best_split);
+// M = 512, N = 12288, K = 4096 (QKV with images): 66 us against 85; M = 64, N = 4096, K = 4096: 12.5 us against 84.
 //
 // Layout: eight waves (four for the 32 x 32 tile) in a WM x WN grid, v_mfma_f32_16x16x32_bf16 / 16x16x128_f8f6f4, W
 // fragment first, so that a lane's accumulator quad is four consecutive columns of one output row.  The epilogue
@@ -27,7 +27,7 @@ namespace {
 
 constexpr int kLds = 160 * 1024;
 constexpr int kMaxSplitK = 8;      // most ranges of K
-constexpr int kKeyNorms = 64 / 8 * 2;      // what pack_piece leaves of a piece's 64 keys: a float per eight keys and head (up to two)
+constexpr int kKeyNorms = 64 / 8 * 2;      // floats that pack_keys leaves of 64 keys: one per eight keys and head (up to two); KSQ holds TM / 64 such pieces
 
 template <int TM, int TN, int WM, int WN>
 struct Geo {
@@ -421,6 +421,8 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
             load_residual<EPI>(p, row < tile.m_end ? row : tile.m_end - 1, cc, res[it]);
         }
     }
+    // (128 x 256 QKV tiles run out of scalar registers from here on: 20, with e4m3 operands 26, go into a vector register's lanes once behind the
+    // k-loop and come back once per 128 columns, some 60 instructions of a wave; the k-loop has none of it)
     KeyTables<TM / 64 ? TM / 64 : 1> tables;
     if (EPI == CDM_EPI_QKV_PACK && n0 + TN > p.d_q && n0 < p.d_q + p.d_kv) request_tables(p, tile, tid, tables);
 
@@ -568,12 +570,18 @@ namespace {
 // Measured with weights that no cache holds:
 //     tile       fixed  per k-tile   example (M = 512, N = 4096, K = 16384, bf16: us, at the 256 x 256 tile 287)
 //     256 x 256   18    1.08 / 1.37
-//     128 x 256   10    0.64 / 0.84  211
-//     128 x 128    7    0.50 / 0.53  142
-//      64 x 128    5    0.40         113
-//      64 x 64     4.5  0.25         138 (two rounds)
-//      32 x 32     4.5  0.14         220 (eight tiles per CU)
+//     128 x 256   10    0.64 / 0.84  204
+//     128 x 128    7    0.50 / 0.53  139
+//      64 x 128    5    0.40         111
+//      64 x 64     4.5  0.25         136 (two rounds)
+//      32 x 32     4.5  0.14         240 (eight tiles per CU)
 // e4m3 k-tiles take the same time (twice the elements per 128 bytes at twice the matrix rate).
+// The fixed parts are of launches that stand alone; back to back in a recorded graph, fitted over 250 launches, they are 9, 5.4, 4.6, 3.5, 3.0 and
+// 2.5 us, the slopes within 12 % of the table's.  What counts is which shape comes out: over 16 layers of K = 1024 .. 16384 and 16
+// row counts from 16 to 1637, weights that no cache holds, 240 of 256 choices are within 4 % of the fastest whole launch or ahead of it, the rest
+// mostly 64 x 64 tiles where 32 x 32 are up to 13 % faster (M = 512, N = K = 1024: 7.4 / 6.5 us); the farthest is SwiGLU to 4096 at K = 1024,
+// M = 1300 (31.9 / 26.0).  The fitted figures in the table's place set those right and others wrong (M = 96, N = K = 4096: 16.6 us cut,
+// 19.7 whole): the time hangs on the weights' bytes per CU as well, which the estimate does not see.
 struct ShapeCost { TileShape s; double fixed, half, full; };
 const ShapeCost kShapes[] = {{{256, 256, 4, 2}, 18.0, 1.08, 1.37}, {{128, 256, 2, 4}, 10.0, 0.64, 0.84},
                              {{128, 128, 4, 2}, 7.0, 0.50, 0.53},  {{64, 128, 2, 4}, 5.0, 0.40, 0.40},
@@ -607,11 +615,11 @@ Best best_shape(const int64_t* rows, int n_seg, int64_t N, double kt, int epilog
 // Launches with few tiles and a long K: every tile once per range of K, fp32 sums in scratch memory and a pass over them
 // (finish_split_kernel: its launch, and the sums written and read at about 8 TB/s).  Whole launch against the cut one, us, fp32
 // residual, weights that no cache holds:
-//     N = 4096, K = 16384:  M = 128  74.8 / 56.2   256  75.0 / 59.7   512  114 / 81.9   768  148 / 125   1024  153 / 135
-//     N = 2048, K = 8192:   M = 64   20.8 / 15.8   256  35.6 / 24.4   512  35.7 / 32.1
-//     N = 4096, K = 4096:   M = 128  22.0 / 19.2;  N = 1024, K = 4096: M = 512 20.0 / 18.5
-// Cut launches stream the weights at 2.4 - 3 TB/s at most (M = 16 and 64 at K = 16384: 55 us against 39 and 46 whole), so such
-// a rate bounds the estimate.  Against 64 bits the sums are closer than uncut ones (K = 16384: 2.8e-7 in four ranges, 5.8e-7).
+//     N = 4096, K = 16384:  M = 128  71.2 / 49.8   256  73.2 / 56.5   512  111 / 79.1   768  140 / 122   1024  146 / 133
+//     N = 2048, K = 8192:   M = 64   20.2 / 16.3   256  33.3 / 23.8   512  35.5 / 31.8
+//     N = 4096, K = 4096:   M = 128  19.5 / 18.3;  N = 1024, K = 4096: M = 512 16.8 / 18.0
+// (with weights that a cache holds the cuts of shorter sums lose: N = 1024, K = 4096, M = 512 14.8 / 17.6; N = 2048, K = 4096, M = 256 14.5 / 17.7).
+// Cut launches stream the weights at 2.4 - 3 TB/s at most (M = 96 at K = 16384: 45 us), so such a rate bounds the estimate.  Against 64 bits the sums are closer than uncut ones (K = 16384: 2.8e-7 in four ranges, 5.8e-7).
 struct SplitK { TileShape s; int parts; double us; int64_t bytes; };
 SplitK best_split(const GemmParams& p, const int64_t* rows, double kt, int epilogue) {
     SplitK best{{}, 1, 1e30, 0};
@@ -668,8 +676,8 @@ int32_t launch_split_k(GemmParams& p, int epilogue, const GemmPlan& plan, void* 
 
 // How a launch is cut: one shape for all of it, or - where 256 x 256 tiles end in a poorly filled round - whole rounds of
 // those tiles and a second launch for the rows behind them in the shape that suits it.  N = 4096, one launch of 256 x 256
-// tiles against the cut: M = 4352 (1.06 rounds) 184 -> 141 us at K = 4096, 667 -> 459 at K = 16384; M = 9000 (2.25) 295 ->
-// 264 and 1043 -> 907; M = 14080 (3.44) 427 -> 414 and 1453 -> 1381; M = 11000 (2.69) keeps one launch.
+// tiles against the cut: M = 4352 (1.06 rounds) 187 -> 138 us at K = 4096, 673 -> 475 at K = 16384; M = 9000 (2.25) 314 ->
+// 278 and 1076 -> 929; M = 14080 (3.44) 431 -> 412 and 1486 -> 1416; M = 11000 (2.69) keeps one launch.
 // The second launch costs about 5 us of its own (it starts when the first has drained).
 GemmPlan plan_gemm(const GemmParams& p, int epilogue, bool fp8, int64_t scratch_bytes) {
     const int v = cdm_get_variant(1);
