@@ -797,7 +797,8 @@ def copy_runs(dsts: Sequence[torch.Tensor], srcs: Sequence[torch.Tensor]) -> Non
     for d, s in zip(dsts, srcs):
         if (type(s) is torch.Tensor and type(d) is torch.Tensor and s.get_device() == device and d.get_device() == device
                 and s.dtype == d.dtype and s.shape == d.shape and s.is_contiguous() and d.is_contiguous()
-                and not (s.requires_grad or d.requires_grad or s.is_neg() or s.is_conj() or d.is_inference())):
+                and not (s.requires_grad or d.requires_grad or s.is_neg() or s.is_conj())
+                and (not d.is_inference() or torch.is_inference_mode_enabled())):
             a, b, n = s.data_ptr(), d.data_ptr(), s.nbytes
             if n <= (1 << 22 if (a | b) & 15 else 1 << 24):
                 todo.append((a, b, n, d))

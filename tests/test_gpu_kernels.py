@@ -1919,7 +1919,7 @@ def test_copy_runs_keeps_the_order_and_what_copies_do():
     ops.copy_runs([], [])
 
 
-def test_copy_runs_is_seen_where_copies_are():
+def test_copy_runs_is_seen_where_copies_are(monkeypatch):
     """Modes see ``copy_``, a tangent goes along, the targets' version counters rise, and what may not be written stays refused."""
     from torch.overrides import TorchFunctionMode
     from torch.utils._python_dispatch import TorchDispatchMode
@@ -1949,9 +1949,17 @@ def test_copy_runs_is_seen_where_copies_are():
         out = torch.zeros(64, device=dev())
         ops.copy_runs([out], [torch.autograd.forward_ad.make_dual(src[0], src[1])])
         assert torch.equal(torch.autograd.forward_ad.unpack_dual(out).tangent, src[1])
+    launched, inner = 0, ops._copy_runs
+
+    def launch(todo):
+        nonlocal launched
+        launched += bool(todo)
+        inner(todo)
+    monkeypatch.setattr(ops, "_copy_runs", launch)
     with torch.inference_mode():
         kept = torch.zeros(64, device=dev())
-        ops.copy_runs([kept], src[:1])
+        ops.copy_runs([kept, dst[0]], [src[0], src[1]])
+        assert launched == 1 and torch.equal(kept, src[0]) and torch.equal(dst[0], src[1])
     with pytest.raises(RuntimeError):
         ops.copy_runs([kept], src[1:])
 
