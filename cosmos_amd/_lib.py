@@ -11,6 +11,8 @@ library instead (tests and measurement aids only).
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -18,6 +20,7 @@ from . import build as _build
 
 _LOCK = threading.Lock()
 _LIB = None
+_HOST = None                               # the extension module of the argument checks
 _XLIB = None                               # the cross-check build, loaded on the first set_variant
 _VARIANTS = {"attn": 0, "gemm": 0}         # what set_variant last selected
 
@@ -104,7 +107,23 @@ def _bind(path: str, signatures: dict):
     for name, (res, args) in signatures.items():
         fn = getattr(lib, name)     # AttributeError here = the library does not export the ABI
         fn.restype, fn.argtypes = res, args
+    host = _host_module()
+    import torch
+    lib.host = host.Host(lib._handle, torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream)      # the same launchers behind native argument checks (csrc/host.cpp)
     return lib
+
+
+def _host_module():
+    """The extension module of the argument checks (built first if it is missing or stale; there is no way around it)."""
+    global _HOST
+    if _HOST is None:
+        import torch      # noqa: F401      (its libraries are what the module is linked against)
+        _fresh(_build.HOST_PATH)
+        loader = importlib.machinery.ExtensionFileLoader("_host", _build.HOST_PATH)
+        spec = importlib.util.spec_from_file_location("_host", _build.HOST_PATH, loader=loader)
+        _HOST = importlib.util.module_from_spec(spec)
+        loader.exec_module(_HOST)
+    return _HOST
 
 
 def _fresh(path: str) -> None:

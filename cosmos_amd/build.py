@@ -13,6 +13,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
@@ -27,6 +28,9 @@ SOURCES = ["api.hip", "norm.hip", "rope.hip", "gemm.hip", "gemm_tile.hip", "attn
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Xclang", "-target-feature", "-Xclang",
          "-packed-fp32-ops", "-Wno-unused-command-line-argument"]
 CROSSCHECK_FLAGS = ["-DCDM_CROSSCHECK"]
+# the Python side's argument checks and calls (an extension module of the host compiler's, against torch's headers)
+HOST_PATH = os.path.join(LIB_DIR, "_host.so")
+HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden"]
 
 
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
@@ -37,13 +41,13 @@ def source_hash() -> str:
     """16 hex digits over everything a library is built from: kernels, shared headers, the public header and the
     compiler flags."""
     h = hashlib.sha256()
-    files = [os.path.join(CSRC, f) for f in sorted(os.listdir(CSRC)) if f.endswith((".hip", ".h"))]
+    files = [os.path.join(CSRC, f) for f in sorted(os.listdir(CSRC)) if f.endswith((".hip", ".h", ".cpp"))]
     files += [os.path.join(INCLUDE, f) for f in sorted(os.listdir(INCLUDE)) if f.endswith(".h")]
     for path in files:
         h.update(os.path.basename(path).encode() + b"\0")
         with open(path, "rb") as fh:
             h.update(fh.read())
-    h.update("\0".join(FLAGS + ["|"] + CROSSCHECK_FLAGS).encode())
+    h.update("\0".join(FLAGS + ["|"] + CROSSCHECK_FLAGS + ["|"] + HOST_FLAGS).encode())
     return h.hexdigest()[:16]
 
 
@@ -75,8 +79,20 @@ def _compile(job) -> str:
     return obj
 
 
+def _compile_host(out: str, want: str) -> None:
+    import torch
+    root = os.path.dirname(torch.__file__)
+    abi = f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"
+    cmd = [os.environ.get("CXX", "g++"), *HOST_FLAGS, abi, f'-DCDM_SOURCE_HASH="{want}"', "-I" + os.path.join(root, "include"),
+           "-I" + os.path.join(root, "include", "torch", "csrc", "api", "include"), "-I" + sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "host.cpp"), "-L" + os.path.join(root, "lib"), "-lc10", "-ltorch_cpu", "-ltorch_python", "-o", out]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"the host compiler failed for host.cpp:\n{r.stderr[-4000:]}")
+
+
 def build(verbose: bool = True, only_if_stale: bool = False) -> str:
-    """Compile every HIP source for gfx950 and link both shared libraries.  Recompiles every time it is called, unless
+    """Compile every HIP source for gfx950 and link both shared libraries, and the Python side's extension module.  Recompiles every time it is called, unless
     ``only_if_stale`` is set and both libraries already carry the hash of the present sources (the loader's case).
     Builds go to a temporary directory and are moved into place under a file lock, so that processes which find a
     stale library at the same time neither overwrite each other's objects nor load a half-written file."""
@@ -85,7 +101,7 @@ def build(verbose: bool = True, only_if_stale: bool = False) -> str:
     with open(os.path.join(LIB_DIR, ".build.lock"), "w") as lock:
         fcntl.flock(lock, fcntl.LOCK_EX)
         try:
-            if only_if_stale and built_hash(LIB_PATH) == want and built_hash(CROSSCHECK_PATH) == want:
+            if only_if_stale and all(built_hash(p) == want for p in (LIB_PATH, CROSSCHECK_PATH, HOST_PATH)):
                 return LIB_PATH             # another process built it while this one waited for the lock
             tmp = tempfile.mkdtemp(prefix=".build-", dir=LIB_DIR)
             try:
@@ -94,8 +110,11 @@ def build(verbose: bool = True, only_if_stale: bool = False) -> str:
                 for _, extra, out_dir in targets:
                     os.makedirs(out_dir)
                     jobs += [(src, extra, out_dir, want) for src in SOURCES]
+                host = os.path.join(tmp, os.path.basename(HOST_PATH))
                 with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1, len(jobs))) as ex:
+                    host_job = ex.submit(_compile_host, host, want)
                     objs = list(ex.map(_compile, jobs))
+                    host_job.result()
                 for i, (path, _, out_dir) in enumerate(targets):
                     so = os.path.join(out_dir, os.path.basename(path))
                     cmd = [_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", so, *objs[i * len(SOURCES):(i + 1) * len(SOURCES)]]
@@ -104,6 +123,7 @@ def build(verbose: bool = True, only_if_stale: bool = False) -> str:
                         raise RuntimeError(f"link failed:\n{r.stderr[-4000:]}")
                 for path, _, out_dir in targets:
                     os.replace(os.path.join(out_dir, os.path.basename(path)), path)
+                os.replace(host, HOST_PATH)
             finally:
                 shutil.rmtree(tmp, ignore_errors=True)
         finally:

@@ -1,0 +1,515 @@
+// Argument checks and calls of the launchers a forward is made of, for Python (cosmos_amd/ops.py).
+//
+// Bound by the interpreter: an operator's checks, pointer arrays and foreign call took 8 - 14 us in Python, where a small stack's
+// kernels take 9 us each.  Here they take about one, so that such a stack no longer waits for the host.  A method takes a call only
+// if every argument is as the general path in Python demands and of the plainest kind (tensors and parameters themselves, no
+// subclass; lists and tuples; whole numbers); for anything else it returns None, and the general path raises what it raises, or
+// accepts what it accepts.  Nothing is kept from one call for the next.
+#include <dlfcn.h>
+
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/core/Tensor.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/cosmos_dm.h"
+
+namespace {
+
+struct NotTaken {};
+constexpr int kMax = 16;      // token runs, or blocks, of one call
+constexpr at::ScalarType kBf16 = at::kBFloat16, kF32 = at::kFloat;
+
+void need(bool ok) { if (!ok) throw NotTaken{}; }
+
+const at::Tensor& tensor(PyObject* o) {
+    need(THPVariable_CheckExact(o));      // a tensor or parameter itself: a subclass's attributes may be its own
+    const at::Tensor& t = THPVariable_Unpack(o);
+    need(t.is_cuda());
+    return t;
+}
+
+// rows (or, with ndim 1, a vector) of one type, contiguous along the last dimension
+const at::Tensor& rows(PyObject* o, at::ScalarType type, int ndim = 2) {
+    const at::Tensor& t = tensor(o);
+    need(t.scalar_type() == type && t.dim() == ndim && t.stride(ndim - 1) == 1);
+    return t;
+}
+
+// contiguous fp32 values, n of them; None: no values
+const float* values(PyObject* o, int64_t n) {
+    if (o == Py_None) return nullptr;
+    const at::Tensor& t = tensor(o);
+    need(t.scalar_type() == kF32 && t.numel() == n && t.is_contiguous());
+    return static_cast<const float*>(t.data_ptr());
+}
+
+int64_t whole(PyObject* o) {
+    need(PyLong_CheckExact(o));
+    int overflow = 0;
+    const long long v = PyLong_AsLongLongAndOverflow(o, &overflow);
+    need(overflow == 0);
+    return v;
+}
+int32_t whole32(PyObject* o) {
+    const int64_t v = whole(o);
+    need(v == (int32_t)v);
+    return (int32_t)v;
+}
+float real(PyObject* o) {
+    need(PyFloat_CheckExact(o));
+    return (float)PyFloat_AS_DOUBLE(o);
+}
+
+struct List {      // the entries of a list or tuple
+    PyObject** at;
+    int n;
+    explicit List(PyObject* o) {
+        need(PyList_CheckExact(o) || PyTuple_CheckExact(o));
+        const Py_ssize_t size = PySequence_Fast_GET_SIZE(o);
+        need(size > 0 && size <= kMax);
+        n = (int)size;
+        at = PySequence_Fast_ITEMS(o);
+    }
+};
+
+struct Runs {      // token runs (start, length)
+    int64_t start[kMax], len[kMax], end = 0, total = 0;
+    int n;
+    explicit Runs(PyObject* o) {
+        const List l(o);
+        n = l.n;
+        for (int i = 0; i < n; ++i) {
+            need(PyTuple_CheckExact(l.at[i]) && PyTuple_GET_SIZE(l.at[i]) == 2);
+            start[i] = whole(PyTuple_GET_ITEM(l.at[i], 0));
+            len[i] = whole(PyTuple_GET_ITEM(l.at[i], 1));
+            need(start[i] >= 0 && len[i] >= 0 && start[i] < (1ll << 40) && len[i] < (1ll << 40));
+            if (start[i] + len[i] > end) end = start[i] + len[i];
+            total += len[i];
+        }
+    }
+};
+
+struct Weights {      // bf16 matrices of one shape and row stride
+    const void* p[kMax];
+    int64_t out, in, ld;
+    Weights(PyObject* o, int n, const Weights* like = nullptr) {
+        const List l(o);
+        need(l.n == n);
+        for (int i = 0; i < n; ++i) {
+            const at::Tensor& w = rows(l.at[i], kBf16);
+            if (i == 0) { out = w.size(0); in = w.size(1); ld = w.stride(0); }
+            need(w.size(0) == out && w.size(1) == in && w.stride(0) == ld);
+            p[i] = w.data_ptr();
+        }
+        if (like) need(out == like->out && in == like->in && ld == like->ld);
+    }
+};
+
+struct Vectors {      // fp32 vectors of n values, or None, one per run
+    const float* p[kMax];
+    Vectors(PyObject* o, int runs, int64_t n) {
+        const List l(o);
+        need(l.n == runs);
+        for (int i = 0; i < runs; ++i) p[i] = values(l.at[i], n);
+    }
+};
+
+struct QkNorm {      // None or (q_weight, k_weight, segment ends, eps)
+    cdm_qk_norm v{};
+    int64_t ends[kMax];
+    const cdm_qk_norm* p = nullptr;
+    QkNorm(PyObject* o, int64_t head_dim) {
+        if (o == Py_None) return;
+        need(PyTuple_CheckExact(o) && PyTuple_GET_SIZE(o) == 4);
+        const List e(PyTuple_GET_ITEM(o, 2));
+        for (int i = 0; i < e.n; ++i) ends[i] = whole(e.at[i]);
+        v.q_weight = values(PyTuple_GET_ITEM(o, 0), e.n * head_dim);
+        v.k_weight = values(PyTuple_GET_ITEM(o, 1), e.n * head_dim);
+        v.seg_end = ends;
+        v.n_seg = e.n;
+        v.eps = real(PyTuple_GET_ITEM(o, 3));
+        p = &v;
+    }
+};
+
+// the launchers of one loaded library
+struct Host {
+    PyObject_HEAD
+    PyObject *get_device, *get_stream;      // torch's: the current device, and its current stream's handle
+    decltype(&cdm_adaln_rmsnorm_grouped) norm;
+    decltype(&cdm_adaln_rmsnorm_join) join;
+    decltype(&cdm_gemm_bf16) gemm;
+    decltype(&cdm_grouped_gemm_bf16) grouped;
+    decltype(&cdm_grouped_gemm_runs_bf16) grouped_runs;
+    decltype(&cdm_grouped_gemm_qkv_pack_bf16) qkv;
+    decltype(&cdm_grouped_gemm_qkv_pack_runs_bf16) qkv_runs;
+    decltype(&cdm_attn_workspace_bytes) images;
+    decltype(&cdm_attn_fwd_bf16) attention;
+    decltype(&cdm_attn_fwd_packed_bf16) packed;
+    decltype(&cdm_timestep_mlp_f32) mlp;
+    decltype(&cdm_adaln_modulation_bf16) modulation;
+};
+
+// the current HIP stream of the current device; asked for last, when everything else is in order
+void* stream_of(const Host* h) {
+    PyObject* device = PyObject_CallNoArgs(h->get_device);
+    need(device);
+    PyObject* stream = PyObject_CallOneArg(h->get_stream, device);
+    Py_DECREF(device);
+    need(stream);
+    const uintptr_t v = (uintptr_t)PyLong_AsUnsignedLongLong(stream);
+    Py_DECREF(stream);
+    need(!PyErr_Occurred());
+    return reinterpret_cast<void*>(v);
+}
+
+template <class F>
+int32_t unlocked(F&& launch) {      // the launch itself, without the interpreter's lock (a full queue may make it wait)
+    int32_t rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = launch();
+    Py_END_ALLOW_THREADS
+    return rc;
+}
+
+template <int N, class F>
+PyObject* call(PyObject* const* args, Py_ssize_t n, F&& body) {
+    if (n != N) {
+        PyErr_Format(PyExc_TypeError, "%d arguments expected, got %zd", N, n);
+        return nullptr;
+    }
+    int32_t rc;
+    try {
+        if (at::impl::torch_function_mode_enabled()) Py_RETURN_NONE;      // a mode sees what the general path asks of tensors
+        rc = body();
+    } catch (...) {      // not a call for this path: the general one raises what is to be raised
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    return PyLong_FromLong(rc);
+}
+
+Host* self_of(PyObject* o) { return reinterpret_cast<Host*>(o); }
+
+// x, ws, shifts, scales, runs, eps, out, out_s, sources (out is bf16: e4m3 rows go the general way)
+PyObject* h_norm(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    return call<9>(a, n, [&] {
+        Host* h = self_of(self);
+        const at::Tensor& x = tensor(a[0]);
+        const bool f32 = x.scalar_type() == kF32;
+        need((f32 || x.scalar_type() == kBf16) && x.dim() == 2 && x.is_contiguous() && x.stride(1) == 1);
+        const int64_t rows_x = x.size(0), d = x.size(1);
+        const Runs r(a[4]);
+        need(r.end <= rows_x);
+        const at::Tensor& out = rows(a[6], kBf16);
+        need(out.is_contiguous() && out.size(0) == rows_x && out.size(1) == d && a[7] == Py_None);
+        const List wl(a[1]);
+        need(wl.n == r.n);
+        const void* w[kMax];
+        for (int i = 0; i < r.n; ++i) {
+            const at::Tensor& t = rows(wl.at[i], kBf16, 1);
+            need(t.size(0) == d);
+            w[i] = t.data_ptr();
+        }
+        const Vectors shift(a[2], r.n, d), scale(a[3], r.n, d);
+        const float eps = real(a[5]);
+        void *px = x.data_ptr(), *po = out.data_ptr();
+        if (a[8] == Py_None) {
+            void* st = stream_of(h);
+            return unlocked([&] { return h->norm(px, f32, w, shift.p, scale.p, r.start, r.len, r.n, po, nullptr, d, eps, st); });
+        }
+        const List sl(a[8]);
+        need(f32 && sl.n == r.n);
+        const void* src[kMax];
+        for (int i = 0; i < r.n; ++i) {
+            const at::Tensor& t = rows(sl.at[i], kBf16);
+            need(t.is_contiguous() && t.size(0) == r.len[i] && t.size(1) == d);
+            src[i] = t.data_ptr();
+        }
+        void* st = stream_of(h);
+        return unlocked([&] { return h->join(src, (float*)px, w, shift.p, scale.p, r.start, r.len, r.n, po, nullptr, d, eps, st); });
+    });
+}
+
+// (out and residual are fp32 rows under the fp32 residual epilogue, bf16 under every other)
+at::ScalarType row_type(int32_t epilogue) { return epilogue == CDM_EPI_GATE_RESIDUAL_F32 ? kF32 : kBf16; }
+
+// a, w, w2, epilogue, residual, gate, cos, sin, rope_cols, head_dim, out
+PyObject* h_gemm(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    return call<11>(a, n, [&] {
+        Host* h = self_of(self);
+        const at::Tensor &x = rows(a[0], kBf16), &w = rows(a[1], kBf16);
+        const int32_t epi = whole32(a[3]), head_dim = whole32(a[9]);
+        const at::ScalarType ot = row_type(epi);
+        const at::Tensor& out = rows(a[10], ot);
+        const int64_t M = x.size(0), K = x.size(1), N = w.size(0), half = head_dim / 2, rope_cols = whole(a[8]);
+        need(w.size(1) == K && out.size(0) == M && out.size(1) == N && head_dim >= 0);
+        const void* w2 = nullptr;
+        if (a[2] != Py_None) {
+            const at::Tensor& t = rows(a[2], kBf16);
+            need(t.size(0) == N && t.size(1) == K && t.stride(0) == w.stride(0));
+            w2 = t.data_ptr();
+        }
+        const void* res = nullptr;
+        int64_t ldr = 0;
+        if (a[4] != Py_None) {
+            const at::Tensor& t = rows(a[4], ot);
+            res = t.data_ptr();
+            ldr = t.stride(0);
+        }
+        const float *gate = values(a[5], N), *cos = values(a[6], M * half), *sin = values(a[7], M * half);
+        void *px = x.data_ptr(), *pw = w.data_ptr(), *po = out.data_ptr(), *st = stream_of(h);
+        const int64_t lda = x.stride(0), ldw = w.stride(0), ldc = out.stride(0);
+        return unlocked([&] { return h->gemm(px, lda, pw, ldw, w2, po, ldc, M, N, K, epi, res, ldr, gate, cos, sin, rope_cols, head_dim, st); });
+    });
+}
+
+// a, ws, runs, w2s, epilogue, residual, gates, cos, sin, rope_cols, head_dim, out
+PyObject* h_grouped(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    return call<12>(a, n, [&] {
+        Host* h = self_of(self);
+        const Runs r(a[2]);
+        const Weights w(a[1], r.n);
+        const at::Tensor& x = rows(a[0], kBf16);
+        const int32_t epi = whole32(a[4]), head_dim = whole32(a[10]);
+        const at::ScalarType ot = row_type(epi);
+        const at::Tensor& out = rows(a[11], ot);
+        const int64_t M = x.size(0), K = x.size(1), half = head_dim / 2, rope_cols = whole(a[9]);
+        need(head_dim >= 0);
+        const void* const* w2 = nullptr;
+        alignas(Weights) char mem[sizeof(Weights)];
+        if (a[3] != Py_None) w2 = (new (mem) Weights(a[3], r.n, &w))->p;
+        const void* res = nullptr;
+        int64_t ldr = 0;
+        if (a[5] != Py_None) {
+            const at::Tensor& t = rows(a[5], ot);
+            res = t.data_ptr();
+            ldr = t.stride(0);
+        }
+        const float* const* gates = nullptr;
+        alignas(Vectors) char gmem[sizeof(Vectors)];
+        if (a[6] != Py_None) gates = (new (gmem) Vectors(a[6], r.n, w.out))->p;
+        const float *cos = values(a[7], M * half), *sin = values(a[8], M * half);
+        void *px = x.data_ptr(), *po = out.data_ptr(), *st = stream_of(h);
+        const int64_t lda = x.stride(0), ldc = out.stride(0);
+        return unlocked([&] { return h->grouped(px, lda, w.p, w.ld, w2, po, ldc, r.start, r.len, r.n, w.out, K, epi, res, ldr, gates, cos, sin,
+                                                rope_cols, head_dim, st); });
+    });
+}
+
+struct Sources {      // the rows of every run in tensors of their own
+    const void* p[kMax];
+    int64_t k, ld = 0;
+    Sources(PyObject* o, const Runs& r) {
+        const List l(o);
+        need(l.n == r.n);
+        bool any = false;
+        for (int i = 0; i < r.n; ++i) {
+            const at::Tensor& t = rows(l.at[i], kBf16);
+            if (i == 0) { k = t.size(1); ld = t.stride(0); }
+            need(t.size(0) == r.len[i] && t.size(1) == k);
+            if (r.len[i] > 0) {
+                if (!any) ld = t.stride(0);
+                need(t.stride(0) == ld);
+                any = true;
+            }
+            p[i] = t.data_ptr();
+        }
+    }
+};
+
+// sources, ws, runs, out
+PyObject* h_grouped_runs(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    return call<4>(a, n, [&] {
+        Host* h = self_of(self);
+        const Runs r(a[2]);
+        const Weights w(a[1], r.n);
+        const Sources x(a[0], r);
+        const at::Tensor& out = rows(a[3], kBf16);
+        need(out.size(0) >= r.end && out.size(1) == w.out);
+        void *po = out.data_ptr(), *st = stream_of(h);
+        const int64_t ldc = out.stride(0);
+        return unlocked([&] { return h->grouped_runs(x.p, x.ld, w.p, w.ld, po, ldc, r.start, r.len, r.n, w.out, x.k, st); });
+    });
+}
+
+// a (rows, or a list of the runs' rows), ws, runs, n_heads, n_kv_heads, head_dim, q_out, workspace, cos, sin, qk_norm
+PyObject* h_qkv(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    return call<11>(a, n, [&] {
+        Host* h = self_of(self);
+        const Runs r(a[2]);
+        const Weights w(a[1], r.n);
+        const int32_t heads = whole32(a[3]), kv = whole32(a[4]), hd = whole32(a[5]);
+        need(heads > 0 && kv > 0 && hd > 0 && w.out == ((int64_t)heads + 2 * (int64_t)kv) * hd);
+        const at::Tensor &q = rows(a[6], kBf16), &ws = rows(a[7], at::kByte, 1);
+        const float *cos = values(a[8], r.total * (hd / 2)), *sin = values(a[9], r.total * (hd / 2));
+        const QkNorm qn(a[10], hd);
+        void *pq = q.data_ptr(), *pws = ws.data_ptr();
+        const int64_t ldq = q.stride(0), bytes = ws.numel();
+        if (THPVariable_CheckExact(a[0])) {
+            const at::Tensor& x = rows(a[0], kBf16);
+            void* px = x.data_ptr();
+            const int64_t lda = x.stride(0), K = x.size(1);
+            void* st = stream_of(h);
+            return unlocked([&] { return h->qkv(px, lda, w.p, w.ld, pq, ldq, r.start, r.len, r.n, K, heads, kv, hd, cos, sin, qn.p, pws, bytes, st); });
+        }
+        const Sources x(a[0], r);
+        void* st = stream_of(h);
+        return unlocked([&] { return h->qkv_runs(x.p, x.ld, w.p, w.ld, pq, ldq, r.start, r.len, r.n, x.k, heads, kv, hd, cos, sin, qn.p, pws, bytes, st); });
+    });
+}
+
+// q, workspace, n_heads, n_kv_heads, head_dim, out, cos, sin, qk_norm, prefix, causal_prefix (no row maxima asked for, and
+// what the workspace holds beyond the images is the scratch)
+PyObject* h_packed(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    return call<11>(a, n, [&] {
+        Host* h = self_of(self);
+        const at::Tensor &q = rows(a[0], kBf16), &ws = rows(a[1], at::kByte, 1), &out = rows(a[5], kBf16);
+        const int32_t heads = whole32(a[2]), kv = whole32(a[3]), hd = whole32(a[4]);
+        need(heads > 0 && kv > 0 && hd > 0);
+        const int64_t N = q.size(0), half = hd / 2, causal = whole(a[10]), need_bytes = h->images(N, kv, hd), have = ws.numel();
+        const float *cos = values(a[6], N * half), *sin = values(a[7], N * half);
+        const QkNorm qn(a[8], hd);
+        void* prefix = nullptr;
+        int64_t n_prefix = 0;
+        if (a[9] != Py_None) {
+            need(PyTuple_CheckExact(a[9]) && PyTuple_GET_SIZE(a[9]) == 2);
+            const at::Tensor& t = rows(PyTuple_GET_ITEM(a[9], 0), at::kByte, 1);
+            n_prefix = whole(PyTuple_GET_ITEM(a[9], 1));
+            need(n_prefix >= 0 && t.numel() >= h->images(n_prefix, kv, hd));
+            prefix = t.data_ptr();
+        }
+        need(have >= need_bytes);
+        const int64_t used = (need_bytes + 255) / 256 * 256, extra = have > used ? have - used : 0;
+        char* pws = static_cast<char*>(ws.data_ptr());
+        void *pq = q.data_ptr(), *po = out.data_ptr(), *st = stream_of(h);
+        const int64_t ldq = q.stride(0), ldo = out.stride(0);
+        return unlocked([&] { return h->packed(pq, ldq, cos, sin, pws, po, ldo, N, heads, kv, hd, qn.p, prefix, n_prefix, causal, nullptr,
+                                               extra ? pws + used : nullptr, extra, st); });
+    });
+}
+
+// q, k, v, n_heads, n_kv_heads, head_dim, out, workspace, cos, sin, qk_norm, causal_prefix
+PyObject* h_attention(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    return call<12>(a, n, [&] {
+        Host* h = self_of(self);
+        const at::Tensor &q = rows(a[0], kBf16), &k = rows(a[1], kBf16), &v = rows(a[2], kBf16), &out = rows(a[6], kBf16), &ws = rows(a[7], at::kByte, 1);
+        const int32_t heads = whole32(a[3]), kv = whole32(a[4]), hd = whole32(a[5]);
+        need(heads > 0 && kv > 0 && hd > 0);
+        const int64_t N = q.size(0), d = (int64_t)heads * hd, dkv = (int64_t)kv * hd, half = hd / 2, causal = whole(a[11]);
+        need(q.size(1) == d && k.size(0) == N && k.size(1) == dkv && v.size(0) == N && v.size(1) == dkv);
+        const float *cos = values(a[8], N * half), *sin = values(a[9], N * half);
+        const QkNorm qn(a[10], hd);
+        void *pq = q.data_ptr(), *pk = k.data_ptr(), *pv = v.data_ptr(), *po = out.data_ptr(), *pws = ws.data_ptr(), *st = stream_of(h);
+        const int64_t ldq = q.stride(0), ldk = k.stride(0), ldv = v.stride(0), ldo = out.stride(0), bytes = ws.numel();
+        return unlocked([&] { return h->attention(pq, ldq, pk, ldk, pv, ldv, cos, sin, po, ldo, N, heads, kv, hd, pws, bytes, qn.p, causal, st); });
+    });
+}
+
+// t, w1, b1, w2, b2, both [2, d]
+PyObject* h_mlp(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    return call<6>(a, n, [&] {
+        Host* h = self_of(self);
+        const at::Tensor &w1 = rows(a[1], kF32), &w2 = rows(a[3], kF32), &both = rows(a[5], kF32);
+        const int64_t d = w1.size(0), freq = w1.size(1);
+        need(w2.size(0) == d && w2.size(1) == d && w1.is_contiguous() && w2.is_contiguous() && both.is_contiguous() && both.numel() == 2 * d);
+        const float *t = values(a[0], 1), *b1 = values(a[2], d), *b2 = values(a[4], d), *p1 = (float*)w1.data_ptr(), *p2 = (float*)w2.data_ptr();
+        float* po = static_cast<float*>(both.data_ptr());
+        void* st = stream_of(h);
+        return unlocked([&] { return h->mlp(t, p1, b1, p2, b2, po, po + d, freq, d, st); });
+    });
+}
+
+// c, ws, bs, out [blocks, n_out]
+PyObject* h_modulation(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+    return call<4>(a, n, [&] {
+        Host* h = self_of(self);
+        const List wl(a[1]), bl(a[2]);
+        need(wl.n == bl.n);
+        const void *w[kMax], *b[kMax];
+        int64_t n_out = 0, d = 0;
+        for (int i = 0; i < wl.n; ++i) {
+            const at::Tensor &tw = rows(wl.at[i], kBf16), &tb = rows(bl.at[i], kBf16, 1);
+            if (i == 0) { n_out = tw.size(0); d = tw.size(1); }
+            need(tw.size(0) == n_out && tw.size(1) == d && tw.is_contiguous() && tb.size(0) == n_out);
+            w[i] = tw.data_ptr();
+            b[i] = tb.data_ptr();
+        }
+        const float* c = values(a[0], d);
+        const at::Tensor& out = rows(a[3], kF32);
+        need(out.is_contiguous() && out.size(0) == wl.n && out.size(1) == n_out);
+        float* po = static_cast<float*>(out.data_ptr());
+        void* st = stream_of(h);
+        return unlocked([&] { return h->modulation(c, w, b, wl.n, po, d, n_out, st); });
+    });
+}
+
+#define METHOD(name) {#name, (PyCFunction)(void (*)(void))h_##name, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {METHOD(norm), METHOD(gemm), METHOD(grouped), METHOD(grouped_runs), METHOD(qkv), METHOD(packed), METHOD(attention),
+                         METHOD(mlp), METHOD(modulation), {nullptr, nullptr, 0, nullptr}};
+#undef METHOD
+
+void host_dealloc(PyObject* o) {
+    PyTypeObject* type = Py_TYPE(o);
+    Py_XDECREF(self_of(o)->get_device);
+    Py_XDECREF(self_of(o)->get_stream);
+    type->tp_free(o);
+    Py_DECREF(type);
+}
+
+// Host(handle, get_device, get_stream): the launchers of the library behind a dlopen handle
+PyObject* host_new(PyTypeObject* type, PyObject* args, PyObject*) {
+    unsigned long long handle;
+    PyObject *get_device, *get_stream;
+    if (!PyArg_ParseTuple(args, "KOO", &handle, &get_device, &get_stream)) return nullptr;
+    PyObject* o = type->tp_alloc(type, 0);
+    if (!o) return nullptr;
+    Host* h = self_of(o);
+    Py_INCREF(h->get_device = get_device);
+    Py_INCREF(h->get_stream = get_stream);
+    bool ok = true;
+    auto find = [&](auto& fn, const char* name) {
+        fn = reinterpret_cast<std::remove_reference_t<decltype(fn)>>(dlsym(reinterpret_cast<void*>((uintptr_t)handle), name));
+        if (!fn && ok) {
+            ok = false;
+            PyErr_Format(PyExc_RuntimeError, "the library does not export %s", name);
+        }
+    };
+    find(h->norm, "cdm_adaln_rmsnorm_grouped");
+    find(h->join, "cdm_adaln_rmsnorm_join");
+    find(h->gemm, "cdm_gemm_bf16");
+    find(h->grouped, "cdm_grouped_gemm_bf16");
+    find(h->grouped_runs, "cdm_grouped_gemm_runs_bf16");
+    find(h->qkv, "cdm_grouped_gemm_qkv_pack_bf16");
+    find(h->qkv_runs, "cdm_grouped_gemm_qkv_pack_runs_bf16");
+    find(h->images, "cdm_attn_workspace_bytes");
+    find(h->attention, "cdm_attn_fwd_bf16");
+    find(h->packed, "cdm_attn_fwd_packed_bf16");
+    find(h->mlp, "cdm_timestep_mlp_f32");
+    find(h->modulation, "cdm_adaln_modulation_bf16");
+    if (!ok) {
+        Py_DECREF(o);
+        return nullptr;
+    }
+    return o;
+}
+
+PyType_Slot slots[] = {{Py_tp_new, (void*)host_new}, {Py_tp_dealloc, (void*)host_dealloc}, {Py_tp_methods, (void*)methods}, {0, nullptr}};
+PyType_Spec spec = {"cosmos_amd._host.Host", sizeof(Host), 0, Py_TPFLAGS_DEFAULT, slots};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "checks and calls of the HIP library's launchers", -1, nullptr, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+__attribute__((used)) const char kSourceHash[] = "CDM_SRC_HASH=" CDM_SOURCE_HASH;
+
+PyMODINIT_FUNC PyInit__host() {
+    PyObject* m = PyModule_Create(&module);
+    if (!m) return nullptr;
+    PyObject* type = PyType_FromSpec(&spec);
+    if (!type || PyModule_AddObject(m, "Host", type) < 0) {
+        Py_XDECREF(type);
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

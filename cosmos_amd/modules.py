@@ -400,10 +400,11 @@ def _routed_linear(a, sa, weights, qweights, weights2, segments, *, out, epilogu
     """Per-modality linear over contiguous token segments: one grouped launch over all segments."""
     if qweights is None and len(segments) == 1:
         (s0, ln, b, _), = segments
-        rows = lambda t: t if t is None or (s0 == 0 and t.shape[0] == ln) else t[s0:s0 + ln]
-        ops.gemm(rows(a), _entry(weights, b), w2=_entry(weights2, b) if weights2 is not None else None, epilogue=epilogue, residual=rows(residual),
-                 gate=gates[0] if gates is not None else None, cos=rows(cos), sin=rows(sin), rope_cols=rope_cols, head_dim=head_dim,
-                 out=rows(out))
+        if s0 or a.shape[0] != ln or out.shape[0] != ln or (residual is not None and residual.shape[0] != ln) or cos is not None or sin is not None:
+            rows = lambda t: t if t is None or (s0 == 0 and t.shape[0] == ln) else t[s0:s0 + ln]
+            a, residual, cos, sin, out = rows(a), rows(residual), rows(cos), rows(sin), rows(out)
+        ops.gemm(a, _entry(weights, b), w2=_entry(weights2, b) if weights2 is not None else None, epilogue=epilogue, residual=residual,
+                 gate=gates[0] if gates is not None else None, cos=cos, sin=sin, rope_cols=rope_cols, head_dim=head_dim, out=out)
         return
     segl = [(s, l) for (s, l, _, _) in segments]
     if qweights is None:

@@ -168,6 +168,10 @@ def adaln_rmsnorm_grouped(x: torch.Tensor, ws: Sequence[torch.Tensor], shifts: S
     its own weights and modulation, in one launch; ``out`` [n, d] bf16 (e4m3 with ``out_s`` [n] fp32).  With ``sources`` (run
     g's rows, contiguous [len, d] bf16) x is an fp32 output as well: the runs joined."""
     lib = _lib.load()
+    rc = lib.host.norm(x, ws, shifts, scales, segments, eps, out, out_s, sources)
+    if rc is not None:
+        _lib.check(rc, "cdm_adaln_rmsnorm_grouped")
+        return
     n, d = x.shape
     f32 = x.dtype == torch.float32
     if not x.is_contiguous() or not out.is_contiguous() or out.shape != x.shape or (out_s is not None and out_s.shape != (n,)):
@@ -316,12 +320,14 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, w2: Optional[torch.Tensor] = None,
     scratch = gemm_scratch_bytes((M,), N, K, epi) if epi in _MAY_SPLIT_K and w2 is None and cos is None and sin is None else 0
     if scratch:
         return _gemm_cut_along_k(a, [w], [(0, M)], epi, odt, residual, [gate], out, scratch)
-    rc = lib.cdm_gemm_bf16(_chk(a, "a", torch.bfloat16, 2), a.stride(0), _chk(w, "w", torch.bfloat16, 2), w.stride(0),
-                           _chk(w2, "w2", torch.bfloat16, 2), _chk(out, "out", odt, 2), out.stride(0),
-                           M, N, K, epi, _chk(residual, "residual", odt, 2),
-                           residual.stride(0) if residual is not None else 0, _f32vec(gate, "gate", N),
-                           _f32vec(cos, "cos", M * half), _f32vec(sin, "sin", M * half), int(rope_cols), int(head_dim),
-                           _stream())
+    rc = lib.host.gemm(a, w, w2, epi, residual, gate, cos, sin, int(rope_cols), int(head_dim), out)
+    if rc is None:
+        rc = lib.cdm_gemm_bf16(_chk(a, "a", torch.bfloat16, 2), a.stride(0), _chk(w, "w", torch.bfloat16, 2), w.stride(0),
+                               _chk(w2, "w2", torch.bfloat16, 2), _chk(out, "out", odt, 2), out.stride(0),
+                               M, N, K, epi, _chk(residual, "residual", odt, 2),
+                               residual.stride(0) if residual is not None else 0, _f32vec(gate, "gate", N),
+                               _f32vec(cos, "cos", M * half), _f32vec(sin, "sin", M * half), int(rope_cols), int(head_dim),
+                               _stream())
     _lib.check(rc, "cdm_gemm_bf16")
     return out
 
@@ -404,22 +410,18 @@ def grouped_gemm(a: torch.Tensor, ws: Sequence[torch.Tensor], segments: Sequence
     for w in list(ws) + list(w2s or []):
         if w.shape != ws[0].shape or w.stride(0) != ldw:
             raise ValueError("all segment weights must share shape and row stride")
-    PP = C.c_void_p * n_seg
-    wp = PP(*[_chk(w, "w", torch.bfloat16, 2) for w in ws])
+    PP, I64 = C.c_void_p * n_seg, C.c_int64 * n_seg
     if runs is not None:
-        ap, lda = _run_ptrs(runs, segments)
-        I64 = C.c_int64 * n_seg
-        if out.shape[0] < max(int(s) + int(l) for s, l in segments) or out.shape[1] != N:
-            raise ValueError("out shape mismatch")
-        rc = lib.cdm_grouped_gemm_runs_bf16(ap, lda, wp, ldw, _chk(out, "out", torch.bfloat16, 2), out.stride(0),
-                                            I64(*[int(s) for s, _ in segments]), I64(*[int(l) for _, l in segments]), n_seg, N, K,
-                                            _stream())
+        rc = lib.host.grouped_runs(runs, ws, segments, out)
+        if rc is None:
+            ap, lda = _run_ptrs(runs, segments)
+            if out.shape[0] < max(int(s) + int(l) for s, l in segments) or out.shape[1] != N:
+                raise ValueError("out shape mismatch")
+            rc = lib.cdm_grouped_gemm_runs_bf16(ap, lda, PP(*[_chk(w, "w", torch.bfloat16, 2) for w in ws]), ldw,
+                                                _chk(out, "out", torch.bfloat16, 2), out.stride(0), I64(*[int(s) for s, _ in segments]),
+                                                I64(*[int(l) for _, l in segments]), n_seg, N, K, _stream())
         _lib.check(rc, "cdm_grouped_gemm_runs_bf16")
         return out
-    w2p = PP(*[_chk(w, "w2", torch.bfloat16, 2) for w in w2s]) if w2s is not None else None
-    gp = PP(*[(_f32vec(g, "gate", N) or None) for g in gates]) if gates is not None else None
-    I64 = C.c_int64 * n_seg
-    st, ln = I64(*[int(s) for s, _ in segments]), I64(*[int(l) for _, l in segments])
     half = head_dim // 2 if head_dim else 0
     epi, odt = _epilogue(epilogue, out, residual)
     # operands that the epilogue does not use are checked below all the same
@@ -427,12 +429,16 @@ def grouped_gemm(a: torch.Tensor, ws: Sequence[torch.Tensor], segments: Sequence
     scratch = gemm_scratch_bytes(tuple(int(l) for _, l in segments), N, K, epi) if may_split else 0
     if scratch:
         return _gemm_cut_along_k(a, ws, segments, epi, odt, residual, gates, out, scratch)
-    rc = lib.cdm_grouped_gemm_bf16(_chk(a, "a", torch.bfloat16, 2), a.stride(0), wp, ldw, w2p,
-                                   _chk(out, "out", odt, 2), out.stride(0), st, ln, n_seg, N, K,
-                                   epi, _chk(residual, "residual", odt, 2),
-                                   residual.stride(0) if residual is not None else 0, gp,
-                                   _f32vec(cos, "cos", M * half), _f32vec(sin, "sin", M * half), int(rope_cols),
-                                   int(head_dim), _stream())
+    rc = lib.host.grouped(a, ws, segments, w2s, epi, residual, gates, cos, sin, int(rope_cols), int(head_dim), out)
+    if rc is None:
+        wp = PP(*[_chk(w, "w", torch.bfloat16, 2) for w in ws])
+        w2p = PP(*[_chk(w, "w2", torch.bfloat16, 2) for w in w2s]) if w2s is not None else None
+        gp = PP(*[(_f32vec(g, "gate", N) or None) for g in gates]) if gates is not None else None
+        rc = lib.cdm_grouped_gemm_bf16(_chk(a, "a", torch.bfloat16, 2), a.stride(0), wp, ldw, w2p, _chk(out, "out", odt, 2), out.stride(0),
+                                       I64(*[int(s) for s, _ in segments]), I64(*[int(l) for _, l in segments]), n_seg, N, K, epi,
+                                       _chk(residual, "residual", odt, 2), residual.stride(0) if residual is not None else 0, gp,
+                                       _f32vec(cos, "cos", M * half), _f32vec(sin, "sin", M * half), int(rope_cols), int(head_dim),
+                                       _stream())
     _lib.check(rc, "cdm_grouped_gemm_bf16")
     return out
 
@@ -489,6 +495,11 @@ def gemm_qkv_pack(a: torch.Tensor, sa: Optional[torch.Tensor], ws: Sequence[torc
     given.  Raises where the fused form does not apply (``qkv_pack_applies`` tells beforehand).  ``a`` may be a list of the
     segments' rows (bf16)."""
     lib = _lib.load()
+    if sa is None:
+        rc = lib.host.qkv(a, ws, segments, n_heads, n_kv_heads, head_dim, q_out, workspace, cos, sin, qk_norm)
+        if rc is not None:
+            _lib.check(rc, "cdm_grouped_gemm_qkv_pack_bf16")
+            return
     runs = None if isinstance(a, torch.Tensor) else list(a)
     a = a if runs is None else runs[0]
     M, K = a.shape
@@ -624,6 +635,11 @@ def attention_packed(q: torch.Tensor, workspace: torch.Tensor, n_heads: int, hea
     n_kv_heads = n_heads if n_kv_heads is None else int(n_kv_heads)
     if out is None:
         out = torch.empty((n, d), dtype=torch.bfloat16, device=q.device)
+    if row_amax is None and split_scratch is None and _ATTN_TIMER is None:
+        rc = lib.host.packed(q, workspace, n_heads, n_kv_heads, head_dim, out, cos, sin, qk_norm, prefix, causal_prefix)
+        if rc is not None:
+            _lib.check(rc, "cdm_attn_fwd_packed_bf16")
+            return out
     half = head_dim // 2
     qn, _keep = _qk_norm_arg(qk_norm, head_dim)
     pws, npre = (None, 0) if prefix is None else (_chk(prefix[0], "prefix images", torch.uint8, 1), int(prefix[1]))
@@ -680,14 +696,16 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, n_heads: int, h
         workspace = torch.empty((attn_workspace_total_bytes(n, n_heads, n_kv_heads, head_dim),), dtype=torch.uint8,
                                 device=q.device)
     if _ATTN_TIMER is None and _OP_TIMER is None and prefix is None:
-        half = head_dim // 2
-        qn, _keep = _qk_norm_arg(qk_norm, head_dim)
-        rc = lib.cdm_attn_fwd_bf16(_chk(q, "q", torch.bfloat16, 2), q.stride(0), _chk(k, "k", torch.bfloat16, 2),
-                                   k.stride(0), _chk(v, "v", torch.bfloat16, 2), v.stride(0),
-                                   _f32vec(cos, "cos", n * half), _f32vec(sin, "sin", n * half),
-                                   _chk(out, "out", torch.bfloat16, 2), out.stride(0), n, n_heads, n_kv_heads, head_dim,
-                                   _chk(workspace, "workspace", torch.uint8, 1), workspace.numel(), qn,
-                                   int(causal_prefix), _stream())
+        rc = lib.host.attention(q, k, v, n_heads, n_kv_heads, head_dim, out, workspace, cos, sin, qk_norm, causal_prefix)
+        if rc is None:
+            half = head_dim // 2
+            qn, _keep = _qk_norm_arg(qk_norm, head_dim)
+            rc = lib.cdm_attn_fwd_bf16(_chk(q, "q", torch.bfloat16, 2), q.stride(0), _chk(k, "k", torch.bfloat16, 2),
+                                       k.stride(0), _chk(v, "v", torch.bfloat16, 2), v.stride(0),
+                                       _f32vec(cos, "cos", n * half), _f32vec(sin, "sin", n * half),
+                                       _chk(out, "out", torch.bfloat16, 2), out.stride(0), n, n_heads, n_kv_heads, head_dim,
+                                       _chk(workspace, "workspace", torch.uint8, 1), workspace.numel(), qn,
+                                       int(causal_prefix), _stream())
         _lib.check(rc, "cdm_attn_fwd_bf16")
         return out
     # two-stage form: prefix images, or HIP events around the attention kernel alone while timing is on
@@ -716,8 +734,10 @@ def timestep_mlp(t: torch.Tensor, w1: torch.Tensor, b1: torch.Tensor, w2: torch.
         raise ValueError("timestep MLP weights must be contiguous [d, freq_dim] and [d, d]")
     f32 = torch.float32
     both = torch.empty((2, d), dtype=f32, device=w1.device)      # hidden | out
-    rc = lib.cdm_timestep_mlp_f32(_f32vec(t, "t", 1), _chk(w1, "w1", f32, 2), _f32vec(b1, "b1", d), _chk(w2, "w2", f32, 2),
-                                  _f32vec(b2, "b2", d), both.data_ptr(), both.data_ptr() + 4 * d, freq_dim, d, _stream())
+    rc = lib.host.mlp(t, w1, b1, w2, b2, both)
+    if rc is None:
+        rc = lib.cdm_timestep_mlp_f32(_f32vec(t, "t", 1), _chk(w1, "w1", f32, 2), _f32vec(b1, "b1", d), _chk(w2, "w2", f32, 2),
+                                      _f32vec(b2, "b2", d), both.data_ptr(), both.data_ptr() + 4 * d, freq_dim, d, _stream())
     _lib.check(rc, "cdm_timestep_mlp_f32")
     return both[1:]
 
@@ -732,9 +752,11 @@ def adaln_modulation(c: torch.Tensor, ws: Sequence[torch.Tensor], bs: Sequence[t
         raise ValueError("modulation weights must be contiguous and share one shape [n_out, d], biases [n_out]")
     PP = C.c_void_p * len(ws)
     out = torch.empty((len(ws), n_out), dtype=torch.float32, device=c.device)
-    rc = lib.cdm_adaln_modulation_bf16(_f32vec(c, "c", d), PP(*[_chk(w, "w", torch.bfloat16, 2) for w in ws]),
-                                       PP(*[_chk(b, "b", torch.bfloat16, 1) for b in bs]), len(ws), out.data_ptr(), d, n_out,
-                                       _stream())
+    rc = lib.host.modulation(c, ws, bs, out)
+    if rc is None:
+        rc = lib.cdm_adaln_modulation_bf16(_f32vec(c, "c", d), PP(*[_chk(w, "w", torch.bfloat16, 2) for w in ws]),
+                                           PP(*[_chk(b, "b", torch.bfloat16, 1) for b in bs]), len(ws), out.data_ptr(), d, n_out,
+                                           _stream())
     _lib.check(rc, "cdm_adaln_modulation_bf16")
     return out
 

@@ -1,0 +1,167 @@
+"""The native argument checks (csrc/host.cpp) against the general path of ops.py: the same results for every form of a call that
+they take, and the same refusals - they may only pass a call on, never accept or refuse one by themselves."""
+import types
+
+import pytest
+import torch
+
+from cosmos_amd import _lib, ops
+
+METHODS = ("norm", "gemm", "grouped", "grouped_runs", "qkv", "packed", "attention", "mlp", "modulation")
+COUNTS = dict(norm=9, gemm=11, grouped=12, grouped_runs=4, qkv=11, packed=11, attention=12, mlp=6, modulation=4)
+
+
+class General:
+    """Every call goes the general way."""
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+class Counting:
+    """The native methods, counting the calls they took."""
+    def __init__(self, host):
+        self.host, self.taken = host, []
+
+    def __getattr__(self, name):
+        def method(*a):
+            rc = getattr(self.host, name)(*a)
+            if rc is not None:
+                self.taken.append(name)
+            return rc
+        return method
+
+
+@pytest.fixture
+def hosts():
+    lib = _lib.load()
+    real = lib.host
+    yield types.SimpleNamespace(use=lambda h: setattr(lib, "host", h), counting=Counting(real))
+    lib.host = real
+
+
+def test_native_calls_pass_on_what_is_not_theirs():
+    host, cpu = _lib.load().host, torch.zeros((4, 8), dtype=torch.bfloat16)
+    for name in METHODS:
+        for arg in (None, cpu, 3, "x", [cpu], torch.nn.Parameter(cpu)):      # host memory, other types: the general path's to refuse
+            assert getattr(host, name)(*[arg] * COUNTS[name]) is None
+        with pytest.raises(TypeError):
+            getattr(host, name)()
+
+
+def bf(g, *shape, scale=1.0):
+    return (torch.randn(shape, generator=g) * scale).to("cuda", torch.bfloat16)
+
+
+def f32(g, *shape):
+    return torch.randn(shape, generator=g).to("cuda")
+
+
+def wide(t, pad):      # the same values in rows that lie further apart
+    w = torch.zeros((t.shape[0], t.shape[1] + pad), dtype=t.dtype, device=t.device)
+    w[:, :t.shape[1]] = t
+    return w[:, :t.shape[1]]
+
+
+def forms(g):
+    """(name, call) of accepted forms; a call returns its outputs."""
+    K, N = 256, 320
+    a, w, w2, gate, res = bf(g, 70, K), bf(g, N, K, scale=0.05), bf(g, N, K, scale=0.05), f32(g, N), f32(g, 70, N)
+    par = torch.nn.Parameter(w, requires_grad=False)
+    cos, sin = torch.rand((70, 32), generator=g).cuda(), torch.rand((70, 32), generator=g).cuda()
+    yield "gemm", lambda: ops.gemm(a, w)
+    yield "gemm", lambda: ops.gemm(wide(a, 8), wide(w, 64), out=wide(torch.zeros((70, N), dtype=torch.bfloat16, device="cuda"), 8))
+    yield "gemm", lambda: ops.gemm(a, par, w2=w2, epilogue="swiglu")
+    yield "gemm", lambda: ops.gemm(a, w, epilogue="gate_residual", residual=res, gate=gate, out=torch.empty_like(res))
+    yield "gemm", lambda: ops.gemm(a, w, epilogue="gate_residual", residual=wide(bf(torch.Generator().manual_seed(1), 70, N), 8))
+    yield "gemm", lambda: ops.gemm(a, w, epilogue="rope_qk", cos=cos, sin=sin, rope_cols=256, head_dim=64)
+    yield "gemm", lambda: ops.gemm(a[:1], w[:8])
+    segs = [(0, 30), (30, 0), (32, 38)]
+    def grouped(**kw):
+        out = torch.zeros((70, N), dtype=torch.float32 if "residual" in kw else torch.bfloat16, device="cuda")
+        return ops.grouped_gemm(a, [w, w2, w2], segs, out=out, **kw)
+    yield "grouped", lambda: grouped()
+    yield "grouped", lambda: grouped(w2s=[w2, w, w], epilogue="swiglu")
+    yield "grouped", lambda: grouped(epilogue="gate_residual", residual=res, gates=[None, gate, gate])
+    yield "grouped_runs", lambda: ops.grouped_gemm([a[:30], a[40:]], [w, w2], [(0, 30), (30, 30)], out=torch.zeros((60, N), dtype=torch.bfloat16, device="cuda"))
+    d = 512
+    x, xb, nw, sc, sh = f32(g, 40, d), bf(g, 40, d), bf(g, d), f32(g, d), f32(g, d)
+    def norm(x, sources=None):
+        x, out = x.clone(), torch.zeros((40, d), dtype=torch.bfloat16, device="cuda")
+        ops.adaln_rmsnorm_grouped(x, [nw, nw], [sh, None], [None, sc], [(0, 7), (7, 33)], 1e-6, out, None, sources)
+        return out, x
+    yield "norm", lambda: norm(x)
+    yield "norm", lambda: norm(xb)
+    yield "norm", lambda: norm(x, [xb[:7], xb[7:]])
+    for hd, H, Hkv, n in ((128, 2, 1, 64 + 13), (64, 4, 2, 100)):
+        qkv_w = bf(g, (H + 2 * Hkv) * hd, K, scale=0.05)
+        rows, c, s = bf(g, n, K), torch.rand((n, hd // 2), generator=g).cuda(), torch.rand((n, hd // 2), generator=g).cuda()
+        qn, kn = 1 + 0.1 * f32(g, 2, hd), 1 + 0.1 * f32(g, 2, hd)
+        def attend(split, norm, prefix, hd=hd, H=H, Hkv=Hkv, n=n, qkv_w=qkv_w, rows=rows, c=c, s=s, qn=qn, kn=kn):
+            ws = torch.zeros((ops.attn_workspace_total_bytes(n, H, Hkv, hd),), dtype=torch.uint8, device="cuda")
+            q, o = torch.zeros((n, H * hd + 64), dtype=torch.bfloat16, device="cuda"), torch.zeros((n, H * hd), dtype=torch.bfloat16, device="cuda")
+            segs = [(0, 64), (64, n - 64)]
+            qk = (qn, kn, [64, n], 1e-6) if norm else None
+            ops.gemm_qkv_pack([rows[:64], rows[64:]] if split else rows, None, [qkv_w, qkv_w], None, segs, H, Hkv, hd, q[:, :H * hd], ws, c, s, qk)
+            first = (ws.clone(), n) if prefix else None
+            return ops.attention_packed(q[:, :H * hd], ws, H, hd, o, c, s, qk, first, 0, Hkv), q, ws
+        yield "qkv packed", lambda f=attend: f(False, False, False)
+        yield "qkv packed", lambda f=attend: f(True, True, True)
+        rowsq = bf(g, n, (H + 2 * Hkv) * hd)
+        parts = (rowsq[:, :H * hd], rowsq[:, H * hd:(H + Hkv) * hd], rowsq[:, (H + Hkv) * hd:])
+        yield "attention", lambda p=parts, H=H, hd=hd, Hkv=Hkv: ops.attention(*p, H, hd, n_kv_heads=Hkv)
+        yield "attention", lambda p=parts, H=H, hd=hd, Hkv=Hkv, c=c, s=s, n=n, qn=qn, kn=kn: ops.attention(*p, H, hd, cos=c, sin=s, n_kv_heads=Hkv,
+                                                                                                           qk_norm=(qn, kn, [64, n], 1e-6), causal_prefix=9)
+    t, w1, b1, wt, b2 = torch.tensor([371.5], device="cuda"), f32(g, 64, 32), f32(g, 64), f32(g, 64, 64), f32(g, 64)
+    yield "mlp", lambda: ops.timestep_mlp(t, w1, b1, wt, b2)
+    m = [bf(g, 48, 64) for _ in range(3)]
+    yield "modulation", lambda: ops.adaln_modulation(b1, m, [bf(torch.Generator().manual_seed(i), 48) for i in range(3)])
+
+
+@pytest.mark.gpu
+def test_native_calls_equal_the_general_path(hosts):
+    made = [list(forms(torch.Generator().manual_seed(5))) for _ in range(2)]
+    for i, ((name, native), (_, general)) in enumerate(zip(*made)):
+        hosts.counting.taken.clear()
+        hosts.use(hosts.counting)
+        got = native()
+        assert hosts.counting.taken == name.split(), f"form {i}: {name}, taken {hosts.counting.taken}"
+        hosts.use(General())
+        want = general()
+        for x, y in zip(got if isinstance(got, tuple) else (got,), want if isinstance(want, tuple) else (want,)):
+            assert x.dtype == y.dtype and torch.equal(x, y), f"form {i}: {name}"
+
+
+class Sub(torch.Tensor):
+    pass
+
+
+@pytest.mark.gpu
+def test_native_calls_leave_refusals_to_the_general_path(hosts):
+    """Refused or accepted, a call that is not of the plain kind ends as it does without the native checks."""
+    g = torch.Generator().manual_seed(6)
+    a, w, res = bf(g, 16, 256), bf(g, 64, 256), f32(g, 16, 64)
+    x, nw, out = f32(g, 16, 256), bf(g, 256), torch.zeros((16, 256), dtype=torch.bfloat16, device="cuda")
+    qkv, ws = bf(g, 64, 512), torch.zeros(16, dtype=torch.uint8, device="cuda")
+    calls = [lambda: ops.gemm(a.float(), w), lambda: ops.gemm(a, w.t()), lambda: ops.gemm(a, w.cpu()), lambda: ops.gemm(a, w[:, :128]),
+             lambda: ops.gemm(a, w, gate=torch.zeros(8, device="cuda"), epilogue="gate_residual", residual=res.bfloat16()),
+             lambda: ops.gemm(a, w, epilogue="gate_residual"), lambda: ops.gemm(a, w, out=res), lambda: ops.gemm(a[:, :100], w[:, :100]),
+             lambda: ops.gemm(a.as_subclass(Sub), w), lambda: ops.gemm(a, w, rope_cols=2.0), lambda: ops.gemm(a[:0], w),
+             lambda: ops.grouped_gemm(a, [w, w], [(0, 8), (8, 9)]), lambda: ops.grouped_gemm(a, [w], [(0, 16.0)]), lambda: ops.grouped_gemm(a, (w,), ((0, 16),)),
+             lambda: ops.grouped_gemm([a], [w], [(0, 15)], out=res.bfloat16()), lambda: ops.grouped_gemm(a, [w], [(0, 16)], gates=[None, None]),
+             lambda: ops.adaln_rmsnorm_grouped(x, [nw], [None], [None], [(0, 17)], 1e-6, out), lambda: ops.adaln_rmsnorm_grouped(x, [nw[:8]], [None], [None], [(0, 16)], 1e-6, out),
+             lambda: ops.adaln_rmsnorm_grouped(x, [nw], [None], [None], [(0, 16)], 1, out), lambda: ops.adaln_rmsnorm_grouped(x, [nw.float()], [None], [None], [(0, 16)], 1e-6, out),
+             lambda: ops.gemm_qkv_pack(a, None, [bf(g, 512, 256)], None, [(0, 16)], 2, 1, 128, qkv[:16], ws),
+             lambda: ops.attention_packed(qkv[:, :128], ws, 1, 128), lambda: ops.attention(qkv[:, :128], qkv[:, :128], qkv[:, :64], 1, 128),
+             lambda: ops.attention(qkv[:, :128], qkv[:, 128:256], qkv[:, 256:384], 1, 128, workspace=ws),
+             lambda: ops.timestep_mlp(torch.zeros(2, device="cuda"), x, nw.float(), x, nw.float()), lambda: ops.adaln_modulation(nw.float(), [w], [w])]
+
+    def outcome(call, host):
+        hosts.use(host)
+        try:
+            r = call()
+            return r if r is None else r.shape
+        except Exception as e:
+            return type(e), str(e)
+    for i, call in enumerate(calls):
+        native, general = outcome(call, hosts.counting), outcome(call, General())
+        assert native == general, f"call {i}: {native} against {general}"
