@@ -308,18 +308,23 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
         for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
     T a[2][KS][MI], b[2][KS][NI];      // fragments of the k-tile at hand and of the next one
-    auto read = [&](int slot, int ks, int set) {
+    // read number r of a k-tile's fragments: k-step by k-step, A before W.  They stand among the first half of the MFMAs that they run
+    // under: in one burst behind the step's barrier both waves of a SIMD issued their reads with the matrix pipe idle.  us per
+    // k-tile with the burst and without (warm weights): 128 x 256 tiles 0.88 / 0.80 on all CUs and 0.62 / 0.57 on half of them,
+    // 128 x 128 0.48 / 0.455 and 0.42 / 0.36; 64 x 128 (0.29) and 64 x 64 (0.185) are bound by the feed alone.  Spread over 3/8 or
+    // all of the MFMAs: the same within the runs' spread.
+    constexpr int RT = KS * (MI + NI), MT = KS * MI * NI;      // reads and MFMAs of a k-tile
+    auto reads_by = [](int i) constexpr { const int n = ((i + 1) * RT * 2 + MT - 1) / MT; return n < RT ? n : RT; };      // ... that stand ahead of MFMA i + 1
+    auto read1 = [&](int slot, int r, int set) {
         const uint32_t s0 = slot * G::STAGE;
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi) a[set][ks][mi] = rd(fa[ks] + s0 + mi * 2048);
-#pragma unroll
-        for (int ni = 0; ni < NI; ++ni) b[set][ks][ni] = rd(fb[ks] + s0 + ni * 2048);
-        __builtin_amdgcn_sched_barrier(0);      // the reads go out ahead of the MFMAs they run under
+        const int ks = r / (MI + NI), f = r % (MI + NI);
+        if (f < MI) a[set][ks][f] = rd(fa[ks] + s0 + f * 2048);
+        else b[set][ks][f - MI] = rd(fb[ks] + s0 + (f - MI) * 2048);
     };
     // the MFMAs of k-step ks; LOADS: its share of the refill of slot `slot` with tile t, one load behind every few MFMAs (a wave
     // that issues its loads back to back sits in the vector-memory issue queue with the matrix pipe idle)
-    auto mma = [&](int set, auto ks_c, auto loads_c, int t, int slot) {
-        constexpr bool LOADS = decltype(loads_c)::value;
+    auto mma = [&](int set, auto ks_c, auto loads_c, auto reads_c, int t, int slot, int next) {
+        constexpr bool LOADS = decltype(loads_c)::value, READS = decltype(reads_c)::value;
         constexpr int ks = decltype(ks_c)::value, NM = MI * NI, GAP = KS * NM / L > 0 ? KS * NM / L : 1;
         int nl = ks * NM / GAP < L ? ks * NM / GAP : L;
 #pragma unroll
@@ -330,6 +335,11 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
                                                                                0 /*B: e4m3*/, 0, 0, 0, 0);
             else
                 acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[set][ks][ni], a[set][ks][mi], acc[mi][ni], 0, 0, 0);
+            if constexpr (READS) {
+#pragma unroll
+                for (int r = reads_by(ks * NM + i - 1); r < reads_by(ks * NM + i); ++r) read1(next, r, 1 - set);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             if (LOADS && (ks * NM + i) % GAP == GAP - 1 && nl < L) {
                 lds_dma16(base[nl] + t * 128, off[nl], l0 + slot * G::STAGE + nl * (NW * 1024));
                 ++nl;
@@ -358,7 +368,6 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
     using std::true_type;
     using C0 = std::integral_constant<int, 0>;
     using C1 = std::integral_constant<int, 1>;
-    constexpr bool BURST = KS * (MI + NI) <= 15;      // more reads than the counter of outstanding ones holds go out in two parts
     int slot = 0;
     // SET: fragment set of the tile at hand
     auto step = [&](auto behind_c, auto refill_c, auto set_c, int t) {
@@ -367,13 +376,8 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
         const int next = slot == S - 1 ? 0 : slot + 1;
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(BEHIND * L) : "memory");
         __builtin_amdgcn_sched_barrier(0);
-        read(next, 0, 1 - SET);
-        if constexpr (KS == 2 && BURST) read(next, 1, 1 - SET);
-        mma(SET, C0{}, refill_c, t + S, slot);
-        if constexpr (KS == 2) {
-            if constexpr (!BURST) read(next, 1, 1 - SET);
-            mma(SET, C1{}, refill_c, t + S, slot);
-        }
+        mma(SET, C0{}, refill_c, true_type{}, t + S, slot, next);
+        if constexpr (KS == 2) mma(SET, C1{}, refill_c, true_type{}, t + S, slot, next);
         slot = next;
     };
     using Deep = std::integral_constant<int, S - 2>;
@@ -381,7 +385,8 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
     if (KT >= S) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * L) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) read(0, ks, 0);
+    for (int r = 0; r < RT; ++r) read1(0, r, 0);
+    __builtin_amdgcn_sched_barrier(0);
     for (int t = 0; t + S < KT; t += 2) {
         step(Deep{}, true_type{}, C0{}, t);
         if (S % 2 == 0 || t + 1 + S < KT) step(Deep{}, true_type{}, C1{}, t + 1);      // KT is even
@@ -400,8 +405,8 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
     tail(std::integral_constant<int, 3>{});
     tail(std::integral_constant<int, 2>{});
     tail(std::integral_constant<int, 1>{});
-    mma(1, C0{}, false_type{}, 0, 0);      // the last tile: an odd index
-    if constexpr (KS == 2) mma(1, C1{}, false_type{}, 0, 0);
+    mma(1, C0{}, false_type{}, false_type{}, 0, 0, 0);      // the last tile: an odd index
+    if constexpr (KS == 2) mma(1, C1{}, false_type{}, false_type{}, 0, 0, 0);
 
     // ---- what the epilogue needs besides the sums is requested here and travels while they are spread, and both 64-key pieces of
     // a tile of keys go through one pass: a captured stack of one block, 1024 tokens x 1024 100.6 -> 99.3 us, an attention layer
