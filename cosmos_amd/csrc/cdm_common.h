@@ -79,6 +79,29 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// op(x, x of the lane 16 or 32 further: lane ^ 16, lane ^ 32), one instruction each instead of a round trip through the LDS unit:
+// with both operands x, v_permlane16_swap leaves the even rows of 16 lanes in one result and the odd ones in the other (32: halves)
+template <class Op>
+__device__ __forceinline__ float with_xor16(float x, Op op) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+template <class Op>
+__device__ __forceinline__ float with_xor32(float x, Op op) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// ... and of lane ^ 1, ^ 2 and ^ 8, and of lane ^ 4 where the four lanes of a quad hold the same (its instruction mirrors eight lanes)
+#define CDM_DPP(x, CTRL) __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true))
+template <class Op>
+__device__ __forceinline__ float with_xor1(float x, Op op) { return op(x, CDM_DPP(x, 0xb1)); }
+template <class Op>
+__device__ __forceinline__ float with_xor2(float x, Op op) { return op(x, CDM_DPP(x, 0x4e)); }
+template <class Op>
+__device__ __forceinline__ float with_xor4_of_quads(float x, Op op) { return op(x, CDM_DPP(x, 0x141)); }
+template <class Op>
+__device__ __forceinline__ float with_xor8(float x, Op op) { return op(x, CDM_DPP(x, 0x128)); }
+
 // One 16-byte-per-lane direct-to-LDS load, written as inline assembly so that the compiler's wait-count
 // insertion does not see an LDS write it would have to guard conservatively across a loop back-edge (it would
 // put s_waitcnt vmcnt(0) in front of fragment reads and drain a multi-stage pipeline).  Every wait on these

@@ -23,6 +23,9 @@ struct GemmSeg {
     const float* knw;                    // QKV_PACK only: the segment's K-norm weight row [head_dim] fp32, or null
 };
 
+// Tile images of a range of keys: [K / V heads][tiles] of each kind
+struct KeyImages { char* k; char* v; float* norm; int tiles; };
+
 struct GemmParams {
     int64_t lda, ldw;                    // operand strides in BYTES
     const float* sa;                     // fp8 only: per-row scale of A, indexed by the global row
@@ -33,8 +36,10 @@ struct GemmParams {
     int rope_cols, head_dim;
     // CDM_EPI_QKV_PACK: columns [0, d_q) are Q (written to C), [d_q, d_q + d_kv) K and the rest V; K and V leave as the
     // attention kernel's tile images (64 keys x 128 channels per K / V head), with the largest key norm of every tile
-    char* kp; char* vp; float* kmax;
-    int d_q, d_kv, n_key_tiles;
+    // (rows from key_cut on in `keys`, whose first key is row key_cut; those ahead of it in `first_keys`)
+    KeyImages keys, first_keys;
+    int key_cut;
+    int d_q, d_kv;
     float k_eps;                         // epsilon of the per-head RMSNorm of K (segments with a weight row)
     // CDM_EPI_SWIGLU, optional: [M, amax_ld] fp32, entry (row, c) = largest |output| of the row within output columns
     // 64 c .. 64 c + 63 (as stored): what a per-row quantiser of the output needs, without a pass of its own
@@ -108,6 +113,13 @@ __device__ __forceinline__ bool locate_tile(const GemmParams& p, Tile& t) {
     t.A = uniform_ptr(sg.A); t.W = uniform_ptr(sg.W); t.W2 = uniform_ptr(sg.W2);
     t.gate = uniform_ptr(sg.gate); t.sw = uniform_ptr(sg.sw); t.sw2 = uniform_ptr(sg.sw2); t.knw = uniform_ptr(sg.knw);
     return true;
+}
+
+// QKV_PACK: where the 64 keys from a (wave-uniform) row on go, `tile` of every head of `at`
+struct KeyPlace { KeyImages at; int tile; };
+__device__ __forceinline__ KeyPlace key_place(const GemmParams& p, int row) {
+    const bool rest = row >= p.key_cut;
+    return KeyPlace{rest ? p.keys : p.first_keys, (rest ? row - p.key_cut : row) >> 6};
 }
 
 // Chunk swizzle of a 128-byte tile row in LDS: 16-byte chunk c of row r lives at position c ^ swz16(r).  A fragment read

@@ -105,54 +105,68 @@ __device__ __forceinline__ void pack_keys(const GemmParams& p, const Tile& t, co
     static_assert(NT == 512, "a key per eight threads and piece");
     const int hd = p.head_dim, half = hd >> 1, head0 = (col0 - p.d_q) >> (hd == 128 ? 7 : 6);
     const int64_t tile_bytes = (int64_t)hd * 128;
+    const KeyPlace place = key_place(p, t.m0);
     const int j = tid & 7, hh = hd == 128 ? 0 : j >> 2, i0 = (hd == 128 ? j : (j & 3)) * 8, key = tid >> 3;
+    // The pieces go through every stage together, and sums over lanes by DPP: one piece behind the other, with nine exchanges through
+    // the LDS unit each, were a serial chain in the epilogue that a launch of one round ends with.  With V's reads no longer one branch each
+    // (pack_values), us: M = 1637, N = 3072, K = 2048 26.6 -> 26.0, M = 512, N = 12288, K = 4096 57.5 -> 56.0, M = 1024, N = 3072, K = 1024 11.3 -> 11.0.
+    const auto add = [](float x, float y) { return x + y; };
+    const auto max = [](float x, float y) { return fmaxf(x, y); };
+    float a[PC][8], b[PC][8];
 #pragma unroll
     for (int pc = 0; pc < PC; ++pc) {
-        const int row0 = t.m0 + pc * 64, row = row0 + key;      // first key of the image (a multiple of 64)
-        if (row0 >= t.m_end) break;
-        char* img = p.kp + ((int64_t)(head0 + hh) * p.n_key_tiles + (row0 >> 6)) * tile_bytes;
-        float a[8], b[8];
+        const char* src = rows + (pc * 64 + key) * PITCH + (c0 + hh * hd + i0) * 4;
+        load8(src, a[pc]);
+        load8(src + half * 4, b[pc]);
+    }
+    if constexpr (FP8) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) a[e] = b[e] = 0.0f;      // padding keys of a ragged last tile are zero in the images
-        if (row < t.m_end) {
-            const char* src = rows + (pc * 64 + key) * PITCH + (c0 + hh * hd + i0) * 4;
-            load8(src, a);
-            load8(src + half * 4, b);
-            if constexpr (FP8) {
-                const float sr = p.sa[row];
-                dequant8<true>(a, t.sw, col0 + hh * hd + i0, sr);
-                dequant8<true>(b, t.sw, col0 + hh * hd + i0 + half, sr);
-            }
-            if (t.knw != nullptr) {
-                float ss = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) ss += a[e] * a[e] + b[e] * b[e];
-                ss += __shfl_xor(ss, 1, 64);
-                ss += __shfl_xor(ss, 2, 64);
-                if (hd == 128) ss += __shfl_xor(ss, 4, 64);
-                const float rn = rsqrtf(ss * (hd == 128 ? 1.0f / 128.0f : 1.0f / 64.0f) + p.k_eps);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) { a[e] *= rn * k.w1[e]; b[e] *= rn * k.w2[e]; }
-            }
-            if (p.cos != nullptr)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) rotate_pair(a[e], b[e], k.c[pc][e], k.s[pc][e]);
+        for (int pc = 0; pc < PC; ++pc) {
+            const int row = t.m0 + pc * 64 + key;
+            const float sr = p.sa[row < t.m_end ? row : t.m_end - 1];
+            dequant8<true>(a[pc], t.sw, col0 + hh * hd + i0, sr);
+            dequant8<true>(b[pc], t.sw, col0 + hh * hd + i0 + half, sr);
         }
-        const uint4 ua = pack8(a), ub = pack8(b);
-        // K image, chunk-major [hd / 8 chunks][64 keys][16 bytes]
-        *reinterpret_cast<uint4*>(img + ((i0 >> 3) * 64 + key) * 16) = ua;
-        *reinterpret_cast<uint4*>(img + (((i0 + half) >> 3) * 64 + key) * 16) = ub;
+    }
+    if (t.knw != nullptr) {
+#pragma unroll
+        for (int pc = 0; pc < PC; ++pc) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += a[pc][e] * a[pc][e] + b[pc][e] * b[pc][e];
+            ss = with_xor2(with_xor1(ss, add), add);
+            if (hd == 128) ss = with_xor4_of_quads(ss, add);
+            const float rn = rsqrtf(ss * (hd == 128 ? 1.0f / 128.0f : 1.0f / 64.0f) + p.k_eps);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { a[pc][e] *= rn * k.w1[e]; b[pc][e] *= rn * k.w2[e]; }
+        }
+    }
+    if (p.cos != nullptr)
+#pragma unroll
+        for (int pc = 0; pc < PC; ++pc)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) rotate_pair(a[pc][e], b[pc][e], k.c[pc][e], k.s[pc][e]);
+#pragma unroll
+    for (int pc = 0; pc < PC; ++pc) {
+        const int row0 = t.m0 + pc * 64;      // first key of the image
+        if (row0 + key >= t.m_end)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) a[pc][e] = b[pc][e] = 0.0f;      // padding keys of a ragged last tile are zero in the images
+        const uint4 ua = pack8(a[pc]), ub = pack8(b[pc]);
+        if (row0 < t.m_end) {
+            char* img = place.at.k + ((int64_t)(head0 + hh) * place.at.tiles + place.tile + pc) * tile_bytes;
+            // K image, chunk-major [hd / 8 chunks][64 keys][16 bytes]
+            *reinterpret_cast<uint4*>(img + ((i0 >> 3) * 64 + key) * 16) = ua;
+            *reinterpret_cast<uint4*>(img + (((i0 + half) >> 3) * 64 + key) * 16) = ub;
+        }
         const uint32_t w[8] = {ua.x, ua.y, ua.z, ua.w, ub.x, ub.y, ub.z, ub.w};
         float sq = 0.0f;      // squared norm of the key as stored
 #pragma unroll
         for (int e = 0; e < 8; ++e) { const float lo = bf16lo(w[e]), hi = bf16hi(w[e]); sq += lo * lo + hi * hi; }
-        sq += __shfl_xor(sq, 1, 64);
-        sq += __shfl_xor(sq, 2, 64);
-        if (hd == 128) sq += __shfl_xor(sq, 4, 64);
+        sq = with_xor2(with_xor1(sq, add), add);
+        if (hd == 128) sq = with_xor4_of_quads(sq, add);
         // the largest among the eight keys of this wave instruction (hd 64: lanes 0-3 and 4-7 of every eight are two heads)
-        sq = fmaxf(sq, __shfl_xor(sq, 8, 64));
-        sq = fmaxf(sq, __shfl_xor(sq, 16, 64));
-        sq = fmaxf(sq, __shfl_xor(sq, 32, 64));
+        sq = with_xor32(with_xor16(with_xor8(sq, max), max), max);
         const int lane = tid & 63;
         if (lane == 0 || (lane == 4 && hd == 64)) ksq[pc * kKeyNorms + (key >> 3) * 2 + (lane >> 2)] = sq;
     }
@@ -162,7 +176,7 @@ __device__ __forceinline__ void pack_keys(const GemmParams& p, const Tile& t, co
         float m = 0.0f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) m = fmaxf(m, ksq[pc * kKeyNorms + 2 * i + (tid & 1)]);
-        p.kmax[(int64_t)(head0 + (tid & 1)) * p.n_key_tiles + ((t.m0 + pc * 64) >> 6)] = sqrtf(m);
+        place.at.norm[(int64_t)(head0 + (tid & 1)) * place.at.tiles + place.tile + pc] = sqrtf(m);
     }
     __syncthreads();
 }
@@ -174,22 +188,21 @@ __device__ __forceinline__ void pack_values(const GemmParams& p, const Tile& t, 
     const int hd = p.head_dim, head0 = (col0 - p.d_q - p.d_kv) >> (hd == 128 ? 7 : 6);
     const int h = tid & 127, hh = hd == 128 ? 0 : h >> 6;
     const float wsc = FP8 ? t.sw[col0 + h] : 1.0f;
+    const KeyPlace place = key_place(p, t.m0);
 #pragma unroll
     for (int pc = 0; pc < PC; ++pc) {
         const int row0 = t.m0 + pc * 64;
         if (row0 >= t.m_end) break;
-        char* img = p.vp + ((int64_t)(head0 + hh) * p.n_key_tiles + (row0 >> 6)) * ((int64_t)hd * 128);
+        char* img = place.at.v + ((int64_t)(head0 + hh) * place.at.tiles + place.tile + pc) * ((int64_t)hd * 128);
 #pragma unroll
         for (int c = tid >> 7; c < 8; c += NT / 128) {
             float v[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const int key = 32 * (c >> 2) + 4 * (c & 3) + 16 * (e >> 2) + (e & 3);
-                v[e] = 0.0f;
-                if (row0 + key < t.m_end) {
-                    v[e] = *reinterpret_cast<const float*>(rows + (pc * 64 + key) * PITCH + (c0 + h) * 4);
-                    if constexpr (FP8) v[e] *= p.sa[row0 + key] * wsc;
-                }
+                const int key = 32 * (c >> 2) + 4 * (c & 3) + 16 * (e >> 2) + (e & 3), row = row0 + key;
+                v[e] = *reinterpret_cast<const float*>(rows + (pc * 64 + key) * PITCH + (c0 + h) * 4);
+                if constexpr (FP8) v[e] *= p.sa[row < t.m_end ? row : t.m_end - 1] * wsc;
+                v[e] = row < t.m_end ? v[e] : 0.0f;      // (a branch per key would be eight waits in a row)
             }
             *reinterpret_cast<uint4*>(img + (c * hd + (h & (hd - 1))) * 16) = pack8(v);
         }
