@@ -27,11 +27,21 @@ __global__ __launch_bounds__(256) void timestep_sinusoid_kernel(const float* __r
 // One row through a linear layer in fp32, y = [silu](W x + b) with W [n_out, K]: the two halves of the timestep's MLP.  With
 // FREQ x is not read but built: the sinusoid of t, every workgroup for itself (K cosines and sines cost less than the
 // launch that would share them), and the activation follows.  A wave owns one output row, 16 bytes per lane four deep.
-// Bound by the weights' read (W2: 4 d^2 bytes, 67 MB at d = 4096) or, at small widths, by the launch alone.
+// Bound by the weights' read (W2: 4 d^2 bytes, 67 MB at d = 4096) or, at small widths, by the launch and one round trip to memory: the
+// row's first chunks and its bias are requested ahead of x (both launches, d = 1024 / 2048 / 4096: 5.4 / 6.4 / 16.4 -> 4.9 / 5.9 / 15.3 us).
 template <bool FREQ>
 __global__ __launch_bounds__(64 * kWaves) void linear_row_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                  const float* __restrict__ b, float* __restrict__ y, int K, int n_out) {
     extern __shared__ float s[];         // K values
+    const int lane = threadIdx.x & 63, row = blockIdx.x * kWaves + (threadIdx.x >> 6), at = row < n_out ? row : n_out - 1;
+    const float4* wr = reinterpret_cast<const float4*>(w + (int64_t)at * K);
+    constexpr int PRE = 4;               // chunks of the row (and its bias) that travel while x is built or read
+    float4 pre[PRE];
+    const int last = (K >> 2) - 1;
+#pragma unroll
+    for (int k = 0; k < PRE; ++k) pre[k] = wr[lane + 64 * k < last ? lane + 64 * k : last];
+    const float bias = b[at];
+    asm volatile("" ::: "memory");
     if (FREQ) {
         const float tv = x[0];
         const int half = K >> 1;
@@ -43,18 +53,20 @@ __global__ __launch_bounds__(64 * kWaves) void linear_row_kernel(const float* __
     } else {
         for (int i = threadIdx.x; i < K >> 2; i += 64 * kWaves) reinterpret_cast<float4*>(s)[i] = reinterpret_cast<const float4*>(x)[i];
     }
-    const int lane = threadIdx.x & 63, row = blockIdx.x * kWaves + (threadIdx.x >> 6);
-    const float4* wr = reinterpret_cast<const float4*>(w + (int64_t)(row < n_out ? row : n_out - 1) * K);
     float acc = 0.0f;
     __syncthreads();
-#pragma unroll 4
-    for (int i = lane; i < K >> 2; i += 64) {
-        const float4 v = wr[i], u = reinterpret_cast<const float4*>(s)[i];
+    auto add = [&](const float4& v, int i) {
+        const float4 u = reinterpret_cast<const float4*>(s)[i];
         acc += v.x * u.x + v.y * u.y + v.z * u.z + v.w * u.w;
-    }
+    };
+#pragma unroll
+    for (int k = 0; k < PRE; ++k)
+        if (lane + 64 * k <= last) add(pre[k], lane + 64 * k);
+#pragma unroll 4
+    for (int i = lane + 64 * PRE; i <= last; i += 64) add(wr[i], i);
     acc = wave_sum(acc);
     if (lane == 0 && row < n_out) {
-        const float v = acc + b[row];
+        const float v = acc + bias;
         y[row] = FREQ ? silu_exact(v) : v;
     }
 }
@@ -69,7 +81,8 @@ struct ModParams {
 
 // out[l] = W_l silu(c) + b_l for every block l.  The vector is rounded to bf16 ahead of the activation and behind it, and the
 // result to bf16, as the bf16 linear layer it stands for does; sums are fp32.
-// PRE: how many chunks of 64 x 16 bytes of its rows a wave requests ahead of the activation (d >= 512 PRE)
+// PRE: how many chunks of 64 x 16 bytes of its rows a wave requests ahead of the activation (d >= 512 PRE).  The biases are requested there
+// too, and one lane per row finishes it: one block of d = 1024 4.8 -> 4.0 us, of d = 2048 11.3 -> 10.5.
 template <int PRE>
 __global__ __launch_bounds__(64 * kWaves) void modulation_kernel(const ModParams p) {
     extern __shared__ float s[];         // silu(c), d values
@@ -85,6 +98,7 @@ __global__ __launch_bounds__(64 * kWaves) void modulation_kernel(const ModParams
     for (int k = 0; k < PRE; ++k)
 #pragma unroll
         for (int r = 0; r < kRows; ++r) pre[k][r] = wr[r][lane + 64 * k];
+    const float bias = lane < kRows ? bf16lo(p.b[blk][row0 + lane < p.n_out ? row0 + lane : p.n_out - 1]) : 0.0f;
     asm volatile("" ::: "memory");
     for (int i = threadIdx.x; i < p.d; i += 64 * kWaves) {
         const float c = bf16lo(pack_bf16x2(p.c[i], 0.0f));
@@ -110,11 +124,12 @@ __global__ __launch_bounds__(64 * kWaves) void modulation_kernel(const ModParams
         add(v, i);
     }
 #pragma unroll
-    for (int r = 0; r < kRows; ++r) {
-        acc[r] = wave_sum(acc[r]);
-        const int row = row0 + r;
-        if (lane == 0 && row < p.n_out)
-            p.out[(int64_t)blk * p.n_out + row] = bf16lo(pack_bf16x2(acc[r] + bf16lo(p.b[blk][row]), 0.0f));
+    for (int r = 0; r < kRows; ++r) acc[r] = wave_sum(acc[r]);
+    if (lane < kRows && row0 + lane < p.n_out) {      // lane r stores row r
+        float v = acc[0];
+#pragma unroll
+        for (int r = 1; r < kRows; ++r) v = lane == r ? acc[r] : v;
+        p.out[(int64_t)blk * p.n_out + row0 + lane] = bf16lo(pack_bf16x2(v + bias, 0.0f));
     }
 }
 
@@ -168,7 +183,8 @@ extern "C" int32_t cdm_adaln_modulation_bf16(const float* c, const void* const* 
         p.out = out + (int64_t)at * n_out;
         // from d = 4096 on (16 activations per thread) the first weights travel under the activation; at smaller widths the
         // registers that takes cost more waves than it hides.  Two / four / eight blocks, us without and with it: d = 4096 86.7 / 155 /
-        // 293 and 77.9 / 144 / 268 (6.0 TB/s), d = 2048 24.9 / 42.7 / 76.1 and 28.0 / 48.8 / 86.9
+        // 293 and 77.9 / 144 / 268 (6.0 TB/s), d = 2048 24.9 / 42.7 / 76.1 and 28.0 / 48.8 / 86.9; two chunks instead of four, one / two / four blocks:
+        // d = 2048 10.6 / 22.0 / 37.0 and 11.4 / 21.8 / 40.5, d = 1024 4.1 / 4.5 / 10.9 and 4.3 / 5.0 / 12.3
         if (d >= 4096) modulation_kernel<4><<<(unsigned)(nb * p.per_block), 64 * kWaves, (size_t)d * 4, (hipStream_t)stream>>>(p);
         else modulation_kernel<0><<<(unsigned)(nb * p.per_block), 64 * kWaves, (size_t)d * 4, (hipStream_t)stream>>>(p);
         if ((rc = cdm_check_launch("adaln_modulation"))) return rc;
