@@ -553,7 +553,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __shared__ __attribute__((aligned(1024))) char s_ring[5 * kGranule];
 
     Tile tile;
-    if (!locate_tile<BM, 4>(p, tile)) return;
+    if (!locate_tile<BM, 4, EPI == kPartial>(p, tile)) return;
     const int tn = tile.tn;
 
     const int lane = threadIdx.x & 63;
@@ -576,8 +576,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         bn = (n0 + bn) < p.N ? bn : p.N - 1 - n0;
         ob[j] = (uint32_t)(bn * (int)p.ldw + chunk * 16);
     }
-    const char* abase = reinterpret_cast<const char*>(tile.A) + (int64_t)m0 * p.lda;
-    const char* wbase = reinterpret_cast<const char*>(tile.W) + (int64_t)n0 * p.ldw;
+    int KT = p.K / (FP8 ? 128 : 64), kt0 = 0;   // k-tiles of 128 bytes (at least 2, host-checked)
+    if constexpr (EPI == kPartial) {      // this part's k-tiles: an even number, as a whole K's is
+        const int pairs = KT >> 1;
+        kt0 = (int)((int64_t)pairs * tile.part / p.k_split) * 2;
+        KT = (int)((int64_t)pairs * (tile.part + 1) / p.k_split) * 2 - kt0;
+    }
+    const char* abase = reinterpret_cast<const char*>(tile.A) + (int64_t)m0 * p.lda + (int64_t)kt0 * 128;
+    const char* wbase = reinterpret_cast<const char*>(tile.W) + (int64_t)n0 * p.ldw + (int64_t)kt0 * 128;
     const char* w2base = EPI == CDM_EPI_SWIGLU ? reinterpret_cast<const char*>(tile.W2) + (int64_t)n0 * p.ldw : wbase;
     const uint32_t l0 = lds_addr_of(s_ring) + wave * 1024;
 
@@ -587,7 +593,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int ni = 0; ni < 8; ++ni) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int KT = p.K / (FP8 ? 128 : 64);   // k-tiles of 128 bytes (at least 2, host-checked)
     auto gload = [&](int t, int op, int slot, int j) {
         const int ko = (t < KT ? t : KT - 1) * 128;
         if (op == 0) {
@@ -713,6 +718,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // surplus loads must not outlive the workgroup's LDS; after the barrier no wave reads the ring any more and
     // each wave owns an eighth of it as the staging area of its epilogue
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if constexpr (EPI == kPartial) {
+#pragma unroll
+        for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < 8; ++ni) store_partial(p, tile, m0 + (wm * 4 + mi) * 16, n0 + (wn * 8 + ni) * 16, lane, acc[mi][ni]);
+        return;
+    }
     epilogue<EPI, FP8>(p, tile, Acc16<4>{acc}, m0 + wm * 64, n0, wn, lane, s_ring + wave * (64 * kStagePitch));
 }
 
@@ -997,6 +1009,12 @@ int32_t qkv_pack(const char* who, const void* A, int64_t lda, const float* sa, c
 }
 
 }  // namespace
+
+namespace cdm_gemm {
+
+void launch_ring_partial(const GemmParams& p, int grid, hipStream_t st) { gemm_ring_kernel<kPartial, false><<<grid, 512, 0, st>>>(p); }
+
+}  // namespace cdm_gemm
 
 extern "C" int32_t cdm_grouped_gemm_qkv_pack_bf16(const void* A, int64_t lda, const void* const* W, int64_t ldw, void* Q,
                                                   int64_t ldq, const int64_t* seg_start, const int64_t* seg_len,

@@ -44,8 +44,8 @@ struct GemmParams {
     // CDM_EPI_SWIGLU, optional: [M, amax_ld] fp32, entry (row, c) = largest |output| of the row within output columns
     // 64 c .. 64 c + 63 (as stored): what a per-row quantiser of the output needs, without a pass of its own
     float* row_amax; int64_t amax_ld;
-    // Launches cut along K (gemm_tile.hip): part i of k_split leaves fp32 sums of its k-tiles, [k_split][part_rows][N], row 0 =
-    // token row part_row0
+    // Launches cut along K (gemm_tile.hip): part i of k_split leaves fp32 sums of its k-tiles (partial_at), [k_split][part_rows x N],
+    // from token row part_row0 on
     float* partial; int k_split, part_rows, part_row0;
     // CDM_EPI_GATE_RESIDUAL_F32, optional: rows c16_row0 .. + c16_rows - 1 of the result as bf16 too, from row 0 of C16 on
     bf16_t* C16; int64_t ldc16; int c16_row0, c16_rows;
@@ -115,6 +115,20 @@ __device__ __forceinline__ bool locate_tile(const GemmParams& p, Tile& t) {
     return true;
 }
 
+constexpr int kPartial = 100;      // "epilogue" of a launch cut along K: the fp32 sums of its k-tiles
+
+// ... of a 16 x 16 block, which its lanes hold as four columns of a row each.  A segment's rows lie 16 by 16 (the last ones fewer, R), inside
+// them [N / 4 column quads][R rows][4]: what a wave stores is one run of 1 KB, and a part takes exactly rows x N values.
+__device__ __forceinline__ int64_t partial_at(const GemmParams& p, int part, int row0, int m_end, int row, int col) {
+    const int R = m_end - row0 < 16 ? m_end - row0 : 16;
+    return ((int64_t)part * p.part_rows + (row0 - p.part_row0)) * p.N + ((int64_t)(col >> 2) * R + row) * 4;
+}
+__device__ __forceinline__ void store_partial(const GemmParams& p, const Tile& t, int row0, int col0, int lane, const f32x4& v) {
+    const int row = lane & 15, col = col0 + 4 * (lane >> 4);
+    if (row0 + row < t.m_end && col < p.N)      // N is a multiple of 8: four columns are in or out together
+        *reinterpret_cast<f32x4*>(p.partial + partial_at(p, t.part, row0, t.m_end, row, col)) = v;
+}
+
 // QKV_PACK: where the 64 keys from a (wave-uniform) row on go, `tile` of every head of `at`
 struct KeyPlace { KeyImages at; int tile; };
 __device__ __forceinline__ KeyPlace key_place(const GemmParams& p, int row) {
@@ -150,6 +164,7 @@ struct GemmPlan {
 };
 // scratch_bytes: what the caller brought for a launch cut along K (bf16 operands only)
 GemmPlan plan_gemm(const GemmParams& p, int epilogue, bool fp8, int64_t scratch_bytes);
+void launch_ring_partial(const GemmParams& p, int grid, hipStream_t st);      // 256 x 256 tiles of a launch cut along K (gemm.hip)
 int32_t launch_split_k(GemmParams& p, int epilogue, const GemmPlan& plan, void* scratch, hipStream_t st);
 int32_t launch_tile(GemmParams& p, int epilogue, bool fp8, TileShape shape, hipStream_t st);      // (with p.touch)
 

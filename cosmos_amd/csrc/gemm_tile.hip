@@ -209,8 +209,6 @@ __device__ __forceinline__ void pack_values(const GemmParams& p, const Tile& t, 
     }
 }
 
-constexpr int kPartial = 100;      // "epilogue" of a launch cut along K: the fp32 sums of its k-tiles
-
 // eight columns of the residual, and of its gate (1 without one)
 template <int EPI>
 __device__ __forceinline__ void load_residual(const GemmParams& p, int row, int col, float (&r)[8]) {
@@ -475,6 +473,14 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
     KeyTables<TM / 64 ? TM / 64 : 1> tables;
     if (EPI == CDM_EPI_QKV_PACK && n0 + TN > p.d_q && n0 < p.d_q + p.d_kv) request_tables(p, tile, tid, tables);
 
+    if constexpr (EPI == kPartial) {
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni) store_partial(p, tile, m0 + (wm * MI + mi) * 16, n0 + (wn * NI + ni) * 16, lane, acc[mi][ni]);
+        return;
+    }
+
     // ---- accumulators -> fp32 rows in LDS (every wave is done with the ring)
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
@@ -538,12 +544,6 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
         }
         float v[8];
         load8(smem + rl * G::PITCH + cl * 4, v);
-        if constexpr (EPI == kPartial) {
-            float* P = p.partial + ((int64_t)tile.part * p.part_rows + (row - p.part_row0)) * p.N + col;
-            *reinterpret_cast<float4*>(P) = make_float4(v[0], v[1], v[2], v[3]);
-            *reinterpret_cast<float4*>(P + 4) = make_float4(v[4], v[5], v[6], v[7]);
-            continue;
-        }
         if constexpr (EPI != CDM_EPI_GATE_RESIDUAL_F32) dequant8<FP8>(v, tile.sw, col, sr);
         if constexpr (EPI == CDM_EPI_ROPE_QK) {
             if (col < p.rope_cols) {      // whole heads: tile columns start on head boundaries
@@ -567,27 +567,33 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
 }
 
 // The sums of a launch cut along K, added part by part, through the epilogue.  Bound by reading them (k_split * 4 bytes per
-// value, most of it from the memory-side cache): one eight-column chunk per thread.
+// value, most of it from the memory-side cache): eight columns of a row per thread.  The sums come from the accumulators as they lie, in
+// runs of 1 KB; through the LDS to whole rows first M = 512, N = 2048, K = 8192 takes 32.5 us instead of 30.7, M = 333, N = 4096, K = 16384 with warm weights 57.6
+// instead of 53.8, and as rows straight from the registers (64 bytes a row) 256 x 256 tiles lose 3 - 5 us.
 template <int EPI>
 __global__ __launch_bounds__(256) void finish_split_kernel(const GemmParams p) {
-    const int cpr = p.N >> 3;
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int r = (int)(idx / cpr), col = (int)(idx % cpr) * 8;
-    if (r >= p.part_rows) return;
-    const int row = p.part_row0 + r;
+    const int64_t cpr = p.N >> 3, idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int near = (int)(idx / cpr);      // a row of this thread's segment: its rows' sums lie together
+    if (near >= p.part_rows) return;
+    int m_start = 0, m_end = 0;
     const float* gate = nullptr;
-    bool in = false;
     for (int i = 0; i < p.n_seg; ++i)
-        if (row >= p.seg[i].m_start && row < p.seg[i].m_end) { in = true; gate = p.seg[i].gate; }
-    if (!in) return;
+        if (p.part_row0 + near >= p.seg[i].m_start && p.part_row0 + near < p.seg[i].m_end) { m_start = p.seg[i].m_start; m_end = p.seg[i].m_end; gate = p.seg[i].gate; }
+    const int64_t in_seg = idx - (int64_t)(m_start - p.part_row0) * cpr;
+    const int block = (int)(in_seg / (16 * cpr)), row0 = m_start + 16 * block, in_block = (int)(in_seg - block * 16 * cpr);
+    const int R = m_end - row0 < 16 ? m_end - row0 : 16, pair = in_block / R, row = row0 + (in_block - pair * R), col = pair * 8;
     float v[8];
     float g[8], r0[8];
     load_gate(gate, col, g);
     load_residual<EPI>(p, row, col, r0);
-    load8(p.partial + (int64_t)r * p.N + col, v);
+    const float* src = p.partial + partial_at(p, 0, row0, m_end, row - row0, col);
+    const int64_t part = (int64_t)p.part_rows * p.N;
+    unpack4(*reinterpret_cast<const float4*>(src), v);
+    unpack4(*reinterpret_cast<const float4*>(src + R * 4), v + 4);
     for (int i = 1; i < p.k_split; ++i) {
         float w[8];
-        load8(p.partial + ((int64_t)i * p.part_rows + r) * p.N + col, w);
+        unpack4(*reinterpret_cast<const float4*>(src + i * part), w);
+        unpack4(*reinterpret_cast<const float4*>(src + i * part + R * 4), w + 4);
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] += w[e];
     }
@@ -701,8 +707,11 @@ Best best_touched(const int64_t* rows, int n_seg, int64_t N, double kt, double w
 // Launches with few tiles and a long K: every tile once per range of K, fp32 sums in scratch memory and a pass over them
 // (finish_split_kernel: its launch, and the sums written and read at about 8 TB/s).  Whole launch against the cut one, us, fp32
 // residual, weights that no cache holds:
-//     N = 4096, K = 16384:  M = 128  71.2 / 49.8   256  73.2 / 56.5   512  111 / 79.1   768  140 / 122   1024  146 / 133
-//     N = 2048, K = 8192:   M = 64   20.2 / 16.3   256  33.3 / 23.8   512  35.5 / 31.8
+//     N = 4096, K = 16384:  M = 128  71.2 / 49.8   256  73.2 / 56.5   512  111 / 79.1
+// In 256 x 256 tiles, whose k-tiles cost a fifth less per product, against the best cut in smaller ones (the same layer): M = 700 96 / 113, 768 96 / 118,
+// 1024 119 / 130, 1152 140 / 180 (uncut), 1280 142 / 174; prompts through 8 layers of 4096: 720 rows 3.55 -> 3.34 ms, 768 3.62 -> 3.38, 1024 4.07 -> 3.85 (half of that on the slowest boxes).
+// At 512 they are even in a loop of this layer and behind in a prompt (8.29 / 8.39 ms): the estimate keeps to the smaller ones.
+//     N = 2048, K = 8192:   M = 64   20.2 / 16.3   256  33.3 / 23.8   512  35.5 / 30.7
 //     N = 4096, K = 4096:   M = 128  19.5 / 18.3;  N = 1024, K = 4096: M = 512 16.8 / 18.0
 // (with weights that a cache holds the cuts of shorter sums lose: N = 1024, K = 4096, M = 512 14.8 / 17.6; N = 2048, K = 4096, M = 256 14.5 / 17.7).
 // Cut launches stream the weights at 2.4 - 3 TB/s at most (M = 96 at K = 16384: 45 us), so such a rate bounds the estimate.  Against 64 bits the sums are closer than uncut ones (K = 16384: 2.8e-7 in four ranges, 5.8e-7).
@@ -719,12 +728,13 @@ SplitK best_split(const GemmParams& p, const int64_t* rows, double kt, int epilo
     }
     if (filled != hi - lo) return best;                                     // gaps between the segments
     for (const ShapeCost& c : kShapes) {
-        if (c.s.tm == 256 || c.s.tm == 32) continue;
+        if (c.s.tm == 32) continue;
         int64_t n = 0;
         for (int i = 0; i < p.n_seg; ++i) n += (rows[i] + c.s.tm - 1) / c.s.tm;
+        if (c.s.tm == 256 && 10 * (hi - lo) < 9 * 256 * n) continue;      // too many rows that do not exist: M = 420 72.9 us against 70.2, 640 96 / 93, 900 119.5 / 118.8
         n *= (p.N + c.s.tn - 1) / c.s.tn;
         for (int s = 2; s <= kMaxSplitK; ++s) {
-            if (kt < 12.0 * s || n * s > 512) break;
+            if (kt < 12.0 * s || n * s > (c.s.tm == 256 ? 256 : 512)) break;      // (two rounds of 256 x 256: M = 1536, N = 4096, K = 16384 204 us, uncut 185)
             const int64_t bytes = (hi - lo) * p.N * 4 * s;
             const double weights = (double)p.N * kt * 128.0 * p.n_seg / 2.9e6, run = estimate(c, n * s, kt / s);
             const double us = (run > weights ? run : weights) + 5.5 + 2.0 * (double)bytes / 8e6;
@@ -751,8 +761,9 @@ int32_t launch_split_k(GemmParams& p, int epilogue, const GemmPlan& plan, void* 
         hi = p.seg[i].m_end > hi ? p.seg[i].m_end : hi;
     }
     p.total_tiles = total; p.part_row0 = lo; p.part_rows = hi - lo;
-    int32_t rc = launch_epi<kPartial, false>(p, s, (total * p.k_split + 7) / 8 * 8, st);
-    if (rc) return rc;
+    const int parts = (total * p.k_split + 7) / 8 * 8;
+    if (s.tm == 256) launch_ring_partial(p, parts, st);
+    else if (int32_t rc = launch_epi<kPartial, false>(p, s, parts, st)) return rc;
     const unsigned grid = (unsigned)(((int64_t)p.part_rows * (p.N / 8) + 255) / 256);
     if (epilogue == CDM_EPI_NONE) finish_split_kernel<CDM_EPI_NONE><<<grid, 256, 0, st>>>(p);
     else if (epilogue == CDM_EPI_GATE_RESIDUAL) finish_split_kernel<CDM_EPI_GATE_RESIDUAL><<<grid, 256, 0, st>>>(p);

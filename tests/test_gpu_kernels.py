@@ -204,6 +204,34 @@ def test_gemm_in_an_odd_number_of_ranges(M, parts):
     assert not torch.equal(cut, whole) and err(cut) <= 1.01 * err(whole), (err(cut), err(whole))
 
 
+@pytest.mark.parametrize("lens,N,parts", [((700,), 4096, 5), ((250, 509), 4104, 5), ((510, 246), 4096, 5), ((1011,), 4096, 4), ((1152,), 4096, 3)])
+def test_gemm_cut_along_k_in_large_tiles(lens, N, parts):
+    """Ranges of K in 256 x 256 tiles: ragged rows (16-row blocks of 12, 10, 13, 14, 6 and 3 rows) and columns, segments, rows that leave as bf16
+    too.  Bounds as in test_gemm_cut_along_k, the error as in test_gemm_in_an_odd_number_of_ranges."""
+    g, M, K = gen(sum(lens) + N), sum(lens), 16384
+    a = torch.randn((M, K), generator=g).to(dev(), torch.bfloat16)
+    ws = [(torch.randn((N, K), generator=g) * K ** -0.5).to(dev(), torch.bfloat16) for _ in lens]
+    segs = [(sum(lens[:i]), n) for i, n in enumerate(lens)]
+    r, gates = torch.randn((M, N), generator=g).to(dev()), [None if i == 1 else torch.randn(N, generator=g).to(dev()) for i in range(len(lens))]
+    assert ops.gemm_scratch_bytes(tuple(lens), N, K, ops.EPI_GATE_RESIDUAL_F32) == parts * M * N * 4
+    want = torch.cat([r[s:s + n].double() + (1.0 if gt is None else gt.double()) * (a[s:s + n].double() @ w.double().t())
+                      for (s, n), w, gt in zip(segs, ws, gates)])
+    got, rows16 = r.clone(), torch.empty((M - 3, N), dtype=torch.bfloat16, device=dev())
+    ops.residual_gemm_(got, a, ws, segs, gates, rows16, 3)
+    err = lambda o: (o.double() - want).norm().item()
+    assert bool(((got.double() - want).abs() <= 1e-5).all()) and torch.equal(rows16, got[3:].to(torch.bfloat16))
+    run = lambda res, **kw: ops.grouped_gemm(a, ws, segs, epilogue="gate_residual", residual=res, gates=gates, out=torch.empty_like(res))
+    assert torch.equal(run(r), got)
+    r16 = r.to(torch.bfloat16)
+    assert bool(((run(r16).double() - (want - r.double() + r16.double())).abs() <= 1e-5 + want.abs() * 2.0 ** -8 + 2.0 ** -9).all())
+    prev = ops.set_variant("gemm", 2)                       # the same tiles, uncut
+    try:
+        whole = run(r)
+    finally:
+        ops.set_variant("gemm", prev)
+    assert err(got) <= 1.01 * err(whole)
+
+
 @pytest.mark.parametrize("K", [512, 8192])
 def test_grouped_gemm_of_wider_weights(K):
     """Weights with more columns than the rows have: their first K columns, cut along K or not."""
