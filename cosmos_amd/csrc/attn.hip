@@ -1123,7 +1123,7 @@ __global__ __launch_bounds__(256) void pack_kv_kernel(const bf16_t* __restrict__
                                                       const bf16_t* __restrict__ v, int64_t ldv,
                                                       const float* __restrict__ cos, const float* __restrict__ sin,
                                                       const QkNormDev kn, char* __restrict__ kp, char* __restrict__ vp,
-                                                      float* __restrict__ kmax, int n_tokens, int n_tiles) {
+                                                      float* __restrict__ kmax, int n_tokens, int n_tiles, bool by_xcd) {
     __shared__ bf16_t tile[64][HD + 2];
     __shared__ float wave_kmax[4];
     float ksq_max = 0.0f;      // largest squared norm among the keys this thread has helped with
@@ -1131,8 +1131,10 @@ __global__ __launch_bounds__(256) void pack_kv_kernel(const bf16_t* __restrict__
     constexpr int HALF = HD / 2;
     constexpr int TILE_BYTES = BN * HD * 2;
     // heads vary fastest over the grid: the K / V rows of neighbouring heads are adjacent in memory, so the
-    // workgroups that run together share DRAM pages and cache lines
-    const int tile_idx = blockIdx.y, head = blockIdx.x;
+    // workgroups that run together share DRAM pages and cache lines.  by_xcd: a head's images are written by the XCD whose workgroups
+    // attend with it (ids are dealt round-robin, an XCD owns neighbouring heads) and stay in its L2.
+    const int n_kv = gridDim.x, x = blockIdx.x, head = by_xcd ? (x & 7) * (n_kv >> 3) + (x >> 3) : x;
+    const int tile_idx = blockIdx.y;
     const int t0 = tile_idx * 64;
     char* kt = kp + ((int64_t)head * n_tiles + tile_idx) * TILE_BYTES;
     char* vt = vp + ((int64_t)head * n_tiles + tile_idx) * TILE_BYTES;
@@ -1357,13 +1359,17 @@ extern "C" int32_t cdm_attn_pack_kv_bf16(const void* k, int64_t ldk, const void*
     const int64_t img = image_bytes(n_tokens, n_heads, head_dim);
     char* ws = (char*)workspace;
     dim3 grid(n_heads, n_tiles);
+    // as long as an XCD's images fit its 4 MB of L2.  Re-tiling and attention, us, without and with it: 16 heads x 128, 640 / 1024 / 1637 tokens 17.7 / 23.8 /
+    // 40.4 and 15.8 / 20.4 / 36.9, 32 x 128 27.6 / 34.1 / 63.8 and 24.5 / 31.7 / 61.7, 16 x 64 13.1 / 16.2 / 26.8 and 12.4 / 14.6 / 24.5; nothing at
+    // 8 heads, which lie so anyway; beyond the L2 (32 x 128, 7040 tokens) 660 and 670
+    const bool by_xcd = n_heads % 8 == 0 && 2 * img / 8 <= 4 << 20;
     hipStream_t st = (hipStream_t)stream;
     if (head_dim == 128)
         pack_kv_kernel<128><<<grid, 256, 0, st>>>((const bf16_t*)k, ldk, (const bf16_t*)v, ldv, cos, sin, kn, ws, ws + img,
-                                                  (float*)(ws + 2 * img), (int)n_tokens, n_tiles);
+                                                  (float*)(ws + 2 * img), (int)n_tokens, n_tiles, by_xcd);
     else
         pack_kv_kernel<64><<<grid, 256, 0, st>>>((const bf16_t*)k, ldk, (const bf16_t*)v, ldv, cos, sin, kn, ws, ws + img,
-                                                 (float*)(ws + 2 * img), (int)n_tokens, n_tiles);
+                                                 (float*)(ws + 2 * img), (int)n_tokens, n_tiles, by_xcd);
     return cdm_check_launch("attn_pack_kv");
 }
 

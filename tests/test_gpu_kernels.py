@@ -1014,6 +1014,23 @@ def test_qkv_pack_with_a_cut(lens, cut, H, Hkv, K, qkn, hd, apart):
         ops.attention_packed(q_out, img, H, hd, None, cos, sin, norm, n_kv_heads=Hkv, cut=n)
 
 
+@pytest.mark.parametrize("H,hd,n", [(8, 64, 1), (16, 64, 70), (24, 128, 130), (12, 128, 130), (16, 128, 4096), (16, 128, 4097)])
+def test_images_lie_by_head_whoever_writes_them(H, hd, n):
+    """Re-tiling of K and V: workgroups are dealt out by XCD or not (whole eighths of the heads, up to 4 MB of images an eighth: 4096
+    tokens of 2 x 128 are the last), the images of a head are those of a call for this head alone."""
+    g = gen(H + n)
+    k, v = rand_bf16((n, H * hd), g)[0], rand_bf16((n, H * hd), g)[0]
+    img = ops.attention_pack_kv(k, v, H, hd, torch.zeros(ops.attn_workspace_bytes(n, H, hd), dtype=torch.uint8, device=dev()))
+    tiles = (n + 63) // 64
+    one, all_heads = tiles * 64 * hd * 2, tiles * 64 * hd * 2 * H
+    for h in (0, 1, H // 2, H - 1):
+        cols = slice(h * hd, (h + 1) * hd)
+        ref = ops.attention_pack_kv(k[:, cols], v[:, cols], 1, hd, torch.zeros(ops.attn_workspace_bytes(n, 1, hd), dtype=torch.uint8, device=dev()))
+        assert torch.equal(img[h * one:(h + 1) * one], ref[:one]) and torch.equal(img[all_heads + h * one:all_heads + (h + 1) * one], ref[one:2 * one])
+        norms = lambda t, at: t[at:at + 4 * tiles]
+        assert torch.equal(norms(img, 2 * all_heads + 4 * h * tiles), norms(ref, 2 * one))
+
+
 # ------------------------------------------------------------------ attention
 @pytest.mark.parametrize("variant", [0, 1])
 @pytest.mark.parametrize("n,H,hd", [(64, 2, 64), (256, 1, 128), (1000, 3, 128), (321, 2, 64), (1, 1, 128), (130, 2, 128), (65, 1, 64),
