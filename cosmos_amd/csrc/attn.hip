@@ -309,7 +309,6 @@ struct PackedParams {
     const float* cos; const float* sin;   // optional rotary tables [n_tokens, HD/2] applied to Q at load
     QkNormDev qn;                          // optional per-head RMSNorm of Q, applied before the rotation
     int n_tokens, n_heads, n_qblocks;
-    int n_keys;                  // keys of kp / vp: all tokens, or those behind the prefix where that holds the others
     uint64_t kv_magic;           // ceil(2^32 / query heads per K / V head): head * kv_magic >> 32 is the K / V head (heads < 2^16)
     int always_max;              // cross-check: take the row maxima of every tile whatever the norm bound says
     float scale_log2e;           // factor on Q ahead of its rounding to bf16: log2(e)/sqrt(HD), or only its power of two
@@ -322,6 +321,7 @@ struct PackedParams {
     void* part_o;                // [8 * split_tail * split][256][HD], fp32 where part_f32, bf16 otherwise
     int part_f32;
     float* part_lse;             // [8 * split_tail * split][256]   log2 of the unit's sum of exponentials, reference added
+    int n_keys;                  // keys of kp / vp: all tokens, or those behind the prefix where that holds the others
 };
 
 // QS = query sub-tiles (of 32 rows = two 16-row blocks) per wave: QS = 1 -> 8 waves, two per SIMD, 256 registers each;
@@ -494,6 +494,7 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
     // the in-phase waves needs: the out-of-phase waves read the first fragments of V(j) BEFORE barrier j, so V(j)
     // has to be complete at barrier j - 1
     constexpr int RING = 3, RING_V = 4;
+    if constexpr (HD == 64) asm volatile(".rept 11\n\ts_nop 0\n\t.endr");      // (the place of the loop, see there)
     __shared__ __attribute__((aligned(1024))) char sk[RING * TILE_BYTES];
     __shared__ __attribute__((aligned(1024))) char sv[RING_V * TILE_BYTES];
     __shared__ float s_km[kMaxKm];       // largest key norm of every tile of this K / V head, prefix tiles first (set-up only)
@@ -727,6 +728,11 @@ __global__ __launch_bounds__(512 / QS) __attribute__((amdgpu_waves_per_eu(2 / QS
         ks_cur = ks_next;                                                                                       \
         ks_next = ks_next == 2 ? 0 : ks_next + 1;                                                               \
     }
+    // Where the loop's 6 KB begin counts for half a percent (a mix of 4- and 8-byte instructions against the fetch of 32 bytes): 8 bytes behind such a
+    // boundary head_dim 128 takes 36.71 ms at 56,320 tokens x 32 heads, elsewhere 36.78 - 36.95.  The compiler's 36 bytes between here and
+    // the loop are part of the sum.  At head_dim 64 a statement here changes the loop itself, so the kernel's first instructions shift it to 4 bytes
+    // behind a boundary of 64 (14,080 x 16, another box: 721 - 724 us there, 728 at 24 bytes).
+    if constexpr (HD == 128) asm volatile(".p2align 8\n\t.rept 9\n\ts_nop 0\n\t.endr");
     for (int j = 0; j < NTW; ++j) {
         CDM_ATTN_STEP(s_a, s_b)
         if (++j >= NTW) break;
