@@ -271,6 +271,12 @@ __device__ __forceinline__ void epilogue(const GemmParams& p, const Tile& t, ACC
                 acc.set(rs, cs, 3, acc.get(rs, cs, 3) * (sr * w4.w));
             }
         }
+        if (EPI == CDM_EPI_QKV_PACK && !FP8 && region == 1 && p.key_cut > 0) {      // see key_cut
+#pragma unroll
+            for (int cs = 0; cs < CS; ++cs)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc.set(rs, cs, e, (float)(__bf16)acc.get(rs, cs, e));
+        }
         if (EPI == CDM_EPI_QKV_PACK && region == 1 && t.knw != nullptr) {
             // per-head RMSNorm of K on the fp32 accumulators, ahead of the rotation: the wave's 128 columns are one head,
             // a key's channels are spread over the four quarter-waves (lanes r, r + 16, r + 32, r + 48 share the row)

@@ -37,6 +37,8 @@ struct GemmParams {
     // CDM_EPI_QKV_PACK: columns [0, d_q) are Q (written to C), [d_q, d_q + d_kv) K and the rest V; K and V leave as the
     // attention kernel's tile images (64 keys x 128 channels per K / V head), with the largest key norm of every tile
     // (rows from key_cut on in `keys`, whose first key is row key_cut; those ahead of it in `first_keys`)
+    // With a cut, K is rounded to bf16 ahead of its norm and rotation, as in the rows that the re-tiling kernel reads: such layers
+    // took that kernel's way before, and without the rounding their outputs differ from it by 5e-3 - 6e-3 where attention averages many keys.
     KeyImages keys, first_keys;
     int key_cut;
     int d_q, d_kv;

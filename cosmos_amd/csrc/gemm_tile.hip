@@ -128,6 +128,12 @@ __device__ __forceinline__ void pack_keys(const GemmParams& p, const Tile& t, co
             dequant8<true>(b[pc], t.sw, col0 + hh * hd + i0 + half, sr);
         }
     }
+    if (!FP8 && p.key_cut > 0) {
+#pragma unroll
+        for (int pc = 0; pc < PC; ++pc)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { a[pc][e] = (float)(__bf16)a[pc][e]; b[pc][e] = (float)(__bf16)b[pc][e]; }      // see key_cut
+    }
     if (t.knw != nullptr) {
 #pragma unroll
         for (int pc = 0; pc < PC; ++pc) {
