@@ -715,7 +715,7 @@ Best best_touched(const int64_t* rows, int n_seg, int64_t N, double kt, double w
 // residual, weights that no cache holds:
 //     N = 4096, K = 16384:  M = 128  71.2 / 49.8   256  73.2 / 56.5   512  111 / 79.1
 // In 256 x 256 tiles, whose k-tiles cost a fifth less per product, against the best cut in smaller ones (the same layer): M = 700 96 / 113, 768 96 / 118,
-// 1024 119 / 130, 1152 140 / 180 (uncut), 1280 142 / 174; prompts through 8 layers of 4096: 720 rows 3.55 -> 3.34 ms, 768 3.62 -> 3.38, 1024 4.07 -> 3.85 (half of that on the slowest boxes).
+// 1024 119 / 130, 1152 140 / 180 (uncut), 1280 142 / 174; prompts through 8 layers of 4096: 720 rows 3.55 -> 3.34 ms, 768 3.62 -> 3.38, 1024 4.07 -> 3.85 (half of that on the slowest cards).
 // At 512 they are even in a loop of this layer and behind in a prompt (8.29 / 8.39 ms): the estimate keeps to the smaller ones.
 //     N = 2048, K = 8192:   M = 64   20.2 / 16.3   256  33.3 / 23.8   512  35.5 / 30.7
 //     N = 4096, K = 4096:   M = 128  19.5 / 18.3;  N = 1024, K = 4096: M = 512 16.8 / 18.0
